@@ -1,0 +1,579 @@
+// cgpersist.hpp -- the CG iteration of one system as a persistent kernel: the
+// Krylov vectors stay in registers and LDS between the iterations, and the
+// workgroups exchange nothing but dot-product partials and one vector.
+//
+// What bounds the kernel-per-phase iteration (cgkernels.hpp) is, on systems that
+// fill the chip, bytes: of the 168 bytes per row of an FP64 iteration 96 are
+// vector reads and writes that only exist because each phase is a launch of its
+// own; on small systems it is the chain of dependent loads and the reduction
+// that every launch repeats (4-6 us per kernel).  One kernel for many iterations
+// needs neither.  The 256 CUs hold 128 MB of registers and 40 MB of LDS, so the
+// vectors of a system of up to 2^21 rows fit on the chip:
+//
+//  * a workgroup of 1024 threads per CU takes four tiles of 256 threads, the
+//    tiles (rows, order, partial sums) of cgkernels.hpp; a thread keeps r and q of
+//    its RPT rows in registers, p and d in LDS, g in either;
+//  * the matrix rows stay in registers where they fit (RES of the RPT rows: all
+//    of them up to 2 FP64 or 4 FP32 rows per thread); the others are read every
+//    iteration (72 bytes per FP64 row, 48 FP32);
+//  * a column of the tile's own rows (83 % of them in a Z-order tile of 256 rows,
+//    92 % of 2048) is read from LDS.  For the others, each tile publishes r of its
+//    rows that have such a column (the pattern is symmetric, so they are the ones
+//    others read) after the update and p after the direction, and the reader
+//    evaluates p' = r + beta p, the expression of the row's owner, so p' itself is
+//    needed by nobody before the next reduction: two grid exchanges per iteration.
+//
+// Grid reduction without atomics or fences: a workgroup publishes its partial
+// sums as 64-bit words, half payload and half sequence number, and the readers
+// poll the words themselves.  So the value and its arrival are one word, nothing
+// has to be reset, and every workgroup adds the same numbers in the order of
+// sum_slots (see GridSum): the bits are those of the kernel-per-phase form.
+// Measured with 1024-thread workgroups, a 128-byte line per slot: 1.4 us for 64
+// workgroups, 2.3 for 256 (3.1 with the slots 16 bytes apart: writers of one line
+// wait for each other); with an agent-scope fence in every wave the same exchange
+// took 31-86 us for 256 (each fence is an L2 write-back or invalidate).  The
+// published vectors therefore go through agent-scope relaxed stores and loads,
+// which pass the per-XCD L2s.  Either the words carry the iteration's tag too
+// (TAGGED: small systems, where the 1.2 us of waiting for the stores counts), or a
+// wave waits for its stores to complete (vmcnt) before the workgroup's barrier,
+// behind which its partial sum is published.
+//
+// The launch is cooperative, so its workgroups are resident together.  Every
+// wait is bounded by a clock: a workgroup that waits longer than kSyncSeconds
+// sets stop = kStopSync and ends, and so do the others.
+//
+// Measured per iteration (pressure equation on jittered cubes, kernel-by-kernel
+// form -> this one): FP64 32^3 10.9 -> 6.8 us, 64^3 21.6 -> 10.2, 96^3 39.6 ->
+// 19.8, 128^3 65.9 -> 42.8; FP32 32^3 10.9 -> 6.2, 64^3 16.4 -> 8.5, 96^3 27.3 ->
+// 13.4, 128^3 42.5 -> 26.3.  At 128^3 FP64 27 of the 43 us are the matrix stream
+// (5.6 TB/s), 11 the two exchanges with their waits for the slowest workgroup.
+#pragma once
+
+#include "cgkernels.hpp"
+
+namespace fvhip {
+namespace {
+
+constexpr int kPersistThreads = 1024;  // four tiles of kCgBlock threads
+constexpr int kPersistSub = kPersistThreads / kCgBlock;
+constexpr int kPersistGroups = kCgMaxTiles / kPersistSub;  // workgroups at most
+constexpr int kSlotWords = 16;  // up to two doubles as half-payload words; a 128-byte line per slot
+constexpr int kSlotBuffer = (kPersistGroups + 8) * kSlotWords;  // workgroups and groups of them
+constexpr int kStopSync = 4;           // CgState::stop after a timed-out wait
+constexpr unsigned long long kSyncSeconds = 20;
+constexpr unsigned long long kClockHz = 100000000ull;  // wall_clock64: 100 MHz
+
+// Arguments by value: the kernel reads them from scalar registers instead of
+// chasing the launch description and the system description in memory.
+template <typename S>
+struct CgPersist {
+    int32_t N, tiles, rowsPerTile;
+    int32_t iters;        // iterations this launch may run
+    uint32_t tag0;        // sequence number of its first exchange
+    const int32_t* sellCol;  // slices of one width W: entry k of row i at
+    const S* sval;           // (i / 64) * 64 W + 64 k + i % 64
+    const S* g;
+    S *d, *r, *p, *p2;
+    unsigned long long* rtag;  // published r with its iteration's tag (TAGGED)
+    CgState* st;
+    unsigned long long* slots;  // 2 * kSlotBuffer
+};
+
+template <typename T>
+__device__ __forceinline__ void put_shared(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T get_shared(const T* p) {
+    return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Keeps x in its register as it is: without this the compiler turns the 32-bit
+// offsets, which do not change between iterations, into 64-bit addresses held
+// across the loop (two registers each, and the rows no longer fit).
+__device__ __forceinline__ void opaque(uint32_t& x) { asm volatile("" : "+v"(x)); }
+
+// A value that is the same in every lane, in scalar registers.
+__device__ __forceinline__ double uniform(double x) {
+    const long long b = __double_as_longlong(x);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)b);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The byte at base + off, a 32-bit offset: one scalar base and one vector
+// register per address.
+template <typename T>
+__device__ __forceinline__ T* at_byte(T* base, uint32_t off) {
+    return reinterpret_cast<T*>(reinterpret_cast<char*>(base) + off);
+}
+template <typename T>
+__device__ __forceinline__ const T* at_byte(const T* base, uint32_t off) {
+    return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + off);
+}
+
+// A published value that carries its tag: one 64-bit word in FP32, two in FP64.
+// The reader sees from the words themselves whether they have arrived, so the
+// writer need not wait for its stores before it tells the others.
+template <typename S>
+struct Tagged {
+    static constexpr int n = (int)(sizeof(S) / 4);
+    unsigned long long w[n];
+    __device__ __forceinline__ static void store(unsigned long long* at, S x, uint32_t tag) {
+        if constexpr (n == 1) {
+            put_shared(at, (unsigned long long)__float_as_uint(x) << 32 | tag);
+        } else {
+            const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+            put_shared(at, b << 32 | tag);
+            put_shared(at + 1, (b & 0xffffffff00000000ull) | tag);
+        }
+    }
+    __device__ __forceinline__ void load(const unsigned long long* at) {
+        for (int j = 0; j < n; ++j) w[j] = get_shared(at + j);
+    }
+    __device__ __forceinline__ bool is(uint32_t tag) const {
+        bool ok = true;
+        for (int j = 0; j < n; ++j) ok = ok && (uint32_t)w[j] == tag;
+        return ok;
+    }
+    __device__ __forceinline__ S value() const {
+        if constexpr (n == 1)
+            return __uint_as_float((uint32_t)(w[0] >> 32));
+        else
+            return __longlong_as_double(
+                (long long)(w[0] >> 32 | (w[n - 1] & 0xffffffff00000000ull)));
+    }
+    // Loads until the words carry the tag; false after kSyncSeconds.
+    __device__ __forceinline__ bool wait(const unsigned long long* at, uint32_t tag) {
+        const unsigned long long t0 = wall_clock64();
+        do {
+            load(at);
+            if (is(tag)) return true;
+        } while (wall_clock64() - t0 < kSyncSeconds * kClockHz);
+        return false;
+    }
+};
+
+// Lane l of the lower half of a group of 2 * OFF lanes: x of lane l + OFF (what
+// __shfl_down gives those lanes; the others get something).  Register moves
+// between lanes, where __shfl_down goes through the LDS unit (about 130 cycles a
+// step, and a reduction is a chain of six).
+template <int OFF>
+__device__ __forceinline__ uint32_t lane_down(uint32_t x) {
+    if constexpr (OFF == 32)
+        return __builtin_amdgcn_permlane32_swap(x, x, false, false)[1];
+    else if constexpr (OFF == 16)
+        return __builtin_amdgcn_permlane16_swap(x, x, false, false)[1];
+    else  // row_shl:OFF
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x100 + OFF, 0xf, 0xf, true);
+}
+template <int OFF>
+__device__ __forceinline__ double lane_down(double x) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const uint32_t lo = lane_down<OFF>((uint32_t)b), hi = lane_down<OFF>((uint32_t)(b >> 32));
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+// Lane 0 of each group of 2 * OFF lanes: the group's sum, in the order of a
+// __shfl_down tree (offsets OFF, OFF / 2, ..., 1).
+template <int OFF>
+__device__ __forceinline__ double lane_sum(double x) {
+    x += lane_down<OFF>(x);
+    if constexpr (OFF > 1)
+        return lane_sum<OFF / 2>(x);
+    else
+        return x;
+}
+// x of one lane, in every lane
+__device__ __forceinline__ double from_lane(double x, int lane) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const uint32_t lo = __builtin_amdgcn_readlane((int)b, lane);
+    const uint32_t hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+struct PersistLds {
+    double wave[2][kPersistThreads / 64];  // wave sums of this workgroup's tiles
+    double tot[2][2];                      // by parity of the exchange: the grid's sums
+    int bad;
+};
+
+// One workgroup's place in the grid exchange.  sum_slots adds the slots of a
+// system's tiles as 256 threads: thread t takes t, t + 256, ... and the threads
+// are added by a tree per wave of 64 (offsets 32, 16, ..., 1) and then wave by
+// wave.  The tiles are dealt to the workgroups so that each of them, and each
+// group of them, holds a whole branch of that tree:
+//  * more than 256 tiles (256 workgroups): a workgroup holds thread t's tiles;
+//    the 32 workgroups of XCD x (hardware workgroup i runs on XCD i % 8) hold the
+//    threads of wave x / 2 with parity x % 2, the branch below the last step.
+//    The first of them collects its group's sums and publishes theirs, and every
+//    workgroup reads the eight group sums: the two hops take as long as polling
+//    all 256 slots does on an idle device (2.4 us), with a sixteenth of the
+//    polling, which otherwise slows the stores it waits for;
+//  * up to 256 tiles (64 workgroups): a workgroup holds tiles l, l + 16, l + 32,
+//    l + 48 of a wave, the branch of the first two steps, and every workgroup
+//    reads all slots.
+struct GridSum {
+    unsigned long long* slots;
+    uint32_t tag;
+    int slot;    // this workgroup's slot
+    int nslots;  // workgroups of the grid
+    bool large;
+
+    __device__ static void publish(unsigned long long* s, double x, uint32_t tag) {
+        const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+        put_shared(s, b << 32 | tag);
+        put_shared(s + 1, (b & 0xffffffff00000000ull) | tag);
+    }
+    // The values of slot s once they carry the tag; false after kSyncSeconds.
+    template <int NV>
+    __device__ static bool collect(const unsigned long long* s, uint32_t tag, double (&v)[NV]) {
+        unsigned long long w[2 * NV], t0 = 0;
+        for (int tries = 0;; ++tries) {
+            bool ok = true;
+            for (int j = 0; j < 2 * NV; ++j) w[j] = get_shared(s + j);
+            for (int j = 0; j < 2 * NV; ++j) ok = ok && (uint32_t)w[j] == tag;
+            if (ok) break;
+            if ((tries & 63) == 63) {
+                const unsigned long long t = wall_clock64();
+                if (!t0) t0 = t;
+                if (t - t0 > kSyncSeconds * kClockHz) return false;
+            }
+        }
+        for (int j = 0; j < NV; ++j)
+            v[j] = __longlong_as_double(
+                (long long)(w[2 * j] >> 32 | (w[2 * j + 1] & 0xffffffff00000000ull)));
+        return true;
+    }
+
+    // The sum over the grid of every thread's v[], in the order of write_slot
+    // and sum_slots.  PUBLISHED: this wave's put_shared stores are complete for
+    // every workgroup once it returns.  False after a timed-out wait.
+    template <int NV, bool PUBLISHED>
+    __device__ bool sum(double (&v)[NV], double (&tot)[NV], PersistLds& L) {
+        const int tid = (int)threadIdx.x, lane = tid & 63, wid = tid >> 6;
+        for (int j = 0; j < NV; ++j) v[j] = lane_sum<32>(v[j]);
+        if (lane == 0)
+            for (int j = 0; j < NV; ++j) L.wave[j][wid] = v[j];
+        if (PUBLISHED) __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        double* const out = L.tot[tag & 1];
+        if (wid == 0) {
+            unsigned long long* const buf = slots + (size_t)(tag & 1) * kSlotBuffer;
+            // lane k: the partial of tile k, its waves in order (lanes past 3 repeat tile 3)
+            double a[NV];
+            for (int j = 0; j < NV; ++j) {
+                double part = 0.0;
+                const int k = min(lane, kPersistSub - 1);
+                for (int w = 0; w < kCgBlock / 64; ++w)
+                    part += L.wave[j][k * (kCgBlock / 64) + w];
+                const double p0 = from_lane(part, 0), p1 = from_lane(part, 1),
+                             p2 = from_lane(part, 2), p3 = from_lane(part, 3);
+                a[j] = large ? ((p0 + p1) + p2) + p3 : (p0 + p2) + (p1 + p3);
+            }
+            if (lane == 0)
+                for (int j = 0; j < NV; ++j)
+                    publish(buf + (size_t)slot * kSlotWords + 2 * j, a[j], tag);
+            bool ok = true;
+            const unsigned long long* from = buf;  // the slots every workgroup reads
+            int count = nslots;
+            if (large) {
+                const int group = slot & 7;  // slots of a group: group + 8 * member
+                unsigned long long* const gbuf = buf + (size_t)kPersistGroups * kSlotWords;
+                if (slot < 8) {
+                    double m[NV];
+                    for (int j = 0; j < NV; ++j) m[j] = 0.0;
+                    if (lane < kPersistGroups / 8)
+                        ok = collect<NV>(buf + (size_t)(group + 8 * lane) * kSlotWords, tag, m);
+                    for (int j = 0; j < NV; ++j) m[j] = lane_sum<16>(m[j]);
+                    if (lane == 0)
+                        for (int j = 0; j < NV; ++j)
+                            publish(gbuf + (size_t)group * kSlotWords + 2 * j, m[j], tag);
+                }
+                from = gbuf;
+                count = 8;
+            }
+            double g[NV];
+            for (int j = 0; j < NV; ++j) g[j] = 0.0;
+            if (ok && lane < count) ok = collect<NV>(from + (size_t)lane * kSlotWords, tag, g);
+            for (int j = 0; j < NV; ++j) {
+                double r = 0.0;
+                if (large) {  // lanes 2 w and 2 w + 1: the last step of wave w's tree
+                    g[j] = lane_sum<1>(g[j]);
+                    for (int w = 0; w < 4; ++w) r += from_lane(g[j], 2 * w);
+                } else {      // lanes 16 w ...: the last four steps
+                    g[j] = lane_sum<8>(g[j]);
+                    for (int w = 0; w < 4; ++w) r += from_lane(g[j], 16 * w);
+                }
+                if (lane == 0) out[j] = r;
+            }
+            if (!ok) L.bad = 1;
+        }
+        __syncthreads();
+        for (int j = 0; j < NV; ++j) tot[j] = uniform(out[j]);
+        ++tag;
+        return L.bad == 0;
+    }
+};
+
+// RPT: rows per thread (the rows a tile gives a thread, rounded up to a power
+// of two); W: entries of every slice of the sliced ELL; RES: rows of each thread
+// whose values and columns stay in registers; GLDS: g in LDS too (else in
+// registers).  p and d are in LDS: the SpMV reads p there for the columns of
+// this workgroup's own rows.  Rows past a tile's end take part as zeros; the
+// vectors are allocated to a multiple of 64 rows, so the rows of the last slice
+// past N are stored too (as zeros).
+template <typename S, int RPT, int W, int RES, bool GLDS, bool TAGGED>
+__global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
+    __shared__ PersistLds L;
+    __shared__ S lp[RPT * kPersistThreads], ld[RPT * kPersistThreads],
+        lg[GLDS ? RPT * kPersistThreads : 1];
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    // a tile is four waves and its rows are dealt in waves of 64, so its bounds
+    // are the same in every lane: kept in scalar registers
+    const int sub = __builtin_amdgcn_readfirstlane(tid / kCgBlock);
+    GridSum gs;
+    gs.slots = A.slots;
+    gs.tag = A.tag0;
+    gs.slot = (int)blockIdx.x;
+    gs.nslots = (int)gridDim.x;
+    gs.large = A.tiles > kCgBlock;
+    const int R = A.rowsPerTile;
+    int tile;  // see GridSum
+    if (gs.large) {
+        const int x = gs.slot & 7;
+        tile = 64 * (x >> 1) + 2 * (gs.slot >> 3) + (x & 1) + kCgBlock * sub;
+    } else {
+        tile = 64 * (gs.slot >> 4) + (gs.slot & 15) + 16 * sub;
+    }
+    // this tile's rows [cbase, cbase + R) have their p in LDS, from lofs on
+    const uint32_t cbase = (uint32_t)tile * R, lofs = (uint32_t)sub * (RPT * kCgBlock);
+    CgState* const st = A.st;
+    const int entry = st->stop;
+    const bool lead = gs.slot == 0 && tid == 0;
+    if (entry) {
+        if (lead) st->done = entry;  // as the update kernel of a stopped system
+        return;
+    }
+    if (tid == 0) L.bad = 0;
+    const int row0 = tile * R;
+    const int row1 = tile < A.tiles ? min(row0 + R, (A.N + 63) & ~63) : row0;
+    // this wave's first row; its row u is iw + 256 u + lane, of slice (iw + 256 u) / 64
+    const int iw = row0 + __builtin_amdgcn_readfirstlane(tid & (kCgBlock - 64));
+    auto live = [&](int u) { return iw + u * kCgBlock < row1; };
+    uint32_t lb = (uint32_t)lane * sizeof(S);
+    auto mine = [&](auto* vec, int u) { return at_byte(vec + (iw + u * kCgBlock), lb); };
+    auto mine2 = [&](int u) {  // row u's place in rtag: twice the bytes of a value
+        return at_byte(A.rtag + (int64_t)(iw + u * kCgBlock) * (int)(sizeof(S) / 4), 2 * lb);
+    };
+    const uint32_t lown = (uint32_t)(iw - (int)cbase) + lofs;  // LDS place of row u: lown + 256 u + lane
+    auto lds = [&](S* vec, int u) -> S& { return *at_byte(vec + lown + u * kCgBlock, lb); };
+    auto value = [&](int u, int k) {
+        return *at_byte(A.sval + ((int64_t)(iw + u * kCgBlock) * W + 64 * k), lb);
+    };
+    // a column as the byte offset of its p in LDS, or (top bit set) of its row in the vectors
+    constexpr uint32_t kFar = 0x80000000u;
+    auto column = [&](int u, int k) {
+        const uint32_t c = (uint32_t)*at_byte(
+            A.sellCol + ((int64_t)(iw + u * kCgBlock) * W + 64 * k), (uint32_t)lane * 4u);
+        const uint32_t l = c - cbase;
+        return l < (uint32_t)R ? (l + lofs) * (uint32_t)sizeof(S) : c * (uint32_t)sizeof(S) | kFar;
+    };
+
+    // Bit u: row u has a far column.  The pattern is symmetric, so those are the
+    // rows that other workgroups read, and only they are published.
+    uint32_t shown = 0;
+
+    S rv[RPT], qv[RPT], gr[GLDS ? 1 : RPT];
+    S mv[RES ? RES : 1][W];
+    uint32_t mc[RES ? RES : 1][W];
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+        rv[u] = qv[u] = S(0);
+        S p0 = S(0), d0 = S(0), g0 = S(0);
+        if (u < RES)
+            for (int k = 0; k < W; ++k) {
+                mv[u][k] = S(0);
+                mc[u][k] = 0;
+            }
+        if (live(u)) {
+            if (u < RES) {
+#pragma unroll
+                for (int k = 0; k < W; ++k) {
+                    mv[u][k] = value(u, k);
+                    mc[u][k] = column(u, k);
+                    shown |= mc[u][k] >> 31 << u;
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < W; ++k) shown |= column(u, k) >> 31 << u;
+            }
+            if (iw + u * kCgBlock + lane < A.N) {
+                rv[u] = *mine(A.r, u);
+                p0 = *mine(A.p, u);
+                d0 = *mine(A.d, u);
+                g0 = *mine(A.g, u);
+            }
+            lds(lp, u) = p0;
+            lds(ld, u) = d0;
+            if constexpr (GLDS) lds(lg, u) = g0;
+        }
+        if constexpr (!GLDS) gr[u] = g0;
+    }
+    const double bnorm = uniform(st->bnorm), tol = uniform(st->tol), atol = uniform(st->atol),
+                 delta = uniform(st->delta), rrep = uniform(st->rrep);
+    const int maxit = __builtin_amdgcn_readfirstlane(st->maxit);
+    double rho = uniform(st->rho), rhoPrev = uniform(st->rhoPrev), alpha = uniform(st->alpha),
+           res = uniform(st->res);
+    int it = __builtin_amdgcn_readfirstlane(st->it), stop = 0;
+    S beta = S(0);
+    uint32_t rtag = 0;
+    S *pold = A.p, *pnew = A.p2;  // the direction before this iteration's, and the next one's place
+    bool ok = true;
+    __syncthreads();
+    for (int n = 0; n < A.iters; ++n) {
+        opaque(lb);
+        for (int u = 0; u < RES; ++u)
+            for (int k = 0; k < W; ++k) opaque(mc[u][k]);
+        // q = As p, p.q.  A far column's p: as published for the launch's first
+        // iteration, afterwards from its published r and old p
+        double v1[1] = {0.0}, t1[1];
+        auto row = [&](int u, const S (&v)[W], const uint32_t (&c)[W], auto next) {
+            S x[W], y[W];
+            Tagged<S> t[TAGGED ? W : 1];
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                if (c[k] & kFar) {
+                    const uint32_t o = c[k] & ~kFar;
+                    y[k] = get_shared(at_byte(pold, o));
+                    if constexpr (TAGGED)
+                        t[k].load(at_byte(A.rtag, 2 * o));
+                    else
+                        x[k] = n ? get_shared(at_byte(A.r, o)) : S(0);
+                } else {
+                    x[k] = *at_byte(lp, c[k]);
+                }
+            }
+            next();
+            const S own = lds(lp, u);
+            S sum = own;
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                if (c[k] & kFar) {
+                    if constexpr (TAGGED) {
+                        if (n && !t[k].is(rtag) &&
+                            !t[k].wait(at_byte(A.rtag, 2 * (c[k] & ~kFar)), rtag))
+                            L.bad = 1;
+                        x[k] = t[k].value();
+                    }
+                    x[k] = n ? x[k] + beta * y[k] : y[k];
+                }
+                sum += v[k] * x[k];
+            }
+            qv[u] = sum;
+            v1[0] += (double)own * (double)sum;
+        };
+        // streamed rows: the next row's columns are in flight during this row, whose
+        // values are loaded beside the far columns' vectors
+        uint32_t cn[W];
+        auto fetch = [&](int u) {
+#pragma unroll
+            for (int k = 0; k < W; ++k) cn[k] = column(u, k);
+        };
+        if (RES < RPT && live(RES)) fetch(RES);
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            if (u < RES) {
+                row(u, mv[u], mc[u], [] {});
+            } else {
+                S v[W];
+                uint32_t c[W];
+#pragma unroll
+                for (int k = 0; k < W; ++k) {
+                    c[k] = cn[k];
+                    v[k] = value(u, k);
+                }
+                row(u, v, c, [&] {
+                    if (u + 1 < RPT && live(u + 1)) fetch(u + 1);
+                });
+            }
+        }
+        if (!(ok = gs.sum<1, true>(v1, t1, L))) break;
+        // alpha; d += alpha p, r -= alpha q, ||G r||^2 and r.r
+        alpha = rho / t1[0];
+        ++it;
+        rhoPrev = rho;
+        const S a = (S)alpha;
+        rtag = gs.tag;
+        double v2[2] = {0.0, 0.0}, t2[2];
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            const S ri = rv[u] - a * qv[u];
+            rv[u] = ri;
+            if (shown >> u & 1) {
+                if constexpr (TAGGED)
+                    Tagged<S>::store(mine2(u), ri, rtag);
+                else
+                    put_shared(mine(A.r, u), ri);
+            }
+            lds(ld, u) = lds(ld, u) + a * lds(lp, u);
+            S gi;
+            if constexpr (GLDS)
+                gi = lds(lg, u);
+            else
+                gi = gr[u];
+            const double ur = (double)ri * (double)gi;
+            v2[0] += ur * ur;
+            v2[1] += (double)ri * (double)ri;
+        }
+        if (!(ok = gs.sum<2, !TAGGED>(v2, t2, L))) break;
+        // the stop decision (cg_decide) and the next direction
+        const double rn = sqrt(t2[0]);
+        res = rn / bnorm;
+        rho = t2[1];
+        if (res <= tol || rn <= atol || it >= maxit || !(res == res) ||
+            (delta > 0.0 && rn < delta * rrep)) {
+            stop = 1;
+            break;
+        }
+        beta = (S)(rho / rhoPrev);
+        if (n) {
+            S* const t = pold;
+            pold = pnew;
+            pnew = t;
+        }
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            const S pi = rv[u] + beta * lds(lp, u);
+            lds(lp, u) = pi;
+            if (shown >> u & 1) put_shared(mine(pnew, u), pi);
+        }
+        __syncthreads();
+    }
+    if (!ok) {
+        if (tid == 0) st->stop = kStopSync;
+        return;
+    }
+#pragma unroll
+    for (int u = 0; u < RPT; ++u)
+        if (live(u)) {
+            *mine(A.r, u) = rv[u];
+            *mine(A.p, u) = lds(lp, u);
+            *mine(A.d, u) = lds(ld, u);
+        }
+    if (lead) {
+        st->rho = rho;
+        st->rhoPrev = rhoPrev;
+        st->alpha = alpha;
+        st->res = res;
+        st->it = it;
+        st->stop = stop;
+        st->done = 0;
+        st->pbuf = 0;
+    }
+}
+
+}  // namespace
+}  // namespace fvhip

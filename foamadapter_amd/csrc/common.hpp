@@ -91,6 +91,9 @@ struct fv_ctx {
     static constexpr size_t kPollBytes = 4096;
     void* pollHost = nullptr;
     hipEvent_t pollEv[2] = {};
+    // another context of the same owner works on the device at the same time (the
+    // server's two lanes): no kernel of this one may hold every CU for long
+    bool shared = false;
 };
 
 namespace fvhip {

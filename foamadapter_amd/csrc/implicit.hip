@@ -464,11 +464,14 @@ int fv_sparsity_create(fv_mesh* m, fv_sparsity** out) {
         // without their diagonal entry: the solvers' scaled matrices have a unit
         // diagonal, which their SpMVs add themselves
         const int64_t C = fv_sparsity::kSlice, nS = (N + C - 1) / C;
+        int32_t widest = 0;
+        for (int64_t r = 0; r < N; ++r) widest = std::max(widest, rowOffs[r + 1] - rowOffs[r] - 1);
+        sp->sellWidth = widest <= 4 ? 4 : widest <= 6 ? 6 : 0;
         auto sliced = [&](fvhip::DBuf<int64_t>& offOut, fvhip::DBuf<int32_t>& colOut,
                           fvhip::DBuf<int32_t>& srcOut) -> int64_t {
             std::vector<int64_t> soff(nS + 1, 0);
             for (int64_t s = 0; s < nS; ++s) {
-                int32_t wmax = 0;
+                int32_t wmax = sp->sellWidth;
                 for (int64_t r = s * C; r < std::min<int64_t>(N, (s + 1) * C); ++r)
                     wmax = std::max(wmax, rowOffs[r + 1] - rowOffs[r] - 1);
                 soff[s + 1] = soff[s] + C * wmax;
@@ -488,7 +491,8 @@ int fv_sparsity_create(fv_mesh* m, fv_sparsity** out) {
                         }
                     for (; k < wdt; ++k) {
                         const int64_t pos = soff[s] + k * C + l;
-                        scol[pos] = r < N ? (int32_t)r : 0;
+                        // the row itself, or the last one: a column of the same slice
+                        scol[pos] = (int32_t)std::min(r, N - 1);
                         ssrc[pos] = -1;
                     }
                 }

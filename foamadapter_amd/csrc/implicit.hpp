@@ -21,6 +21,11 @@ struct fv_sparsity {
     // wavefront each; entry k of row 64s+l at sellOff[s] + 64k + l): column and
     // source CSR index (-1 for padding)
     static constexpr int kSlice = 64;
+    // When no row has more than 6 off-diagonal entries (hexahedra) every slice has
+    // the same width, 4 or 6: entry k of row i is at (i / 64) * 64 w + 64 k + i % 64
+    // and the persistent CG reads it without slice offsets.  0: slices as wide as
+    // their longest row.
+    int32_t sellWidth = 0;
     int64_t sellTotal = 0;
     fvhip::DBuf<int64_t> sellOff;
     fvhip::DBuf<int32_t> sellCol, sellSrc;

@@ -618,6 +618,7 @@ int fv_server_create(int device, const fv_server_opts* opts, fv_server** out) {
         s->batch->useGraph = opts->use_graph != 0;
         if (s->opts.batched && s->opts.solo_rows > 0) {
             check(fv_ctx_create(device, 0, &s->soloCtx));
+            s->ctx->shared = s->soloCtx->shared = true;  // the lanes share the device
             s->soloWorker = std::thread(solo_loop, s);
         }
         s->worker = std::thread(worker_loop, s);

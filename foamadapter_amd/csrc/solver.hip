@@ -8,11 +8,13 @@
 // implicit tiles of the one system (at most kCgMaxTiles tiles, rows in multiples of 64).
 // All scalars live on the device; kernels turn into no-ops once the stop flag is
 // set, and the host polls the flag every `check` iterations, so a solve needs
-// no host round trip per iteration.  The workspace stays with the linear
+// no host round trip per iteration.  Systems of up to 2^21 rows with at most 6
+// off-diagonal entries per row run many iterations per launch instead
+// (cgpersist.hpp, the same bits).  The workspace stays with the linear
 // system, so repeated solves (time steps) allocate nothing, and a repeated
 // solve launches the previous solve's schedule at once -- as a captured
 // hipGraph once the same schedule has come five times in a row.
-#include "cgkernels.hpp"
+#include "cgpersist.hpp"
 
 #include <cmath>
 #include <deque>
@@ -43,6 +45,13 @@ struct CgWork : fv_solver_cache {
     int seenCount = 0;  // consecutive solves with seenKey
     int lastIters = 0;  // iterations of the previous solve (time steps repeat them)
     std::vector<int> lastRounds;  // FP32 iterations per round of the previous mixed solve
+    // persistent form (null: this system runs kernel by kernel)
+    void (*persist)(CgPersist<S>) = nullptr;
+    int persistGrid = 0, persistIters = 0;
+    int lastLaunches = 0;  // persistent launches of the previous mixed solve
+    int lastTotal = 0;     // iterations of the previous solve, in either form
+    DBuf<unsigned long long> slots, rtag;
+    uint32_t tag = 1;
 
     CgWork(fv_ctx* c, const fv_linsys* ls) {
         const fv_sparsity* sp = ls->sp;
@@ -50,12 +59,14 @@ struct CgWork : fv_solver_cache {
         const int R = cg_tile_rows(N, kB);
         const int tiles = (N + R - 1) / R;
         G = cg_grid(tiles);
-        r.alloc(c, N);
-        p.alloc(c, N);
-        p2.alloc(c, N);
+        // whole slices: the persistent kernel stores the last one's rows past N too
+        const size_t N64 = ((size_t)N + 63) / 64 * 64;
+        r.alloc(c, N64);
+        p.alloc(c, N64);
+        p2.alloc(c, N64);
         q.alloc(c, N);
         g.alloc(c, N);
-        dbuf.alloc(c, N);
+        dbuf.alloc(c, N64);
         sval.alloc(c, sp->sellTotal);
         r64.alloc(c, N);
         pq.alloc(c, tiles);
@@ -91,6 +102,90 @@ struct CgWork : fv_solver_cache {
         gdev.upload(c, &grid, 1);
         FV_HIP(hipStreamSynchronize(c->stream));
         red = CgPartials{pq.p, rz.p, rb.p};
+        if (!c->shared) choose_persist(c, sp, tiles, R);
+    }
+
+    // The persistent kernel for this system, when there is one: slices of one
+    // width, at most 8 rows per thread (2^21 rows; beyond, the vectors do not fit
+    // the registers), and a device that keeps its workgroups resident together.
+    void choose_persist(fv_ctx* c, const fv_sparsity* sp, int tiles, int R) {
+        const int rpt = (R + kB - 1) / kB;
+        if (sp->sellWidth == 6)
+            persist = persist_kernel<6>(rpt);
+        else if (sp->sellWidth == 4)
+            persist = persist_kernel<4>(rpt);
+        if (!persist) return;
+        persistGrid = tiles > kCgBlock ? kPersistGroups
+                                       : 16 * (tiles / 64) + std::min(tiles % 64, 16);
+        int perCu = 0, cus = 0, coop = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, persist, kPersistThreads, 0) !=
+                hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) !=
+                hipSuccess ||
+            hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) !=
+                hipSuccess ||
+            !coop || (int64_t)perCu * cus < persistGrid) {
+            (void)hipGetLastError();
+            persist = nullptr;
+            return;
+        }
+        // a launch holds the device for about 2 ms (an iteration takes 6 to 40 us,
+        // from the smallest to the largest of these systems), so that the work of
+        // other streams gets in between
+        persistIters = (int)(2000.0 / (6.0 + 32.0 * h.N / (1 << 21)));
+        slots.alloc(c, 2 * (size_t)kSlotBuffer);
+        if (rpt <= (sizeof(S) == 8 ? 2 : 4))  // the TAGGED kernels
+            rtag.alloc(c, ((size_t)h.N + 63) / 64 * 64 * (sizeof(S) / 4));
+        clear_tags(c->stream);
+    }
+    // A cooperative launch costs about 17 us more than a plain one and is not
+    // replayed as a graph, and an iteration saves 4 us on the smallest systems: a
+    // system whose previous solve took fewer than kPersistMin iterations keeps the
+    // kernel-by-kernel form (32^3 heat step of 5 iterations: 157 us, 178 persistent).
+    static constexpr int kPersistMin = 12;
+    bool use_persist() const { return persist && (lastTotal == 0 || lastTotal >= kPersistMin); }
+    // no word of the exchange carries a tag that is still to come
+    void clear_tags(hipStream_t s) {
+        FV_HIP(hipMemsetAsync(slots.p, 0, slots.n * sizeof(unsigned long long), s));
+        if (rtag.n) FV_HIP(hipMemsetAsync(rtag.p, 0, rtag.n * sizeof(unsigned long long), s));
+        tag = 1;
+    }
+    // RES, the rows whose matrix stays in registers, is what fits beside the vectors
+    // in the 128 registers of a 1024-thread workgroup without spills.
+    template <int W>
+    static auto persist_kernel(int rpt) -> void (*)(CgPersist<S>) {
+        if (rpt <= 1) return kc_persist<S, 1, W, 1, false, true>;
+        if (rpt <= 2) return kc_persist<S, 2, W, 2, true, true>;
+        if constexpr (sizeof(S) == 8) {
+            if (rpt <= 4) return kc_persist<S, 4, W, 2, true, false>;
+            if (rpt <= 8) return kc_persist<S, 8, W, 0, false, false>;
+        } else {
+            if (rpt <= 4) return kc_persist<S, 4, W, 4, true, true>;
+            if (rpt <= 8) return kc_persist<S, 8, W, 4, true, false>;
+        }
+        return nullptr;
+    }
+    // Up to persistIters iterations in one launch; false if the device refuses it.
+    bool run_persist(hipStream_t s) {
+        const uint32_t uses = 3 * (uint32_t)persistIters + 3;
+        if (tag > 0xffffffffu - uses) clear_tags(s);  // sequence numbers start over
+        CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persistIters, tag, h.sellCol, h.sval,
+                       h.g, h.d, h.r, h.p, h.p2, rtag.p, h.st, slots.p};
+        void* args[] = {&a};
+        if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(persist), dim3(persistGrid),
+                                       dim3(kPersistThreads), args, 0, s) != hipSuccess) {
+            (void)hipGetLastError();
+            persist = nullptr;
+            return false;
+        }
+        tag += uses;
+        return true;
+    }
+    void check_persist(const CgState& h) {
+        if (h.stop != kStopSync) return;
+        persist = nullptr;
+        throw Error{FV_EDEVICE, "persistent CG: the workgroups did not meet in " +
+                                    std::to_string(kSyncSeconds) + " s"};
     }
 
     ~CgWork() override { drop_graph(); }
@@ -353,6 +448,46 @@ CgState run_cg(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, int check,
     return h;
 }
 
+// run_cg with the persistent kernel: a launch ends at the stop by itself, so
+// nothing has to be predicted.  A system whose previous solve fitted one launch
+// gets the correction and the explicit residual queued behind it and is read
+// once; otherwise two launches are kept queued until one has stopped.  False
+// (and nothing done) if the device refuses the launch.
+bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, double atol,
+                    double* true_res, CgState* out) {
+    hipStream_t s = ctx->stream;
+    w.prep(s);
+    w.start(s, tol, maxit, 0.0, atol);
+    if (!w.run_persist(s)) return false;
+    CgState h{}, t{};
+    bool haveTrue = false;
+    if (w.lastIters > 0 && w.lastIters <= w.persistIters) {
+        w.finish(s);
+        w.enqueue_true_residual(s);
+        FV_LAUNCH_CHECK();
+        h = w.state2(s, &t);
+        haveTrue = h.stop != 0;
+    }
+    if (!h.stop) {
+        PollPipe pp{static_cast<CgState*>(ctx_poll_host(ctx)), ctx};
+        pp.push(s, w.st.p);
+        while (!h.stop) {
+            while (pp.npend < 2) {
+                FV_REQUIRE(w.run_persist(s), "a cooperative launch was refused");
+                pp.push(s, w.st.p);
+            }
+            h = pp.pop();
+        }
+        while (pp.npend) h = pp.pop();
+        w.finish(s);
+    }
+    w.check_persist(h);
+    w.lastIters = std::max(h.it, 1);
+    *true_res = haveTrue ? t.res : w.true_residual(s);
+    *out = h;
+    return true;
+}
+
 // ---- mixed precision: FP32 CG with FP64 residual replacement ---------------
 //
 // The FP32 CG accumulates its correction d (FP32); it stops when the FP32
@@ -499,6 +634,51 @@ IrOut run_mixed(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, int chunk,
     return IrOut{h.res0, h.res, h.bnorm, h.it, h.nrep};
 }
 
+// run_mixed with the persistent kernel: a round is one launch, which ends at the
+// drop trigger, the tolerance or its iterations, and the replacement kernels,
+// which act only on a stopped CG.  As many rounds as the previous solve took are
+// queued at once, otherwise two at a time.
+bool run_mixed_persist(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, double delta,
+                       double atol, IrOut* out) {
+    hipStream_t s = ctx->stream;
+    w.prep(s);
+    w.start(s, tol, maxit, delta, atol);
+    if (!w.run_persist(s)) return false;
+    w.replacement(s);
+    int rounds = 1;
+    auto round = [&] {
+        FV_REQUIRE(w.run_persist(s), "a cooperative launch was refused");
+        w.replacement(s);
+        FV_LAUNCH_CHECK();
+        ++rounds;
+    };
+    CgState h{};
+    auto done = [&] { return h.stop >= 2 || h.it >= maxit; };
+    if (w.lastLaunches > 0) {
+        while (rounds < w.lastLaunches) round();
+        h = w.state(s);
+    }
+    if (!done()) {
+        PollPipe pp{static_cast<CgState*>(ctx_poll_host(ctx)), ctx};
+        int seen = rounds - 1;
+        pp.push(s, w.st.p);
+        while (!done()) {
+            while (pp.npend < 2) {
+                round();
+                pp.push(s, w.st.p);
+            }
+            h = pp.pop();
+            ++seen;
+        }
+        while (pp.npend) h = pp.pop();
+        rounds = seen;
+    }
+    w.check_persist(h);
+    if (h.stop == 2) w.lastLaunches = rounds;
+    *out = IrOut{h.res0, h.res, h.bnorm, h.it, h.nrep};
+    return true;
+}
+
 }  // namespace
 
 extern "C" {
@@ -518,8 +698,11 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
             CgWork<double>& w = work_of<double>(ls, false);
             w.bind(ctx, x);
             double tr = 0.0;
-            CgState h =
-                run_cg(ctx, w, o->rel_tol, o->max_iter, check, o->abs_tol, o->eager != 0, &tr);
+            CgState h{};
+            if (o->eager || !w.use_persist() ||
+                !run_cg_persist(ctx, w, o->rel_tol, o->max_iter, o->abs_tol, &tr, &h))
+                h = run_cg(ctx, w, o->rel_tol, o->max_iter, check, o->abs_tol, o->eager != 0, &tr);
+            w.lastTotal = h.it;
             local.init_res = h.res0;
             local.final_res = h.res;
             bnorm = h.bnorm;
@@ -529,11 +712,17 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
         } else if (o->mode == FV_SOLVE_F32_IR) {
             CgWork<float>& w = work_of<float>(ls, true);
             w.bind(ctx, x);
-            IrOut r = run_mixed(ctx, w, o->rel_tol, o->max_iter,
-                                o->check_every > 0 ? o->check_every : 64,
-                                o->inner_rel_tol > 0.0 ? o->inner_rel_tol : kIrDelta,
-                                o->max_outer > 0 ? o->max_outer : (1 << 30), o->abs_tol,
-                                o->eager != 0);
+            IrOut r{};
+            const double delta = o->inner_rel_tol > 0.0 ? o->inner_rel_tol : kIrDelta;
+            // max_outer counts rounds of check_every iterations: those solves run
+            // kernel by kernel
+            if (o->eager || o->max_outer > 0 || !w.use_persist() ||
+                !run_mixed_persist(ctx, w, o->rel_tol, o->max_iter, delta, o->abs_tol, &r))
+                r = run_mixed(ctx, w, o->rel_tol, o->max_iter,
+                              o->check_every > 0 ? o->check_every : 64, delta,
+                              o->max_outer > 0 ? o->max_outer : (1 << 30), o->abs_tol,
+                              o->eager != 0);
+            w.lastTotal = r.iters;
             local.init_res = r.init_res;
             local.final_res = r.res;
             bnorm = r.bnorm;

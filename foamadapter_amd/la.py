@@ -202,8 +202,8 @@ def solver_opts(solver: dict | None) -> _lib.FvSolveOpts:
     relTol -> relative_residual_norm, maxIter -> iteration, default 1000, tolerance ->
     absolute_residual_norm), or its mapped Ginkgo form, to solver options.
     'precision': 'mixed' selects FP32 CG inside FP64 iterative refinement;
-    'graph': False launches a repeated CG solve kernel by kernel instead of
-    replaying it as a captured hipGraph (the same bits)."""
+    'graph': False launches a CG solve kernel by kernel instead of as a persistent
+    kernel or a captured hipGraph (the same bits)."""
     d = dict(solver or {})
     crit = d.get("criteria", {})
     o = _lib.FvSolveOpts()

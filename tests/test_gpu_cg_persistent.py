@@ -1,0 +1,75 @@
+"""The persistent CG kernel against the kernel-by-kernel form ("graph": False), bit for
+bit: both add every dot product in the same order, so the solutions, the iteration counts
+and the residuals are the same numbers.  The sizes sit at the edges of what the kernel
+distinguishes: tiles of 256 rows (the last one ragged), 64 workgroups of up to 256 tiles or
+256 workgroups beyond, 1, 2, 4 and 8 rows per thread, slices of 4 (plane meshes) and 6
+entries, and solves of several launches."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # dims, iteration limit
+    ((3, 3, 3), 200),          # one ragged tile
+    ((16, 16, 1), 200),        # one whole tile, 4 entries a row
+    ((17, 16, 16), 400),       # 17 tiles: a second tile in one workgroup
+    ((65, 16, 16), 2000),      # 65 tiles: the second wave of slots begins
+    ((256, 16, 16), 700),      # 256 tiles: the last grid of 64 workgroups
+    ((257, 16, 16), 700),      # 257: 256 workgroups, all but one with one tile
+    ((64, 32, 32), 2000),      # the same two, converging
+    ((41, 40, 40), 2000),
+    ((64, 64, 65), 60),        # 2 rows per thread
+    ((700, 500, 1), 60),       # the same, 4 entries a row
+    ((101, 100, 61), 40),      # 3 rows per thread (kernel of 4), last slice ragged
+    ((128, 128, 70), 30),      # 5 rows per thread (kernel of 8)
+]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import foamadapter_amd as fa
+    with fa.Context(0) as c:
+        yield c
+
+
+def _system(ctx, dims):
+    import foamadapter_amd as fa
+    from foamadapter_amd import dsl, fvcc
+    poly = fa.PolyMesh.hex(dims, jitter=0.2 if min(dims) > 1 else 0.0, jitter_seed=5)
+    if min(dims) == 1:  # a plane mesh: no finite-volume faces on its two sides
+        for p in poly.patches[4:]:
+            p.type = "empty"
+    m = fa.Mesh.from_poly(ctx, poly, renumber=len(dims) == 3 and min(dims) > 40)
+    N, F, B = m.n_cells, m.n_internal_faces, m.n_boundary_faces
+    bc = fa.BoundaryConditions(m, ["fixedValue"] + ["zeroGradient"] * (m.n_patches - 1))
+    p = fvcc.VolumeField(m, ctx.zeros((N,)), ctx.zeros((B,)), bc, "p")
+    gamma = fvcc.SurfaceField(m, ctx.uniform(F + B, 0.5, 2.0, 11, 0))
+    phi = fvcc.SurfaceField(m, ctx.uniform(F + B, -1.0, 1.0, 11, 1))
+    return m, dsl.assemble(dsl.imp.laplacian(gamma, p) - dsl.exp.div(phi), p, 0.0, 1.0)
+
+
+@pytest.mark.parametrize("precision", ["double", "mixed"])
+@pytest.mark.parametrize("dims,limit", CASES, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_persistent_is_bitwise_the_kernel_by_kernel_form(ctx, dims, limit, precision):
+    from foamadapter_amd import la
+    print(dims, limit, precision, flush=True)
+    m, ls = _system(ctx, dims)
+    got = []
+    # eager first, then the persistent form three times: a first solve, and repeats of it
+    for graph in (False, True, True, True):
+        x = ctx.zeros((m.n_cells,))
+        st = la.solve_cg(ls, x, {"relTol": 1e-8, "maxIter": limit, "precision": precision, "graph": graph},
+                         raise_on_noconverge=False)
+        got.append((x.numpy(), st.numIter, st.finalResNorm, st.status))
+    assert got[0][1] >= 12  # fewer iterations in the solve before run kernel by kernel
+    for g in got[1:]:
+        if precision == "mixed" and got[0][3] != 0 and got[0][1] < limit:
+            # cut by its limit after a residual replacement: the kernel-by-kernel form
+            # counts the iterations it had queued behind the replacement's stop towards
+            # the limit, the persistent one runs as many as it was given
+            assert g[1] == limit and g[3] == got[0][3]
+            continue
+        assert g[1:] == got[0][1:]
+        assert np.array_equal(g[0], got[0][0])
+    m.close()

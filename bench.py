@@ -64,14 +64,14 @@ OPS = ["interp_linear", "grad", "div_linear", "div_upwind", "laplacian", "sngrad
 KERNEL_OF = {
     ("interp_linear", "f64"): "k_interp4<double>", ("interp_linear", "f32"): "k_interp4<float>",
     ("sngrad", "f64"): "k_sngrad4<double>", ("sngrad", "f32"): "k_sngrad4<float>",
-    ("grad", "f64"): "k_gather<double, GradOp<double>, 256, 256>",
-    ("grad", "f32"): "k_gather<float, GradOp<float>, 256, 256>",
-    ("div_linear", "f64"): "k_gather<double, DivOp<double, 0>, 512, 512>",
-    ("div_linear", "f32"): "k_gather<float, DivOp<float, 0>, 1024, 512>",
-    ("div_upwind", "f64"): "k_gather<double, DivOp<double, 1>, 512, 512>",
-    ("div_upwind", "f32"): "k_gather<float, DivOp<float, 1>, 1024, 512>",
-    ("laplacian", "f64"): "k_gather<double, LapOp<double>, 256, 256>",
-    ("laplacian", "f32"): "k_gather<float, LapOp<float>, 1024, 512>",
+    ("grad", "f64"): "k_gather<double, GradOp<double>, 256, 256, 1>",
+    ("grad", "f32"): "k_gather<float, GradOp<float>, 256, 256, 1>",
+    ("div_linear", "f64"): "k_gather<double, DivOp<double, 0>, 512, 512, 1>",
+    ("div_linear", "f32"): "k_gather<float, DivOp<float, 0>, 1024, 512, 1>",
+    ("div_upwind", "f64"): "k_gather<double, DivOp<double, 1>, 512, 512, 1>",
+    ("div_upwind", "f32"): "k_gather<float, DivOp<float, 1>, 1024, 512, 1>",
+    ("laplacian", "f64"): "k_gather<double, LapOp<double>, 256, 256, 1>",
+    ("laplacian", "f32"): "k_gather<float, LapOp<float>, 1024, 512, 1>",
 }
 TRAFFIC_PROFILE = ROOT / "profiles" / "faceops_sweep_256cube.md"
 # the sources whose kernels the traffic profile measured; the profile records

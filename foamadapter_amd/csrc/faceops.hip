@@ -431,7 +431,9 @@ __device__ inline void sort_keys(uint16_t (&k)[K]) {
 // order (external lower, inner lower, own, boundary) and divides by V.  A
 // workgroup whose faces do not fit the LDS arrays takes the per-cell path of
 // gather_cell instead; both give the same bits.
-template <typename S, typename Op, int CELLS, int THREADS>
+// XE: external list records each thread holds at once (2: the wide form of the
+// 256-cell workgroup, see gather_wide_ext).
+template <typename S, typename Op, int CELLS, int THREADS, int XE>
 __global__ __launch_bounds__(THREADS) void k_gather(int N, int nBlocks, int run, Split t,
                                                     Lists L, ExGeo<S> xg, Op op,
                                                     const S* __restrict__ V, S coeff,
@@ -439,8 +441,8 @@ __global__ __launch_bounds__(THREADS) void k_gather(int N, int nBlocks, int run,
     constexpr int NC = Op::NC;
     constexpr int kUL = Op::kFacesPerPass;
     constexpr int kMaxUp = max_up<CELLS>();
-    constexpr int kMaxExt = gather_max_ext(CELLS);
-    constexpr int kMaxBnd = gather_max_bnd(CELLS);
+    constexpr int kMaxExt = XE == 1 ? gather_max_ext(CELLS) : gather_wide_ext();
+    constexpr int kMaxBnd = XE == 1 ? gather_max_bnd(CELLS) : gather_wide_bnd();
     constexpr int kMaxLow = gather_max_low(CELLS);  // inner lower faces per cell, in LDS
     __shared__ S fluxU[NC][kMaxUp];
     __shared__ S fluxE[NC][kMaxExt];
@@ -507,17 +509,30 @@ __global__ __launch_bounds__(THREADS) void k_gather(int N, int nBlocks, int run,
     // first pass also takes this thread's list records (at most one external
     // lower face and one boundary face: the lists of a fitting workgroup hold
     // no more records than it has threads).
-    static_assert(kMaxExt <= THREADS && kMaxBnd <= THREADS, "one list record per thread");
+    static_assert(XE > 1 || (kMaxExt <= THREADS && kMaxBnd <= THREADS), "one list record per thread");
     const int ke = e0 + (int)threadIdx.x, kb = b0 + (int)threadIdx.x;
-    const bool hasE = fits && ke < e1, hasB = fits && kb < b1;
+    const bool hasB = fits && kb < b1;
     // Every lane reads records (past its workgroup's range: the first record
     // after it, at most the zero record past the last workgroup), so no lane
     // branches around these loads; lanes without a record ignore them.
-    const int kec = min(ke, e1), kbc = min(kb, b1);
-    const int ef = L.extFace[kec], eo = L.extOwn[kec], ecl = L.extCell[kec];
-    const int ecp = L.extCell[max(kec - 1, e0)], ecn = L.extCell[max(min(kec + 1, e1 - 1), e0)];
-    const int bf = L.bndFace[kbc], bcl = L.bndCell[kbc];
-    const int bcp = L.bndCell[max(kbc - 1, b0)], bcn = L.bndCell[max(min(kbc + 1, b1 - 1), b0)];
+    // face, owner, cell, the cells of the records before and after
+    struct Rec {
+        int f, o, c, cp, cn;
+    };
+    auto record = [&](int k) -> Rec {
+        const int kc = min(k, e1);
+        return {L.extFace[kc], L.extOwn[kc], L.extCell[kc], L.extCell[max(kc - 1, e0)],
+                L.extCell[max(min(kc + 1, e1 - 1), e0)]};
+    };
+    Rec er[XE];
+#pragma unroll
+    for (int x = 0; x < XE; ++x) er[x] = record(ke + x * THREADS);
+    auto brecord = [&](int k) -> Rec {
+        const int kc = min(k, b1);
+        return {L.bndFace[kc], 0, L.bndCell[kc], L.bndCell[max(kc - 1, b0)],
+                L.bndCell[max(min(kc + 1, b1 - 1), b0)]};
+    };
+    const Rec br = brecord(kb);
     for (int l = threadIdx.x; l < CELLS; l += THREADS) {
         exS[l] = exE[l] = bS[l] = bE[l] = 0;
         lowN[l] = 0;
@@ -536,24 +551,41 @@ __global__ __launch_bounds__(THREADS) void k_gather(int N, int nBlocks, int run,
     }
     __syncthreads();
     // This thread's list faces: loads, contribution into LDS, the cell ranges.
+    auto put_ext = [&](int k, const Rec& r, const In& in) {
+        S sv[NC];
+        op.make(in, sv);
+        for (int j = 0; j < NC; ++j) fluxE[j][k - e0] = sv[j];
+        if (k == e0 || r.cp != r.c) exS[r.c] = (uint16_t)(k - e0);
+        if (k == e1 - 1 || r.cn != r.c) exE[r.c] = (uint16_t)(k - e0 + 1);
+    };
+    auto put_bnd = [&](int k, const Rec& r, const BIn& in) {
+        S sv[NC];
+        op.bmake(in, sv);
+        for (int j = 0; j < NC; ++j) fluxB[j][k - b0] = sv[j];
+        if (k == b0 || r.cp != r.c) bS[r.c] = (uint16_t)(k - b0);
+        if (k == b1 - 1 || r.cn != r.c) bE[r.c] = (uint16_t)(k - b0 + 1);
+    };
     auto list_faces = [&] {
-        In ein{};
+        In ein[XE]{};
         BIn bin{};
-        if (hasE) ein = op.eload(ke, ef, eo, c0 + ecl, xg);
-        if (hasB) bin = op.bload(bf, c0 + bcl);
-        if (hasE) {
-            S sv[NC];
-            op.make(ein, sv);
-            for (int j = 0; j < NC; ++j) fluxE[j][ke - e0] = sv[j];
-            if (ke == e0 || ecp != ecl) exS[ecl] = (uint16_t)(ke - e0);
-            if (ke == e1 - 1 || ecn != ecl) exE[ecl] = (uint16_t)(ke - e0 + 1);
-        }
-        if (hasB) {
-            S sv[NC];
-            op.bmake(bin, sv);
-            for (int j = 0; j < NC; ++j) fluxB[j][kb - b0] = sv[j];
-            if (kb == b0 || bcp != bcl) bS[bcl] = (uint16_t)(kb - b0);
-            if (kb == b1 - 1 || bcn != bcl) bE[bcl] = (uint16_t)(kb - b0 + 1);
+#pragma unroll
+        for (int x = 0; x < XE; ++x)
+            if (fits && ke + x * THREADS < e1)
+                ein[x] = op.eload(ke + x * THREADS, er[x].f, er[x].o, c0 + er[x].c, xg);
+        if (hasB) bin = op.bload(br.f, c0 + br.c);
+#pragma unroll
+        for (int x = 0; x < XE; ++x)
+            if (fits && ke + x * THREADS < e1) put_ext(ke + x * THREADS, er[x], ein[x]);
+        if (hasB) put_bnd(kb, br, bin);
+        if constexpr (XE > 1) {  // the few records past those
+            for (int k = ke + XE * THREADS; fits && k < e1; k += THREADS) {
+                const Rec r = record(k);
+                put_ext(k, r, op.eload(k, r.f, r.o, c0 + r.c, xg));
+            }
+            for (int k = kb + THREADS; fits && k < b1; k += THREADS) {
+                const Rec r = brecord(k);
+                put_bnd(k, r, op.bload(r.f, c0 + r.c));
+            }
         }
     };
     // One pass over this thread's kUL own faces from i0 (nUp > 0).  The loads
@@ -660,7 +692,7 @@ Split split_of(const fv_mesh* m) {
             m->lowFace.p, m->lowOwn.p, m->bOff.p,     m->bFace.p};
 }
 
-template <typename S, typename Op, int CELLS, int THREADS>
+template <typename S, typename Op, int CELLS, int THREADS, int XE = 1>
 void launch_gather_t(fv_ctx* ctx, const fv_mesh* m, const Op& op, const S* V, S coeff, S* out) {
     const int nBlocks = (m->nCells + CELLS - 1) / CELLS;
     // the lists are built once per mesh and workgroup size (a cache on the mesh)
@@ -672,7 +704,7 @@ void launch_gather_t(fv_ctx* ctx, const fv_mesh* m, const Op& op, const S* V, S 
         xg = {gl.exW.p, gl.exMagSf.p, gl.exNodc.p, gl.exSf.p};
     else
         xg = {gl.exW32.p, gl.exMagSf32.p, gl.exNodc32.p, gl.exSf32.p};
-    k_gather<S, Op, CELLS, THREADS><<<gather_grid(nBlocks, m->gatherRun), THREADS, 0, ctx->stream>>>(
+    k_gather<S, Op, CELLS, THREADS, XE><<<gather_grid(nBlocks, m->gatherRun), THREADS, 0, ctx->stream>>>(
         m->nCells, nBlocks, m->gatherRun, split_of(m), L, xg, op, V, coeff, out);
     FV_LAUNCH_CHECK();
 }
@@ -695,7 +727,12 @@ void launch_gather(fv_ctx* ctx, const fv_mesh* m, const Op& op, const S* V, S co
     switch (cells) {
         case 1024: launch_gather_t<S, Op, 1024, 512>(ctx, m, op, V, coeff, out); break;
         case 512: launch_gather_t<S, Op, 512, 512>(ctx, m, op, V, coeff, out); break;
-        default: launch_gather_t<S, Op, 256, 256>(ctx, m, op, V, coeff, out); break;
+        default:
+            if (gather_wide(gather_lists(const_cast<fv_mesh*>(m), 256, sizeof(S) == 4)))
+                launch_gather_t<S, Op, 256, 256, 2>(ctx, m, op, V, coeff, out);
+            else
+                launch_gather_t<S, Op, 256, 256>(ctx, m, op, V, coeff, out);
+            break;
     }
 }
 

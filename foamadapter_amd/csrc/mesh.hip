@@ -304,7 +304,7 @@ const GatherLists& gather_lists(fv_mesh* m, int cells, bool f32) {
     const int64_t nBlocks = (N + cells - 1) / cells;
     std::vector<int32_t> eo(nBlocks + 1, 0), ef, ew, bo(nBlocks + 1, 0), bf;
     std::vector<uint16_t> ec, bc;
-    int64_t nOverflow = 0;
+    int64_t nOverflow = 0, nOverflowWide = 0;
     for (int64_t blk = 0; blk < nBlocks; ++blk) {
         const int64_t c0 = blk * cells, c1 = std::min<int64_t>(c0 + cells, N);
         int innerMax = 0;
@@ -324,14 +324,16 @@ const GatherLists& gather_lists(fv_mesh* m, int cells, bool f32) {
         }
         eo[blk + 1] = (int32_t)ef.size();
         bo[blk + 1] = (int32_t)bf.size();
-        const bool fits = ownStart[c1] - ownStart[c0] <= gather_max_up(cells) &&
-                          eo[blk + 1] - eo[blk] <= gather_max_ext(cells) &&
-                          bo[blk + 1] - bo[blk] <= gather_max_bnd(cells) &&
+        const int32_t nE = eo[blk + 1] - eo[blk];
+        const int32_t nB = bo[blk + 1] - bo[blk];
+        const bool rest = ownStart[c1] - ownStart[c0] <= gather_max_up(cells) &&
                           innerMax <= gather_max_low(cells);
-        nOverflow += fits ? 0 : 1;
+        nOverflow += rest && nE <= gather_max_ext(cells) && nB <= gather_max_bnd(cells) ? 0 : 1;
+        nOverflowWide += rest && nE <= gather_wide_ext() && nB <= gather_wide_bnd() ? 0 : 1;
     }
     L.nBlocks = nBlocks;
     L.nOverflow = nOverflow;
+    L.nOverflowWide = nOverflowWide;
     L.nExt = (int64_t)ef.size();
     // the zero records past the last block
     ef.push_back(0);
@@ -615,7 +617,7 @@ int fv_mesh_gather_stats(fv_mesh* m, int cells, int64_t* counts2) {
         FV_REQUIRE(m->upperTri, "the staged gather needs upper-triangular face order");
         const GatherLists& L = gather_lists(m, cells);
         counts2[0] = L.nBlocks;
-        counts2[1] = L.nOverflow;
+        counts2[1] = gather_wide(L) ? L.nOverflowWide : L.nOverflow;
     });
 }
 

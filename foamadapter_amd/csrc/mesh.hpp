@@ -48,6 +48,7 @@ struct GatherLists {
     // than gather_max_low lower faces from inside the workgroup): they take the
     // per-cell path, same bits, slower
     int64_t nBlocks = 0, nOverflow = 0;
+    int64_t nOverflowWide = 0;  // the same for the wide form (256 cells only)
 };
 
 // LDS capacities of the staged gather for a CELLS-cell workgroup (faces owned,
@@ -60,6 +61,12 @@ struct GatherLists {
 // boundary list holds CELLS/2, so corner and edge bricks stay on the fast path.
 constexpr int gather_max_up(int cells) { return cells * 3 + cells / 4; }
 constexpr int gather_max_ext(int cells) { return cells < 512 ? cells : 512; }
+// The wide form of the 256-cell workgroup, for meshes numbered in lines (a block
+// mesher's order): 256 consecutive cells have up to 256 lower faces to the plane
+// before, as many to the line before and one to the cell before; those of the
+// first and last planes have 256 boundary faces and a few at the lines' ends.
+constexpr int gather_wide_ext() { return 2 * 256 + 16; }
+constexpr int gather_wide_bnd() { return 256 + 32; }
 constexpr int gather_max_bnd(int cells) { return cells / 2; }
 // Inner lower faces per cell: 8 (a hex cell has 3; polyhedra up to 8), 4 for
 // 1024-cell workgroups, whose LDS then fits four workgroups per CU (a mesh with
@@ -111,6 +118,14 @@ const GatherLists& gather_lists(fv_mesh* m, int cells, bool f32 = false);
 // order, or forced by fv_mesh_set_gather); kDefaultGatherCells stands for the
 // per-operator default of the staged gather (its Op::kDefaultCells).
 constexpr int kDefaultGatherCells = 512;
+// Whether the 256-cell workgroups run in their wide form: where more than 1 % of
+// them would take the per-cell path otherwise (97x83x61 cells in block order, FP64,
+// per-cell path -> wide form: gradient 34.6 -> 23.6 us, linear divergence 25.5 ->
+// 16.4, upwind 17.7 -> 14.4, laplacian 32.7 -> 19.0).  The larger lists cost a
+// workgroup per CU, so meshes that do without them keep the default.
+inline bool gather_wide(const GatherLists& L) {
+    return L.cells == 256 && L.nOverflow * 100 > L.nBlocks && L.nOverflowWide < L.nOverflow;
+}
 inline int gather_cells(const fv_mesh* m) {
     if (!m->upperTri) return 0;
     switch (m->gatherMode) {

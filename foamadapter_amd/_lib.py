@@ -74,6 +74,12 @@ class FvSolveOpts(C.Structure):
                 ("check_every", C.c_int32), ("abs_tol", C.c_double), ("eager", C.c_int32)]
 
 
+class FvTerm(C.Structure):
+    _fields_ = [("kind", C.c_int32), ("scheme", C.c_int32), ("coeff", C.c_double),
+                ("dt", C.c_double), ("field", C.c_void_p), ("bc", C.c_void_p),
+                ("d_Tb", C.c_void_p), ("d_Tg", C.c_void_p)]
+
+
 class FvSolverStats(C.Structure):
     _fields_ = [("init_res", C.c_double), ("final_res", C.c_double), ("iters", C.c_int32),
                 ("outer_iters", C.c_int32), ("true_res", C.c_double)]
@@ -138,6 +144,7 @@ _SIGS = {
     "fv_assemble_ddt_euler": [_vp, _vp, _d, _d],
     "fv_assemble_source": [_vp, _vp, _d],
     "fv_assemble_explicit": [_vp, _vp, _d],
+    "fv_assemble_terms": [_vp, C.POINTER(FvTerm), C.c_int, C.c_int, _vp, C.POINTER(C.c_int)],
     "fv_assemble_laplacian": [_vp, _vp, _vp, _vp, _vp, _d],
     "fv_assemble_div": [_vp, C.c_int, _vp, _vp, _vp, _vp, _d],
     "fv_assemble_ddt_laplacian": [_vp, _vp, _d, _vp, _vp, _vp, _vp, _d],

@@ -136,4 +136,30 @@ inline int gather_cells(const fv_mesh* m) {
         default: return kDefaultGatherCells;
     }
 }
+
+// Sorts 8 (or 4) keys ascending in registers: the 19-comparator network for 8
+// inputs, layers (0,2)(1,3)(4,6)(5,7) / (0,4)(1,5)(2,6)(3,7) /
+// (0,1)(2,3)(4,5)(6,7) / (2,4)(3,5) / (1,4)(3,6) / (1,2)(3,4)(5,6); the
+// 5-comparator one for 4, (0,1)(2,3) / (0,2)(1,3) / (1,2).
+template <int K>
+__device__ inline void sort_keys(uint16_t (&k)[K]) {
+    static_assert(K == 8 || K == 4, "per-cell lower-face lists hold 8 or 4 entries");
+    auto cx = [&](int a, int b) {
+        const uint16_t x = k[a], y = k[b];
+        k[a] = x < y ? x : y;
+        k[b] = x < y ? y : x;
+    };
+    if constexpr (K == 8) {
+        cx(0, 2); cx(1, 3); cx(4, 6); cx(5, 7);
+        cx(0, 4); cx(1, 5); cx(2, 6); cx(3, 7);
+        cx(0, 1); cx(2, 3); cx(4, 5); cx(6, 7);
+        cx(2, 4); cx(3, 5);
+        cx(1, 4); cx(3, 6);
+        cx(1, 2); cx(3, 4); cx(5, 6);
+    } else {
+        cx(0, 1); cx(2, 3);
+        cx(0, 2); cx(1, 3);
+        cx(1, 2);
+    }
+}
 }  // namespace fvhip

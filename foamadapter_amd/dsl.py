@@ -11,11 +11,12 @@ field's old-time copy, which solve() refreshes after each solve.
 """
 from __future__ import annotations
 
+import ctypes as C
 from dataclasses import dataclass, field
 
 import numpy as np
 
-from ._lib import FV_LINEAR, FV_UPWIND, call, lib
+from ._lib import FV_LINEAR, FV_UPWIND, FvTerm, call, lib
 from . import fvcc
 from .la import LinearSystem, SparsityPattern, SolverStats, solve_cg
 from .runtime import DeviceArray
@@ -128,6 +129,45 @@ def _on_component(expr: Expression, psi, psi_k) -> Expression:
                        for t in expr.terms])
 
 
+_TERM_KINDS = {"ddt": 0, "div": 1, "laplacian": 2, "source": 3, "exp_div": 4}
+
+
+def _assemble_fused(expr: Expression, psi: fvcc.VolumeField, dt: float, ls: LinearSystem,
+                    rhs3: DeviceArray | None = None) -> bool:
+    """The whole equation in one pass (fv_assemble_terms); False when the library
+    has none for its terms, which are then assembled one by one."""
+    terms = (FvTerm * max(len(expr.terms), 1))()
+    for i, tm in enumerate(expr.terms):
+        k = _TERM_KINDS.get(tm.kind)
+        if k is None or (tm.kind == "exp_div" and tm.args[1] is not None):
+            return False
+        t = terms[i]
+        t.kind, t.coeff = k, tm.coeff
+        if k == 0:
+            if tm.args[0] is not psi:
+                return False
+            if psi.old_time is None:
+                psi.old_time = fvcc.VolumeField(psi.mesh, _copy(psi.internal), None)
+            t.field, t.dt = psi.old_time.internal.ptr.value, float(dt)
+            continue
+        a, f = tm.args
+        if k == 3:
+            t.field = (a.internal if isinstance(a, fvcc.VolumeField) else a).ptr.value
+            continue
+        t.field = a.values.ptr.value
+        if k < 3:
+            if psi.ncomp > 1 and f is not psi:  # another field's boundary arrays are not [B, 3]
+                return False
+            t.scheme = FV_UPWIND if tm.scheme == "upwind" else FV_LINEAR
+            t.bc = f.bcs.handle.value
+            t.d_Tb = f.boundary.ptr.value
+            t.d_Tg = f.boundary_gradient.ptr.value if f.boundary_gradient is not None else None
+    done = C.c_int()
+    call("fv_assemble_terms", ls.handle, terms, len(expr.terms), psi.ncomp, _ptr_or_none(rhs3),
+         C.byref(done))
+    return bool(done.value)
+
+
 def assemble(expr: Expression, psi: fvcc.VolumeField, t: float, dt: float,
              ls: LinearSystem | None = None) -> LinearSystem:
     """Expression::assemble(t, dt, sparsity, ls) (expression.hpp:69-73).
@@ -143,6 +183,8 @@ def assemble(expr: Expression, psi: fvcc.VolumeField, t: float, dt: float,
     mesh = psi.mesh
     ctx = mesh.ctx
     ls = ls or _linsys(mesh)
+    if _assemble_fused(expr, psi, dt, ls):
+        return ls
     ls.zero()
     tmp = None
     for term in expr.terms:
@@ -186,6 +228,9 @@ def _assemble_vec(expr, psi, t, dt, ls):
     if psi.old_time is None and any(tm.kind == "ddt" for tm in expr.terms):
         psi.old_time = fvcc.VolumeField(mesh, _copy(psi.internal), None)
     rhs3 = ctx.empty((mesh.n_cells, psi.ncomp))
+    if psi.ncomp == 3 and _assemble_fused(expr, psi, dt, ls, rhs3):
+        ls.rhs3 = rhs3
+        return ls
     rhs = ctx.empty((mesh.n_cells,))
     for k in reversed(range(psi.ncomp)):          # component 0 last: its system stays in ls
         pk = psi.component(k)

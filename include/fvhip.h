@@ -323,6 +323,32 @@ int fv_assemble_source(fv_linsys* ls, const void* d_coeff_field, double coeff);
  * the equation (dsl::exp terms of an Expression, neoIcoFoam.cpp:145):
  * rhs -= coeff*E*V. */
 int fv_assemble_explicit(fv_linsys* ls, const void* d_E, double coeff);
+/* The terms of one equation in one pass (dsl::Expression assembled as a whole,
+ * expression.hpp:69-73): what fv_linsys_zero and the single-term calls give in the
+ * order of the list, the same bits, with ncomp = 3 the three right-hand sides of a
+ * Vec3 equation in d_rhs3 ([N, 3], fields [N, 3] and boundary arrays [B, 3]
+ * interleaved; the system's own rhs and boundary coefficients hold component 0).
+ * Sets *done = 1, or to 0 and leaves the system alone when it has no such pass
+ * for the list: it takes ddt, div, laplacian, source and explicit div (the
+ * surfaceIntegrate of a face flux, subtracted as fv_assemble_explicit does; not
+ * beside div nor for three components) in this order, each at most once, with a div
+ * or laplacian among them, both of one field, on a mesh in upper-triangular order. */
+enum {
+    FV_TERM_DDT_EULER = 0,    /* field: T_old; dt              */
+    FV_TERM_DIV = 1,          /* field: phi; scheme, bc, Tb, Tg */
+    FV_TERM_LAPLACIAN = 2,    /* field: gamma; bc, Tb, Tg       */
+    FV_TERM_SOURCE = 3,       /* field: coefficients [N]        */
+    FV_TERM_EXPLICIT_DIV = 4, /* field: phi                     */
+};
+typedef struct {
+    int32_t kind, scheme;
+    double coeff, dt;
+    const void* field;
+    const fv_bc* bc;
+    const void *d_Tb, *d_Tg;  /* boundary values; boundary gradients or NULL */
+} fv_term;
+int fv_assemble_terms(fv_linsys* ls, const fv_term* terms, int n, int ncomp, void* d_rhs3,
+                      int* done);
 /* LaplacianOperator(Implicit, gamma, T, "Gauss linear uncorrected").implicitOperation(ls)
  * (test_implicitOperators.cpp:242-249): off-diagonals coeff*gamma|Sf|nonOrthDeltaCoeffs,
  * diagonal minus their sum, boundary faces folded into diag/rhs. */

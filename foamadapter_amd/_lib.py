@@ -153,8 +153,10 @@ _SIGS = {
     "fv_residual": [_vp, _vp, _vp],
     "fv_compute_rau": [_vp, _vp, _vp],
     "fv_compute_hbya": [_vp, _vp, _vp, _vp, _vp, _vp],
+    "fv_compute_rau_hbya": [_vp, _vp, _vp, _vp, _vp, _vp, _vp],
     "fv_update_face_velocity": [_vp, _vp, _vp, _vp],
     "fv_update_velocity": [_vp, _vp, _vp, _vp, _vp, _vp],
+    "fv_update_velocity_grad": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, C.POINTER(C.c_int)],
     "fv_constrain_hbya": [_vp, _vp, _vp],
     "fv_linsys_boundary_coeffs": [_vp, C.POINTER(_vp), C.POINTER(_vp)],
     "fv_courant_number": [_vp, _vp, _vp, _d, C.POINTER(_d)],

@@ -10,6 +10,8 @@ is passed alongside as a [N, 3] device array.
 """
 from __future__ import annotations
 
+import ctypes as C
+
 from . import fvcc
 from ._lib import call
 from .la import LinearSystem
@@ -32,11 +34,11 @@ def computeRAUandHByA(ls: LinearSystem, b3: DeviceArray, U: fvcc.VolumeField
     sum runs in ascending face order (no atomics), boundary values extrapolated."""
     m = ls.mesh
     ctx = m.ctx
-    rAU = computeRAU(ls)
+    rau, raub = ctx.empty((m.n_cells,)), ctx.empty((m.n_boundary_faces,))
     h = ctx.empty((m.n_cells, 3))
     hb = ctx.empty((m.n_boundary_faces, 3))
-    call("fv_compute_hbya", ls.handle, b3.ptr, U.internal.ptr, rAU.internal.ptr, h.ptr, hb.ptr)
-    return rAU, fvcc.VolumeField(m, h, hb, None, "HbyA")
+    call("fv_compute_rau_hbya", ls.handle, b3.ptr, U.internal.ptr, rau.ptr, raub.ptr, h.ptr, hb.ptr)
+    return fvcc.VolumeField(m, rau, raub, None, "rAU"), fvcc.VolumeField(m, h, hb, None, "HbyA")
 
 
 def constrainHbyA(U: fvcc.VolumeField, p: fvcc.VolumeField | None, hByA: fvcc.VolumeField):
@@ -56,6 +58,11 @@ def updateVelocity(hByA: fvcc.VolumeField, rAU: fvcc.VolumeField, p: fvcc.Volume
                    U: fvcc.VolumeField):
     """U = HbyA - rAU grad(p) (:197-211)."""
     m = U.mesh
+    done = C.c_int()
+    call("fv_update_velocity_grad", m.ctx.handle, m.handle, hByA.internal.ptr, rAU.internal.ptr,
+         p.internal.ptr, p.boundary.ptr, U.internal.ptr, C.byref(done))
+    if done.value:
+        return
     gradP = fvcc.GaussGreenGrad(m.ctx, m).grad(p)
     call("fv_update_velocity", m.ctx.handle, m.handle, hByA.internal.ptr, rAU.internal.ptr,
          gradP.ptr, U.internal.ptr)

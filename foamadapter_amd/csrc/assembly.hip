@@ -15,7 +15,11 @@
 //
 // The sums of every term run over the cell's faces in the order of the single-term
 // kernels of implicit.hip and the terms are added in the equation's order, so the
-// values are the same bits.  Workgroups whose faces do not fit the LDS lists take
+// values are the same bits.  150x140x130 cells: the momentum matrix with its three
+// right-hand sides 2.1 ms term by term -> 151 us (718 MB at least: 4.8 TB/s), the
+// pressure equation with its explicit divergence 390 -> 107 us (520 MB); 194 and 150
+// before the rows went through LDS and the bricks were dealt to the XCDs in runs.
+// Workgroups whose faces do not fit the LDS lists take
 // the same walk with the coefficients recomputed per cell.
 #include <type_traits>
 
@@ -48,7 +52,7 @@ struct Terms {
 };
 
 struct MeshIn {
-    int N, F, nBlocks;
+    int N, F, nBlocks, run;
     const int32_t *nbr, *ownStart, *lowOff, *lowFace, *bOff, *bFace, *rowOffs;
     const double *V, *w, *magSf, *nodc, *magSfb, *dcb;
     // lists of the staged gather, 256 cells per workgroup
@@ -77,7 +81,13 @@ __global__ __launch_bounds__(kCells) void k_assemble(MeshIn m, Terms t, Out o) {
     __shared__ uint16_t exS[kCells], exE[kCells], lowL[kMaxLow][kCells];
     __shared__ int lowN[kCells];
     __shared__ int overflow;
-    const int tid = (int)threadIdx.x, lb = (int)blockIdx.x;
+    // the workgroup's rows, one contiguous range of the matrix: written by the cells'
+    // threads entry by entry here, and from here with consecutive lanes on
+    // consecutive entries (kRows entries fit, 8 per row; more are written directly)
+    constexpr int kRows = 8 * kCells;
+    __shared__ double rows[kRows];
+    const int tid = (int)threadIdx.x, lb = brick_of((int)blockIdx.x, m.run);
+    if (lb >= m.nBlocks) return;
     const int c0 = lb * kCells, c1 = min(c0 + kCells, m.N), c = c0 + tid;
     const int fs = m.ownStart[c0], nF = m.ownStart[c1] - fs;
     const int e0 = m.extOff[lb], e1 = m.extOff[lb + 1];
@@ -118,97 +128,99 @@ __global__ __launch_bounds__(kCells) void k_assemble(MeshIn m, Terms t, Out o) {
         if (LAP) v[kL] = a.nodc * (a.gamma * a.magSf);
         if (EDIV) v[kE] = a.ephi;
     };
-    for (int l = tid; l < kCells; l += kCells) {
-        exS[l] = exE[l] = 0;
-        lowN[l] = 0;
+    auto eload = [&](int k, int f) {
+        In a{};
+        if (DIV) {
+            a.phi = t.phi[f];
+            if (t.scheme == FV_LINEAR) a.w = m.exW[k];
+        }
+        if (LAP) {
+            a.gamma = t.gamma[f];
+            a.magSf = m.exMagSf[k];
+            a.nodc = m.exNodc[k];
+        }
+        if (EDIV) a.ephi = t.ephi[f];
+        return a;
+    };
+    auto eput = [&](int k, int cl, int cp, int cn, const In& a) {
+        double v[NV];
+        make(a, v);
+#pragma unroll
+        for (int j = 0; j < NV; ++j) fE[j][k - e0] = v[j];
+        if (k == e0 || cp != cl) exS[cl] = (uint16_t)(k - e0);
+        if (k == e1 - 1 || cn != cl) exE[cl] = (uint16_t)(k - e0 + 1);
+    };
+    // the list records and the first pass's faces are loaded before the barrier
+    int ef[XE], ec[XE], ep[XE], en[XE];
+#pragma unroll
+    for (int x = 0; x < XE; ++x) {
+        const int k = min(e0 + tid + x * kCells, e1);  // at most the zero record past the lists
+        ef[x] = m.extFace[k];
+        ec[x] = m.extCell[k];
+        ep[x] = m.extCell[max(k - 1, e0)];
+        en[x] = m.extCell[max(min(k + 1, e1 - 1), e0)];
     }
+    const int nUp = fits ? nF : 0;
+    int nn[kUL];
+    In fin[kUL];
+    auto own_load = [&](int i0) {
+#pragma unroll
+        for (int q = 0; q < kUL; ++q) nn[q] = m.nbr[fs + min(i0 + q * kCells, nUp - 1)];
+#pragma unroll
+        for (int q = 0; q < kUL; ++q) fin[q] = load(fs + min(i0 + q * kCells, nUp - 1));
+    };
+    auto own_put = [&](int i0) {
+#pragma unroll
+        for (int q = 0; q < kUL; ++q) {
+            const int i = i0 + q * kCells;
+            if (i >= nUp) break;
+            double v[NV];
+            make(fin[q], v);
+#pragma unroll
+            for (int j = 0; j < NV; ++j) fU[j][i] = v[j];
+            if (nn[q] < c1) {
+                const int nl = nn[q] - c0;
+                const int s = atomicAdd(&lowN[nl], 1);
+                if (s < kMaxLow)
+                    lowL[s][nl] = (uint16_t)i;
+                else
+                    overflow = 1;
+            }
+        }
+    };
+    if (nUp > 0) own_load(tid);
+    In ein[XE];
+#pragma unroll
+    for (int x = 0; x < XE; ++x)
+        if (fits && e0 + tid + x * kCells < e1) ein[x] = eload(e0 + tid + x * kCells, ef[x]);
+    exS[tid] = exE[tid] = 0;
+    lowN[tid] = 0;
     if (tid == 0) overflow = fits ? 0 : 1;
     __syncthreads();
     if (fits) {
-        // external lower faces: XE records per thread at once
-        int ef[XE], ec[XE], ep[XE], en[XE];
-        In ein[XE];
 #pragma unroll
-        for (int x = 0; x < XE; ++x) {
-            const int k = min(e0 + tid + x * kCells, e1);  // at most the zero record past the lists
-            ef[x] = m.extFace[k];
-            ec[x] = m.extCell[k];
-            ep[x] = m.extCell[max(k - 1, e0)];
-            en[x] = m.extCell[max(min(k + 1, e1 - 1), e0)];
-        }
-        auto eload = [&](int k, int f) {
-            In a{};
-            if (DIV) {
-                a.phi = t.phi[f];
-                if (t.scheme == FV_LINEAR) a.w = m.exW[k];
-            }
-            if (LAP) {
-                a.gamma = t.gamma[f];
-                a.magSf = m.exMagSf[k];
-                a.nodc = m.exNodc[k];
-            }
-            if (EDIV) a.ephi = t.ephi[f];
-            return a;
-        };
-        auto eput = [&](int k, int cl, int cp, int cn, const In& a) {
-            double v[NV];
-            make(a, v);
-#pragma unroll
-            for (int j = 0; j < NV; ++j) fE[j][k - e0] = v[j];
-            if (k == e0 || cp != cl) exS[cl] = (uint16_t)(k - e0);
-            if (k == e1 - 1 || cn != cl) exE[cl] = (uint16_t)(k - e0 + 1);
-        };
-        bool first = true;
-        // own faces, kUL per thread and pass; the first pass also takes the lists
-        for (int i0 = tid; first || i0 < nF; i0 += kUL * kCells) {
-            int nn[kUL];
-            In fin[kUL];
-            if (nF > 0) {
-#pragma unroll
-                for (int q = 0; q < kUL; ++q) nn[q] = m.nbr[fs + min(i0 + q * kCells, nF - 1)];
-#pragma unroll
-                for (int q = 0; q < kUL; ++q) fin[q] = load(fs + min(i0 + q * kCells, nF - 1));
-            }
-            if (first) {
-                first = false;
-#pragma unroll
-                for (int x = 0; x < XE; ++x)
-                    if (e0 + tid + x * kCells < e1) ein[x] = eload(e0 + tid + x * kCells, ef[x]);
-#pragma unroll
-                for (int x = 0; x < XE; ++x)
-                    if (e0 + tid + x * kCells < e1)
-                        eput(e0 + tid + x * kCells, ec[x], ep[x], en[x], ein[x]);
-            }
-#pragma unroll
-            for (int q = 0; q < kUL; ++q) {
-                const int i = i0 + q * kCells;
-                if (i >= nF) break;
-                double v[NV];
-                make(fin[q], v);
-#pragma unroll
-                for (int j = 0; j < NV; ++j) fU[j][i] = v[j];
-                if (nn[q] < c1) {
-                    const int nl = nn[q] - c0;
-                    const int s = atomicAdd(&lowN[nl], 1);
-                    if (s < kMaxLow)
-                        lowL[s][nl] = (uint16_t)i;
-                    else
-                        overflow = 1;
-                }
-            }
+        for (int x = 0; x < XE; ++x)
+            if (e0 + tid + x * kCells < e1)
+                eput(e0 + tid + x * kCells, ec[x], ep[x], en[x], ein[x]);
+        own_put(tid);
+        for (int i0 = tid + kUL * kCells; i0 < nUp; i0 += kUL * kCells) {
+            own_load(i0);
+            own_put(i0);
         }
         if (XE > 1)
             for (int k = e0 + tid + XE * kCells; k < e1; k += kCells)
                 eput(k, m.extCell[k], m.extCell[max(k - 1, e0)], m.extCell[min(k + 1, e1 - 1)],
                      eload(k, m.extFace[k]));
     }
+    const int rbase = m.rowOffs[c0], rn = m.rowOffs[c1] - rbase;
+    const bool staged = rn <= kRows;
     __syncthreads();
-    if (c >= c1) return;
+    if (c < c1) {
 
     double dDiv = 0.0, dLap = 0.0, acc = 0.0, bDiv[NC], bLap[NC];
 #pragma unroll
     for (int k = 0; k < NC; ++k) bDiv[k] = bLap[k] = 0.0;
-    double* out = o.values + row;
+    double* out = staged ? rows + (row - rbase) : o.values + row;
     auto entry = [&](double cd, double cl) {
         double x = 0.0;
         if (DIV) x += t.cDiv * cd;
@@ -310,6 +322,10 @@ __global__ __launch_bounds__(kCells) void k_assemble(MeshIn m, Terms t, Out o) {
         if (q == 0) o.rhs[c] = r;
         if (NC > 1) o.rhs3[(int64_t)NC * c + q] = r;
     }
+    }
+    if (!staged) return;
+    __syncthreads();
+    for (int i = tid; i < rn; i += kCells) o.values[rbase + i] = rows[i];
 }
 
 }  // namespace
@@ -370,7 +386,7 @@ extern "C" int fv_assemble_terms(fv_linsys* ls, const fv_term* terms, int n, int
         if (!(div || lap) || (ediv && (div || ncomp > 1))) return;
         const GatherLists& L = gather_lists(m, kCells);
         const fv_sparsity* sp = ls->sp;
-        const MeshIn in{m->nCells,   m->nInt,     (int)L.nBlocks, m->nbr.p,   m->ownStart.p,
+        const MeshIn in{m->nCells,   m->nInt,     (int)L.nBlocks, m->gatherRun, m->nbr.p,   m->ownStart.p,
                         m->lowOff.p, m->lowFace.p, m->bOff.p,     m->bFace.p, sp->rowOffs.p,
                         m->V.p,      m->w.p,       m->magSf.p,    m->nodc.p,  m->magSfb.p,
                         m->dcb.p,    L.extOff.p,   L.extFace.p,   L.extCell.p, L.exW.p,
@@ -383,9 +399,9 @@ extern "C" int fv_assemble_terms(fv_linsys* ls, const fv_term* terms, int n, int
                            kEd = decltype(E)::value;
             constexpr int kC = decltype(C)::value;
             if (wide)
-                k_assemble<kDiv, kLap, kEd, kC, 2><<<in.nBlocks, kCells, 0, s>>>(in, t, out);
+                k_assemble<kDiv, kLap, kEd, kC, 2><<<gather_grid(in.nBlocks, in.run), kCells, 0, s>>>(in, t, out);
             else
-                k_assemble<kDiv, kLap, kEd, kC, 1><<<in.nBlocks, kCells, 0, s>>>(in, t, out);
+                k_assemble<kDiv, kLap, kEd, kC, 1><<<gather_grid(in.nBlocks, in.run), kCells, 0, s>>>(in, t, out);
         };
         using Y = std::true_type;
         using X = std::false_type;

@@ -488,9 +488,8 @@ __global__ __launch_bounds__(kCgBlock) void kc_resid(const CgGrid<S>* __restrict
     if (!cg_locate(g, Pp, row0, row1, slot)) return;
     const CgSys<S>& P = *Pp;
     if (!START && P.st->stop != 1) return;
-    // a row's first kRE entries have their loads issued together (values and
-    // columns, then the gathers of x), as in the SpMV; same summation order
-    constexpr int kRE = 8;
+    __shared__ double prod[kCsrLds];
+    static_assert(kCgBlock == kCsrBlock, "one row per thread and block");
     const int32_t* __restrict__ ro = P.rowOffs;
     const int32_t* __restrict__ ci = P.colIdxs;
     const double* __restrict__ va = P.vals;
@@ -499,29 +498,24 @@ __global__ __launch_bounds__(kCgBlock) void kc_resid(const CgGrid<S>* __restrict
     double* __restrict__ r64 = P.r64;
     double rr = 0.0, bb = 0.0;
     const int r1 = min(row1, P.N);
-    for (int i = row0 + threadIdx.x; i < r1; i += kCgBlock) {
-        const int k0 = ro[i], k1 = ro[i + 1];
-        const double bi = rhs[i];
-        double v[kRE], xg[kRE];
-        int c[kRE];
-#pragma unroll
-        for (int k = 0; k < kRE; ++k)
-            if (k0 + k < k1) {
-                v[k] = va[k0 + k];
-                c[k] = ci[k0 + k];
-            }
-#pragma unroll
-        for (int k = 0; k < kRE; ++k)
-            if (k0 + k < k1) xg[k] = xv[c[k]];
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < kRE; ++k)
-            if (k0 + k < k1) s += v[k] * xg[k];
-        for (int k = k0 + kRE; k < k1; ++k) s += va[k] * xv[ci[k]];
-        const double ri = bi - s;
-        r64[i] = ri;
-        rr += ri * ri;
-        bb += bi * bi;
+    for (int i0 = row0; i0 < r1; i0 += kCgBlock) {
+        const int i = i0 + (int)threadIdx.x, ic = min(i, r1 - 1);
+        const int k0 = ro[ic], k1 = ro[ic + 1], base = ro[i0];
+        const double bi = rhs[ic];
+        const bool staged = csr_products(ro, ci, va, xv, i0, min(i0 + kCgBlock, r1), prod);
+        __syncthreads();
+        if (i < r1) {
+            double s = 0.0;
+            if (staged)
+                for (int k = k0; k < k1; ++k) s += prod[k - base];
+            else
+                for (int k = k0; k < k1; ++k) s += va[k] * xv[ci[k]];
+            const double ri = bi - s;
+            r64[i] = ri;
+            rr += ri * ri;
+            bb += bi * bi;
+        }
+        __syncthreads();
     }
     double v[2] = {rr, bb};
     write_slot<2>(v, red.rb, slot, sh);

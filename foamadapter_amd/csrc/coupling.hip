@@ -49,65 +49,85 @@ __global__ __launch_bounds__(kBlock) void k_rau(int N, int B, const int32_t* __r
 }
 
 // HbyA_c = (b_c - sum_f A(c, other) U_other) * rAU_c / V_c, the sum in ascending
-// face order starting from zero (H is accumulated, then b added)
-__global__ __launch_bounds__(kBlock) void k_hbya(int N, int F, const int32_t* __restrict__ off,
-                                                 const int32_t* __restrict__ idx,
-                                                 const int32_t* __restrict__ oth,
-                                                 const int32_t* __restrict__ slot,
-                                                 const int32_t* __restrict__ rowOffs,
+// face order starting from zero (H is accumulated, then b added).  The columns of
+// a row ascend in that order, so the row is walked without the stencil: the block's
+// values and columns go through LDS (see csr_products), and a row's neighbour
+// velocities are loaded kE entries at a time.  RAU: rAU = V / diag(A) is computed
+// here too and written.
+template <bool RAU>
+__global__ __launch_bounds__(kBlock) void k_hbya(int N, const int32_t* __restrict__ rowOffs,
+                                                 const int32_t* __restrict__ cols,
+                                                 const int32_t* __restrict__ diag,
                                                  const double* __restrict__ values,
                                                  const double* __restrict__ b3,
                                                  const double* __restrict__ U,
-                                                 const double* __restrict__ rau,
                                                  const double* __restrict__ V,
+                                                 double* __restrict__ rau,
                                                  double* __restrict__ hbya) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= N) return;
-    const int row = rowOffs[c];
-    double h0 = 0.0, h1 = 0.0, h2 = 0.0;
-    const int k0 = off[c], e1 = off[c + 1];
-    // the first kE stencil entries: indices, then their coefficients and the
-    // neighbours' velocities, loaded in two rounds before the sums, which run
-    // in stencil order (boundary faces carry no off-diagonal)
-    constexpr int kE = 8;
-    int ie[kE], oe[kE], se[kE];
+    static_assert(kBlock == kCsrBlock, "one row per thread");
+    __shared__ double va[kCsrLds];
+    __shared__ int32_t co[kCsrLds];
+    const int i0 = blockIdx.x * kBlock, i1 = min(i0 + kBlock, N);
+    const int c = i0 + (int)threadIdx.x, cc = min(c, N - 1);
+    const int base = rowOffs[i0], n = rowOffs[i1] - base;
+    const int k0 = rowOffs[cc] - base, k1 = rowOffs[cc + 1] - base, dg = k0 + diag[cc];
+    const double vol = V[cc];
+    const int64_t i = 3 * (int64_t)cc;
+    const double q0 = b3[i], q1 = b3[i + 1], q2 = b3[i + 2];
+    const bool staged = n <= kCsrLds;
+    if (staged) {
+        const int t = (int)threadIdx.x;
+        double v[kCsrU];
+        int32_t w[kCsrU];
 #pragma unroll
-    for (int j = 0; j < kE; ++j)
-        if (k0 + j < e1) {
-            ie[j] = idx[k0 + j];
-            oe[j] = oth[k0 + j];
-            se[j] = slot[k0 + j];
+        for (int u = 0; u < kCsrU; ++u) {
+            const int k = base + min(t + u * kBlock, n - 1);
+            v[u] = values[k];
+            w[u] = cols[k];
         }
-    double av[kE], u0[kE], u1[kE], u2[kE];
 #pragma unroll
-    for (int j = 0; j < kE; ++j)
-        if (k0 + j < e1 && ie[j] < F) {
-            const int64_t o = 3 * (int64_t)oe[j];
-            av[j] = values[row + se[j]];
+        for (int u = 0; u < kCsrU; ++u)
+            if (t + u * kBlock < n) {
+                va[t + u * kBlock] = v[u];
+                co[t + u * kBlock] = w[u];
+            }
+    }
+    __syncthreads();
+    if (c >= N) return;
+    auto value = [&](int k) { return staged ? va[k] : values[base + k]; };
+    auto column = [&](int k) { return staged ? co[k] : cols[base + k]; };
+    double h0 = 0.0, h1 = 0.0, h2 = 0.0;
+    constexpr int kE = 7;
+    for (int k = k0; k < k1; k += kE) {
+        double a[kE], u0[kE], u1[kE], u2[kE];
+#pragma unroll
+        for (int j = 0; j < kE; ++j) {
+            const int kk = min(k + j, k1 - 1);
+            const int64_t o = 3 * (int64_t)column(kk);
+            a[j] = value(kk);
             u0[j] = U[o];
             u1[j] = U[o + 1];
             u2[j] = U[o + 2];
         }
 #pragma unroll
-    for (int j = 0; j < kE; ++j)
-        if (k0 + j < e1 && ie[j] < F) {
-            h0 -= av[j] * u0[j];
-            h1 -= av[j] * u1[j];
-            h2 -= av[j] * u2[j];
-        }
-    for (int k = k0 + kE; k < e1; ++k) {  // cells with more than kE faces
-        if (idx[k] >= F) continue;
-        const double a = values[row + slot[k]];
-        const int64_t o = 3 * (int64_t)oth[k];
-        h0 -= a * U[o];
-        h1 -= a * U[o + 1];
-        h2 -= a * U[o + 2];
+        for (int j = 0; j < kE; ++j)
+            if (k + j < k1 && k + j != dg) {
+                h0 -= a[j] * u0[j];
+                h1 -= a[j] * u1[j];
+                h2 -= a[j] * u2[j];
+            }
     }
-    const double s = rau[c] / V[c];
-    const int64_t i = 3 * (int64_t)c;
-    hbya[i] = (h0 + b3[i]) * s;
-    hbya[i + 1] = (h1 + b3[i + 1]) * s;
-    hbya[i + 2] = (h2 + b3[i + 2]) * s;
+    double ra;
+    if (RAU) {
+        ra = vol / value(dg);
+        rau[c] = ra;
+    } else {
+        ra = rau[c];
+    }
+    const double s = ra / vol;
+    hbya[i] = (h0 + q0) * s;
+    hbya[i + 1] = (h1 + q1) * s;
+    hbya[i + 2] = (h2 + q2) * s;
 }
 
 // boundary values of a cell field, extrapolated: out_b = in_P (ncomp components)
@@ -119,6 +139,20 @@ __global__ __launch_bounds__(kBlock) void k_extrapolate(int B, int ncomp,
     if (b >= B) return;
     const int64_t c = faceCells[b];
     for (int j = 0; j < ncomp; ++j) out[(int64_t)ncomp * b + j] = in[ncomp * c + j];
+}
+
+// the same for rAU and HbyA at once (either may be null)
+__global__ __launch_bounds__(kBlock) void k_extrapolate2(int B, const int32_t* __restrict__ faceCells,
+                                                         const double* __restrict__ rau,
+                                                         double* __restrict__ raub,
+                                                         const double* __restrict__ h,
+                                                         double* __restrict__ hb) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= B) return;
+    const int64_t c = faceCells[b];
+    if (raub) raub[b] = rau[c];
+    if (hb)
+        for (int j = 0; j < 3; ++j) hb[3 * (int64_t)b + j] = h[3 * c + j];
 }
 
 // phi_f = pred_f - (A(nbr,own) p_N - A(own,nbr) p_P); phi_b = pred_b - (bRhs - bMat p_P)
@@ -260,13 +294,31 @@ int fv_compute_hbya(fv_linsys* ls, const void* d_b3, const void* d_U, const void
         const fv_sparsity* sp = ls->sp;
         const fv_mesh* m = sp->mesh;
         hipStream_t s = m->ctx->stream;
-        k_hbya<<<grid_for(m->nCells, kBlock), kBlock, 0, s>>>(
-            m->nCells, m->nInt, m->cfOff.p, m->cfIdx.p, m->cfOther.p, sp->entrySlot.p,
-            sp->rowOffs.p, ls->values.p, (const double*)d_b3, (const double*)d_U,
-            (const double*)d_rau, m->V.p, (double*)d_hbya);
+        k_hbya<false><<<grid_for(m->nCells, kBlock), kBlock, 0, s>>>(
+            m->nCells, sp->rowOffs.p, sp->colIdxs.p, sp->diagOffset.p, ls->values.p,
+            (const double*)d_b3, (const double*)d_U, m->V.p, (double*)d_rau, (double*)d_hbya);
         if (d_hbya_b && m->nB)
             k_extrapolate<<<grid_for(m->nB, kBlock), kBlock, 0, s>>>(
                 m->nB, 3, m->faceCells.p, (const double*)d_hbya, (double*)d_hbya_b);
+        FV_LAUNCH_CHECK();
+    });
+}
+
+int fv_compute_rau_hbya(fv_linsys* ls, const void* d_b3, const void* d_U, void* d_rau,
+                        void* d_rau_b, void* d_hbya, void* d_hbya_b) {
+    return guarded([&] {
+        check_ls(ls);
+        FV_REQUIRE(d_b3 && d_U && d_rau && d_hbya, "NULL argument");
+        const fv_sparsity* sp = ls->sp;
+        const fv_mesh* m = sp->mesh;
+        hipStream_t s = m->ctx->stream;
+        k_hbya<true><<<grid_for(m->nCells, kBlock), kBlock, 0, s>>>(
+            m->nCells, sp->rowOffs.p, sp->colIdxs.p, sp->diagOffset.p, ls->values.p,
+            (const double*)d_b3, (const double*)d_U, m->V.p, (double*)d_rau, (double*)d_hbya);
+        if (m->nB && (d_rau_b || d_hbya_b))
+            k_extrapolate2<<<grid_for(m->nB, kBlock), kBlock, 0, s>>>(
+                m->nB, m->faceCells.p, (const double*)d_rau, (double*)d_rau_b,
+                (const double*)d_hbya, (double*)d_hbya_b);
         FV_LAUNCH_CHECK();
     });
 }

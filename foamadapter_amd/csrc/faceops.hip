@@ -182,17 +182,6 @@ __global__ __launch_bounds__(kBlock) void k_laplacian(
 // again, then ran shortly before on the same XCD and are still in its L2.
 // Measured at 256^3, runs of 8 cut the L2 misses of the gathers by 6-18% at
 // the same speed; run = 1 is the natural order.
-__device__ __forceinline__ int brick_of(int h, int run) {
-    if (run <= 1) return h;
-    const int x = h & 7, s = h >> 3;
-    return ((s / run) * 8 + x) * run + s % run;
-}
-inline int gather_grid(int nBlocks, int run) {
-    if (run <= 1) return nBlocks;
-    const int g = 8 * run;
-    return (nBlocks + g - 1) / g * g;
-}
-
 // LDS face slots of a CELLS-cell workgroup: 3 owned faces per hex cell plus slack;
 // faces beyond it (unusual meshes) are recomputed in phase 2
 template <int CELLS>
@@ -218,6 +207,10 @@ struct FaceOp {
     // workgroups: 3 beats 4 and 2 -- loads in flight against registers)
     static constexpr int kFacesPerPass = 3;
     __device__ const D& self() const { return *static_cast<const D*>(this); }
+    // what becomes of component j of cell c's result
+    __device__ void put(S* __restrict__ out, int c, int j, S r) const {
+        out[(int64_t)NC * c + j] = r;
+    }
     __device__ void face(int f, int o, int n, S* v) const { self().make(self().load(f, o, n), v); }
     __device__ void bface(int b, int c, S* v) const { self().bmake(self().bload(b, c), v); }
 };
@@ -258,6 +251,16 @@ struct GradOp : FaceOp<S, GradOp<S>, 3> {
         v[0] = a.sx * a.tb;
         v[1] = a.sy * a.tb;
         v[2] = a.sz * a.tb;
+    }
+};
+
+// U = HbyA - rAU * grad(p): the gradient is used where it arises instead of being
+// written and read back (48 bytes per cell; 150x140x130 cells 128 -> 97 us).
+struct VelocityOp : GradOp<double> {
+    const double *hbya, *rau;
+    __device__ void put(double* __restrict__ U, int c, int j, double g) const {
+        const int64_t i = 3 * (int64_t)c + j;
+        U[i] = hbya[i] - rau[c] * g;
     }
 };
 
@@ -387,7 +390,7 @@ __device__ inline void gather_cell(int c, int fs, int nUp, const Split& t, const
         op.bface(t.bFace[k], c, v);
         for (int j = 0; j < NC; ++j) acc[j] += v[j];
     }
-    for (int j = 0; j < NC; ++j) out[(int64_t)NC * c + j] = coeff * (acc[j] / vol);
+    for (int j = 0; j < NC; ++j) op.put(out, c, j, coeff * (acc[j] / vol));
 }
 
 struct Lists {
@@ -657,7 +660,7 @@ __global__ __launch_bounds__(THREADS) void k_gather(int N, int nBlocks, int run,
             for (int j = 0; j < NC; ++j) acc[j] += v[j];
         }
         const S vol = vols[q];
-        for (int j = 0; j < NC; ++j) out[(int64_t)NC * c + j] = coeff * (acc[j] / vol);
+        for (int j = 0; j < NC; ++j) op.put(out, c, j, coeff * (acc[j] / vol));
     }
 }
 
@@ -993,6 +996,23 @@ int fv_grad_gauss(fv_ctx* ctx, const fv_mesh* mc, fv_prec prec, double coeff, co
         else
             run_grad<float>(ctx, m, geo32(m), (const float*)T, (const float*)Tb, (float)coeff,
                             (float*)out);
+    });
+}
+
+int fv_update_velocity_grad(fv_ctx* ctx, const fv_mesh* mc, const void* d_hbya, const void* d_rau,
+                            const void* d_p, const void* d_pb, void* d_U, int* done) {
+    return guarded([&] {
+        fv_mesh* m = const_cast<fv_mesh*>(mc);
+        check_common(ctx, m, FV_F64);
+        FV_REQUIRE(d_hbya && d_rau && d_p && (d_pb || m->nB == 0) && d_U && done, "NULL argument");
+        *done = 0;
+        if (!gather_cells(m)) return;  // the stencil walk has no such form
+        const Geo<double> g = geo64(m);
+        launch_gather<double>(ctx, m,
+                              VelocityOp{{{}, (const double*)d_p, g.w, g.Sf, g.Sfb, (const double*)d_pb},
+                                         (const double*)d_hbya, (const double*)d_rau},
+                              g.V, 1.0, (double*)d_U);
+        *done = 1;
     });
 }
 

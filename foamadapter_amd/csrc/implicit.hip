@@ -359,19 +359,28 @@ __global__ void k_set_reference(const int32_t* __restrict__ rowOffs,
     }
 }
 
-// res = A.x - b, one thread per row, row entries summed in column order
+// res = A.x - b, a block of 256 rows per workgroup, row entries summed in column order
 __global__ __launch_bounds__(kBlock) void k_residual(int N, const int32_t* __restrict__ rowOffs,
                                                      const int32_t* __restrict__ col,
                                                      const double* __restrict__ values,
                                                      const double* __restrict__ b,
                                                      const double* __restrict__ x,
                                                      double* __restrict__ res) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    static_assert(kBlock == kCsrBlock, "one row per thread");
+    __shared__ double prod[kCsrLds];
+    const int i0 = blockIdx.x * kBlock, i1 = min(i0 + kBlock, N);
+    const int r = i0 + (int)threadIdx.x, rc = min(r, N - 1);
+    const int k0 = rowOffs[rc], k1 = rowOffs[rc + 1], base = rowOffs[i0];
+    const double bi = b[rc];
+    const bool staged = csr_products(rowOffs, col, values, x, i0, i1, prod);
+    __syncthreads();
     if (r >= N) return;
     double s = 0.0;
-    const int e = rowOffs[r + 1];
-    for (int k = rowOffs[r]; k < e; ++k) s += values[k] * x[col[k]];
-    res[r] = s - b[r];
+    if (staged)
+        for (int k = k0; k < k1; ++k) s += prod[k - base];
+    else
+        for (int k = k0; k < k1; ++k) s += values[k] * x[col[k]];
+    res[r] = s - bi;
 }
 
 fv_mesh* mesh_of(const fv_linsys* ls) { return ls->sp->mesh; }

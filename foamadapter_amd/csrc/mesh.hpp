@@ -137,6 +137,19 @@ inline int gather_cells(const fv_mesh* m) {
     }
 }
 
+// The brick of hardware block h when each XCD takes runs of `run` consecutive bricks
+// (see the staged gathers of faceops.hip), and the grid that covers nBlocks of them.
+__device__ __forceinline__ int brick_of(int h, int run) {
+    if (run <= 1) return h;
+    const int x = h & 7, s = h >> 3;
+    return ((s / run) * 8 + x) * run + s % run;
+}
+inline int gather_grid(int nBlocks, int run) {
+    if (run <= 1) return nBlocks;
+    const int g = 8 * run;
+    return (nBlocks + g - 1) / g * g;
+}
+
 // Sorts 8 (or 4) keys ascending in registers: the 19-comparator network for 8
 // inputs, layers (0,2)(1,3)(4,6)(5,7) / (0,4)(1,5)(2,6)(3,7) /
 // (0,1)(2,3)(4,5)(6,7) / (2,4)(3,5) / (1,4)(3,6) / (1,2)(3,4)(5,6); the

@@ -434,6 +434,9 @@ int fv_compute_rau(fv_linsys* ls, void* d_rau, void* d_rau_b);
  * values extrapolated into d_hbya_b [3B] (may be NULL). */
 int fv_compute_hbya(fv_linsys* ls, const void* d_b3, const void* d_U, const void* d_rau,
                     void* d_hbya, void* d_hbya_b);
+/* fv_compute_rau and fv_compute_hbya in one pass over the matrix (the same bits). */
+int fv_compute_rau_hbya(fv_linsys* ls, const void* d_b3, const void* d_U, void* d_rau,
+                        void* d_rau_b, void* d_hbya, void* d_hbya_b);
 /* updateFaceVelocity (:122-195) on the assembled pressure system ls:
  * phi_f = pred_f - (A(N,P) p_N - A(P,N) p_P) on internal faces and
  * phi_b = pred_b - (bRhs_b - bMat_b p_P) on boundary faces, where bMat/bRhs are
@@ -443,6 +446,11 @@ int fv_update_face_velocity(fv_linsys* ls, const void* d_phi_pred, const void* d
 /* updateVelocity (:197-211): U = HbyA - rAU * gradP (gradP from fv_grad_gauss). */
 int fv_update_velocity(fv_ctx* ctx, const fv_mesh* mesh, const void* d_hbya, const void* d_rau,
                        const void* d_gradp, void* d_U);
+/* fv_grad_gauss of p (d_pb: its boundary values) and fv_update_velocity with it in one
+ * pass (the same bits).  Sets *done = 1, or to 0 and does nothing on a mesh whose
+ * gradient runs as a stencil walk. */
+int fv_update_velocity_grad(fv_ctx* ctx, const fv_mesh* m, const void* d_hbya, const void* d_rau,
+                            const void* d_p, const void* d_pb, void* d_U, int* done);
 /* constrainHbyA (:14-36): HbyA_b = U_b on the faces of patches whose velocity
  * condition is not assignable (fixedValue); other faces keep their value. */
 int fv_constrain_hbya(const fv_bc* u_bc, const void* d_Ub, void* d_hbya_b);

@@ -47,10 +47,11 @@ def test_rows_by_blocks(ctx, name):
             s += va[k] * x[ci[k]]
         res[i] = s - b[i]
     assert np.array_equal(ls.residual(T.internal).numpy(), res)
-    # the solver's own, ||b - A x|| / ||b|| before its first iteration
+    # the solver's own, ||b - A x|| / ||b|| of a solve that may not iterate (the
+    # kernel-by-kernel form reads no state then and reports the final residual only)
     st = la.solve_cg(ls, T.internal, {"relTol": 1e-30, "maxIter": 0}, raise_on_noconverge=False)
     ref = np.linalg.norm(res) / np.linalg.norm(b)
-    assert abs(st.initResNorm - ref) <= 4 * N * 2.3e-16 * ref  # two sums of N squares
+    assert abs((st.initResNorm or st.trueResNorm) - ref) <= 4 * N * 2.3e-16 * ref  # two sums of N squares
 
     u3, b3 = ctx.uniform(3 * N, -1, 1, 3, 4), ctx.uniform(3 * N, -1, 1, 3, 5)
     u3.shape = b3.shape = (N, 3)

@@ -219,6 +219,17 @@ struct GridSum {
     int nslots;  // workgroups of the grid
     bool large;
 
+    // Takes this workgroup's place in a grid over `tiles` tiles and returns the tile
+    // of its part sub.
+    __device__ int place(int tiles, int sub) {
+        slot = (int)blockIdx.x;
+        nslots = (int)gridDim.x;
+        large = tiles > kCgBlock;
+        if (!large) return 64 * (slot >> 4) + (slot & 15) + 16 * sub;
+        const int x = slot & 7;
+        return 64 * (x >> 1) + 2 * (slot >> 3) + (x & 1) + kCgBlock * sub;
+    }
+
     __device__ static void publish(unsigned long long* s, double x, uint32_t tag) {
         const unsigned long long b = (unsigned long long)__double_as_longlong(x);
         put_shared(s, b << 32 | tag);
@@ -334,17 +345,8 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     GridSum gs;
     gs.slots = A.slots;
     gs.tag = A.tag0;
-    gs.slot = (int)blockIdx.x;
-    gs.nslots = (int)gridDim.x;
-    gs.large = A.tiles > kCgBlock;
     const int R = A.rowsPerTile;
-    int tile;  // see GridSum
-    if (gs.large) {
-        const int x = gs.slot & 7;
-        tile = 64 * (x >> 1) + 2 * (gs.slot >> 3) + (x & 1) + kCgBlock * sub;
-    } else {
-        tile = 64 * (gs.slot >> 4) + (gs.slot & 15) + 16 * sub;
-    }
+    const int tile = gs.place(A.tiles, sub);
     // this tile's rows [cbase, cbase + R) have their p in LDS, from lofs on
     const uint32_t cbase = (uint32_t)tile * R, lofs = (uint32_t)sub * (RPT * kCgBlock);
     CgState* const st = A.st;
@@ -573,6 +575,24 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
         st->done = 0;
         st->pbuf = 0;
     }
+}
+
+// Workgroups of a persistent launch over `tiles` tiles
+inline int persist_grid(int tiles) {
+    return tiles > kCgBlock ? kPersistGroups : 16 * (tiles / 64) + (tiles % 64 < 16 ? tiles % 64 : 16);
+}
+
+// Whether the device keeps the workgroups of such a launch resident together.
+inline bool persist_fits(const void* kernel, int device, int grid) {
+    int perCu = 0, cus = 0, coop = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, kernel, kPersistThreads, 0) !=
+            hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return coop && (int64_t)perCu * cus >= grid;
 }
 
 }  // namespace

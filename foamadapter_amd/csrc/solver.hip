@@ -115,17 +115,8 @@ struct CgWork : fv_solver_cache {
         else if (sp->sellWidth == 4)
             persist = persist_kernel<4>(rpt);
         if (!persist) return;
-        persistGrid = tiles > kCgBlock ? kPersistGroups
-                                       : 16 * (tiles / 64) + std::min(tiles % 64, 16);
-        int perCu = 0, cus = 0, coop = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, persist, kPersistThreads, 0) !=
-                hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) !=
-                hipSuccess ||
-            hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) !=
-                hipSuccess ||
-            !coop || (int64_t)perCu * cus < persistGrid) {
-            (void)hipGetLastError();
+        persistGrid = persist_grid(tiles);
+        if (!persist_fits(reinterpret_cast<const void*>(persist), c->device, persistGrid)) {
             persist = nullptr;
             return;
         }

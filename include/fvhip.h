@@ -392,11 +392,10 @@ typedef struct {
     int32_t check_every;  /* host polls the stop flag every this many iterations */
     double abs_tol;       /* also stop when ||r|| <= abs_tol (criteria absolute_residual_norm,
                              fvSolution.cpp:139-144); 0: off */
-    int32_t eager;        /* fv_solve_cg: 1 launches the kernels of every phase one by one;
-                             0 (default) runs many iterations in one persistent kernel
-                             where the system fits the chip, and else replays a repeated
-                             solve as a hipGraph once the same schedule repeats (same bits
-                             either way) */
+    int32_t eager;        /* 1 launches the kernels of every phase one by one; 0 (default)
+                             runs many iterations in one persistent kernel where the
+                             system fits the chip, and else (CG) replays a repeated solve
+                             as a hipGraph once the same schedule repeats (same bits) */
 } fv_solve_opts;
 typedef struct {
     double init_res;      /* SolverStats::initResNorm, relative */

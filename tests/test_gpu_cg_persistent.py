@@ -1,9 +1,9 @@
-"""The persistent CG kernel against the kernel-by-kernel form ("graph": False), bit for
+"""The persistent CG and BiCGStab kernels against the kernel-by-kernel form ("graph": False), bit for
 bit: both add every dot product in the same order, so the solutions, the iteration counts
 and the residuals are the same numbers.  The sizes sit at the edges of what the kernel
 distinguishes: tiles of 256 rows (the last one ragged), 64 workgroups of up to 256 tiles or
 256 workgroups beyond, 1, 2, 4 and 8 rows per thread, slices of 4 (plane meshes) and 6
-entries, and solves of several launches."""
+entries, and solves of several launches (for BiCGStab, solves that go on where a launch ended)."""
 import numpy as np
 import pytest
 
@@ -70,6 +70,42 @@ def test_persistent_is_bitwise_the_kernel_by_kernel_form(ctx, dims, limit, preci
             # the limit, the persistent one runs as many as it was given
             assert g[1] == limit and g[3] == got[0][3]
             continue
+        assert g[1:] == got[0][1:]
+        assert np.array_equal(g[0], got[0][0])
+    m.close()
+
+
+BI_CASES = [
+    ((3, 3, 3), 100), ((16, 16, 1), 200), ((17, 16, 16), 100), ((65, 16, 16), 400), ((64, 32, 32), 400),
+    ((41, 40, 40), 400),
+    ((64, 64, 65), 130),       # 2 rows per thread, two launches
+    ((700, 500, 1), 130),      # the same, 4 entries a row
+    ((101, 100, 61), 130),     # 3 rows per thread (kernel of 4), last slice ragged
+]
+
+
+@pytest.mark.parametrize("kind", ["advection", "diffusion"])
+@pytest.mark.parametrize("dims,limit", BI_CASES, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_persistent_bicgstab_is_bitwise_the_kernel_by_kernel_form(ctx, dims, limit, kind):
+    from foamadapter_amd import dsl, fvcc, la
+    print(dims, limit, kind, flush=True)
+    m, ls = _system(ctx, dims)
+    N, F, B = m.n_cells, m.n_internal_faces, m.n_boundary_faces
+    if kind == "advection":  # non-symmetric, a few iterations
+        import foamadapter_amd as fa
+        T = fvcc.VolumeField(m, ctx.uniform(N, -1, 1, 12, 0), ctx.uniform(B, -1, 1, 12, 1),
+                             fa.BoundaryConditions(m, ["fixedValue"] * m.n_patches), "T")
+        phi = fvcc.SurfaceField(m, ctx.uniform(F + B, -1e-6, 1e-6, 12, 2))
+        gamma = fvcc.SurfaceField(m, ctx.uniform(F + B, 0.5, 2.0, 12, 3))
+        dt = 0.5 * float(m.get("V").mean()) ** (2.0 / 3.0)
+        dsl.assemble(dsl.imp.ddt(T) + dsl.imp.div(phi, T, "upwind") - dsl.imp.laplacian(gamma, T), T, 0.0, dt, ls)
+    got = []
+    for graph in (False, True, True):
+        x = ctx.uniform(N, -1, 1, 12, 4)
+        st = la.solve_cg(ls, x, {"solver": "PBiCGStab", "relTol": 1e-9, "maxIter": limit, "graph": graph},
+                         raise_on_noconverge=False)
+        got.append((x.numpy(), st.numIter, st.initResNorm, st.finalResNorm, st.trueResNorm, st.status))
+    for g in got[1:]:
         assert g[1:] == got[0][1:]
         assert np.array_equal(g[0], got[0][0])
     m.close()

@@ -303,8 +303,8 @@ struct BiPersist {
     int32_t maxit;
     uint32_t tag0;
     double tol, atol;
-    const int32_t *rowOffs, *diag, *sellCol;
-    const double *vals, *rhs;
+    const int32_t* sellCol;
+    CsrSystem m;
     double* sval;  // scaled values of the rows whose matrix does not stay in registers
     double *x, *r, *rhat, *p, *p2, *v, *v2;
     BiState* st;
@@ -341,7 +341,6 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
     auto mine = [&](auto* vec, int u) { return at_byte(vec + (iw + u * kB), lb); };
     const uint32_t lown = (uint32_t)(iw - (int)cbase) + lofs;
     auto lds = [&](double* vec, int u) -> double& { return *at_byte(vec + lown + u * kB, lb); };
-    constexpr uint32_t kFar = 0x80000000u;
     auto column = [&](int u, int k) {  // byte offset in LDS, or (top bit) in the vectors
         const uint32_t c = (uint32_t)*at_byte(
             A.sellCol + ((int64_t)(iw + u * kB) * W + 64 * k), (uint32_t)lane * 4u);
@@ -370,77 +369,15 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
         if (inN(u)) {
             x0 = *mine(A.x, u);
             const int i = iw + u * kB + lane;
-            d0 = 1.0 / A.vals[A.rowOffs[i] + A.diag[i]];
+            d0 = 1.0 / A.m.vals[A.m.rowOffs[i] + A.m.diag[i]];
         }
         lds(lx, u) = x0;
         lds(li, u) = d0;
     }
-    // b - A x of the own rows (x: LDS, or X for a far column), each handed to
-    // out(u, row's residual, row's b); KEEP: the scaled values and columns too
-    double* const raw = l0 + sub * kRaw;
-    auto residual = [&](auto keep, auto farx, auto out) {
-        constexpr bool KEEP = decltype(keep)::value;
-#pragma unroll
-        for (int u = 0; u < RPT; ++u) {
-            __syncthreads();  // the rows before this (and x) are in place / done with
-            const int i0 = row0 + u * kB, i1 = min(min(i0 + kB, row1), A.N);
-            int b = 0;
-            if (i0 < i1) {
-                b = A.rowOffs[i0];
-                const int n = A.rowOffs[i1] - b;
-                for (int k = tid & (kB - 1); k < n; k += kB) raw[k] = A.vals[b + k];
-            }
-            __syncthreads();
-            if (live(u)) {
-                const int i = iw + u * kB + lane;
-                const bool in = i < A.N;
-                const int o = in ? A.rowOffs[i] - b : 0, len = in ? A.rowOffs[i + 1] - b - o : 0;
-                const int dg = in ? A.diag[i] : 0;
-                uint32_t c[W];
-                double xg[W];
-#pragma unroll
-                for (int k = 0; k < W; ++k) c[k] = column(u, k);
-#pragma unroll
-                for (int k = 0; k < W; ++k)
-                    xg[k] = c[k] & kFar ? farx(c[k] & ~kFar) : *at_byte(lx, c[k]);
-                const double dx = in ? raw[o + dg] * lds(lx, u) : 0.0;
-                double s = 0.0;
-#pragma unroll
-                for (int k = 0; k <= W; ++k) {  // column order, the diagonal at dg
-                    if (k == dg && k < len) s += dx;
-                    if (k < W && k + 1 < len) {
-                        const double a = raw[o + k + (k >= dg ? 1 : 0)];
-                        s += a * xg[k];
-                    }
-                }
-                if (KEEP) {
-#pragma unroll
-                    for (int k = 0; k < W; ++k) {
-                        double a = 0.0;
-                        if (k + 1 < len) {
-                            double dj;
-                            if (c[k] & kFar) {
-                                const uint32_t j = (c[k] & ~kFar) / 8u;
-                                dj = 1.0 / A.vals[A.rowOffs[j] + A.diag[j]];
-                            } else {
-                                dj = *at_byte(li, c[k]);
-                            }
-                            a = raw[o + k + (k >= dg ? 1 : 0)] * dj;
-                        }
-                        if (u < RES) {
-                            mv[u][k] = a;
-                            mc[u][k] = c[k];
-                        } else {
-                            *svalAt(u, k) = a;
-                        }
-                        shown |= c[k] >> 31 << u;
-                    }
-                }
-                const double bi = in ? A.rhs[i] : 0.0;
-                out(u, in ? bi - s : 0.0, bi);
-            }
-        }
-        __syncthreads();
+    auto residual = [&](auto far, auto out) {
+        tile_residual<RPT, W>(
+            A.m, A.N, row0, row1, iw, l0 + sub * kRaw, live, column,
+            [&](uint32_t o) { return *at_byte(lx, o); }, far, [&](int u) { return lds(lx, u); }, out);
     };
 
     double bnorm, res, rho, alpha = 1.0, omega = 1.0, rhoPrev = 1.0, res0;
@@ -449,8 +386,27 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
     bool ok = true;
     {
         double s2[2] = {0.0, 0.0}, t2[2];
-        residual(std::true_type{}, [&](uint32_t o) { return *at_byte(A.x, o); },
-                 [&](int u, double ri, double bi) {
+        residual([&](uint32_t o) { return *at_byte(A.x, o); },
+                 [&](int u, bool, double ri, double bi, const double (&a)[W],
+                     const uint32_t (&c)[W]) {
+#pragma unroll
+                     for (int k = 0; k < W; ++k) {  // a_ij / a_jj
+                         double dj;
+                         if (c[k] & kFar) {
+                             const uint32_t j = (c[k] & ~kFar) / 8u;
+                             dj = 1.0 / A.m.vals[A.m.rowOffs[j] + A.m.diag[j]];
+                         } else {
+                             dj = *at_byte(li, c[k]);
+                         }
+                         const double v = a[k] != 0.0 ? a[k] * dj : 0.0;
+                         if (u < RES) {
+                             mv[u][k] = v;
+                             mc[u][k] = c[k];
+                         } else {
+                             *svalAt(u, k) = v;
+                         }
+                         shown |= c[k] >> 31 << u;
+                     }
                      s2[0] += ri * ri;
                      s2[1] += bi * bi;
                      if (A.fresh) rv[u] = hv[u] = ri;
@@ -647,9 +603,9 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
             double none[1] = {0.0}, all[1], s1[1] = {0.0};
             ok = gs.sum<1, true>(none, all, L);
             if (ok) {
-                residual(std::false_type{},
-                         [&](uint32_t o) { return get_shared(at_byte(A.x, o)); },
-                         [&](int, double ri, double) { s1[0] += ri * ri; });
+                residual([&](uint32_t o) { return get_shared(at_byte(A.x, o)); },
+                         [&](int, bool, double ri, double, const double (&)[W],
+                             const uint32_t (&)[W]) { s1[0] += ri * ri; });
                 ok = gs.sum<1, false>(s1, all, L);
                 trueRes = sqrt(all[0]) / bnorm;
             }
@@ -721,7 +677,7 @@ struct BiWork : fv_solver_cache {
             tag = 1;
         }
         BiPersist a{h.N, h.ntiles, h.rowsPerBlock, persistIters, fresh ? 1 : 0, o->max_iter, tag,
-                    o->rel_tol, o->abs_tol, h.rowOffs, diag, h.sellCol, h.vals, h.rhs, sval.p, x,
+                    o->rel_tol, o->abs_tol, h.sellCol, CsrSystem{h.rowOffs, diag, h.vals, h.rhs}, sval.p, x,
                     h.r, h.rhat, h.p, h.s, h.v, h.t, h.st, slots.p};
         void* args[] = {&a};
         if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(persist), dim3(persistGrid),

@@ -63,6 +63,13 @@ constexpr int kStopSync = 4;           // CgState::stop after a timed-out wait
 constexpr unsigned long long kSyncSeconds = 20;
 constexpr unsigned long long kClockHz = 100000000ull;  // wall_clock64: 100 MHz
 
+// The assembled system, for the persistent forms that scale the matrix and take
+// explicit residuals themselves.
+struct CsrSystem {
+    const int32_t *rowOffs, *diag;
+    const double *vals, *rhs;
+};
+
 // Arguments by value: the kernel reads them from scalar registers instead of
 // chasing the launch description and the system description in memory.
 template <typename S>
@@ -77,6 +84,12 @@ struct CgPersist {
     unsigned long long* rtag;  // published r with its iteration's tag (TAGGED)
     CgState* st;
     unsigned long long* slots;  // 2 * kSlotBuffer
+    // WHOLE: the system, its solution, and the solve's limits; fresh: start from x,
+    // else go on where a launch ran out of iterations
+    CsrSystem m;
+    double* x;
+    double tol, atol;
+    int32_t maxit, fresh;
 };
 
 template <typename T>
@@ -326,6 +339,63 @@ struct GridSum {
     }
 };
 
+// Top bit of a column's byte offset: a row of another tile (an offset into the
+// vectors instead of the LDS)
+constexpr uint32_t kFar = 0x80000000u;
+
+// b - A x of a tile's rows, their entries in column order, 256 rows at a time: the
+// matrix rows are read coalesced into raw ((W + 1) * 256 doubles of LDS) and taken
+// from there.  column(u, k): the columns; near(o), far(o), own(u): x at an LDS
+// offset, at a vector offset, of this thread's row u.  out(u, in, r, b, a, c) gets
+// each row's residual and right-hand side (zero past N) and its off-diagonal
+// values and columns.  Every thread of the workgroup calls it; barriers before the
+// first and after the last use of raw.
+template <int RPT, int W, typename Live, typename Col, typename Near, typename Far, typename Own,
+          typename Out>
+__device__ __forceinline__ void tile_residual(const CsrSystem& m, int N, int row0, int row1, int iw,
+                                              double* raw, Live live, Col column, Near near,
+                                              Far far, Own own, Out out) {
+    const int lane = (int)threadIdx.x & 63;
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+        __syncthreads();
+        const int i0 = row0 + u * kCgBlock, i1 = min(min(i0 + kCgBlock, row1), N);
+        int b = 0;
+        if (i0 < i1) {
+            b = m.rowOffs[i0];
+            const int n = m.rowOffs[i1] - b;
+            for (int k = (int)threadIdx.x & (kCgBlock - 1); k < n; k += kCgBlock)
+                raw[k] = m.vals[b + k];
+        }
+        __syncthreads();
+        if (live(u)) {
+            const int i = iw + u * kCgBlock + lane;
+            const bool in = i < N;
+            const int o = in ? m.rowOffs[i] - b : 0, len = in ? m.rowOffs[i + 1] - b - o : 0;
+            const int dg = in ? m.diag[i] : 0;
+            const double bi = in ? m.rhs[i] : 0.0;
+            uint32_t c[W];
+            double a[W], x[W];
+#pragma unroll
+            for (int k = 0; k < W; ++k) c[k] = column(u, k);
+#pragma unroll
+            for (int k = 0; k < W; ++k) x[k] = c[k] & kFar ? far(c[k] & ~kFar) : near(c[k]);
+            const double dx = in ? raw[o + dg] * own(u) : 0.0;
+            double s = 0.0;
+#pragma unroll
+            for (int k = 0; k <= W; ++k) {  // the diagonal comes before entry dg
+                if (k == dg && in) s += dx;
+                if (k < W) {
+                    a[k] = k + 1 < len ? raw[o + k + (k >= dg ? 1 : 0)] : 0.0;
+                    if (k + 1 < len) s += a[k] * x[k];
+                }
+            }
+            out(u, in, in ? bi - s : 0.0, bi, a, c);
+        }
+    }
+    __syncthreads();
+}
+
 // RPT: rows per thread (the rows a tile gives a thread, rounded up to a power
 // of two); W: entries of every slice of the sliced ELL; RES: rows of each thread
 // whose values and columns stay in registers; GLDS: g in LDS too (else in
@@ -333,11 +403,20 @@ struct GridSum {
 // this workgroup's own rows.  Rows past a tile's end take part as zeros; the
 // vectors are allocated to a multiple of 64 rows, so the rows of the last slice
 // past N are stored too (as zeros).
-template <typename S, int RPT, int W, int RES, bool GLDS, bool TAGGED>
+// WHOLE (FP64): the launch also scales the matrix (from the CSR, also when it goes
+// on), takes the initial residual, and after the stop adds the correction to x and
+// takes the explicit residual, which goes to CgState::rrep: on small systems the
+// nine launches around the iterations cost as much as they do (32^3 heat step of 5
+// iterations 144 us with the start and end as kernels in a replayed graph, 103 whole;
+// 16^3 Poisson of 125 iterations 0.82 -> 0.73 ms).
+template <typename S, int RPT, int W, int RES, bool GLDS, bool TAGGED, bool WHOLE>
 __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     __shared__ PersistLds L;
     __shared__ S lp[RPT * kPersistThreads], ld[RPT * kPersistThreads],
         lg[GLDS ? RPT * kPersistThreads : 1];
+    constexpr int kRaw = WHOLE ? (W + 1) * kCgBlock : 1;
+    __shared__ double raw[kPersistSub * kRaw];
+    static_assert(!WHOLE || (sizeof(S) == 8 && GLDS), "whole solves are FP64 with g in LDS");
     const int tid = (int)threadIdx.x, lane = tid & 63;
     // a tile is four waves and its rows are dealt in waves of 64, so its bounds
     // are the same in every lane: kept in scalar registers
@@ -350,11 +429,13 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     // this tile's rows [cbase, cbase + R) have their p in LDS, from lofs on
     const uint32_t cbase = (uint32_t)tile * R, lofs = (uint32_t)sub * (RPT * kCgBlock);
     CgState* const st = A.st;
-    const int entry = st->stop;
     const bool lead = gs.slot == 0 && tid == 0;
-    if (entry) {
-        if (lead) st->done = entry;  // as the update kernel of a stopped system
-        return;
+    if (!WHOLE || !A.fresh) {
+        const int entry = st->stop;
+        if (entry) {
+            if (lead) st->done = entry;  // as the update kernel of a stopped system
+            return;
+        }
     }
     if (tid == 0) L.bad = 0;
     const int row0 = tile * R;
@@ -372,8 +453,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     auto value = [&](int u, int k) {
         return *at_byte(A.sval + ((int64_t)(iw + u * kCgBlock) * W + 64 * k), lb);
     };
-    // a column as the byte offset of its p in LDS, or (top bit set) of its row in the vectors
-    constexpr uint32_t kFar = 0x80000000u;
+    // a column as the byte offset of its p in LDS, or (kFar) of its row in the vectors
     auto column = [&](int u, int k) {
         const uint32_t c = (uint32_t)*at_byte(
             A.sellCol + ((int64_t)(iw + u * kCgBlock) * W + 64 * k), (uint32_t)lane * 4u);
@@ -391,48 +471,151 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
 #pragma unroll
     for (int u = 0; u < RPT; ++u) {
         rv[u] = qv[u] = S(0);
-        S p0 = S(0), d0 = S(0), g0 = S(0);
         if (u < RES)
             for (int k = 0; k < W; ++k) {
                 mv[u][k] = S(0);
                 mc[u][k] = 0;
             }
-        if (live(u)) {
-            if (u < RES) {
-#pragma unroll
-                for (int k = 0; k < W; ++k) {
-                    mv[u][k] = value(u, k);
-                    mc[u][k] = column(u, k);
-                    shown |= mc[u][k] >> 31 << u;
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < W; ++k) shown |= column(u, k) >> 31 << u;
-            }
-            if (iw + u * kCgBlock + lane < A.N) {
-                rv[u] = *mine(A.r, u);
-                p0 = *mine(A.p, u);
-                d0 = *mine(A.d, u);
-                g0 = *mine(A.g, u);
-            }
-            lds(lp, u) = p0;
-            lds(ld, u) = d0;
-            if constexpr (GLDS) lds(lg, u) = g0;
-        }
-        if constexpr (!GLDS) gr[u] = g0;
+        if constexpr (!GLDS) gr[u] = S(0);
     }
-    const double bnorm = uniform(st->bnorm), tol = uniform(st->tol), atol = uniform(st->atol),
-                 delta = uniform(st->delta), rrep = uniform(st->rrep);
-    const int maxit = __builtin_amdgcn_readfirstlane(st->maxit);
-    double rho = uniform(st->rho), rhoPrev = uniform(st->rhoPrev), alpha = uniform(st->alpha),
-           res = uniform(st->res);
-    int it = __builtin_amdgcn_readfirstlane(st->it), stop = 0;
+    double bnorm, tol, atol, delta, rrep, rho, rhoPrev, alpha, res, res0;
+    int maxit, it, stop = 0;
+    bool ok = true;
+    [[maybe_unused]] auto residual = [&](auto far, auto out) {
+        tile_residual<RPT, W>(
+            A.m, A.N, row0, row1, iw, raw + sub * kRaw, live, column,
+            [&](uint32_t o) { return *at_byte(lp, o); }, far, [&](int u) { return lds(lp, u); }, out);
+    };
+    if constexpr (!WHOLE) {
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            S p0 = S(0), d0 = S(0), g0 = S(0);
+            if (live(u)) {
+                if (u < RES) {
+#pragma unroll
+                    for (int k = 0; k < W; ++k) {
+                        mv[u][k] = value(u, k);
+                        mc[u][k] = column(u, k);
+                        shown |= mc[u][k] >> 31 << u;
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < W; ++k) shown |= column(u, k) >> 31 << u;
+                }
+                if (iw + u * kCgBlock + lane < A.N) {
+                    rv[u] = *mine(A.r, u);
+                    p0 = *mine(A.p, u);
+                    d0 = *mine(A.d, u);
+                    g0 = *mine(A.g, u);
+                }
+                lds(lp, u) = p0;
+                lds(ld, u) = d0;
+                if constexpr (GLDS) lds(lg, u) = g0;
+            }
+            if constexpr (!GLDS) gr[u] = g0;
+        }
+    } else {
+        // x (in p's place) and g of the own rows, as kc_start_tile
+        const double first = A.m.vals[A.m.rowOffs[0] + A.m.diag[0]];
+        auto root = [&](double di) {
+            const bool good =
+                di != 0.0 && (di > 0.0) == (first > 0.0) && fabs(di) <= 1.7976931348623157e308;
+            return good ? copysign(sqrt(fabs(di)), di) : (double)NAN;
+        };
+#pragma unroll
+        for (int u = 0; u < RPT; ++u)
+            if (live(u)) {
+                const int i = iw + u * kCgBlock + lane;
+                const bool in = i < A.N;
+                lds(lp, u) = in ? *mine(A.x, u) : 0.0;
+                lds(lg, u) = in ? root(A.m.vals[A.m.rowOffs[i] + A.m.diag[i]]) : 0.0;
+                lds(ld, u) = !A.fresh && in ? *mine(A.d, u) : 0.0;
+            }
+        double s2[2] = {0.0, 0.0}, t2[2];
+        residual([&](uint32_t o) { return *at_byte(A.x, o); },
+                 [&](int u, bool in, double ri, double bi, const double (&a)[W],
+                     const uint32_t (&c)[W]) {
+                     const double gi = in ? lds(lg, u) : 1.0;
+#pragma unroll
+                     for (int k = 0; k < W; ++k) {  // as kc_scale_tile
+                         double gj;
+                         if (c[k] & kFar) {
+                             const uint32_t j = (c[k] & ~kFar) / 8u;
+                             gj = root(A.m.vals[A.m.rowOffs[j] + A.m.diag[j]]);
+                         } else {
+                             gj = *at_byte(lg, c[k]);
+                         }
+                         const double v = a[k] != 0.0 ? a[k] / (gi * fabs(gj)) : 0.0;
+                         if (u < RES) {
+                             mv[u][k] = v;
+                             mc[u][k] = c[k];
+                         } else {
+                             *at_byte(const_cast<double*>(A.sval) +
+                                          ((int64_t)(iw + u * kCgBlock) * W + 64 * k), lb) = v;
+                         }
+                         shown |= c[k] >> 31 << u;
+                     }
+                     rv[u] = ri;
+                     s2[0] += ri * ri;
+                     s2[1] += bi * bi;
+                 });
+        if (A.fresh) {
+            // ||b||, the relative residual; r = G^-1 r64, p = r, ||G r||^2 and r.r
+            if ((ok = gs.sum<2, false>(s2, t2, L))) {
+                bnorm = sqrt(t2[1]);
+                if (!(bnorm > 0.0)) bnorm = 1.0;
+                res = res0 = sqrt(t2[0]) / bnorm;
+                double s3[2] = {0.0, 0.0};
+#pragma unroll
+                for (int u = 0; u < RPT; ++u)
+                    if (live(u)) {
+                        const bool in = iw + u * kCgBlock + lane < A.N;
+                        const double gi = lds(lg, u);
+                        const double ri = in ? rv[u] / gi : 0.0;
+                        rv[u] = ri;
+                        lds(lp, u) = ri;
+                        if (shown >> u & 1) put_shared(mine(A.p, u), ri);
+                        const double ur = ri * gi;
+                        s3[0] += ur * ur;
+                        s3[1] += ri * ri;
+                    }
+                ok = gs.sum<2, true>(s3, t2, L);
+                rho = t2[1];
+                rhoPrev = alpha = 0.0;
+                it = 0;
+                // the decision of kc_direction after a start
+                const bool conv = res <= A.tol || res * bnorm <= A.atol;
+                stop = conv ? 2 : !(res <= 1.7976931348623157e308) ? 3 : A.maxit <= 0 ? 1 : 0;
+            }
+        } else {
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < RPT; ++u)
+                if (live(u)) {
+                    rv[u] = *mine(A.r, u);
+                    lds(lp, u) = *mine(A.p, u);
+                }
+        }
+    }
+    if (!WHOLE || !A.fresh) {
+        bnorm = uniform(st->bnorm);
+        rho = uniform(st->rho);
+        rhoPrev = uniform(st->rhoPrev);
+        alpha = uniform(st->alpha);
+        res = uniform(st->res);
+        res0 = uniform(st->res0);
+        it = __builtin_amdgcn_readfirstlane(st->it);
+    }
+    tol = WHOLE ? A.tol : uniform(st->tol);
+    atol = WHOLE ? A.atol : uniform(st->atol);
+    maxit = WHOLE ? A.maxit : __builtin_amdgcn_readfirstlane(st->maxit);
+    delta = WHOLE ? 0.0 : uniform(st->delta);
+    rrep = WHOLE ? 0.0 : uniform(st->rrep);
     S beta = S(0);
     uint32_t rtag = 0;
     S *pold = A.p, *pnew = A.p2;  // the direction before this iteration's, and the next one's place
-    bool ok = true;
     __syncthreads();
-    for (int n = 0; n < A.iters; ++n) {
+    for (int n = 0; ok && !stop && n < A.iters; ++n) {
         opaque(lb);
         for (int u = 0; u < RES; ++u)
             for (int k = 0; k < W; ++k) opaque(mc[u][k]);
@@ -554,17 +737,41 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
         }
         __syncthreads();
     }
+    if constexpr (WHOLE) {
+        if (ok && stop) {  // x += |G|^-1 d, the explicit residual of the result
+#pragma unroll
+            for (int u = 0; u < RPT; ++u)
+                if (live(u) && iw + u * kCgBlock + lane < A.N) {
+                    const double x = *mine(A.x, u) + lds(ld, u) / fabs(lds(lg, u));
+                    lds(lp, u) = x;
+                    if (shown >> u & 1)
+                        put_shared(mine(A.x, u), x);
+                    else
+                        *mine(A.x, u) = x;
+                }
+            double none[1] = {0.0}, all[1], s1[1] = {0.0};
+            if ((ok = gs.sum<1, true>(none, all, L))) {
+                residual([&](uint32_t o) { return get_shared(at_byte(A.x, o)); },
+                         [&](int, bool, double ri, double, const double (&)[W],
+                             const uint32_t (&)[W]) { s1[0] += ri * ri; });
+                ok = gs.sum<1, false>(s1, all, L);
+                rrep = sqrt(all[0]) / bnorm;
+            }
+        }
+    }
     if (!ok) {
         if (tid == 0) st->stop = kStopSync;
         return;
     }
+    if (!WHOLE || !stop) {
 #pragma unroll
-    for (int u = 0; u < RPT; ++u)
-        if (live(u)) {
-            *mine(A.r, u) = rv[u];
-            *mine(A.p, u) = lds(lp, u);
-            *mine(A.d, u) = lds(ld, u);
-        }
+        for (int u = 0; u < RPT; ++u)
+            if (live(u)) {
+                *mine(A.r, u) = rv[u];
+                *mine(A.p, u) = lds(lp, u);
+                *mine(A.d, u) = lds(ld, u);
+            }
+    }
     if (lead) {
         st->rho = rho;
         st->rhoPrev = rhoPrev;
@@ -574,6 +781,11 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
         st->stop = stop;
         st->done = 0;
         st->pbuf = 0;
+        if (WHOLE) {
+            st->bnorm = bnorm;
+            st->res0 = res0;
+            st->rrep = rrep;
+        }
     }
 }
 

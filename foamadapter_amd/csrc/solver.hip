@@ -47,6 +47,7 @@ struct CgWork : fv_solver_cache {
     std::vector<int> lastRounds;  // FP32 iterations per round of the previous mixed solve
     // persistent form (null: this system runs kernel by kernel)
     void (*persist)(CgPersist<S>) = nullptr;
+    bool whole = false;  // a launch does everything from the scaling to the residual
     int persistGrid = 0, persistIters = 0;
     int lastLaunches = 0;  // persistent launches of the previous mixed solve
     int lastTotal = 0;     // iterations of the previous solve, in either form
@@ -120,6 +121,7 @@ struct CgWork : fv_solver_cache {
             persist = nullptr;
             return;
         }
+        whole = sizeof(S) == 8 && rpt <= 2;
         // a launch holds the device for about 2 ms (an iteration takes 6 to 40 us,
         // from the smallest to the largest of these systems), so that the work of
         // other streams gets in between
@@ -130,11 +132,14 @@ struct CgWork : fv_solver_cache {
         clear_tags(c->stream);
     }
     // A cooperative launch costs about 17 us more than a plain one and is not
-    // replayed as a graph, and an iteration saves 4 us on the smallest systems: a
-    // system whose previous solve took fewer than kPersistMin iterations keeps the
-    // kernel-by-kernel form (32^3 heat step of 5 iterations: 157 us, 178 persistent).
+    // replayed as a graph, and an iteration saves 4 us on the smallest systems: unless
+    // it is whole, a system whose previous solve took fewer than kPersistMin
+    // iterations keeps the kernel-by-kernel form (32^3 heat step of 5 iterations: 157
+    // us, 178 with the iterations alone persistent, 103 whole).
     static constexpr int kPersistMin = 12;
-    bool use_persist() const { return persist && (lastTotal == 0 || lastTotal >= kPersistMin); }
+    bool use_persist() const {
+        return persist && (whole || lastTotal == 0 || lastTotal >= kPersistMin);
+    }
     // no word of the exchange carries a tag that is still to come
     void clear_tags(hipStream_t s) {
         FV_HIP(hipMemsetAsync(slots.p, 0, slots.n * sizeof(unsigned long long), s));
@@ -145,23 +150,29 @@ struct CgWork : fv_solver_cache {
     // in the 128 registers of a 1024-thread workgroup without spills.
     template <int W>
     static auto persist_kernel(int rpt) -> void (*)(CgPersist<S>) {
-        if (rpt <= 1) return kc_persist<S, 1, W, 1, false, true>;
-        if (rpt <= 2) return kc_persist<S, 2, W, 2, true, true>;
         if constexpr (sizeof(S) == 8) {
-            if (rpt <= 4) return kc_persist<S, 4, W, 2, true, false>;
-            if (rpt <= 8) return kc_persist<S, 8, W, 0, false, false>;
+            if (rpt <= 1) return kc_persist<S, 1, W, 1, true, true, true>;
+            if (rpt <= 2) return kc_persist<S, 2, W, 2, true, true, true>;
+            if (rpt <= 4) return kc_persist<S, 4, W, 2, true, false, false>;
+            if (rpt <= 8) return kc_persist<S, 8, W, 0, false, false, false>;
         } else {
-            if (rpt <= 4) return kc_persist<S, 4, W, 4, true, true>;
-            if (rpt <= 8) return kc_persist<S, 8, W, 4, true, false>;
+            if (rpt <= 1) return kc_persist<S, 1, W, 1, false, true, false>;
+            if (rpt <= 2) return kc_persist<S, 2, W, 2, true, true, false>;
+            if (rpt <= 4) return kc_persist<S, 4, W, 4, true, true, false>;
+            if (rpt <= 8) return kc_persist<S, 8, W, 4, true, false, false>;
         }
         return nullptr;
     }
     // Up to persistIters iterations in one launch; false if the device refuses it.
-    bool run_persist(hipStream_t s) {
-        const uint32_t uses = 3 * (uint32_t)persistIters + 3;
+    // (whole: x, the limits and whether the solve starts.)
+    bool run_persist(hipStream_t s, double* x = nullptr, double tol = 0.0, double atol = 0.0,
+                     int maxit = 0, bool fresh = false) {
+        const uint32_t uses = 2 * (uint32_t)persistIters + 8;
         if (tag > 0xffffffffu - uses) clear_tags(s);  // sequence numbers start over
         CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persistIters, tag, h.sellCol, h.sval,
-                       h.g, h.d, h.r, h.p, h.p2, rtag.p, h.st, slots.p};
+                       h.g, h.d, h.r, h.p, h.p2, rtag.p, h.st, slots.p,
+                       CsrSystem{h.rowOffs, h.diag, h.vals, h.rhs}, x, tol, atol, maxit,
+                       fresh ? 1 : 0};
         void* args[] = {&a};
         if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(persist), dim3(persistGrid),
                                        dim3(kPersistThreads), args, 0, s) != hipSuccess) {
@@ -440,13 +451,33 @@ CgState run_cg(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, int check,
 }
 
 // run_cg with the persistent kernel: a launch ends at the stop by itself, so
-// nothing has to be predicted.  A system whose previous solve fitted one launch
+// nothing has to be predicted.  A whole solve is one launch and one read (of pinned
+// memory) unless it runs out of a launch's iterations.  Else, a system whose previous solve fitted one launch
 // gets the correction and the explicit residual queued behind it and is read
 // once; otherwise two launches are kept queued until one has stopped.  False
 // (and nothing done) if the device refuses the launch.
 bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, double atol,
-                    double* true_res, CgState* out) {
+                    double* x, double* true_res, CgState* out) {
     hipStream_t s = ctx->stream;
+    if (w.whole) {
+        CgState* const host = static_cast<CgState*>(ctx_poll_host(ctx));
+        bool fresh = true;
+        do {
+            if (!w.run_persist(s, x, tol, atol, maxit, fresh)) {
+                FV_REQUIRE(fresh, "a cooperative launch was refused");
+                return false;
+            }
+            fresh = false;
+            FV_HIP(hipMemcpyAsync(host, w.st.p, sizeof *host, hipMemcpyDeviceToHost, s));
+            FV_HIP(hipStreamSynchronize(s));
+        } while (!host->stop);
+        *out = *host;
+        w.check_persist(*out);
+        w.lastIters = std::max(out->it, 1);
+        *true_res = out->rrep;
+        return true;
+    }
+    w.bind(ctx, x);
     w.prep(s);
     w.start(s, tol, maxit, 0.0, atol);
     if (!w.run_persist(s)) return false;
@@ -687,12 +718,13 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
         double bnorm = 0.0;
         if (o->mode == FV_SOLVE_F64) {
             CgWork<double>& w = work_of<double>(ls, false);
-            w.bind(ctx, x);
             double tr = 0.0;
             CgState h{};
             if (o->eager || !w.use_persist() ||
-                !run_cg_persist(ctx, w, o->rel_tol, o->max_iter, o->abs_tol, &tr, &h))
+                !run_cg_persist(ctx, w, o->rel_tol, o->max_iter, o->abs_tol, x, &tr, &h)) {
+                w.bind(ctx, x);
                 h = run_cg(ctx, w, o->rel_tol, o->max_iter, check, o->abs_tol, o->eager != 0, &tr);
+            }
             w.lastTotal = h.it;
             local.init_res = h.res0;
             local.final_res = h.res;

@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -109,7 +110,6 @@ void build_tables(fv_batch* b) {
         p.ntiles = (int)ht.size() - p.tile0;
         p.sellOff = sp->sellOff.p;
         p.sellCol = sp->sellCol.p;
-        p.sellSrc = sp->sellSrc.p;
         p.diag = sp->diagOffset.p;
         p.sval = (const S*)m->sval.p;
         p.rowOffs = sp->rowOffs.p;
@@ -210,7 +210,7 @@ void enqueue_chunk(fv_batch* b) {
     // FP64 residual replacement of the systems that stopped in this chunk
     kc_accum<S, 0><<<G, kB, 0, s>>>(g);
     kc_resid<S, 0><<<G, kB, 0, s>>>(g, red);
-    kc_replace<S, 0><<<G, kB, 0, s>>>(g, red);
+    kc_replace<S><<<G, kB, 0, s>>>(g, red);
     kc_direction<S, 1><<<G, kB, 0, s>>>(g, red, 0);
 }
 
@@ -237,8 +237,11 @@ void run_chunk(fv_batch* b) {
     FV_HIP(hipGraphLaunch(b->graphExec, s));
 }
 
+// Starts the members that need it; false if none does.  Nothing waits here: the step's
+// synchronisation does, and the tables (launch description, start parameters, tiles, in
+// one upload) stay in b->hostStart until then.
 template <typename S>
-void start_members(fv_batch* b) {
+bool start_members(fv_batch* b) {
     fv_ctx* ctx = b->ctx;
     hipStream_t s = ctx->stream;
     std::vector<CgTile> st;
@@ -256,36 +259,28 @@ void start_members(fv_batch* b) {
         }
         slot += member_tiles(b, m);
     }
-    if (st.empty()) return;
-    if (b->startTiles.n < st.size() * sizeof(CgTile))
-        b->startTiles.alloc(ctx, next_pow2((int)st.size()) * sizeof(CgTile));
-    if (b->startParams.n < prm.size() * sizeof(CgStartParam))
-        b->startParams.alloc(ctx, next_pow2((int)prm.size()) * sizeof(CgStartParam));
-    if (!b->startGridDev.p) b->startGridDev.alloc(ctx, sizeof(CgGrid<S>));
-    FV_HIP(hipMemcpyAsync(b->startTiles.p, st.data(), st.size() * sizeof(CgTile),
-                          hipMemcpyHostToDevice, s));
-    FV_HIP(hipMemcpyAsync(b->startParams.p, prm.data(), prm.size() * sizeof(CgStartParam),
-                          hipMemcpyHostToDevice, s));
-    const CgGrid<S> hg{(const CgTile*)b->startTiles.p, (const CgSys<S>*)b->probs.p,
-                       (int)st.size(), 0};
-    FV_HIP(hipMemcpyAsync(b->startGridDev.p, &hg, sizeof hg, hipMemcpyHostToDevice, s));
-    const auto* g = (const CgGrid<S>*)b->startGridDev.p;
+    if (st.empty()) return false;
+    constexpr size_t oPrm = 64;
+    static_assert(sizeof(CgGrid<S>) <= oPrm, "launch description");
+    const size_t oTiles = oPrm + prm.size() * sizeof(CgStartParam);
+    const size_t bytes = oTiles + st.size() * sizeof(CgTile);
+    if (b->startTab.n < bytes) b->startTab.alloc(ctx, next_pow2((int)bytes));
+    const uint8_t* dev = b->startTab.p;
+    const CgGrid<S> hg{(const CgTile*)(dev + oTiles), (const CgSys<S>*)b->probs.p, (int)st.size(), 0};
+    b->hostStart.resize(bytes);
+    std::memcpy(b->hostStart.data(), &hg, sizeof hg);
+    std::memcpy(b->hostStart.data() + oPrm, prm.data(), prm.size() * sizeof(CgStartParam));
+    std::memcpy(b->hostStart.data() + oTiles, st.data(), st.size() * sizeof(CgTile));
+    FV_HIP(hipMemcpyAsync(b->startTab.p, b->hostStart.data(), bytes, hipMemcpyHostToDevice, s));
+    const auto* g = (const CgGrid<S>*)dev;
     const CgPartials red = partials_of<S>(b);
     const int G = cg_grid((int)st.size());
     FV_HIP(hipEventRecord(b->ev[2], s));
-    kc_start_tile<S, 1><<<G, kB, 0, s>>>(g, (const CgStartParam*)b->startParams.p);
-    kc_scale_tile<S><<<G, kB, 0, s>>>(g);
-    kc_resid<S, 1><<<G, kB, 0, s>>>(g, red);
-    kc_replace<S, 1><<<G, kB, 0, s>>>(g, red);
-    kc_direction<S, 2><<<G, kB, 0, s>>>(g, red, 0);
+    kc_begin<S><<<G, kB, 0, s>>>(g, red, (const CgStartParam*)(dev + oPrm), CgStartParam{});
+    kc_scale<S><<<cg_scale_grid(G, b->tileRows), kB, 0, s>>>(g, red);
     FV_LAUNCH_CHECK();
     FV_HIP(hipEventRecord(b->ev[3], s));
-    // the upload buffer must outlive the launches
-    FV_HIP(hipStreamSynchronize(s));
-    float ms = 0.0f;
-    FV_HIP(hipEventElapsedTime(&ms, b->ev[2], b->ev[3]));
-    b->startMs += ms;
-    ++b->starts;
+    return true;
 }
 
 void make_events(fv_batch* b) {
@@ -299,7 +294,7 @@ void step_t(fv_batch* b, std::vector<CgState>& out) {
     out.clear();
     if (b->members.empty()) return;
     make_events(b);
-    start_members<S>(b);
+    const bool started = start_members<S>(b);
     hipStream_t s = b->ctx->stream;
     FV_HIP(hipEventRecord(b->ev[0], s));
     run_chunk<S>(b);
@@ -312,6 +307,11 @@ void step_t(fv_batch* b, std::vector<CgState>& out) {
     FV_HIP(hipEventElapsedTime(&ms, b->ev[0], b->ev[1]));
     b->chunkMs += ms;
     ++b->chunks;
+    if (started) {
+        FV_HIP(hipEventElapsedTime(&ms, b->ev[2], b->ev[3]));
+        b->startMs += ms;
+        ++b->starts;
+    }
     for (BMember* m : b->members) out.push_back(all[m->slot]);
 }
 

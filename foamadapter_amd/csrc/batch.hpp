@@ -38,8 +38,9 @@ struct fv_batch {
     // grow, and the captured chunk graph stays valid until they do
     fvhip::DBuf<uint8_t> probs;
     fvhip::DBuf<uint8_t> tiles;
-    fvhip::DBuf<uint8_t> startTiles, startParams;
-    fvhip::DBuf<uint8_t> gridDev, startGridDev;  // launch descriptions (CgGrid)
+    fvhip::DBuf<uint8_t> startTab;    // launch description, parameters and tiles of a start
+    std::vector<uint8_t> hostStart;   // what it is uploaded from
+    fvhip::DBuf<uint8_t> gridDev;     // launch description (CgGrid) of the chunk
     fvhip::DBuf<fvhip::CgState> states;
     fvhip::DBuf<double> partials;
     int nTiles = 0, nStartTiles = 0;

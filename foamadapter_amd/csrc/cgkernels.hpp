@@ -62,7 +62,6 @@ struct CgSys {
     const int64_t* sellOff;         // sliced ELL of the off-diagonal entries, 64-row
     const int32_t* sellCol;         // slices, entries column-major
     const S* sval;                  // their scaled values a_ij / (g_i |g_j|)
-    const int32_t* sellSrc;         // CSR index of each sliced-ELL entry (-1: padding)
     const int32_t* diag;            // CSR slot of the diagonal within each row
     const int32_t* rowOffs;         // FP64 CSR (residual replacement)
     const int32_t* colIdxs;
@@ -377,8 +376,7 @@ __global__ __launch_bounds__(kCgBlock) void kc_update(const CgGrid<S>* __restric
 // MODE 0: after an update (stop on the recurrence estimate, the iteration limit,
 //         NaN or the residual-drop trigger);
 // MODE 1: after a residual replacement, for the replaced systems only (stop on
-//         the FP64 residual: 2 converged, 3 non-finite, 1 iteration limit);
-// MODE 2: after the start (replacement of the initial guess; p = z already).
+//         the FP64 residual: 2 converged, 3 non-finite, 1 iteration limit).
 template <typename S, int MODE>
 __global__ __launch_bounds__(kCgBlock) void kc_direction(const CgGrid<S>* __restrict__ g, CgPartials red,
                                                          int pOld) {
@@ -413,7 +411,7 @@ __global__ __launch_bounds__(kCgBlock) void kc_direction(const CgGrid<S>* __rest
             }
         }
     };
-    if (MODE != 2) load(i0);
+    load(i0);
     double tot[2];
     sum_slots<2>(red.rz, P.tile0, P.ntiles, sh, tot);
     const int it = st->it;
@@ -434,7 +432,7 @@ __global__ __launch_bounds__(kCgBlock) void kc_direction(const CgGrid<S>* __rest
             st->rrep = rn;
         st->stop = stop;
     }
-    if (MODE == 2 || stop != 0 || it == 0) return;
+    if (stop != 0 || it == 0) return;
     const S beta = (S)(tot[1] / st->rhoPrev);
     for (int base = i0; base < r1; base += kCgU * kCgBlock) {
         if (base != i0) load(base);
@@ -521,9 +519,9 @@ __global__ __launch_bounds__(kCgBlock) void kc_resid(const CgGrid<S>* __restrict
     write_slot<2>(v, red.rb, slot, sh);
 }
 
-// relative FP64 residual from the resid partials; r = (S) (r64 / g) (z = r),
-// START: p = r and ||b||; partials of ||G r||^2 and r.r
-template <typename S, int START>
+// relative FP64 residual from the resid partials of the systems that stopped;
+// r = (S) (r64 / g) (z = r); partials of ||G r||^2 and r.r
+template <typename S>
 __global__ __launch_bounds__(kCgBlock) void kc_replace(const CgGrid<S>* __restrict__ g, CgPartials red) {
     __shared__ double sh[kCgShared];
     const CgSys<S>* Pp;
@@ -532,38 +530,24 @@ __global__ __launch_bounds__(kCgBlock) void kc_replace(const CgGrid<S>* __restri
     const CgSys<S>& P = *Pp;
     CgState* st = P.st;
     const int stop = st->stop;
-    if (!START && stop != 1) return;
+    if (stop != 1) return;
     double tot[2];
     sum_slots<2>(red.rb, P.tile0, P.ntiles, sh, tot);
-    double bn;
-    if (START) {
-        bn = sqrt(tot[1]);
-        if (!(bn > 0.0)) bn = 1.0;
-    } else {
-        bn = st->bnorm;
-    }
-    const double res = sqrt(tot[0]) / bn;
+    const double res = sqrt(tot[0]) / st->bnorm;
     if (row0 == 0 && threadIdx.x == 0) {
         st->res = res;
         st->done = stop;  // tells the mode-1 direction kernel that this system was replaced
-        if (START) {
-            st->bnorm = bn;
-            st->res0 = res;
-        } else {
-            st->nrep += 1;
-        }
+        st->nrep += 1;
     }
     double rr = 0.0, rz = 0.0;
     const int r1 = min(row1, P.N);
     const S* __restrict__ gv = P.g;  // addresses read once (see kc_direction)
     const double* __restrict__ r64 = P.r64;
     S* __restrict__ rv = P.r;
-    S* __restrict__ pv = P.p;
     for (int i = row0 + threadIdx.x; i < r1; i += kCgBlock) {
         const double gi = (double)gv[i];
         const S ri = (S)(r64[i] / gi);
         rv[i] = ri;
-        if (START) pv[i] = ri;
         const double ur = (double)ri * gi;
         rr += ur * ur;
         rz += (double)ri * (double)ri;
@@ -593,27 +577,74 @@ struct CgStartParam {
     int32_t maxit, pad;
 };
 
-// Start, one workgroup per tile of the (re)starting systems: g_i (the signed
-// square root of the diagonal, NaN for a zero, non-finite or opposite-sign
-// entry), d = 0, and (STATE, first tile) the system's CG state from prm.
-// Tile rows are multiples of 64, so a tile owns whole slices.
-template <typename S, int STATE>
-__global__ __launch_bounds__(kCgBlock) void kc_start_tile(const CgGrid<S>* __restrict__ g,
-                                                          const CgStartParam* __restrict__ prm) {
+// Start, in two kernels over the tiles of the (re)starting systems (tile rows are
+// multiples of 64, so a tile owns whole slices).  They read the matrix rows
+// coalesced, by blocks of 256 (see csr_products), once each.  A 2.7 M row FP32 batch
+// (40 systems, tiles of 4096 rows): 91 + 90 us (340 and 290 MB); as five kernels, two
+// of them walking rows and source indices, 352.
+//
+// kc_begin: g_i (the signed square root of the diagonal, NaN for a zero, non-finite
+// or opposite-sign entry), d = 0, the residual b - A x of the initial guess,
+// r = p = (S) (r64 / g) (z = r), partials of r64.r64 and b.b and of ||G r||^2 and
+// r.r; the first tile writes the system's CG state from prm (by system) or one.
+template <typename S>
+__global__ __launch_bounds__(kCgBlock) void kc_begin(const CgGrid<S>* __restrict__ g, CgPartials red,
+                                                     const CgStartParam* __restrict__ prm,
+                                                     CgStartParam one) {
+    __shared__ double sh[kCgShared];
+    __shared__ double prod[kCsrLds];
     const CgSys<S>* Pp;
     int row0, row1, slot;
     if (!cg_locate(g, Pp, row0, row1, slot)) return;
     const CgSys<S>& P = *Pp;
-    const double d0 = P.vals[P.rowOffs[0] + P.diag[0]];
+    const int32_t* __restrict__ ro = P.rowOffs;
+    const int32_t* __restrict__ ci = P.colIdxs;
+    const int32_t* __restrict__ dg = P.diag;
+    const double* __restrict__ va = P.vals;
+    const double* __restrict__ xv = P.x;
+    const double* __restrict__ rhs = P.rhs;
+    S* __restrict__ gv = P.g;
+    S* __restrict__ dv = P.d;
+    S* __restrict__ rv = P.r;
+    S* __restrict__ pv = P.p;
+    const double d0 = va[ro[0] + dg[0]];
+    double rr = 0.0, bb = 0.0, gr = 0.0, rz = 0.0;
     const int r1 = min(row1, P.N);
-    for (int i = row0 + threadIdx.x; i < r1; i += kCgBlock) {
-        const double di = P.vals[P.rowOffs[i] + P.diag[i]];
-        const bool ok = di != 0.0 && (di > 0.0) == (d0 > 0.0) && fabs(di) <= 1.7976931348623157e308;
-        P.g[i] = ok ? (S)copysign(sqrt(fabs(di)), di) : (S)NAN;
-        P.d[i] = S(0);
+    for (int i0 = row0; i0 < r1; i0 += kCgBlock) {
+        const int i = i0 + (int)threadIdx.x, ic = min(i, r1 - 1);
+        const int k0 = ro[ic], k1 = ro[ic + 1], base = ro[i0];
+        const double bi = rhs[ic], di = va[k0 + dg[ic]];
+        const bool staged = csr_products(ro, ci, va, xv, i0, min(i0 + kCgBlock, r1), prod);
+        __syncthreads();
+        if (i < r1) {
+            double s = 0.0;
+            if (staged)
+                for (int k = k0; k < k1; ++k) s += prod[k - base];
+            else
+                for (int k = k0; k < k1; ++k) s += va[k] * xv[ci[k]];
+            const double r64 = bi - s;
+            const bool ok =
+                di != 0.0 && (di > 0.0) == (d0 > 0.0) && fabs(di) <= 1.7976931348623157e308;
+            const S gs = ok ? (S)copysign(sqrt(fabs(di)), di) : (S)NAN;
+            const double gi = (double)gs;
+            const S ri = (S)(r64 / gi);
+            gv[i] = gs;
+            dv[i] = S(0);
+            rv[i] = ri;
+            pv[i] = ri;
+            rr += r64 * r64;
+            bb += bi * bi;
+            const double ur = (double)ri * gi;
+            gr += ur * ur;
+            rz += (double)ri * (double)ri;
+        }
+        __syncthreads();
     }
-    if (STATE && row0 == 0 && threadIdx.x == 0) {
-        const CgStartParam q = prm[Pp - g->probs];
+    double v[2] = {rr, bb}, w[2] = {gr, rz};
+    write_slot<2>(v, red.rb, slot, sh);
+    write_slot<2>(w, red.rz, slot, sh);
+    if (row0 == 0 && threadIdx.x == 0) {
+        const CgStartParam q = prm ? prm[Pp - g->probs] : one;
         CgState s{};
         s.tol = q.tol;
         s.atol = q.atol;
@@ -623,40 +654,87 @@ __global__ __launch_bounds__(kCgBlock) void kc_start_tile(const CgGrid<S>* __res
     }
 }
 
-// Scaled sliced-ELL values a_ij / (g_i |g_j|) in S of the tile's rows (after
-// kc_start_tile has written g); one thread per row, so the stores of an entry
-// index are coalesced over a slice.
+// kc_scale: the scaled sliced-ELL values a_ij / (g_i |g_j|) in S; the first tile
+// sums the partials of kc_begin and decides on the FP64 residual (2 converged, 3
+// non-finite, 1 iteration limit).  No sum runs over a tile's rows here, so long tiles
+// are split over blockIdx.y, kScaleRows each (tiles of 4096 rows unsplit: 118 us).
+constexpr int kScaleRows = 1024;
+inline dim3 cg_scale_grid(int blocks, int tileRows) {
+    return dim3(blocks, (tileRows + kScaleRows - 1) / kScaleRows);
+}
+
 template <typename S>
-__global__ __launch_bounds__(kCgBlock) void kc_scale_tile(const CgGrid<S>* __restrict__ g) {
+__global__ __launch_bounds__(kCgBlock) void kc_scale(const CgGrid<S>* __restrict__ g, CgPartials red) {
+    __shared__ double sh[kCgShared];
+    __shared__ double raw[kCsrLds];
     const CgSys<S>* Pp;
     int row0, row1, slot;
     if (!cg_locate(g, Pp, row0, row1, slot)) return;
     const CgSys<S>& P = *Pp;
-    S* sval = const_cast<S*>(P.sval);
-    for (int i = row0 + threadIdx.x; i < row1; i += kCgBlock) {
-        const int sl = i >> 6;
-        const int64_t b = P.sellOff[sl] + (i & 63);
-        const int w = (int)((P.sellOff[sl + 1] - P.sellOff[sl]) >> 6);
-        const double gi = i < P.N ? (double)P.g[i] : 1.0;
-        for (int k = 0; k < w; ++k) {
-            const int64_t pos = b + 64 * (int64_t)k;
-            const int32_t j = P.sellSrc[pos];
-            sval[pos] = j >= 0 ? (S)(P.vals[j] / (gi * fabs((double)P.g[P.sellCol[pos]]))) : S(0);
+    if (row0 == 0 && blockIdx.y == 0) {
+        double tb[2], tz[2];
+        sum_slots<2>(red.rb, P.tile0, P.ntiles, sh, tb);
+        sum_slots<2>(red.rz, P.tile0, P.ntiles, sh, tz);
+        if (threadIdx.x == 0) {
+            CgState* st = P.st;
+            double bn = sqrt(tb[1]);
+            if (!(bn > 0.0)) bn = 1.0;
+            const double res = sqrt(tb[0]) / bn;
+            const bool conv = res <= st->tol || res * bn <= st->atol;
+            st->bnorm = bn;
+            st->res0 = st->res = res;
+            st->rho = tz[1];
+            st->rrep = sqrt(tz[0]);
+            st->stop = conv ? 2 : !(res <= 1.7976931348623157e308) ? 3 : st->maxit <= 0 ? 1 : 0;
         }
     }
-}
-
-template <int = 0>
-__global__ void kc_init_state(CgState* st, int n, double tol, int maxit, double delta,
-                              double atol = 0.0) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        CgState s{};
-        s.tol = tol;
-        s.atol = atol;
-        s.maxit = maxit;
-        s.delta = delta;
-        st[i] = s;
+    const int32_t* __restrict__ ro = P.rowOffs;
+    const int32_t* __restrict__ dg = P.diag;
+    const double* __restrict__ va = P.vals;
+    const S* __restrict__ gv = P.g;
+    const int64_t* __restrict__ soff = P.sellOff;
+    const int32_t* __restrict__ scol = P.sellCol;
+    S* __restrict__ sval = const_cast<S*>(P.sval);
+    const int N = P.N;
+    row0 += (int)blockIdx.y * kScaleRows;
+    row1 = min(row1, row0 + kScaleRows);
+    for (int i0 = row0; i0 < row1; i0 += kCgBlock) {
+        const int i = i0 + (int)threadIdx.x, ic = min(i, N - 1);
+        const int base = ro[i0], n = ro[min(min(i0 + kCgBlock, row1), N)] - base;
+        const int o = ro[ic] - base, len = i < N ? ro[ic + 1] - base - o : 0, d = dg[ic];
+        const double gi = i < N ? (double)gv[ic] : 1.0;
+        const int sl = min(i, row1 - 1) >> 6;
+        const int64_t s0 = soff[sl];
+        const int w = i < row1 ? (int)((soff[sl + 1] - s0) >> 6) : 0;
+        const int64_t b = s0 + (i & 63);
+        const bool staged = n <= kCsrLds;
+        if (staged) {
+            double v[kCsrU];
+#pragma unroll
+            for (int u = 0; u < kCsrU; ++u) v[u] = va[base + min((int)threadIdx.x + u * kCgBlock, n - 1)];
+#pragma unroll
+            for (int u = 0; u < kCsrU; ++u)
+                if ((int)threadIdx.x + u * kCgBlock < n) raw[threadIdx.x + u * kCgBlock] = v[u];
+        }
+        __syncthreads();
+        constexpr int kE = 8;  // entries whose columns, then g, are loaded together
+        for (int k = 0; k < w; k += kE) {
+            int c[kE];
+            S gj[kE];
+#pragma unroll
+            for (int j = 0; j < kE; ++j) c[j] = scol[b + 64 * (int64_t)min(k + j, w - 1)];
+#pragma unroll
+            for (int j = 0; j < kE; ++j) gj[j] = gv[c[j]];
+#pragma unroll
+            for (int j = 0; j < kE; ++j)
+                if (k + j < w) {
+                    const int q = o + k + j + (k + j >= d ? 1 : 0);  // entry k + j skips the diagonal
+                    const bool real = k + j + 1 < len;
+                    const double a = real ? (staged ? raw[q] : va[base + q]) : 0.0;
+                    sval[b + 64 * (int64_t)(k + j)] = real ? (S)(a / (gi * fabs((double)gj[j]))) : S(0);
+                }
+        }
+        __syncthreads();
     }
 }
 

@@ -515,7 +515,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
             if constexpr (!GLDS) gr[u] = g0;
         }
     } else {
-        // x (in p's place) and g of the own rows, as kc_start_tile
+        // x (in p's place) and g of the own rows, as kc_begin
         const double first = A.m.vals[A.m.rowOffs[0] + A.m.diag[0]];
         auto root = [&](double di) {
             const bool good =
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
                      const uint32_t (&c)[W]) {
                      const double gi = in ? lds(lg, u) : 1.0;
 #pragma unroll
-                     for (int k = 0; k < W; ++k) {  // as kc_scale_tile
+                     for (int k = 0; k < W; ++k) {  // as kc_scale
                          double gj;
                          if (c[k] & kFar) {
                              const uint32_t j = (c[k] & ~kFar) / 8u;

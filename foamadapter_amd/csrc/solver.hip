@@ -81,7 +81,6 @@ struct CgWork : fv_solver_cache {
         h.ntiles = tiles;
         h.sellOff = sp->sellOff.p;
         h.sellCol = sp->sellCol.p;
-        h.sellSrc = sp->sellSrc.p;
         h.diag = sp->diagOffset.p;
         h.sval = sval.p;
         h.rowOffs = sp->rowOffs.p;
@@ -205,13 +204,6 @@ struct CgWork : fv_solver_cache {
         h.xold = nullptr;
         FV_HIP(hipMemcpyAsync(sys.p, &h, sizeof h, hipMemcpyHostToDevice, c->stream));
     }
-    // Loads the matrix (values may have changed since the last solve): the
-    // diagonal's signed square roots g, d = 0, and the scaled off-diagonal
-    // values in S.
-    void prep(hipStream_t s) {
-        kc_start_tile<S, 0><<<G, kB, 0, s>>>(gdev.p, nullptr);
-        kc_scale_tile<S><<<G, kB, 0, s>>>(gdev.p);
-    }
     // Runs enqueue() -- kernel launches only, whose by-value arguments `key`
     // determines -- eagerly until the same key has come kCaptureAfter times in
     // a row, then as a captured hipGraph, replayed while the key keeps coming.
@@ -250,12 +242,11 @@ struct CgWork : fv_solver_cache {
         FV_HIP(hipGraphLaunch(gexec, s));
     }
 
-    // FP64 residual of the current x, r = (S) (r64 / g), p = r, r.r
+    // Scales the matrix (its values may have changed since the last solve) and takes
+    // the FP64 residual of the current x: r = (S) (r64 / g), p = r.
     void start(hipStream_t s, double tol, int maxit, double delta, double atol) {
-        kc_init_state<<<1, 64, 0, s>>>(st.p, 1, tol, maxit, delta, atol);
-        kc_resid<S, 1><<<G, kB, 0, s>>>(gdev.p, red);
-        kc_replace<S, 1><<<G, kB, 0, s>>>(gdev.p, red);
-        kc_direction<S, 2><<<G, kB, 0, s>>>(gdev.p, red, 0);
+        kc_begin<S><<<G, kB, 0, s>>>(gdev.p, red, nullptr, CgStartParam{tol, delta, atol, maxit, 0});
+        kc_scale<S><<<cg_scale_grid(G, grid.rowsPerBlock), kB, 0, s>>>(gdev.p, red);
     }
     // n iterations: the first with a plain SpMV, the others with the previous
     // direction fused into the SpMV, then the last direction (or, for large
@@ -280,7 +271,7 @@ struct CgWork : fv_solver_cache {
     void replacement(hipStream_t s) {
         kc_accum<S, 0><<<G, kB, 0, s>>>(gdev.p);
         kc_resid<S, 0><<<G, kB, 0, s>>>(gdev.p, red);
-        kc_replace<S, 0><<<G, kB, 0, s>>>(gdev.p, red);
+        kc_replace<S><<<G, kB, 0, s>>>(gdev.p, red);
         kc_direction<S, 1><<<G, kB, 0, s>>>(gdev.p, red, 0);
     }
     CgState state(hipStream_t s) {
@@ -392,7 +383,6 @@ CgState run_cg(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, int check,
     if (w.lastIters > 0) {
         const int n = std::min(w.lastIters, maxit);
         auto seq = [&] {
-            w.prep(s);
             w.start(s, tol, maxit, 0.0, atol);
             w.chunk(s, n);
             w.finish(s);
@@ -407,7 +397,6 @@ CgState run_cg(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, int check,
         h = w.state2(s, &t);
         haveTrue = true;
     } else {
-        w.prep(s);
         w.start(s, tol, maxit, 0.0, atol);
         FV_LAUNCH_CHECK();
     }
@@ -478,7 +467,6 @@ bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, doubl
         return true;
     }
     w.bind(ctx, x);
-    w.prep(s);
     w.start(s, tol, maxit, 0.0, atol);
     if (!w.run_persist(s)) return false;
     CgState h{}, t{};
@@ -589,7 +577,6 @@ IrOut run_mixed(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, int chunk,
         }
         rounds = (int)rr.size();
         auto seq = [&] {
-            w.prep(s);
             w.start(s, tol, maxit, delta, atol);
             for (int n : rr) {
                 w.chunk(s, n);
@@ -613,7 +600,6 @@ IrOut run_mixed(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, int chunk,
         if (h.it > done) sched.push_back(h.it - done);
         done = h.it;
     } else {
-        w.prep(s);
         w.start(s, tol, maxit, delta, atol);
         FV_LAUNCH_CHECK();
     }
@@ -663,7 +649,6 @@ IrOut run_mixed(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, int chunk,
 bool run_mixed_persist(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, double delta,
                        double atol, IrOut* out) {
     hipStream_t s = ctx->stream;
-    w.prep(s);
     w.start(s, tol, maxit, delta, atol);
     if (!w.run_persist(s)) return false;
     w.replacement(s);

@@ -92,3 +92,56 @@ def test_velocity_update(ctx, gather):
     g = fvcc.GaussGreenGrad(ctx, m).grad(p).numpy()
     assert np.array_equal(U.numpy(), h3.numpy() - rau.numpy()[:, None] * g)
     m.close()
+
+
+@pytest.mark.parametrize("precision", ["double", "mixed"])
+@pytest.mark.parametrize("name", ["one", "line", "box", "refined"])
+def test_batch_start(ctx, name, precision):
+    """The start of a batched solve (row residual, scaling, first residual) and the fused
+    heat assembly: two CG iterations from a nonzero x against the same two in FP64 numpy.
+    A row sum of n terms is off by n * eps of its terms; the scaled system is diagonally
+    dominant, so two iterations keep errors at a few times that: bounds 64 and, where
+    vectors are FP32, 64 * 2^-24 of the first correction."""
+    import scipy.sparse as sp
+    import foamadapter_amd as fa
+    from foamadapter_amd import fvcc, la
+    print(name, precision, flush=True)
+    m = fa.Mesh.from_poly(ctx, _poly(name))
+    N, F, B = m.n_cells, m.n_internal_faces, m.n_boundary_faces
+    bc = fa.BoundaryConditions(m, ["fixedValue"] * m.n_patches)
+    T = fvcc.VolumeField(m, ctx.uniform(N, -1, 1, 3, 0), ctx.uniform(B, -1, 1, 3, 1), bc, "T")
+    gam = ctx.upload(np.full(F + B, 1e-2 * float(m.get("V").mean()) ** (2 / 3)))
+    ls = la.LinearSystem(la.SparsityPattern(m))
+    la.HeatAssembly([(ls, T.internal, 1.0, gam, bc, T.boundary, None)]).assemble(-1.0)
+    A, b = ls.scipy(), ls.rhs()
+    if name == "refined":
+        assert A.indptr[256] - A.indptr[0] > 2048
+    x0 = ctx.uniform(N, -1, 1, 3, 7)
+    xh = x0.numpy()
+    bt = la.Batch(ctx, precision, 2048, 2)  # tiles of two kScaleRows, one chunk
+    bt.add(ls, x0)
+    st = bt.solve({"relTol": 1e-30, "maxIter": 2, "innerRelTol": 1e-30}, use_graph=False,
+                  raise_on_noconverge=False)[0]
+    g = np.sqrt(A.diagonal())
+    G = sp.diags(1 / g)
+    As = G @ A @ G
+    r = (b - A @ xh) / g
+    ref0 = np.linalg.norm(r * g) / np.linalg.norm(b)
+    d, p = np.zeros(N), r.copy()
+    rho = r @ r
+    for _ in range(st.numIter):
+        if rho == 0.0:  # one row: solved by the first iteration
+            break
+        q = As @ p
+        a = rho / (p @ q)
+        d, r = d + a * p, r - a * q
+        rho, old = r @ r, rho
+        p = r + rho / old * p
+    eps = 2.0 ** -52 if precision == "double" else 2.0 ** -24
+    assert 1 <= st.numIter <= 2
+    assert abs(st.initResNorm - ref0) <= 64 * N * 2.0 ** -52 * ref0
+    ref = xh + d / g
+    scale = np.abs(xh).max() + np.abs(d / g).max()
+    assert np.abs(x0.numpy() - ref).max() <= 64 * (eps * np.abs(d / g).max() + 2.0 ** -52 * scale)
+    bt.close()
+    m.close()

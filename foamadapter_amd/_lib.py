@@ -132,6 +132,7 @@ _SIGS = {
     "fv_sngrad_uncorrected": [_vp, _vp, C.c_int, _vp, _vp, _vp, _vp, _vp],
     "fv_flux": [_vp, _vp, C.c_int, _vp, _vp, _vp],
     "fv_correct_boundary": [_vp, _vp, C.c_int, _vp, _vp, _vp, _vp],
+    "fv_correct_boundary_vec": [_vp, _vp, C.c_int, C.c_int, _vp, _vp, _vp, _vp],
     "fv_sparsity_create": [_vp, _pp],
     "fv_sparsity_destroy": [_vp],
     "fv_sparsity_sizes": [_vp, _vp],
@@ -159,10 +160,13 @@ _SIGS = {
     "fv_update_velocity_grad": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, C.POINTER(C.c_int)],
     "fv_constrain_hbya": [_vp, _vp, _vp],
     "fv_linsys_boundary_coeffs": [_vp, C.POINTER(_vp), C.POINTER(_vp)],
+    "fv_mean_magnitude": [_vp, _vp, _vp, C.POINTER(_d)],
     "fv_courant_number": [_vp, _vp, _vp, _d, C.POINTER(_d)],
     "fv_courant_number_noalloc": [_vp, _vp, _vp, _d, _vp],
     "fv_set_delta_t": [_d, _d, _d, _d, C.POINTER(_d)],
     "fv_solve_cg": [_vp, _vp, C.POINTER(FvSolveOpts), C.POINTER(FvSolverStats)],
+    "fv_solve_bicgstab_vec": [_vp, C.c_int, _vp, _vp, C.POINTER(FvSolveOpts), C.POINTER(FvSolverStats),
+                              C.POINTER(C.c_int)],
     "fv_solve_bicgstab": [_vp, _vp, C.POINTER(FvSolveOpts), C.POINTER(FvSolverStats)],
     "fv_batch_create": [_vp, C.c_int, C.c_int, C.c_int, _pp],
     "fv_batch_destroy": [_vp],

@@ -23,6 +23,7 @@
 // state field has one writer per kernel and is not read by that kernel.
 #include "cgpersist.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 using namespace fvhip;
@@ -295,8 +296,16 @@ __global__ void kbi_scale(int64_t n, const int32_t* __restrict__ src, const int3
 // (r, and p and v in alternating buffers), and the reader of a far column evaluates
 // its owner's p' = r + beta (p - omega v) or s = r - alpha v, so an iteration has
 // three grid exchanges.  The order of all sums is that of the kernels above (same
-// bits).  Advection step on 110x100x90 cells (31 iterations) 3.20 -> 1.76 ms, the
-// momentum solves of a 64^3 icoFoam step about 0.9 -> 0.4 ms.
+// bits).  Advection step on 110x100x90 cells (31 iterations) 3.20 -> 1.76 ms, an
+// icoFoam step at 64^3 (three momentum solves) 5.01 -> 4.25 ms.
+//
+// A Vec3 equation's right-hand sides and solutions are interleaved: the kernel reads
+// b and the initial x at a stride, keeps the x it publishes in a vector of its own
+// and writes the solution back once it has converged.  The solves of the components
+// are launched one behind another; one that does not converge in its launch, or
+// fails, makes those behind it return at once (prev).  With the boundary values in one
+// launch and the continuity error summed on the device, 45 component copies and two
+// field reads of an icoFoam step at 64^3 went: 4.39 -> 3.55 ms.
 struct BiPersist {
     int32_t N, tiles, rowsPerTile, iters;
     int32_t fresh;  // 1: start from x; 0: go on after `iters` iterations that did not stop
@@ -305,6 +314,10 @@ struct BiPersist {
     double tol, atol;
     const int32_t* sellCol;
     CsrSystem m;
+    int32_t stride;       // of m.rhs, x0 and out
+    const double* x0;     // initial x
+    double* out;          // the solution if it converged (null: x holds it)
+    const BiState* prev;  // component before this one: go on only if it converged
     double* sval;  // scaled values of the rows whose matrix does not stay in registers
     double *x, *r, *rhat, *p, *p2, *v, *v2;
     BiState* st;
@@ -331,6 +344,13 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
     const uint32_t cbase = (uint32_t)tile * R, lofs = (uint32_t)sub * (RPT * kB);
     BiState* const st = A.st;
     if (!A.fresh && st->stop) return;
+    if (A.prev && A.prev->stop != 2) {
+        if (gs.slot == 0 && tid == 0) st->stop = 0;
+        return;
+    }
+    // x at the start of the launch, at stride xs
+    const double* const xin = A.fresh ? A.x0 : A.x;
+    const int xs = A.fresh ? A.stride : 1;
     if (tid == 0) L.bad = 0;
     const int row0 = tile * R;
     const int row1 = tile < A.tiles ? min(row0 + R, (A.N + 63) & ~63) : row0;
@@ -367,8 +387,8 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
         if (!live(u)) break;
         double x0 = 0.0, d0 = 0.0;
         if (inN(u)) {
-            x0 = *mine(A.x, u);
             const int i = iw + u * kB + lane;
+            x0 = xin[(int64_t)i * xs];
             d0 = 1.0 / A.m.vals[A.m.rowOffs[i] + A.m.diag[i]];
         }
         lds(lx, u) = x0;
@@ -377,6 +397,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
     auto residual = [&](auto far, auto out) {
         tile_residual<RPT, W>(
             A.m, A.N, row0, row1, iw, l0 + sub * kRaw, live, column,
+            [&](int i) { return A.m.rhs[(int64_t)i * A.stride]; },
             [&](uint32_t o) { return *at_byte(lx, o); }, far, [&](int u) { return lds(lx, u); }, out);
     };
 
@@ -386,7 +407,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
     bool ok = true;
     {
         double s2[2] = {0.0, 0.0}, t2[2];
-        residual([&](uint32_t o) { return *at_byte(A.x, o); },
+        residual([&](uint32_t o) { return xin[(int64_t)(o / 8u) * xs]; },
                  [&](int u, bool, double ri, double bi, const double (&a)[W],
                      const uint32_t (&c)[W]) {
 #pragma unroll
@@ -591,6 +612,8 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
                     put_shared(mine(A.x, u), lds(lx, u));
                 else
                     *mine(A.x, u) = lds(lx, u);
+                if (A.out && stop == 2)
+                    A.out[(int64_t)(iw + u * kB + lane) * A.stride] = lds(lx, u);
             }
             if (!stop) {
                 *mine(A.r, u) = rv[u];
@@ -632,6 +655,8 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
     }
 }
 
+constexpr int kMaxComp = 3;
+
 // Workspace kept with the linear system between solves
 struct BiWork : fv_solver_cache {
     DBuf<double> sval, dinv, r, rhat, p, v, s, t, parts;
@@ -669,16 +694,27 @@ struct BiWork : fv_solver_cache {
         slots.alloc(c, 2 * (size_t)kSlotBuffer);
         FV_HIP(hipMemsetAsync(slots.p, 0, slots.n * sizeof(unsigned long long), c->stream));
     }
+    // One system of a solve: x in place, or component `comp` of `ncomp` interleaved ones
+    // (rhs, x), whose x between launches is dinv (the persistent form has no other use
+    // for it).
+    struct Target {
+        double* x;
+        const double* rhs;
+        int comp, ncomp;
+    };
     // Up to persistIters iterations; false if the device refuses the launch.
-    bool run_persist(hipStream_t s, double* x, const fv_solve_opts* o, bool fresh) {
+    bool run_persist(hipStream_t s, const Target& t, const fv_solve_opts* o, bool fresh, bool chained = false) {
         const uint32_t uses = 3 * (uint32_t)persistIters + 8;
         if (tag > 0xffffffffu - uses) {  // sequence numbers start over
             FV_HIP(hipMemsetAsync(slots.p, 0, slots.n * sizeof(unsigned long long), s));
             tag = 1;
         }
+        double* const x = t.x + t.comp;
+        BiState* const state = st.p + t.comp;
         BiPersist a{h.N, h.ntiles, h.rowsPerBlock, persistIters, fresh ? 1 : 0, o->max_iter, tag,
-                    o->rel_tol, o->abs_tol, h.sellCol, CsrSystem{h.rowOffs, diag, h.vals, h.rhs}, sval.p, x,
-                    h.r, h.rhat, h.p, h.s, h.v, h.t, h.st, slots.p};
+                    o->rel_tol, o->abs_tol, h.sellCol, CsrSystem{h.rowOffs, diag, h.vals, t.rhs + t.comp},
+                    t.ncomp, x, t.ncomp > 1 ? x : nullptr, chained ? state - 1 : nullptr, sval.p,
+                    t.ncomp > 1 ? dinv.p : x, h.r, h.rhat, h.p, h.s, h.v, h.t, state, slots.p};
         void* args[] = {&a};
         if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(persist), dim3(persistGrid),
                                        dim3(kPersistThreads), args, 0, s) != hipSuccess) {
@@ -701,7 +737,7 @@ struct BiWork : fv_solver_cache {
         for (DBuf<double>* b : {&dinv, &r, &rhat, &p, &v, &s, &t})
             b->alloc(c, ((size_t)N + 63) / 64 * 64);
         parts.alloc(c, 6 * (size_t)tiles);
-        st.alloc(c, 1);
+        st.alloc(c, kMaxComp);
         sys.alloc(c, 1);
         h.N = N;
         h.ntiles = tiles;
@@ -728,41 +764,100 @@ struct BiWork : fv_solver_cache {
         diag = sp->diagOffset.p;
         if (!c->shared) choose_persist(c, sp);
     }
+    // The states after the work queued so far (pinned, valid until the next read)
+    const BiState* states(fv_ctx* c, int n) {
+        static_assert(kMaxComp * sizeof(BiState) <= fv_ctx::kPollBytes, "poll area too small");
+        auto* const host = static_cast<BiState*>(ctx_poll_host(c));
+        FV_HIP(hipMemcpyAsync(host, st.p, n * sizeof(BiState), hipMemcpyDeviceToHost, c->stream));
+        FV_HIP(hipStreamSynchronize(c->stream));
+        return host;
+    }
+    // Goes on until component t.comp, last seen in state h, has stopped.
+    BiState finish_persist(fv_ctx* c, const Target& t, const fv_solve_opts* o, BiState h) {
+        while (!h.stop) {
+            FV_REQUIRE(run_persist(c->stream, t, o, false), "a cooperative launch was refused");
+            h = states(c, t.comp + 1)[t.comp];
+        }
+        if (h.stop == kStopSync) {
+            persist = nullptr;
+            throw Error{FV_EDEVICE, "persistent BiCGStab: the workgroups did not meet in " +
+                                        std::to_string(kSyncSeconds) + " s"};
+        }
+        return h;
+    }
 };
+
+BiWork& bi_work(fv_linsys* ls, const fv_solve_opts* o) {
+    FV_REQUIRE(o->rel_tol >= 0.0 && o->max_iter >= 0 && o->abs_tol >= 0.0, "bad solver options");
+    FV_REQUIRE(o->mode == FV_SOLVE_F64, "BiCGStab runs in FP64 only");
+    auto& slot = ls->cg[2];
+    if (!slot) slot.reset(new BiWork(ls->sp->mesh->ctx, ls));
+    return *static_cast<BiWork*>(slot.get());
+}
+
+// stats of a stopped solve; throws unless it converged
+void bi_finish(const BiState& h, fv_solver_stats& st) {
+    st.init_res = h.res0;
+    st.final_res = h.res;
+    st.iters = h.it;
+    st.outer_iters = 1;
+    if (h.stop == 3)
+        throw Error{FV_ENOCONVERGE, "BiCGStab breakdown at iteration " + std::to_string(h.it)};
+    if (h.stop != 2)
+        throw Error{FV_ENOCONVERGE, "BiCGStab stopped at relative residual " + std::to_string(h.res) +
+                                        " after " + std::to_string(h.it) + " iterations"};
+}
 
 }  // namespace
 
 extern "C" {
 
+int fv_solve_bicgstab_vec(fv_linsys* ls, int ncomp, const void* d_rhs, void* d_x,
+                          const fv_solve_opts* o, fv_solver_stats* stats, int* solved) {
+    if (solved) *solved = 0;
+    return guarded([&] {
+        FV_REQUIRE(ls && ls->sp && d_rhs && d_x && o && stats && solved, "NULL argument");
+        FV_REQUIRE(ncomp >= 1 && ncomp <= kMaxComp, "one to three components");
+        BiWork& w = bi_work(ls, o);
+        fv_ctx* ctx = ls->sp->mesh->ctx;
+        if (o->eager) return;
+        auto target = [&](int k) { return BiWork::Target{(double*)d_x, (const double*)d_rhs, k, ncomp}; };
+        // the system's right-hand side is that of the component solved last
+        auto keep_rhs = [&](int k) {
+            const int rc = fv_component(ctx, FV_F64, ls->sp->nRows, ncomp, k, 0, d_rhs, ls->rhs.p);
+            if (rc != FV_OK) throw Error{rc, fv_last_error()};
+        };
+        int& k = *solved;
+        while (k < ncomp && w.persist) {
+            int n = k;  // components launched
+            while (n < ncomp && w.run_persist(ctx->stream, target(n), o, true, n > k)) ++n;
+            if (n == k) return;
+            BiState h[kMaxComp];
+            std::copy_n(w.states(ctx, n), n, h);
+            for (bool gone_on = false; k < n && !gone_on; ++k) {
+                gone_on = h[k].stop == 0;  // those behind it returned at once
+                h[k] = w.finish_persist(ctx, target(k), o, h[k]);
+                stats[k].true_res = h[k].trueRes;
+                if (h[k].stop != 2) keep_rhs(k);
+                bi_finish(h[k], stats[k]);
+            }
+        }
+        if (k) keep_rhs(k - 1);
+    });
+}
+
 int fv_solve_bicgstab(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stats* stats) {
     fv_solver_stats local{};
     int rc = guarded([&] {
         FV_REQUIRE(ls && ls->sp && d_x && o, "NULL argument");
-        FV_REQUIRE(o->rel_tol >= 0.0 && o->max_iter >= 0 && o->abs_tol >= 0.0,
-                   "bad solver options");
-        FV_REQUIRE(o->mode == FV_SOLVE_F64, "BiCGStab runs in FP64 only");
+        BiWork& w = bi_work(ls, o);
         fv_sparsity* sp = ls->sp;
         fv_ctx* ctx = sp->mesh->ctx;
         hipStream_t s = ctx->stream;
-        auto& slot = ls->cg[2];
-        if (!slot) slot.reset(new BiWork(ctx, ls));
-        BiWork& w = *static_cast<BiWork*>(slot.get());
         BiState h{};
-        if (!o->eager && w.persist && w.run_persist(s, (double*)d_x, o, true)) {
-            BiState* const host = static_cast<BiState*>(ctx_poll_host(ctx));
-            static_assert(sizeof(BiState) <= fv_ctx::kPollBytes, "poll area too small");
-            while (true) {
-                FV_HIP(hipMemcpyAsync(host, w.st.p, sizeof h, hipMemcpyDeviceToHost, s));
-                FV_HIP(hipStreamSynchronize(s));
-                h = *host;
-                if (h.stop) break;
-                FV_REQUIRE(w.run_persist(s, (double*)d_x, o, false), "a cooperative launch was refused");
-            }
-            if (h.stop == kStopSync) {
-                w.persist = nullptr;
-                throw Error{FV_EDEVICE, "persistent BiCGStab: the workgroups did not meet in " +
-                                            std::to_string(kSyncSeconds) + " s"};
-            }
+        const BiWork::Target t{(double*)d_x, ls->rhs.p, 0, 1};
+        if (!o->eager && w.persist && w.run_persist(s, t, o, true)) {
+            h = w.finish_persist(ctx, t, o, *w.states(ctx, 1));
             local.true_res = h.trueRes;
         } else {
             w.h.x = (double*)d_x;
@@ -802,16 +897,7 @@ int fv_solve_bicgstab(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solve
             FV_HIP(hipStreamSynchronize(s));
             local.true_res = h2.res0;
         }
-        local.init_res = h.res0;
-        local.final_res = h.res;
-        local.iters = h.it;
-        local.outer_iters = 1;
-        if (h.stop == 3)
-            throw Error{FV_ENOCONVERGE, "BiCGStab breakdown at iteration " + std::to_string(h.it)};
-        if (h.stop != 2)
-            throw Error{FV_ENOCONVERGE, "BiCGStab stopped at relative residual " +
-                                            std::to_string(h.res) + " after " +
-                                            std::to_string(h.it) + " iterations"};
+        bi_finish(h, local);
     });
     if (stats) *stats = local;
     return rc;

@@ -346,15 +346,16 @@ constexpr uint32_t kFar = 0x80000000u;
 // b - A x of a tile's rows, their entries in column order, 256 rows at a time: the
 // matrix rows are read coalesced into raw ((W + 1) * 256 doubles of LDS) and taken
 // from there.  column(u, k): the columns; near(o), far(o), own(u): x at an LDS
-// offset, at a vector offset, of this thread's row u.  out(u, in, r, b, a, c) gets
+// offset, at a vector offset, of this thread's row u; rhs(i): the right-hand side.
+// out(u, in, r, b, a, c) gets
 // each row's residual and right-hand side (zero past N) and its off-diagonal
 // values and columns.  Every thread of the workgroup calls it; barriers before the
 // first and after the last use of raw.
-template <int RPT, int W, typename Live, typename Col, typename Near, typename Far, typename Own,
-          typename Out>
+template <int RPT, int W, typename Live, typename Col, typename Rhs, typename Near, typename Far,
+          typename Own, typename Out>
 __device__ __forceinline__ void tile_residual(const CsrSystem& m, int N, int row0, int row1, int iw,
-                                              double* raw, Live live, Col column, Near near,
-                                              Far far, Own own, Out out) {
+                                              double* raw, Live live, Col column, Rhs rhs,
+                                              Near near, Far far, Own own, Out out) {
     const int lane = (int)threadIdx.x & 63;
 #pragma unroll
     for (int u = 0; u < RPT; ++u) {
@@ -373,7 +374,7 @@ __device__ __forceinline__ void tile_residual(const CsrSystem& m, int N, int row
             const bool in = i < N;
             const int o = in ? m.rowOffs[i] - b : 0, len = in ? m.rowOffs[i + 1] - b - o : 0;
             const int dg = in ? m.diag[i] : 0;
-            const double bi = in ? m.rhs[i] : 0.0;
+            const double bi = in ? rhs(i) : 0.0;
             uint32_t c[W];
             double a[W], x[W];
 #pragma unroll
@@ -484,7 +485,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     [[maybe_unused]] auto residual = [&](auto far, auto out) {
         tile_residual<RPT, W>(
             A.m, A.N, row0, row1, iw, raw + sub * kRaw, live, column,
-            [&](uint32_t o) { return *at_byte(lp, o); }, far, [&](int u) { return lds(lp, u); }, out);
+            [&](int i) { return A.m.rhs[i]; }, [&](uint32_t o) { return *at_byte(lp, o); }, far, [&](int u) { return lds(lp, u); }, out);
     };
     if constexpr (!WHOLE) {
 #pragma unroll

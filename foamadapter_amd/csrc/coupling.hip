@@ -12,6 +12,7 @@
 // matrix is the scalar system (the reference reads component 0 of its Vec3
 // coefficients, "all the diagonal coefficients are the same"), the right-hand
 // side and the fields are Vec3 (xyz interleaved).
+#include "cgstate.hpp"
 #include "implicit.hpp"
 
 #include <algorithm>
@@ -242,6 +243,28 @@ __global__ __launch_bounds__(kBlock) void k_conum_final(int n, const double* __r
     if (threadIdx.x == 0) *co = 0.5 * sh[0] * dt;
 }
 
+// per block the sums of V |a| and V over its cells; then one block, theirs over all
+// blocks (n of them) and the ratio
+constexpr int kMeanBlocks = 512;
+__global__ __launch_bounds__(kBlock) void k_mean_mag(int N, const double* __restrict__ V,
+                                                     const double* __restrict__ a,
+                                                     double* __restrict__ part) {
+    __shared__ double sh[2 * (kBlock / 64)];
+    double v[2] = {0.0, 0.0};
+    for (int c = blockIdx.x * kBlock + threadIdx.x; c < N; c += gridDim.x * kBlock) {
+        v[0] += V[c] * fabs(a[c]);
+        v[1] += V[c];
+    }
+    write_slot<2>(v, part, (int)blockIdx.x, sh);
+}
+__global__ __launch_bounds__(kBlock) void k_mean_mag_final(int n, const double* __restrict__ part,
+                                                           double* __restrict__ mean) {
+    __shared__ double sh[2 * (kBlock / 64)];
+    double t[2];
+    sum_slots<2>(part, 0, n, sh, t);
+    if (threadIdx.x == 0) *mean = t[0] / t[1];
+}
+
 // Device address of `scratch` on each device, looked up once per device with
 // that device current (a fixed table: the lookup allocates nothing).
 constexpr int kScratchDevices = 64;
@@ -267,6 +290,14 @@ double* scratch_on(int device) {
 }
 
 void check_ls(const fv_linsys* ls) { FV_REQUIRE(ls && ls->sp && ls->sp->mesh, "NULL linear system"); }
+
+// one value through the context's pinned area: a copy into pageable memory is staged
+double read_double(fv_ctx* ctx, const double* d) {
+    auto* const h = static_cast<double*>(ctx_poll_host(ctx));
+    FV_HIP(hipMemcpyAsync(h, d, sizeof *h, hipMemcpyDeviceToHost, ctx->stream));
+    FV_HIP(hipStreamSynchronize(ctx->stream));
+    return *h;
+}
 
 }  // namespace
 
@@ -360,6 +391,19 @@ int fv_constrain_hbya(const fv_bc* ubc, const void* d_Ub, void* d_hbya_b) {
     });
 }
 
+int fv_mean_magnitude(fv_ctx* ctx, const fv_mesh* m, const void* d_div, double* mean) {
+    return guarded([&] {
+        FV_REQUIRE(ctx && m && m->ctx == ctx && d_div && mean, "bad arguments");
+        const int G = std::min(grid_for(m->nCells, kBlock), kMeanBlocks);
+        DBuf<double> part;
+        part.alloc(ctx, 2 * (size_t)G + 1);
+        k_mean_mag<<<G, kBlock, 0, ctx->stream>>>(m->nCells, m->V.p, (const double*)d_div, part.p);
+        k_mean_mag_final<<<1, kBlock, 0, ctx->stream>>>(G, part.p, part.p + 2 * G);
+        FV_LAUNCH_CHECK();
+        *mean = read_double(ctx, part.p + 2 * G);
+    });
+}
+
 int fv_courant_number(fv_ctx* ctx, const fv_mesh* m, const void* d_phi, double dt, double* co) {
     return guarded([&] {
         FV_REQUIRE(ctx && m && m->ctx == ctx && d_phi && co, "bad arguments");
@@ -369,11 +413,9 @@ int fv_courant_number(fv_ctx* ctx, const fv_mesh* m, const void* d_phi, double d
         k_conum<<<G, kBlock, 0, ctx->stream>>>(m->nCells, m->nInt, m->cfOff.p, m->cfIdx.p,
                                                 (const double*)d_phi, m->V.p, bm.p);
         FV_LAUNCH_CHECK();
-        std::vector<double> h(G);
-        bm.download(h.data());
-        double mx = 0.0;
-        for (double v : h) mx = std::max(mx, v);
-        *co = 0.5 * mx * dt;
+        k_conum_final<<<1, kBlock, 0, ctx->stream>>>(G, bm.p, dt, bm.p);
+        FV_LAUNCH_CHECK();
+        *co = read_double(ctx, bm.p);
     });
 }
 

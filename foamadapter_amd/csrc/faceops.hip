@@ -871,8 +871,9 @@ __global__ __launch_bounds__(kBlock) void k_flux(int F, int B, const int32_t* __
 
 // fixedGradient patches: Tb = T_P + g/deltaCoeffs (fixedGradientFvPatchField::evaluate);
 // fixedValue and calculated faces keep their stored value
+// (nc components, interleaved: the kinds are the same for all)
 template <typename S>
-__global__ __launch_bounds__(kBlock) void k_correct_bc(int B, const int32_t* __restrict__ fc,
+__global__ __launch_bounds__(kBlock) void k_correct_bc(int B, int nc, const int32_t* __restrict__ fc,
                                                        const double* __restrict__ dcb,
                                                        const int8_t* __restrict__ kind,
                                                        const S* __restrict__ T,
@@ -880,8 +881,11 @@ __global__ __launch_bounds__(kBlock) void k_correct_bc(int B, const int32_t* __r
                                                        S* __restrict__ Tb) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= B || kind[b] != FV_BC_FIXED_GRADIENT) return;
-    const S g = Tg ? Tg[b] : S(0);
-    Tb[b] = T[fc[b]] + g / (S)dcb[b];
+    const int64_t c = (int64_t)nc * fc[b], f = (int64_t)nc * b;
+    for (int j = 0; j < nc; ++j) {
+        const S g = Tg ? Tg[f + j] : S(0);
+        Tb[f + j] = T[c + j] + g / (S)dcb[b];
+    }
 }
 
 // Operator drivers: the LDS-staged gather on upper-triangular meshes, the
@@ -1113,24 +1117,29 @@ int fv_flux(fv_ctx* ctx, const fv_mesh* mc, fv_prec prec, const void* U, const v
     });
 }
 
-int fv_correct_boundary(fv_ctx* ctx, const fv_mesh* mc, fv_prec prec, const void* T,
-                        const fv_bc* bc, const void* Tg, void* Tb) {
+int fv_correct_boundary_vec(fv_ctx* ctx, const fv_mesh* mc, fv_prec prec, int ncomp, const void* T,
+                            const fv_bc* bc, const void* Tg, void* Tb) {
     return guarded([&] {
         fv_mesh* m = const_cast<fv_mesh*>(mc);
         check_common(ctx, m, prec);
         check_bc(m, bc);
-        FV_REQUIRE(T && (Tb || m->nB == 0), "NULL field");
+        FV_REQUIRE(ncomp >= 1 && T && (Tb || m->nB == 0), "NULL field");
         if (!m->nB) return;
         if (prec == FV_F64)
             k_correct_bc<double><<<grid_for(m->nB, kBlock), kBlock, 0, ctx->stream>>>(
-                m->nB, m->faceCells.p, m->dcb.p, bc->faceKind.p, (const double*)T,
+                m->nB, ncomp, m->faceCells.p, m->dcb.p, bc->faceKind.p, (const double*)T,
                 (const double*)Tg, (double*)Tb);
         else
             k_correct_bc<float><<<grid_for(m->nB, kBlock), kBlock, 0, ctx->stream>>>(
-                m->nB, m->faceCells.p, m->dcb.p, bc->faceKind.p, (const float*)T,
+                m->nB, ncomp, m->faceCells.p, m->dcb.p, bc->faceKind.p, (const float*)T,
                 (const float*)Tg, (float*)Tb);
         FV_LAUNCH_CHECK();
     });
+}
+
+int fv_correct_boundary(fv_ctx* ctx, const fv_mesh* mesh, fv_prec prec, const void* T,
+                        const fv_bc* bc, const void* Tg, void* Tb) {
+    return fv_correct_boundary_vec(ctx, mesh, prec, 1, T, bc, Tg, Tb);
 }
 
 }  // extern "C"

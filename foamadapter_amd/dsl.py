@@ -18,7 +18,7 @@ import numpy as np
 
 from ._lib import FV_LINEAR, FV_UPWIND, FvTerm, call, lib
 from . import fvcc
-from .la import LinearSystem, SparsityPattern, SolverStats, solve_cg
+from .la import LinearSystem, SparsityPattern, SolverStats, solve_cg, solve_components
 from .runtime import DeviceArray
 
 
@@ -244,8 +244,8 @@ def _assemble_vec(expr, psi, t, dt, ls):
 def _solve_vec(ls: LinearSystem, psi: fvcc.VolumeField, solver) -> list[SolverStats]:
     """Each component of psi solved on the shared matrix with its right-hand side."""
     ctx = psi.mesh.ctx
-    stats = []
-    for k in range(psi.ncomp):
+    stats = solve_components(ls, ls.rhs3, psi.internal, solver)
+    for k in range(len(stats), psi.ncomp):
         b = fvcc.component(ls.rhs3, k)
         call("fv_memcpy_d2d", ctx.handle, lib.fv_linsys_rhs(ls.handle), b.ptr, b.nbytes)
         x = fvcc.component(psi.internal, k)

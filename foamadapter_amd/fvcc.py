@@ -72,14 +72,8 @@ class VolumeField:
         component of a Vec3 field)."""
         if self.bcs is None or self.mesh.n_boundary_faces == 0:
             return
-        if self.ncomp > 1:
-            for k in range(self.ncomp):
-                c = self.component(k)
-                c.correct_boundary_conditions()
-                set_component(self.boundary, k, c.boundary)
-            return
-        call("fv_correct_boundary", self.mesh.ctx.handle, self.mesh.handle, prec_of(self.dtype),
-             self.internal.ptr, self.bcs.handle,
+        call("fv_correct_boundary_vec", self.mesh.ctx.handle, self.mesh.handle, prec_of(self.dtype),
+             self.ncomp, self.internal.ptr, self.bcs.handle,
              self.boundary_gradient.ptr if self.boundary_gradient is not None else None,
              self.boundary.ptr)
 

@@ -338,3 +338,19 @@ def solve_cg(ls: LinearSystem, x: DeviceArray, solver: dict | None = None,
     if rc not in (_lib.FV_OK, _lib.FV_ENOCONVERGE) or (rc != _lib.FV_OK and raise_on_noconverge):
         raise _lib.FvError(rc, _lib.last_error())
     return SolverStats(st.init_res, st.final_res, st.iters, st.outer_iters, st.true_res, rc)
+
+
+def solve_components(ls: LinearSystem, rhs: DeviceArray, x: DeviceArray,
+                     solver: dict | None = None) -> list[SolverStats]:
+    """The components of x [N, ncomp] solved in order with their right-hand sides on the
+    shared matrix, as far as fv_solve_bicgstab_vec takes them (none for CG): their stats.
+    solve_cg solves the others."""
+    o = solver_opts(solver)
+    n = x.shape[1]
+    if _method(dict(solver or {})) != "bicgstab" or n > 3 or x.dtype != np.float64:
+        return []
+    st = (_lib.FvSolverStats * n)()
+    solved = C.c_int()
+    call("fv_solve_bicgstab_vec", ls.handle, n, rhs.ptr, x.ptr, C.byref(o), st, C.byref(solved))
+    return [SolverStats(s.init_res, s.final_res, s.iters, s.outer_iters, s.true_res, _lib.FV_OK)
+            for s in st[:solved.value]]

@@ -279,6 +279,9 @@ int fv_sngrad_uncorrected(fv_ctx* ctx, const fv_mesh* mesh, fv_prec prec, const 
  * calculated faces keep their stored values.  Updates d_Tb[B] in place. */
 int fv_correct_boundary(fv_ctx* ctx, const fv_mesh* mesh, fv_prec prec, const void* d_T,
                         const fv_bc* bc, const void* d_Tgrad, void* d_Tb);
+/* The same for an interleaved field of ncomp components per cell and face. */
+int fv_correct_boundary_vec(fv_ctx* ctx, const fv_mesh* mesh, fv_prec prec, int ncomp,
+                            const void* d_T, const fv_bc* bc, const void* d_Tgrad, void* d_Tb);
 /* Face flux phi = Sf . interpolate_linear(U) (FoamAdapter::flux,
  * src/algorithms/pressureVelocityCoupling.cpp:242-264): U[3N], Ub[3B] -> phi[F+B]. */
 int fv_flux(fv_ctx* ctx, const fv_mesh* mesh, fv_prec prec, const void* d_U, const void* d_Ub,
@@ -419,6 +422,16 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* opts, fv_solver_s
  * FV_ENOCONVERGE on the iteration limit or a breakdown (rho or omega zero). */
 int fv_solve_bicgstab(fv_linsys* ls, void* d_x, const fv_solve_opts* opts,
                       fv_solver_stats* stats);
+/* The same for the components of a Vec equation on the shared matrix, in order, with
+ * interleaved right-hand sides d_rhs[N*ncomp] and solutions d_x[N*ncomp] (ncomp <= 3):
+ * component k of d_x is replaced once its solve has converged.  Runs where the solve
+ * is one persistent launch: *solved says how many components were solved, and the
+ * caller solves the rest one by one (all of them where it is 0: opts->eager, wide rows,
+ * systems of over 2^20 rows).  On FV_ENOCONVERGE component *solved did not converge and
+ * the later ones were not touched.  The system's own right-hand side becomes that of
+ * the component solved last. */
+int fv_solve_bicgstab_vec(fv_linsys* ls, int ncomp, const void* d_rhs, void* d_x,
+                          const fv_solve_opts* opts, fv_solver_stats* stats, int* solved);
 
 /* ---- pressure-velocity coupling (src/algorithms/pressureVelocityCoupling.cpp) ---
  * FP64.  The momentum matrix is the scalar system ls (the reference reads
@@ -453,6 +466,9 @@ int fv_update_velocity_grad(fv_ctx* ctx, const fv_mesh* m, const void* d_hbya, c
 /* constrainHbyA (:14-36): HbyA_b = U_b on the faces of patches whose velocity
  * condition is not assignable (fixedValue); other faces keep their value. */
 int fv_constrain_hbya(const fv_bc* u_bc, const void* d_Ub, void* d_hbya_b);
+/* sum_c V_c |div_c| / sum_c V_c of a cell field d_div[N] (OpenFOAM continuityErrs.H:
+ * dt times this for the divergence of the flux), in a fixed order, to the host. */
+int fv_mean_magnitude(fv_ctx* ctx, const fv_mesh* mesh, const void* d_div, double* mean);
 /* Courant number (NeoN computeCoNum, examples/scalarAdvection/scalarAdvection.cpp:69;
  * OpenFOAM CourantNo.H): co = 0.5 * max_c(sum_faces |phi| / V_c) * dt over the
  * internal and boundary faces of each cell, d_phi [F+B] FP64. */

@@ -109,3 +109,75 @@ def test_persistent_bicgstab_is_bitwise_the_kernel_by_kernel_form(ctx, dims, lim
         assert g[1:] == got[0][1:]
         assert np.array_equal(g[0], got[0][0])
     m.close()
+
+
+VEC_CASES = [((3, 3, 3), 100), ((17, 16, 16), 100), ((16, 16, 1), 200),
+             ((41, 40, 40), 400),     # components of several launches
+             ((64, 64, 65), 130),     # 2 rows per thread; the limit ends the first component
+             ((17, 16, 16), 1)]       # no component converges
+
+
+@pytest.mark.parametrize("kind", ["advection", "diffusion"])
+@pytest.mark.parametrize("dims,limit", VEC_CASES, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_vec_components_are_bitwise_the_single_solves(ctx, dims, limit, kind):
+    """The components of a Vec3 equation solved from interleaved arrays against the kernel-by-kernel
+    solves of component copies: solutions, stats, the system's right-hand side, and what an error leaves."""
+    import foamadapter_amd as fa
+    from foamadapter_amd import _lib, dsl, fvcc
+    print(dims, limit, kind, flush=True)
+    m, ls = _system(ctx, dims)
+    N, F, B = m.n_cells, m.n_internal_faces, m.n_boundary_faces
+    if kind == "advection":
+        T = fvcc.VolumeField(m, ctx.uniform(N, -1, 1, 12, 0), ctx.uniform(B, -1, 1, 12, 1),
+                             fa.BoundaryConditions(m, ["fixedValue"] * m.n_patches), "T")
+        phi = fvcc.SurfaceField(m, ctx.uniform(F + B, -1e-6, 1e-6, 12, 2))
+        gamma = fvcc.SurfaceField(m, ctx.uniform(F + B, 0.5, 2.0, 12, 3))
+        dt = 0.5 * float(m.get("V").mean()) ** (2.0 / 3.0)
+        dsl.assemble(dsl.imp.ddt(T) + dsl.imp.div(phi, T, "upwind") - dsl.imp.laplacian(gamma, T), T, 0.0, dt, ls)
+    b3 = ctx.uniform(3 * N, -1, 1, 13, 1)
+    b3.shape = (N, 3)
+    got = []
+    for graph in (False, True, True):
+        x3 = ctx.uniform(3 * N, -1, 1, 13, 2)
+        x3.shape = (N, 3)
+        ls.rhs3 = b3
+        st = err = None
+        try:
+            st = dsl._solve_vec(ls, fvcc.VolumeField(m, x3, None), {"solver": "PBiCGStab", "relTol": 1e-9,
+                                                                    "maxIter": limit, "graph": graph})
+        except _lib.FvError as e:
+            err = str(e)
+        got.append((x3.numpy(), ls.rhs(), st, err))
+    assert (got[0][3] is not None) == (limit == 1 or got[0][2] is None)
+    for g in got[1:]:
+        assert g[2:] == got[0][2:]
+        assert np.array_equal(g[0], got[0][0]) and np.array_equal(g[1], got[0][1])
+    m.close()
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (17, 16, 1), (61, 60, 59)], ids=str)
+def test_vec_boundary_and_mean_magnitude(ctx, dims):
+    import ctypes as C
+    import foamadapter_amd as fa
+    from foamadapter_amd import _lib, fvcc
+    print(dims, flush=True)
+    m = fa.Mesh.from_poly(ctx, fa.PolyMesh.hex(dims, jitter=0.2, jitter_seed=2))
+    N, B = m.n_cells, m.n_boundary_faces
+    kinds = (["fixedGradient", "fixedValue", "zeroGradient"] * m.n_patches)[:m.n_patches]
+    bc = fa.BoundaryConditions(m, kinds)
+    u, ub, ug = (ctx.uniform(3 * n, -1, 1, 14, i) for i, n in enumerate((N, B, B)))
+    u.shape, ub.shape, ug.shape = (N, 3), (B, 3), (B, 3)
+    ref, po, fc, dc = ub.numpy().copy(), m.get("patchOffsets"), m.get("faceCells"), m.get("deltaCoeffs_b")
+    for i, k in enumerate(kinds):
+        if k != "fixedValue":
+            r = slice(po[i], po[i + 1])
+            ref[r] = u.numpy()[fc[r]] + ug.numpy()[r] / dc[r, None]
+    fvcc.VolumeField(m, u, ub, bc, "U", ug).correct_boundary_conditions()
+    assert np.array_equal(ub.numpy(), ref)
+    d = ctx.uniform(N, -1, 1, 14, 5)
+    mean = C.c_double()
+    _lib.call("fv_mean_magnitude", ctx.handle, m.handle, d.ptr, C.byref(mean))
+    V = m.get("V")
+    want = np.sum(V * np.abs(d.numpy())) / np.sum(V)
+    assert abs(mean.value - want) <= 4 * N * 2.3e-16 * want  # two pairs of sums of N terms
+    m.close()

@@ -12,16 +12,23 @@
 //
 //  * a workgroup of 1024 threads per CU takes four tiles of 256 threads, the
 //    tiles (rows, order, partial sums) of cgkernels.hpp; a thread keeps r and q of
-//    its RPT rows in registers, p and d in LDS, g in either;
+//    its RPT rows in registers, p in LDS, d and g in either;
 //  * the matrix rows stay in registers where they fit (RES of the RPT rows: all
 //    of them up to 2 FP64 or 4 FP32 rows per thread); the others are read every
-//    iteration (72 bytes per FP64 row, 48 FP32);
-//  * a column of the tile's own rows (83 % of them in a Z-order tile of 256 rows,
-//    92 % of 2048) is read from LDS.  For the others, each tile publishes r of its
-//    rows that have such a column (the pattern is symmetric, so they are the ones
-//    others read) after the update and p after the direction, and the reader
-//    evaluates p' = r + beta p, the expression of the row's owner, so p' itself is
-//    needed by nobody before the next reduction: two grid exchanges per iteration.
+//    iteration, 60 bytes per FP64 row, 36 FP32: values, and columns as 16-bit LDS
+//    places (k_ghost_plan);
+//  * the rows of other tiles that a tile's columns refer to (its ghosts: 800 to 1300
+//    for 2048 rows in Z order) have places in its LDS as well.  A tile keeps its
+//    ghosts' p itself, by p' = r + beta p, the expression of the row's owner, so all
+//    it reads is their r, which every tile publishes for the rows that others refer
+//    to (the pattern is symmetric: those with ghost columns) after the update: two
+//    grid exchanges per iteration, one read of each ghost, and the product reads
+//    nothing but LDS beside the matrix.  Reading r and the old p of a far column
+//    where the product meets it, as kc_persist_far does, took 42.8 us an iteration
+//    at 128^3 FP64 against 28.0 (its loads, 8 % of the columns, stall the stream);
+//    with 32 registers spilled this form took 32.8, and the wait for a row's loads
+//    before the next is issued costs less than the spills a second row in flight
+//    brings.
 //
 // Grid reduction without atomics or fences: a workgroup publishes its partial
 // sums as 64-bit words, half payload and half sequence number, and the readers
@@ -33,20 +40,22 @@
 // wait for each other); with an agent-scope fence in every wave the same exchange
 // took 31-86 us for 256 (each fence is an L2 write-back or invalidate).  The
 // published vectors therefore go through agent-scope relaxed stores and loads,
-// which pass the per-XCD L2s.  Either the words carry the iteration's tag too
-// (TAGGED: small systems, where the 1.2 us of waiting for the stores counts), or a
-// wave waits for its stores to complete (vmcnt) before the workgroup's barrier,
-// behind which its partial sum is published.
+// which pass the per-XCD L2s, and a wave waits for its stores to complete (vmcnt)
+// before the workgroup's barrier, behind which its partial sum is published.  (Words
+// that carry the iteration's tag, which need no such wait, cost twice the bytes: 5.3
+// -> 5.5 us at 32^3 FP64, 9.5 -> 10.7 at 80^3; in FP32 they gained 0.3 us up to 64^3
+// and lost 0.9 at 96^3.)
 //
 // The launch is cooperative, so its workgroups are resident together.  Every
 // wait is bounded by a clock: a workgroup that waits longer than kSyncSeconds
 // sets stop = kStopSync and ends, and so do the others.
 //
-// Measured per iteration (pressure equation on jittered cubes, kernel-by-kernel
-// form -> this one): FP64 32^3 10.9 -> 6.8 us, 64^3 21.6 -> 10.2, 96^3 39.6 ->
-// 19.8, 128^3 65.9 -> 42.8; FP32 32^3 10.9 -> 6.2, 64^3 16.4 -> 8.5, 96^3 27.3 ->
-// 13.4, 128^3 42.5 -> 26.3.  At 128^3 FP64 27 of the 43 us are the matrix stream
-// (5.6 TB/s), 11 the two exchanges with their waits for the slowest workgroup.
+// Measured per iteration (pressure equation on jittered cubes in Z order,
+// kernel-by-kernel form -> this one): FP64 32^3 10.8 -> 5.3 us, 64^3 21.6 -> 8.1, 96^3
+// 39.6 -> 12.6, 128^3 65.6 -> 28.0; FP32 32^3 10.9 -> 5.8, 64^3 16.4 -> 7.8, 96^3 27.3
+// -> 10.4, 128^3 42.3 -> 15.6.  At 128^3 FP64 12 of the 28 us are the matrix stream
+// (126 MB, from the memory-side cache), 16 the rest: two exchanges (2.4 us each on an
+// idle chip) with their waits for the slowest workgroup, the ghosts, the LDS reads.
 #pragma once
 
 #include "cgkernels.hpp"
@@ -80,8 +89,11 @@ struct CgPersist {
     const int32_t* sellCol;  // slices of one width W: entry k of row i at
     const S* sval;           // (i / 64) * 64 W + 64 k + i % 64
     const S* g;
-    S *d, *r, *p, *p2;
-    unsigned long long* rtag;  // published r with its iteration's tag (TAGGED)
+    S *d, *r, *p;
+    S* p2;                   // (kc_persist_far)
+    const uint32_t* words;   // the columns, see k_ghost_plan; ghosts of each tile
+    const int32_t *ghosts, *count;
+    int32_t ghostStride;
     CgState* st;
     unsigned long long* slots;  // 2 * kSlotBuffer
     // WHOLE: the system, its solution, and the solve's limits; fresh: start from x,
@@ -124,48 +136,6 @@ template <typename T>
 __device__ __forceinline__ const T* at_byte(const T* base, uint32_t off) {
     return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + off);
 }
-
-// A published value that carries its tag: one 64-bit word in FP32, two in FP64.
-// The reader sees from the words themselves whether they have arrived, so the
-// writer need not wait for its stores before it tells the others.
-template <typename S>
-struct Tagged {
-    static constexpr int n = (int)(sizeof(S) / 4);
-    unsigned long long w[n];
-    __device__ __forceinline__ static void store(unsigned long long* at, S x, uint32_t tag) {
-        if constexpr (n == 1) {
-            put_shared(at, (unsigned long long)__float_as_uint(x) << 32 | tag);
-        } else {
-            const unsigned long long b = (unsigned long long)__double_as_longlong(x);
-            put_shared(at, b << 32 | tag);
-            put_shared(at + 1, (b & 0xffffffff00000000ull) | tag);
-        }
-    }
-    __device__ __forceinline__ void load(const unsigned long long* at) {
-        for (int j = 0; j < n; ++j) w[j] = get_shared(at + j);
-    }
-    __device__ __forceinline__ bool is(uint32_t tag) const {
-        bool ok = true;
-        for (int j = 0; j < n; ++j) ok = ok && (uint32_t)w[j] == tag;
-        return ok;
-    }
-    __device__ __forceinline__ S value() const {
-        if constexpr (n == 1)
-            return __uint_as_float((uint32_t)(w[0] >> 32));
-        else
-            return __longlong_as_double(
-                (long long)(w[0] >> 32 | (w[n - 1] & 0xffffffff00000000ull)));
-    }
-    // Loads until the words carry the tag; false after kSyncSeconds.
-    __device__ __forceinline__ bool wait(const unsigned long long* at, uint32_t tag) {
-        const unsigned long long t0 = wall_clock64();
-        do {
-            load(at);
-            if (is(tag)) return true;
-        } while (wall_clock64() - t0 < kSyncSeconds * kClockHz);
-        return false;
-    }
-};
 
 // Lane l of the lower half of a group of 2 * OFF lanes: x of lane l + OFF (what
 // __shfl_down gives those lanes; the others get something).  Register moves
@@ -397,27 +367,79 @@ __device__ __forceinline__ void tile_residual(const CsrSystem& m, int N, int row
     __syncthreads();
 }
 
+// Places of other tiles' rows ("ghosts") a tile's LDS has: as many as its rows can
+// refer to where that fits beside the vectors, else what is left of the 160 KB.
+template <typename S>
+constexpr int ghost_cap(int rpt, int W) {
+    if (sizeof(S) == 8) return rpt == 1 ? (W + 1) * kCgBlock : rpt == 2 ? rpt * kCgBlock * W : rpt == 4 ? 3008 : 1760;
+    return rpt <= 4 ? rpt * kCgBlock * W : 5632;
+}
+
+// The columns of a tile's rows as 16-bit byte offsets in the tile's LDS: its own rows
+// first (`own` places), then its ghosts, numbered in the order of rows blocks of 256,
+// entries, rows; two columns a word, words as the sliced ELL's values (entry pair j
+// of row i at (i / 64) * 32 W + 64 j + i % 64).  ghosts[tile * stride + slot]: the
+// rows they are.  Without words only the counts are taken.
+__global__ __launch_bounds__(kCgBlock) void k_ghost_plan(int N, int R, int W, int own, int size,
+                                                         const int32_t* __restrict__ sellCol,
+                                                         uint32_t* __restrict__ words,
+                                                         int32_t* __restrict__ ghosts, int stride,
+                                                         int32_t* __restrict__ count) {
+    __shared__ int waves[kCgBlock / 64];
+    const int tid = (int)threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int tile = (int)blockIdx.x, row0 = tile * R, row1 = min(row0 + R, (N + 63) & ~63);
+    int base = 0;
+    for (int i0 = row0; i0 < row1; i0 += kCgBlock) {
+        const int i = i0 + tid;
+        const bool in = i < row1;
+        uint32_t word = 0;
+        for (int k = 0; k < W; ++k) {
+            const int c = in ? sellCol[(int64_t)(i >> 6) * 64 * W + 64 * k + lane] : row0;
+            const bool far = (uint32_t)(c - row0) >= (uint32_t)R;
+            const unsigned long long m = __ballot(far);
+            if (lane == 0) waves[wid] = __popcll(m);
+            __syncthreads();
+            int slot = base + __popcll(m & ((1ull << lane) - 1));
+            for (int w = 0; w < kCgBlock / 64; ++w) {
+                if (w < wid) slot += waves[w];
+                base += waves[w];
+            }
+            __syncthreads();
+            if (!words) continue;
+            if (far) ghosts[(int64_t)tile * stride + slot] = c;
+            word |= (uint32_t)((far ? own + slot : c - row0) * size) << (k & 1 ? 16 : 0);
+            if ((k & 1) && in) {
+                words[(int64_t)(i >> 6) * 32 * W + 64 * (k >> 1) + lane] = word;
+                word = 0;
+            }
+        }
+    }
+    if (tid == 0) count[tile] = base;
+}
+
 // RPT: rows per thread (the rows a tile gives a thread, rounded up to a power
 // of two); W: entries of every slice of the sliced ELL; RES: rows of each thread
-// whose values and columns stay in registers; GLDS: g in LDS too (else in
-// registers).  p and d are in LDS: the SpMV reads p there for the columns of
-// this workgroup's own rows.  Rows past a tile's end take part as zeros; the
-// vectors are allocated to a multiple of 64 rows, so the rows of the last slice
-// past N are stored too (as zeros).
+// whose values and columns stay in registers; GL: rows whose g is in LDS too, DLDS: d
+// (else in registers).  p is in LDS, the tile's own rows' and its ghosts'.  Rows past a
+// tile's end take part as zeros; the vectors are allocated to a multiple of 64
+// rows, so the rows of the last slice past N are stored too (as zeros).
 // WHOLE (FP64): the launch also scales the matrix (from the CSR, also when it goes
 // on), takes the initial residual, and after the stop adds the correction to x and
 // takes the explicit residual, which goes to CgState::rrep: on small systems the
 // nine launches around the iterations cost as much as they do (32^3 heat step of 5
 // iterations 144 us with the start and end as kernels in a replayed graph, 103 whole;
 // 16^3 Poisson of 125 iterations 0.82 -> 0.73 ms).
-template <typename S, int RPT, int W, int RES, bool GLDS, bool TAGGED, bool WHOLE>
+template <typename S, int RPT, int W, int RES, int GL, bool DLDS, bool WHOLE>
 __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
+    constexpr int kOwn = RPT * kCgBlock, kTile = kOwn + ghost_cap<S>(RPT, W);
+    static_assert(kTile * sizeof(S) <= 65536, "16-bit columns");
     __shared__ PersistLds L;
-    __shared__ S lp[RPT * kPersistThreads], ld[RPT * kPersistThreads],
-        lg[GLDS ? RPT * kPersistThreads : 1];
-    constexpr int kRaw = WHOLE ? (W + 1) * kCgBlock : 1;
-    __shared__ double raw[kPersistSub * kRaw];
-    static_assert(!WHOLE || (sizeof(S) == 8 && GLDS), "whole solves are FP64 with g in LDS");
+    __shared__ S lp[kPersistSub * kTile], ldAll[DLDS ? kPersistSub * kOwn : 1],
+        lgAll[GL ? kPersistSub * GL * kCgBlock : 1];
+    // the raw matrix rows of 256 rows of the tile (start and end) share the ghosts' LDS
+    static_assert(!WHOLE || (sizeof(S) == 8 && GL == RPT && DLDS && RES == RPT &&
+                             ghost_cap<S>(RPT, W) >= (W + 1) * kCgBlock),
+                  "whole solves are FP64, with the matrix in registers");
     const int tid = (int)threadIdx.x, lane = tid & 63;
     // a tile is four waves and its rows are dealt in waves of 64, so its bounds
     // are the same in every lane: kept in scalar registers
@@ -427,8 +449,6 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     gs.tag = A.tag0;
     const int R = A.rowsPerTile;
     const int tile = gs.place(A.tiles, sub);
-    // this tile's rows [cbase, cbase + R) have their p in LDS, from lofs on
-    const uint32_t cbase = (uint32_t)tile * R, lofs = (uint32_t)sub * (RPT * kCgBlock);
     CgState* const st = A.st;
     const bool lead = gs.slot == 0 && tid == 0;
     if (!WHOLE || !A.fresh) {
@@ -446,9 +466,380 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     auto live = [&](int u) { return iw + u * kCgBlock < row1; };
     uint32_t lb = (uint32_t)lane * sizeof(S);
     auto mine = [&](auto* vec, int u) { return at_byte(vec + (iw + u * kCgBlock), lb); };
-    auto mine2 = [&](int u) {  // row u's place in rtag: twice the bytes of a value
-        return at_byte(A.rtag + (int64_t)(iw + u * kCgBlock) * (int)(sizeof(S) / 4), 2 * lb);
+    S *const tp = lp + sub * kTile, *const ghost = tp + kOwn;
+    S *const ld = ldAll + (DLDS ? sub * kOwn : 0), *const lg = lgAll + sub * (GL * kCgBlock);
+    auto lds = [&](S* vec, int u) -> S& { return *at_byte(vec + (iw - row0) + u * kCgBlock, lb); };
+    auto value = [&](int u, int k) {
+        return *at_byte(A.sval + ((int64_t)(iw + u * kCgBlock) * W + 64 * k), lb);
     };
+    auto pair = [&](int u, int j) {
+        return *at_byte(A.words + ((int64_t)(iw + u * kCgBlock) * (W / 2) + 64 * j), lb / (uint32_t)(sizeof(S) / 4));
+    };
+    auto col = [](const uint32_t (&c)[W / 2], int k) { return k & 1 ? c[k / 2] >> 16 : c[k / 2] & 0xffffu; };
+
+    // Ghost s of the tile is thread s % 256's, which holds the places in the vectors
+    // of its first kGk; its p is kept in LDS and follows p' = r + beta p like its
+    // owner's, so all that a tile reads of another's rows is their r.
+    constexpr int kGk = RPT == 2 || (RPT == 4 && sizeof(S) == 4) ? 6 : 4;
+    const int gt = tid & (kCgBlock - 1), ng = tile < A.tiles ? A.count[tile] : 0;
+    const int32_t* const glist = A.ghosts + (int64_t)(tile < A.tiles ? tile : 0) * A.ghostStride;
+    uint32_t gc[kGk];
+#pragma unroll
+    for (int j = 0; j < kGk; ++j) {
+        const int s = gt + j * kCgBlock;
+        gc[j] = s < ng ? (uint32_t)glist[s] * (uint32_t)sizeof(S) : 0u;
+    }
+    // kGk ghosts at a time: first(j, o) for each, o its byte offset in the vectors,
+    // then then(j, s).  The places of the next kGk are loaded meanwhile.
+    auto each_ghost = [&](auto first, auto then) {
+        uint32_t o[kGk];
+#pragma unroll
+        for (int j = 0; j < kGk; ++j) o[j] = gc[j];
+        for (int s0 = 0; s0 < ng; s0 += kGk * kCgBlock) {
+            uint32_t next[kGk];
+            if (s0 + kGk * kCgBlock < ng) {
+#pragma unroll
+                for (int j = 0; j < kGk; ++j)
+                    next[j] = (uint32_t)glist[min(s0 + (kGk + j) * kCgBlock + gt, ng - 1)] *
+                              (uint32_t)sizeof(S);
+            }
+#pragma unroll
+            for (int j = 0; j < kGk; ++j)
+                if (s0 + j * kCgBlock + gt < ng) first(j, o[j]);
+#pragma unroll
+            for (int j = 0; j < kGk; ++j)
+                if (s0 + j * kCgBlock + gt < ng) then(j, s0 + j * kCgBlock + gt);
+#pragma unroll
+            for (int j = 0; j < kGk; ++j) o[j] = next[j];
+        }
+    };
+
+    // Bit u: row u has a far column.  The pattern is symmetric, so those are the
+    // rows that other workgroups read, and only they are published.
+    uint32_t shown = 0;
+
+    S rv[RPT], qv[RPT], gr[GL < RPT ? RPT - GL : 1], dr[DLDS ? 1 : RPT];
+    S mv[RES ? RES : 1][W];
+    uint32_t mc[RES ? RES : 1][W / 2];
+    auto d_of = [&](int u) -> S& {
+        if constexpr (DLDS)
+            return lds(ld, u);
+        else
+            return dr[u];
+    };
+    auto g_of = [&](int u) -> S& {
+        if (u < GL) return lds(lg, u);
+        return gr[GL < RPT ? u - GL : 0];
+    };
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+        rv[u] = qv[u] = S(0);
+        if (u >= GL) gr[GL < RPT ? u - GL : 0] = S(0);
+        if constexpr (!DLDS) dr[u] = S(0);
+        uint32_t c[W / 2];
+        for (int j = 0; j < W / 2; ++j) c[j] = live(u) ? pair(u, j) : 0u;
+        for (int k = 0; k < W; ++k)
+            if (col(c, k) >= kOwn * sizeof(S)) shown |= 1u << u;
+        if (u < RES) {
+            for (int k = 0; k < W; ++k) mv[u][k] = S(0);
+            for (int j = 0; j < W / 2; ++j) mc[u][j] = c[j];
+        }
+    }
+    double bnorm, tol, atol, delta, rrep, rho, rhoPrev, alpha, res, res0;
+    int maxit, it, stop = 0;
+    bool ok = true;
+    [[maybe_unused]] auto residual = [&](auto far, auto out) {
+        tile_residual<RPT, W>(
+            A.m, A.N, row0, row1, iw, reinterpret_cast<double*>(ghost), live,
+            [&](int u, int k) {
+                const uint32_t c = (uint32_t)*at_byte(
+                    A.sellCol + ((int64_t)(iw + u * kCgBlock) * W + 64 * k), (uint32_t)lane * 4u);
+                const uint32_t l = c - (uint32_t)row0;
+                return l < (uint32_t)R ? l * (uint32_t)sizeof(S) : c * (uint32_t)sizeof(S) | kFar;
+            },
+            [&](int i) { return A.m.rhs[i]; }, [&](uint32_t o) { return *at_byte(tp, o); }, far,
+            [&](int u) { return lds(tp, u); }, out);
+    };
+    if constexpr (!WHOLE) {
+#pragma unroll
+        for (int u = 0; u < RPT; ++u)
+            if (live(u)) {
+                S p0 = S(0), d0 = S(0), g0 = S(0);
+                if (u < RES)
+                    for (int k = 0; k < W; ++k) mv[u][k] = value(u, k);
+                if (iw + u * kCgBlock + lane < A.N) {
+                    rv[u] = *mine(A.r, u);
+                    p0 = *mine(A.p, u);
+                    d0 = *mine(A.d, u);
+                    g0 = *mine(A.g, u);
+                }
+                lds(tp, u) = p0;
+                d_of(u) = d0;
+                g_of(u) = g0;
+            }
+    } else {
+        // x (in p's place) and g of the own rows, as kc_begin
+        const double first = A.m.vals[A.m.rowOffs[0] + A.m.diag[0]];
+        auto root = [&](double di) {
+            const bool good =
+                di != 0.0 && (di > 0.0) == (first > 0.0) && fabs(di) <= 1.7976931348623157e308;
+            return good ? copysign(sqrt(fabs(di)), di) : (double)NAN;
+        };
+#pragma unroll
+        for (int u = 0; u < RPT; ++u)
+            if (live(u)) {
+                const int i = iw + u * kCgBlock + lane;
+                const bool in = i < A.N;
+                lds(tp, u) = in ? *mine(A.x, u) : 0.0;
+                lds(lg, u) = in ? root(A.m.vals[A.m.rowOffs[i] + A.m.diag[i]]) : 0.0;
+                lds(ld, u) = !A.fresh && in ? *mine(A.d, u) : 0.0;
+            }
+        double s2[2] = {0.0, 0.0}, t2[2];
+        residual([&](uint32_t o) { return *at_byte(A.x, o); },
+                 [&](int u, bool in, double ri, double bi, const double (&a)[W],
+                     const uint32_t (&c)[W]) {
+                     const double gi = in ? lds(lg, u) : 1.0;
+#pragma unroll
+                     for (int k = 0; k < W; ++k) {  // as kc_scale
+                         double gj;
+                         if (c[k] & kFar) {
+                             const uint32_t j = (c[k] & ~kFar) / 8u;
+                             gj = root(A.m.vals[A.m.rowOffs[j] + A.m.diag[j]]);
+                         } else {
+                             gj = *at_byte(lg, c[k]);
+                         }
+                         mv[u][k] = a[k] != 0.0 ? a[k] / (gi * fabs(gj)) : 0.0;
+                     }
+                     rv[u] = ri;
+                     s2[0] += ri * ri;
+                     s2[1] += bi * bi;
+                 });
+        if (A.fresh) {
+            // ||b||, the relative residual; r = G^-1 r64, p = r, ||G r||^2 and r.r
+            if ((ok = gs.sum<2, false>(s2, t2, L))) {
+                bnorm = sqrt(t2[1]);
+                if (!(bnorm > 0.0)) bnorm = 1.0;
+                res = res0 = sqrt(t2[0]) / bnorm;
+                double s3[2] = {0.0, 0.0};
+#pragma unroll
+                for (int u = 0; u < RPT; ++u)
+                    if (live(u)) {
+                        const bool in = iw + u * kCgBlock + lane < A.N;
+                        const double gi = lds(lg, u);
+                        const double ri = in ? rv[u] / gi : 0.0;
+                        rv[u] = ri;
+                        lds(tp, u) = ri;
+                        if (shown >> u & 1) put_shared(mine(A.p, u), ri);
+                        const double ur = ri * gi;
+                        s3[0] += ur * ur;
+                        s3[1] += ri * ri;
+                    }
+                ok = gs.sum<2, true>(s3, t2, L);
+                rho = t2[1];
+                rhoPrev = alpha = 0.0;
+                it = 0;
+                // the decision of kc_direction after a start
+                const bool conv = res <= A.tol || res * bnorm <= A.atol;
+                stop = conv ? 2 : !(res <= 1.7976931348623157e308) ? 3 : A.maxit <= 0 ? 1 : 0;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < RPT; ++u)
+                if (live(u)) {
+                    rv[u] = *mine(A.r, u);
+                    lds(tp, u) = *mine(A.p, u);
+                }
+        }
+    }
+    if (!WHOLE || !A.fresh) {
+        bnorm = uniform(st->bnorm);
+        rho = uniform(st->rho);
+        rhoPrev = uniform(st->rhoPrev);
+        alpha = uniform(st->alpha);
+        res = uniform(st->res);
+        res0 = uniform(st->res0);
+        it = __builtin_amdgcn_readfirstlane(st->it);
+    }
+    tol = WHOLE ? A.tol : uniform(st->tol);
+    atol = WHOLE ? A.atol : uniform(st->atol);
+    maxit = WHOLE ? A.maxit : __builtin_amdgcn_readfirstlane(st->maxit);
+    delta = WHOLE ? 0.0 : uniform(st->delta);
+    rrep = WHOLE ? 0.0 : uniform(st->rrep);
+    S beta = S(0);
+    {  // the ghosts' p
+        S x[kGk];
+        each_ghost([&](int j, uint32_t o) { x[j] = get_shared(at_byte(A.p, o)); },
+                   [&](int j, int s) { ghost[s] = x[j]; });
+    }
+    // streamed rows: loaded when the row before is done (the first one of an iteration
+    // at the end of the one before, across its exchanges); the other waves of the SIMD
+    // compute meanwhile, and a second set of registers would not fit
+    S vn[W];
+    uint32_t cn[W / 2];
+    auto fetch = [&](int u) {
+#pragma unroll
+        for (int j = 0; j < W / 2; ++j) cn[j] = pair(u, j);
+#pragma unroll
+        for (int k = 0; k < W; ++k) vn[k] = value(u, k);
+    };
+    if (RES < RPT && live(RES)) fetch(RES);
+    for (int n = 0; ok && !stop && n < A.iters; ++n) {
+        opaque(lb);
+        for (int u = 0; u < RES; ++u)
+            for (int j = 0; j < W / 2; ++j) opaque(mc[u][j]);
+        if (n) {
+            S x[kGk];
+            each_ghost([&](int j, uint32_t o) { x[j] = get_shared(at_byte(A.r, o)); },
+                       [&](int j, int s) { ghost[s] = x[j] + beta * ghost[s]; });
+        }
+        __syncthreads();
+        // q = As p, p.q
+        double v1[1] = {0.0}, t1[1];
+        auto row = [&](int u, const S (&v)[W], const uint32_t (&c)[W / 2]) {
+            S x[W];
+#pragma unroll
+            for (int k = 0; k < W; ++k) x[k] = *at_byte(tp, col(c, k));
+            const S own = lds(tp, u);
+            S sum = own;
+#pragma unroll
+            for (int k = 0; k < W; ++k) sum += v[k] * x[k];
+            qv[u] = sum;
+            v1[0] += (double)own * (double)sum;
+        };
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            if (u < RES) {
+                row(u, mv[u], mc[u]);
+            } else {
+                row(u, vn, cn);
+                if (RPT == 8 && sizeof(S) == 8) __builtin_amdgcn_sched_barrier(0);
+                fetch(u + 1 < RPT && live(u + 1) ? u + 1 : RES);
+            }
+        }
+        if (!(ok = gs.sum<1, false>(v1, t1, L))) break;
+        // alpha; d += alpha p, r -= alpha q, ||G r||^2 and r.r
+        alpha = rho / t1[0];
+        ++it;
+        rhoPrev = rho;
+        const S a = (S)alpha;
+        double v2[2] = {0.0, 0.0}, t2[2];
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            const S ri = rv[u] - a * qv[u];
+            rv[u] = ri;
+            if (shown >> u & 1) put_shared(mine(A.r, u), ri);
+            d_of(u) = d_of(u) + a * lds(tp, u);
+            const double ur = (double)ri * (double)g_of(u);
+            v2[0] += ur * ur;
+            v2[1] += (double)ri * (double)ri;
+        }
+        if (!(ok = gs.sum<2, true>(v2, t2, L))) break;
+        // the stop decision (cg_decide) and the next direction
+        const double rn = sqrt(t2[0]);
+        res = rn / bnorm;
+        rho = t2[1];
+        if (res <= tol || rn <= atol || it >= maxit || !(res == res) ||
+            (delta > 0.0 && rn < delta * rrep)) {
+            stop = 1;
+            break;
+        }
+        beta = (S)(rho / rhoPrev);
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            lds(tp, u) = rv[u] + beta * lds(tp, u);
+        }
+    }
+    if constexpr (WHOLE) {
+        if (ok && stop) {  // x += |G|^-1 d, the explicit residual of the result
+#pragma unroll
+            for (int u = 0; u < RPT; ++u)
+                if (live(u) && iw + u * kCgBlock + lane < A.N) {
+                    const double x = *mine(A.x, u) + lds(ld, u) / fabs(lds(lg, u));
+                    lds(tp, u) = x;
+                    if (shown >> u & 1)
+                        put_shared(mine(A.x, u), x);
+                    else
+                        *mine(A.x, u) = x;
+                }
+            double none[1] = {0.0}, all[1], s1[1] = {0.0};
+            if ((ok = gs.sum<1, true>(none, all, L))) {
+                residual([&](uint32_t o) { return get_shared(at_byte(A.x, o)); },
+                         [&](int, bool, double ri, double, const double (&)[W],
+                             const uint32_t (&)[W]) { s1[0] += ri * ri; });
+                ok = gs.sum<1, false>(s1, all, L);
+                rrep = sqrt(all[0]) / bnorm;
+            }
+        }
+    }
+    if (!ok) {
+        if (tid == 0) st->stop = kStopSync;
+        return;
+    }
+    if (!WHOLE || !stop) {
+#pragma unroll
+        for (int u = 0; u < RPT; ++u)
+            if (live(u)) {
+                *mine(A.r, u) = rv[u];
+                *mine(A.p, u) = lds(tp, u);
+                *mine(A.d, u) = d_of(u);
+            }
+    }
+    if (lead) {
+        st->rho = rho;
+        st->rhoPrev = rhoPrev;
+        st->alpha = alpha;
+        st->res = res;
+        st->it = it;
+        st->stop = stop;
+        st->done = 0;
+        st->pbuf = 0;
+        if (WHOLE) {
+            st->bnorm = bnorm;
+            st->res0 = res0;
+            st->rrep = rrep;
+        }
+    }
+}
+
+// The form for tiles with more ghosts than fit (systems of over 2^20 rows in block
+// order, of over 2^19 whose mesh was not renumbered; 128^3 FP64 in block order
+// 63 us kernel by kernel, 46 here): a far column's p' is evaluated for each entry, from
+// the published r and the published p of the iteration before, and the columns are read
+// as 32-bit row numbers.
+template <typename S, int RPT, int W, int RES, bool GLDS>
+__global__ __launch_bounds__(kPersistThreads) void kc_persist_far(CgPersist<S> A) {
+    __shared__ PersistLds L;
+    __shared__ S lp[RPT * kPersistThreads], ld[RPT * kPersistThreads],
+        lg[GLDS ? RPT * kPersistThreads : 1];
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    // a tile is four waves and its rows are dealt in waves of 64, so its bounds
+    // are the same in every lane: kept in scalar registers
+    const int sub = __builtin_amdgcn_readfirstlane(tid / kCgBlock);
+    GridSum gs;
+    gs.slots = A.slots;
+    gs.tag = A.tag0;
+    const int R = A.rowsPerTile;
+    const int tile = gs.place(A.tiles, sub);
+    // this tile's rows [cbase, cbase + R) have their p in LDS, from lofs on
+    const uint32_t cbase = (uint32_t)tile * R, lofs = (uint32_t)sub * (RPT * kCgBlock);
+    CgState* const st = A.st;
+    const bool lead = gs.slot == 0 && tid == 0;
+    const int entry = st->stop;
+    if (entry) {
+        if (lead) st->done = entry;  // as the update kernel of a stopped system
+        return;
+    }
+    if (tid == 0) L.bad = 0;
+    const int row0 = tile * R;
+    const int row1 = tile < A.tiles ? min(row0 + R, (A.N + 63) & ~63) : row0;
+    // this wave's first row; its row u is iw + 256 u + lane, of slice (iw + 256 u) / 64
+    const int iw = row0 + __builtin_amdgcn_readfirstlane(tid & (kCgBlock - 64));
+    auto live = [&](int u) { return iw + u * kCgBlock < row1; };
+    uint32_t lb = (uint32_t)lane * sizeof(S);
+    auto mine = [&](auto* vec, int u) { return at_byte(vec + (iw + u * kCgBlock), lb); };
     const uint32_t lown = (uint32_t)(iw - (int)cbase) + lofs;  // LDS place of row u: lown + 256 u + lane
     auto lds = [&](S* vec, int u) -> S& { return *at_byte(vec + lown + u * kCgBlock, lb); };
     auto value = [&](int u, int k) {
@@ -479,15 +870,10 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
             }
         if constexpr (!GLDS) gr[u] = S(0);
     }
-    double bnorm, tol, atol, delta, rrep, rho, rhoPrev, alpha, res, res0;
+    double bnorm, tol, atol, delta, rrep, rho, rhoPrev, alpha, res;
     int maxit, it, stop = 0;
     bool ok = true;
-    [[maybe_unused]] auto residual = [&](auto far, auto out) {
-        tile_residual<RPT, W>(
-            A.m, A.N, row0, row1, iw, raw + sub * kRaw, live, column,
-            [&](int i) { return A.m.rhs[i]; }, [&](uint32_t o) { return *at_byte(lp, o); }, far, [&](int u) { return lds(lp, u); }, out);
-    };
-    if constexpr (!WHOLE) {
+    {
 #pragma unroll
         for (int u = 0; u < RPT; ++u) {
             S p0 = S(0), d0 = S(0), g0 = S(0);
@@ -515,105 +901,19 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
             }
             if constexpr (!GLDS) gr[u] = g0;
         }
-    } else {
-        // x (in p's place) and g of the own rows, as kc_begin
-        const double first = A.m.vals[A.m.rowOffs[0] + A.m.diag[0]];
-        auto root = [&](double di) {
-            const bool good =
-                di != 0.0 && (di > 0.0) == (first > 0.0) && fabs(di) <= 1.7976931348623157e308;
-            return good ? copysign(sqrt(fabs(di)), di) : (double)NAN;
-        };
-#pragma unroll
-        for (int u = 0; u < RPT; ++u)
-            if (live(u)) {
-                const int i = iw + u * kCgBlock + lane;
-                const bool in = i < A.N;
-                lds(lp, u) = in ? *mine(A.x, u) : 0.0;
-                lds(lg, u) = in ? root(A.m.vals[A.m.rowOffs[i] + A.m.diag[i]]) : 0.0;
-                lds(ld, u) = !A.fresh && in ? *mine(A.d, u) : 0.0;
-            }
-        double s2[2] = {0.0, 0.0}, t2[2];
-        residual([&](uint32_t o) { return *at_byte(A.x, o); },
-                 [&](int u, bool in, double ri, double bi, const double (&a)[W],
-                     const uint32_t (&c)[W]) {
-                     const double gi = in ? lds(lg, u) : 1.0;
-#pragma unroll
-                     for (int k = 0; k < W; ++k) {  // as kc_scale
-                         double gj;
-                         if (c[k] & kFar) {
-                             const uint32_t j = (c[k] & ~kFar) / 8u;
-                             gj = root(A.m.vals[A.m.rowOffs[j] + A.m.diag[j]]);
-                         } else {
-                             gj = *at_byte(lg, c[k]);
-                         }
-                         const double v = a[k] != 0.0 ? a[k] / (gi * fabs(gj)) : 0.0;
-                         if (u < RES) {
-                             mv[u][k] = v;
-                             mc[u][k] = c[k];
-                         } else {
-                             *at_byte(const_cast<double*>(A.sval) +
-                                          ((int64_t)(iw + u * kCgBlock) * W + 64 * k), lb) = v;
-                         }
-                         shown |= c[k] >> 31 << u;
-                     }
-                     rv[u] = ri;
-                     s2[0] += ri * ri;
-                     s2[1] += bi * bi;
-                 });
-        if (A.fresh) {
-            // ||b||, the relative residual; r = G^-1 r64, p = r, ||G r||^2 and r.r
-            if ((ok = gs.sum<2, false>(s2, t2, L))) {
-                bnorm = sqrt(t2[1]);
-                if (!(bnorm > 0.0)) bnorm = 1.0;
-                res = res0 = sqrt(t2[0]) / bnorm;
-                double s3[2] = {0.0, 0.0};
-#pragma unroll
-                for (int u = 0; u < RPT; ++u)
-                    if (live(u)) {
-                        const bool in = iw + u * kCgBlock + lane < A.N;
-                        const double gi = lds(lg, u);
-                        const double ri = in ? rv[u] / gi : 0.0;
-                        rv[u] = ri;
-                        lds(lp, u) = ri;
-                        if (shown >> u & 1) put_shared(mine(A.p, u), ri);
-                        const double ur = ri * gi;
-                        s3[0] += ur * ur;
-                        s3[1] += ri * ri;
-                    }
-                ok = gs.sum<2, true>(s3, t2, L);
-                rho = t2[1];
-                rhoPrev = alpha = 0.0;
-                it = 0;
-                // the decision of kc_direction after a start
-                const bool conv = res <= A.tol || res * bnorm <= A.atol;
-                stop = conv ? 2 : !(res <= 1.7976931348623157e308) ? 3 : A.maxit <= 0 ? 1 : 0;
-            }
-        } else {
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < RPT; ++u)
-                if (live(u)) {
-                    rv[u] = *mine(A.r, u);
-                    lds(lp, u) = *mine(A.p, u);
-                }
-        }
     }
-    if (!WHOLE || !A.fresh) {
-        bnorm = uniform(st->bnorm);
-        rho = uniform(st->rho);
-        rhoPrev = uniform(st->rhoPrev);
-        alpha = uniform(st->alpha);
-        res = uniform(st->res);
-        res0 = uniform(st->res0);
-        it = __builtin_amdgcn_readfirstlane(st->it);
-    }
-    tol = WHOLE ? A.tol : uniform(st->tol);
-    atol = WHOLE ? A.atol : uniform(st->atol);
-    maxit = WHOLE ? A.maxit : __builtin_amdgcn_readfirstlane(st->maxit);
-    delta = WHOLE ? 0.0 : uniform(st->delta);
-    rrep = WHOLE ? 0.0 : uniform(st->rrep);
+    bnorm = uniform(st->bnorm);
+    rho = uniform(st->rho);
+    rhoPrev = uniform(st->rhoPrev);
+    alpha = uniform(st->alpha);
+    res = uniform(st->res);
+    it = __builtin_amdgcn_readfirstlane(st->it);
+    tol = uniform(st->tol);
+    atol = uniform(st->atol);
+    maxit = __builtin_amdgcn_readfirstlane(st->maxit);
+    delta = uniform(st->delta);
+    rrep = uniform(st->rrep);
     S beta = S(0);
-    uint32_t rtag = 0;
     S *pold = A.p, *pnew = A.p2;  // the direction before this iteration's, and the next one's place
     __syncthreads();
     for (int n = 0; ok && !stop && n < A.iters; ++n) {
@@ -625,16 +925,12 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
         double v1[1] = {0.0}, t1[1];
         auto row = [&](int u, const S (&v)[W], const uint32_t (&c)[W], auto next) {
             S x[W], y[W];
-            Tagged<S> t[TAGGED ? W : 1];
 #pragma unroll
             for (int k = 0; k < W; ++k) {
                 if (c[k] & kFar) {
                     const uint32_t o = c[k] & ~kFar;
                     y[k] = get_shared(at_byte(pold, o));
-                    if constexpr (TAGGED)
-                        t[k].load(at_byte(A.rtag, 2 * o));
-                    else
-                        x[k] = n ? get_shared(at_byte(A.r, o)) : S(0);
+                    x[k] = n ? get_shared(at_byte(A.r, o)) : S(0);
                 } else {
                     x[k] = *at_byte(lp, c[k]);
                 }
@@ -644,15 +940,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
             S sum = own;
 #pragma unroll
             for (int k = 0; k < W; ++k) {
-                if (c[k] & kFar) {
-                    if constexpr (TAGGED) {
-                        if (n && !t[k].is(rtag) &&
-                            !t[k].wait(at_byte(A.rtag, 2 * (c[k] & ~kFar)), rtag))
-                            L.bad = 1;
-                        x[k] = t[k].value();
-                    }
-                    x[k] = n ? x[k] + beta * y[k] : y[k];
-                }
+                if (c[k] & kFar) x[k] = n ? x[k] + beta * y[k] : y[k];
                 sum += v[k] * x[k];
             }
             qv[u] = sum;
@@ -690,19 +978,13 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
         ++it;
         rhoPrev = rho;
         const S a = (S)alpha;
-        rtag = gs.tag;
         double v2[2] = {0.0, 0.0}, t2[2];
 #pragma unroll
         for (int u = 0; u < RPT; ++u) {
             if (!live(u)) break;
             const S ri = rv[u] - a * qv[u];
             rv[u] = ri;
-            if (shown >> u & 1) {
-                if constexpr (TAGGED)
-                    Tagged<S>::store(mine2(u), ri, rtag);
-                else
-                    put_shared(mine(A.r, u), ri);
-            }
+            if (shown >> u & 1) put_shared(mine(A.r, u), ri);
             lds(ld, u) = lds(ld, u) + a * lds(lp, u);
             S gi;
             if constexpr (GLDS)
@@ -713,7 +995,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
             v2[0] += ur * ur;
             v2[1] += (double)ri * (double)ri;
         }
-        if (!(ok = gs.sum<2, !TAGGED>(v2, t2, L))) break;
+        if (!(ok = gs.sum<2, true>(v2, t2, L))) break;
         // the stop decision (cg_decide) and the next direction
         const double rn = sqrt(t2[0]);
         res = rn / bnorm;
@@ -738,41 +1020,17 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
         }
         __syncthreads();
     }
-    if constexpr (WHOLE) {
-        if (ok && stop) {  // x += |G|^-1 d, the explicit residual of the result
-#pragma unroll
-            for (int u = 0; u < RPT; ++u)
-                if (live(u) && iw + u * kCgBlock + lane < A.N) {
-                    const double x = *mine(A.x, u) + lds(ld, u) / fabs(lds(lg, u));
-                    lds(lp, u) = x;
-                    if (shown >> u & 1)
-                        put_shared(mine(A.x, u), x);
-                    else
-                        *mine(A.x, u) = x;
-                }
-            double none[1] = {0.0}, all[1], s1[1] = {0.0};
-            if ((ok = gs.sum<1, true>(none, all, L))) {
-                residual([&](uint32_t o) { return get_shared(at_byte(A.x, o)); },
-                         [&](int, bool, double ri, double, const double (&)[W],
-                             const uint32_t (&)[W]) { s1[0] += ri * ri; });
-                ok = gs.sum<1, false>(s1, all, L);
-                rrep = sqrt(all[0]) / bnorm;
-            }
-        }
-    }
     if (!ok) {
         if (tid == 0) st->stop = kStopSync;
         return;
     }
-    if (!WHOLE || !stop) {
 #pragma unroll
-        for (int u = 0; u < RPT; ++u)
-            if (live(u)) {
-                *mine(A.r, u) = rv[u];
-                *mine(A.p, u) = lds(lp, u);
-                *mine(A.d, u) = lds(ld, u);
-            }
-    }
+    for (int u = 0; u < RPT; ++u)
+        if (live(u)) {
+            *mine(A.r, u) = rv[u];
+            *mine(A.p, u) = lds(lp, u);
+            *mine(A.d, u) = lds(ld, u);
+        }
     if (lead) {
         st->rho = rho;
         st->rhoPrev = rhoPrev;
@@ -782,11 +1040,6 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
         st->stop = stop;
         st->done = 0;
         st->pbuf = 0;
-        if (WHOLE) {
-            st->bnorm = bnorm;
-            st->res0 = res0;
-            st->rrep = rrep;
-        }
     }
 }
 

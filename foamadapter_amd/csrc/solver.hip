@@ -51,7 +51,10 @@ struct CgWork : fv_solver_cache {
     int persistGrid = 0, persistIters = 0;
     int lastLaunches = 0;  // persistent launches of the previous mixed solve
     int lastTotal = 0;     // iterations of the previous solve, in either form
-    DBuf<unsigned long long> slots, rtag;
+    DBuf<unsigned long long> slots;
+    DBuf<uint32_t> words;  // kc_persist's columns and ghosts
+    DBuf<int32_t> ghosts, ghostCount;
+    int ghostStride = 0;
     uint32_t tag = 1;
 
     CgWork(fv_ctx* c, const fv_linsys* ls) {
@@ -110,10 +113,11 @@ struct CgWork : fv_solver_cache {
     // the registers), and a device that keeps its workgroups resident together.
     void choose_persist(fv_ctx* c, const fv_sparsity* sp, int tiles, int R) {
         const int rpt = (R + kB - 1) / kB;
+        if (rpt > 8) return;
         if (sp->sellWidth == 6)
-            persist = persist_kernel<6>(rpt);
+            choose_kernel<6>(c, tiles, R, rpt);
         else if (sp->sellWidth == 4)
-            persist = persist_kernel<4>(rpt);
+            choose_kernel<4>(c, tiles, R, rpt);
         if (!persist) return;
         persistGrid = persist_grid(tiles);
         if (!persist_fits(reinterpret_cast<const void*>(persist), c->device, persistGrid)) {
@@ -126,8 +130,6 @@ struct CgWork : fv_solver_cache {
         // other streams gets in between
         persistIters = (int)(2000.0 / (6.0 + 32.0 * h.N / (1 << 21)));
         slots.alloc(c, 2 * (size_t)kSlotBuffer);
-        if (rpt <= (sizeof(S) == 8 ? 2 : 4))  // the TAGGED kernels
-            rtag.alloc(c, ((size_t)h.N + 63) / 64 * 64 * (sizeof(S) / 4));
         clear_tags(c->stream);
     }
     // A cooperative launch costs about 17 us more than a plain one and is not
@@ -142,25 +144,49 @@ struct CgWork : fv_solver_cache {
     // no word of the exchange carries a tag that is still to come
     void clear_tags(hipStream_t s) {
         FV_HIP(hipMemsetAsync(slots.p, 0, slots.n * sizeof(unsigned long long), s));
-        if (rtag.n) FV_HIP(hipMemsetAsync(rtag.p, 0, rtag.n * sizeof(unsigned long long), s));
         tag = 1;
     }
-    // RES, the rows whose matrix stays in registers, is what fits beside the vectors
-    // in the 128 registers of a 1024-thread workgroup without spills.
+    // RES, the rows whose matrix stays in registers, and where g and d are, is what
+    // fits the 128 registers of a 1024-thread workgroup and its LDS without spills.
     template <int W>
-    static auto persist_kernel(int rpt) -> void (*)(CgPersist<S>) {
-        if constexpr (sizeof(S) == 8) {
-            if (rpt <= 1) return kc_persist<S, 1, W, 1, true, true, true>;
-            if (rpt <= 2) return kc_persist<S, 2, W, 2, true, true, true>;
-            if (rpt <= 4) return kc_persist<S, 4, W, 2, true, false, false>;
-            if (rpt <= 8) return kc_persist<S, 8, W, 0, false, false, false>;
+    void choose_kernel(fv_ctx* c, int tiles, int R, int rpt) {
+        const int n = rpt <= 1 ? 1 : rpt <= 2 ? 2 : rpt <= 4 ? 4 : 8;
+        if (make_ghosts(c, tiles, R, W, n)) {
+            if constexpr (sizeof(S) == 8)
+                persist = n == 1   ? kc_persist<S, 1, W, 1, 1, true, true>
+                          : n == 2 ? kc_persist<S, 2, W, 2, 2, true, true>
+                          : n == 4 ? kc_persist<S, 4, W, 2, 4, false, false>
+                                   : kc_persist<S, 8, W, 0, 5, false, false>;
+            else
+                persist = n == 1   ? kc_persist<S, 1, W, 1, 1, true, false>
+                          : n == 2 ? kc_persist<S, 2, W, 2, 2, true, false>
+                          : n == 4 ? kc_persist<S, 4, W, 4, 4, true, false>
+                                   : kc_persist<S, 8, W, 4, 0, true, false>;
+        } else if constexpr (sizeof(S) == 8) {
+            persist = n == 4 ? kc_persist_far<S, 4, W, 2, true> : kc_persist_far<S, 8, W, 0, false>;
         } else {
-            if (rpt <= 1) return kc_persist<S, 1, W, 1, false, true, false>;
-            if (rpt <= 2) return kc_persist<S, 2, W, 2, true, true, false>;
-            if (rpt <= 4) return kc_persist<S, 4, W, 4, true, true, false>;
-            if (rpt <= 8) return kc_persist<S, 8, W, 4, true, false, false>;
+            persist = kc_persist_far<S, 8, W, 4, true>;
         }
-        return nullptr;
+    }
+    // The ghosts of every tile and the columns that refer to them; false if a tile has
+    // more than fit (never up to 2 FP64 or 4 FP32 rows per thread).
+    bool make_ghosts(fv_ctx* c, int tiles, int R, int W, int rpt) {
+        hipStream_t s = c->stream;
+        ghostCount.alloc(c, tiles);
+        auto plan = [&](uint32_t* w, int32_t* g) {
+            k_ghost_plan<<<tiles, kB, 0, s>>>(h.N, R, W, rpt * kB, (int)sizeof(S), h.sellCol, w, g,
+                                              ghostStride, ghostCount.p);
+            FV_LAUNCH_CHECK();
+        };
+        plan(nullptr, nullptr);
+        std::vector<int32_t> n(tiles);
+        ghostCount.download(n.data());
+        ghostStride = *std::max_element(n.begin(), n.end());
+        if (ghostStride > ghost_cap<S>(rpt, W)) return false;
+        words.alloc(c, ((size_t)h.N + 63) / 64 * 64 * W / 2);
+        ghosts.alloc(c, std::max<size_t>(1, (size_t)tiles * ghostStride));
+        plan(words.p, ghosts.p);
+        return true;
     }
     // Up to persistIters iterations in one launch; false if the device refuses it.
     // (whole: x, the limits and whether the solve starts.)
@@ -169,7 +195,8 @@ struct CgWork : fv_solver_cache {
         const uint32_t uses = 2 * (uint32_t)persistIters + 8;
         if (tag > 0xffffffffu - uses) clear_tags(s);  // sequence numbers start over
         CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persistIters, tag, h.sellCol, h.sval,
-                       h.g, h.d, h.r, h.p, h.p2, rtag.p, h.st, slots.p,
+                       h.g, h.d, h.r, h.p, h.p2, words.p, ghosts.p, ghostCount.p, ghostStride,
+                       h.st, slots.p,
                        CsrSystem{h.rowOffs, h.diag, h.vals, h.rhs}, x, tol, atol, maxit,
                        fresh ? 1 : 0};
         void* args[] = {&a};

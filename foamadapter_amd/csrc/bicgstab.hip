@@ -291,13 +291,14 @@ __global__ void kbi_scale(int64_t n, const int32_t* __restrict__ src, const int3
 // 78 MB, and the launches, reads and no-ops around it take as long again.  Here one
 // cooperative launch scales the matrix, takes the initial residual, iterates and
 // takes the explicit residual of the result, on the tiles, the exchange and the LDS
-// scheme of cgpersist.hpp: r, rhat, v and t of a thread's rows in registers, p, s, x
-// and D^-1 in LDS (up to 4 rows per thread).  What others need of a row is published
-// (r, and p and v in alternating buffers), and the reader of a far column evaluates
-// its owner's p' = r + beta (p - omega v) or s = r - alpha v, so an iteration has
-// three grid exchanges.  The order of all sums is that of the kernels above (same
-// bits).  Advection step on 110x100x90 cells (31 iterations) 3.20 -> 1.76 ms, an
-// icoFoam step at 64^3 (three momentum solves) 5.01 -> 4.25 ms.
+// scheme of cgpersist.hpp: r, rhat, v, t, x and D^-1 of a thread's rows in registers,
+// p and s in LDS, with p, s and v of the tile's ghosts (up to 4 rows per thread).  Each
+// tile publishes v and r of the rows that others refer to, and follows p' = r + beta (p
+// - omega v) and s = r - alpha v for its ghosts, so an iteration has three grid
+// exchanges.  The order of all sums is that of the kernels above (same
+// bits).  Advection step on 110x100x90 cells (about 28 iterations) 2.9 -> 1.18 ms (1.62
+// with the far columns read in the product, as kbi_persist_far does), an icoFoam step
+// at 64^3 (three momentum solves) 5.01 -> 4.25 ms.
 //
 // A Vec3 equation's right-hand sides and solutions are interleaved: the kernel reads
 // b and the initial x at a stride, keeps the x it publishes in a vector of its own
@@ -319,13 +320,341 @@ struct BiPersist {
     double* out;          // the solution if it converged (null: x holds it)
     const BiState* prev;  // component before this one: go on only if it converged
     double* sval;  // scaled values of the rows whose matrix does not stay in registers
-    double *x, *r, *rhat, *p, *p2, *v, *v2;
+    double *x, *r, *rhat, *p, *v;
+    double* v2;  // published v: a launch that goes on reads the ghosts' v of the one before
+    double* p2;  // (kbi_persist_far: p and v alternate)
+    const uint32_t* words;  // the columns, see k_ghost_plan; ghosts of each tile
+    const int32_t *ghosts, *count;
+    int32_t ghostStride;
     BiState* st;
     unsigned long long* slots;
 };
 
+// Places for ghosts in the LDS of a tile (see cgpersist.hpp): p and s of its rows and
+// ghosts, and the ghosts' v.  Enough for tiles of up to 512 rows in any order a mesher
+// writes (1230 at most), and for 1024 rows in Z order (about 950).
+constexpr int bi_ghost_cap(int rpt) { return rpt == 1 ? 1528 : rpt == 2 ? 1360 : 1016; }
+
 template <int RPT, int W, int RES>
 __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
+    constexpr int kOwn = RPT * kB, kCap = bi_ghost_cap(RPT), kTile = kOwn + kCap;
+    constexpr int kLds = 2 * kTile + kCap;  // p | s | ghosts' v
+    __shared__ PersistLds L;
+    __shared__ double l0[kPersistSub * kLds];
+    // the raw matrix rows of 256 rows of the tile (start and end) share the LDS of its
+    // ghosts' s and v; x is where p is then, D^-1 where s is
+    static_assert(2 * kCap >= (W + 1) * kB, "raw rows");
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int sub = __builtin_amdgcn_readfirstlane(tid / kB);
+    GridSum gs;
+    gs.slots = A.slots;
+    gs.tag = A.tag0;
+    const int R = A.rowsPerTile;
+    const int tile = gs.place(A.tiles, sub);
+    BiState* const st = A.st;
+    if (!A.fresh && st->stop) return;
+    if (A.prev && A.prev->stop != 2) {
+        if (gs.slot == 0 && tid == 0) st->stop = 0;
+        return;
+    }
+    // x at the start of the launch, at stride xs
+    const double* const xin = A.fresh ? A.x0 : A.x;
+    const int xs = A.fresh ? A.stride : 1;
+    if (tid == 0) L.bad = 0;
+    const int row0 = tile * R;
+    const int row1 = tile < A.tiles ? min(row0 + R, (A.N + 63) & ~63) : row0;
+    const int iw = row0 + __builtin_amdgcn_readfirstlane(tid & (kB - 64));
+    auto live = [&](int u) { return iw + u * kB < row1; };
+    auto inN = [&](int u) { return iw + u * kB + lane < A.N && live(u); };
+    uint32_t lb = (uint32_t)lane * 8u;
+    auto mine = [&](auto* vec, int u) { return at_byte(vec + (iw + u * kB), lb); };
+    double *const lp = l0 + sub * kLds, *const ls = lp + kTile, *const gp = lp + kOwn,
+                 *const gsv = ls + kOwn, *const gv = ls + kTile;
+    auto lds = [&](double* vec, int u) -> double& { return *at_byte(vec + (iw - row0) + u * kB, lb); };
+    auto svalAt = [&](int u, int k) {
+        return at_byte(A.sval + ((int64_t)(iw + u * kB) * W + 64 * k), lb);
+    };
+    auto pair = [&](int u, int j) {
+        return *at_byte(A.words + ((int64_t)(iw + u * kB) * (W / 2) + 64 * j), lb / 2u);
+    };
+    auto col = [](const uint32_t (&c)[W / 2], int k) { return k & 1 ? c[k / 2] >> 16 : c[k / 2] & 0xffffu; };
+    const GhostWalk<RPT == 4 ? 4 : 6, 8> ghosts(A.ghosts, A.count, A.ghostStride, tile, A.tiles);
+    uint32_t shown = 0;  // bit u: row u has a far column, so others read it
+    double rv[RPT], hv[RPT], vv[RPT], tv[RPT], xr[RPT], di[RPT];
+    double mv[RES ? RES : 1][W];
+    uint32_t mc[RES ? RES : 1][W / 2];
+
+    // x and D^-1 of the own rows
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+        rv[u] = hv[u] = vv[u] = tv[u] = xr[u] = di[u] = 0.0;
+        uint32_t c[W / 2];
+        for (int j = 0; j < W / 2; ++j) c[j] = live(u) ? pair(u, j) : 0u;
+        for (int k = 0; k < W; ++k)
+            if (col(c, k) >= kOwn * 8u) shown |= 1u << u;
+        if (u < RES) {
+            for (int k = 0; k < W; ++k) mv[u][k] = 0.0;
+            for (int j = 0; j < W / 2; ++j) mc[u][j] = c[j];
+        }
+        if (inN(u)) {
+            const int i = iw + u * kB + lane;
+            xr[u] = xin[(int64_t)i * xs];
+            di[u] = 1.0 / A.m.vals[A.m.rowOffs[i] + A.m.diag[i]];
+        }
+        if (live(u)) {
+            lds(lp, u) = xr[u];
+            lds(ls, u) = di[u];
+        }
+    }
+    auto residual = [&](auto far, auto out) {
+        tile_residual<RPT, W>(
+            A.m, A.N, row0, row1, iw, gsv, live,
+            [&](int u, int k) {  // byte offset in LDS, or (top bit) in the vectors
+                const uint32_t c = (uint32_t)*at_byte(
+                    A.sellCol + ((int64_t)(iw + u * kB) * W + 64 * k), (uint32_t)lane * 4u);
+                const uint32_t l = c - (uint32_t)row0;
+                return l < (uint32_t)R ? l * 8u : c * 8u | kFar;
+            },
+            [&](int i) { return A.m.rhs[(int64_t)i * A.stride]; },
+            [&](uint32_t o) { return *at_byte(lp, o); }, far, [&](int u) { return lds(lp, u); }, out);
+    };
+
+    double bnorm, res, rho, alpha = 1.0, omega = 1.0, rhoPrev = 1.0, res0;
+    double rr = 0.0;  // ||r||^2
+    int it = 0, stop = 0;
+    bool ok = true;
+    {
+        double s2[2] = {0.0, 0.0}, t2[2];
+        residual([&](uint32_t o) { return xin[(int64_t)(o / 8u) * xs]; },
+                 [&](int u, bool, double ri, double bi, const double (&a)[W],
+                     const uint32_t (&c)[W]) {
+#pragma unroll
+                     for (int k = 0; k < W; ++k) {  // a_ij / a_jj
+                         double dj;
+                         if (c[k] & kFar) {
+                             const uint32_t j = (c[k] & ~kFar) / 8u;
+                             dj = 1.0 / A.m.vals[A.m.rowOffs[j] + A.m.diag[j]];
+                         } else {
+                             dj = *at_byte(ls, c[k]);
+                         }
+                         const double v = a[k] != 0.0 ? a[k] * dj : 0.0;
+                         if (u < RES)
+                             mv[u][k] = v;
+                         else
+                             *svalAt(u, k) = v;
+                     }
+                     s2[0] += ri * ri;
+                     s2[1] += bi * bi;
+                     if (A.fresh) rv[u] = hv[u] = ri;
+                 });
+        if (A.fresh) {
+#pragma unroll
+            for (int u = 0; u < RPT; ++u)
+                if (shown >> u & 1) put_shared(mine(A.r, u), rv[u]);
+            ok = gs.sum<2, true>(s2, t2, L);
+            bnorm = sqrt(t2[1]);
+            if (!(bnorm > 0.0)) bnorm = 1.0;
+            rr = rho = t2[0];
+            res0 = sqrt(rr) / bnorm;
+        } else {
+            bnorm = uniform(st->bnorm);
+            rho = uniform(st->rho[0]);
+            rhoPrev = uniform(st->rho[1]);
+            alpha = uniform(st->alpha);
+            omega = uniform(st->omega);
+            rr = uniform(st->rr);
+            res0 = uniform(st->res0);
+            it = __builtin_amdgcn_readfirstlane(st->it);
+#pragma unroll
+            for (int u = 0; u < RPT; ++u)
+                if (live(u)) {
+                    rv[u] = *mine(A.r, u);
+                    hv[u] = *mine(A.rhat, u);
+                    vv[u] = *mine(A.v, u);
+                    lds(lp, u) = *mine(A.p, u);
+                }
+            double x[ghosts.K];
+            ghosts.each([&](int j, uint32_t o) { x[j] = get_shared(at_byte(A.p, o)); },
+                        [&](int j, int g) { gp[g] = x[j]; });
+            ghosts.each([&](int j, uint32_t o) { x[j] = get_shared(at_byte(A.v, o)); },
+                        [&](int j, int g) { gv[g] = x[j]; });
+        }
+    }
+    // streamed rows, as in kc_persist: after the last one the first of the next product
+    double vn[W];
+    uint32_t cn[W / 2];
+    auto fetch = [&](int u) {
+#pragma unroll
+        for (int j = 0; j < W / 2; ++j) cn[j] = pair(u, j);
+#pragma unroll
+        for (int k = 0; k < W; ++k) vn[k] = *svalAt(u, k);
+    };
+    // q = As vec of the own rows: the unit diagonal and the off-diagonal entries in
+    // column order
+    auto spmv = [&](double* vec, auto out) {
+        auto row = [&](int u, const double (&v)[W], const uint32_t (&c)[W / 2]) {
+            double x[W];
+#pragma unroll
+            for (int k = 0; k < W; ++k) x[k] = *at_byte(vec, col(c, k));
+            double sum = lds(vec, u);
+#pragma unroll
+            for (int k = 0; k < W; ++k) sum += v[k] * x[k];
+            out(u, sum);
+        };
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            if (u < RES) {
+                row(u, mv[u], mc[u]);
+            } else {
+                row(u, vn, cn);
+                fetch(u + 1 < RPT && live(u + 1) ? u + 1 : RES);
+            }
+        }
+    };
+    if (RES < RPT && live(RES)) fetch(RES);
+    int n = 0;
+    for (; ok; ++n) {
+        opaque(lb);
+        for (int u = 0; u < RES; ++u)
+            for (int j = 0; j < W / 2; ++j) opaque(mc[u][j]);
+        // the decision of kbi_dir
+        const double rn = sqrt(rr);
+        res = rn / bnorm;
+        if (res <= A.tol || rn <= A.atol)
+            stop = 2;
+        else if (!(res == res) || rho == 0.0 || (it > 0 && omega == 0.0))
+            stop = 3;
+        else if (it >= A.maxit)
+            stop = 1;
+        if (stop || n == A.iters) break;
+        const double beta = (rho / rhoPrev) * (alpha / omega);
+        const bool first = it == 0;
+        // p' = r + beta (p - omega v), of the own rows and the ghosts, whose r is kept
+        // in s's place
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            double& pl = lds(lp, u);
+            pl = first ? rv[u] : rv[u] + beta * (pl - omega * vv[u]);
+        }
+        double x[ghosts.K];
+        ghosts.each([&](int j, uint32_t o) { x[j] = get_shared(at_byte(A.r, o)); },
+                    [&](int j, int g) {
+                        gp[g] = first ? x[j] : x[j] + beta * (gp[g] - omega * gv[g]);
+                        gsv[g] = x[j];
+                    });
+        __syncthreads();
+        // v = As p, rhat.v
+        double v1[1] = {0.0}, t1[1];
+        spmv(lp, [&](int u, double q) {
+            vv[u] = q;
+            v1[0] += hv[u] * q;
+        });
+#pragma unroll
+        for (int u = 0; u < RPT; ++u)
+            if (shown >> u & 1) put_shared(mine(A.v2, u), vv[u]);
+        if (!(ok = gs.sum<1, true>(v1, t1, L))) break;
+        // alpha, s = r - alpha v
+        alpha = rho / t1[0];
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            lds(ls, u) = rv[u] - alpha * vv[u];
+        }
+        ghosts.each([&](int j, uint32_t o) { x[j] = get_shared(at_byte(A.v2, o)); },
+                    [&](int j, int g) {
+                        gv[g] = x[j];
+                        gsv[g] = gsv[g] - alpha * x[j];
+                    });
+        __syncthreads();
+        // t = As s, t.s and t.t
+        double v2[2] = {0.0, 0.0}, t2[2];
+        spmv(ls, [&](int u, double q) {
+            tv[u] = q;
+            v2[0] += q * lds(ls, u);
+            v2[1] += q * q;
+        });
+        if (!(ok = gs.sum<2, false>(v2, t2, L))) break;
+        // omega, x += D^-1 (alpha p + omega s), r = s - omega t, r.r and rhat.r
+        omega = t2[1] > 0.0 ? t2[0] / t2[1] : 0.0;
+        ++it;
+        double v3[2] = {0.0, 0.0}, t3[2];
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            const double si = lds(ls, u);
+            xr[u] += di[u] * (alpha * lds(lp, u) + omega * si);
+            const double ri = si - omega * tv[u];
+            rv[u] = ri;
+            if (shown >> u & 1) put_shared(mine(A.r, u), ri);
+            v3[0] += ri * ri;
+            v3[1] += hv[u] * ri;
+        }
+        if (!(ok = gs.sum<2, true>(v3, t3, L))) break;
+        rr = t3[0];
+        rhoPrev = rho;
+        rho = t3[1];
+    }
+    double trueRes = 0.0;
+    if (ok) {
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (!live(u)) break;
+            if (inN(u)) {
+                if (stop && (shown >> u & 1))
+                    put_shared(mine(A.x, u), xr[u]);
+                else
+                    *mine(A.x, u) = xr[u];
+                if (A.out && stop == 2) A.out[(int64_t)(iw + u * kB + lane) * A.stride] = xr[u];
+            }
+            if (!stop) {
+                *mine(A.r, u) = rv[u];
+                *mine(A.rhat, u) = hv[u];
+                *mine(A.v, u) = vv[u];
+                *mine(A.p, u) = lds(lp, u);
+            } else {
+                lds(lp, u) = xr[u];
+            }
+        }
+        if (stop) {  // the explicit residual of the result
+            double none[1] = {0.0}, all[1], s1[1] = {0.0};
+            ok = gs.sum<1, true>(none, all, L);
+            if (ok) {
+                residual([&](uint32_t o) { return get_shared(at_byte(A.x, o)); },
+                         [&](int, bool, double ri, double, const double (&)[W],
+                             const uint32_t (&)[W]) { s1[0] += ri * ri; });
+                ok = gs.sum<1, false>(s1, all, L);
+                trueRes = sqrt(all[0]) / bnorm;
+            }
+        }
+    }
+    if (!ok) {
+        if (tid == 0) st->stop = kStopSync;
+        return;
+    }
+    if (gs.slot == 0 && tid == 0) {
+        BiState o{};
+        o.rho[0] = rho;
+        o.rho[1] = rhoPrev;
+        o.alpha = alpha;
+        o.omega = omega;
+        o.bnorm = bnorm;
+        o.res = res;
+        o.res0 = res0;
+        o.rr = rr;
+        o.trueRes = trueRes;
+        o.it = it;
+        o.stop = stop;
+        *st = o;
+    }
+}
+
+// The form for tiles with more ghosts than fit: the reader of a far column evaluates
+// its owner's p' or s where the product meets it, so p is published too and p and v
+// alternate between two buffers.
+template <int RPT, int W, int RES>
+__global__ __launch_bounds__(kPersistThreads) void kbi_persist_far(BiPersist A) {
     __shared__ PersistLds L;
     // the raw matrix rows of 256 rows of each tile (start and end of the solve) share
     // their LDS with p and s
@@ -669,21 +998,26 @@ struct BiWork : fv_solver_cache {
     int persistGrid = 0, persistIters = 0;
     DBuf<unsigned long long> slots;
     uint32_t tag = 1;
+    GhostPlan plan;
     // 1, 2 or 4 rows per thread (2^20 rows); RES, the rows whose matrix stays in
     // registers, as in the CG
     template <int W>
-    static auto persist_kernel(int rpt) -> void (*)(BiPersist) {
-        if (rpt <= 1) return kbi_persist<1, W, 1>;
-        if (rpt <= 2) return kbi_persist<2, W, 1>;
-        if (rpt <= 4) return kbi_persist<4, W, 0>;
-        return nullptr;
+    void choose_kernel(fv_ctx* c, int rpt) {
+        const int n = rpt <= 1 ? 1 : rpt <= 2 ? 2 : 4;
+        if (plan.make(c, h.N, h.ntiles, h.rowsPerBlock, W, n * kB, 8, bi_ghost_cap(n), h.sellCol))
+            persist = n == 1 ? kbi_persist<1, W, 1> : n == 2 ? kbi_persist<2, W, 2> : kbi_persist<4, W, 0>;
+        else
+            persist = n == 1   ? kbi_persist_far<1, W, 1>
+                      : n == 2 ? kbi_persist_far<2, W, 1>
+                               : kbi_persist_far<4, W, 0>;
     }
     void choose_persist(fv_ctx* c, const fv_sparsity* sp) {
         const int rpt = (h.rowsPerBlock + kB - 1) / kB;
+        if (rpt > 4) return;
         if (sp->sellWidth == 6)
-            persist = persist_kernel<6>(rpt);
+            choose_kernel<6>(c, rpt);
         else if (sp->sellWidth == 4)
-            persist = persist_kernel<4>(rpt);
+            choose_kernel<4>(c, rpt);
         persistGrid = persist_grid(h.ntiles);
         if (!persist || !persist_fits(reinterpret_cast<const void*>(persist), c->device, persistGrid)) {
             persist = nullptr;
@@ -714,7 +1048,8 @@ struct BiWork : fv_solver_cache {
         BiPersist a{h.N, h.ntiles, h.rowsPerBlock, persistIters, fresh ? 1 : 0, o->max_iter, tag,
                     o->rel_tol, o->abs_tol, h.sellCol, CsrSystem{h.rowOffs, diag, h.vals, t.rhs + t.comp},
                     t.ncomp, x, t.ncomp > 1 ? x : nullptr, chained ? state - 1 : nullptr, sval.p,
-                    t.ncomp > 1 ? dinv.p : x, h.r, h.rhat, h.p, h.s, h.v, h.t, state, slots.p};
+                    t.ncomp > 1 ? dinv.p : x, h.r, h.rhat, h.p, h.v, h.t, h.s, plan.words.p,
+                    plan.ghosts.p, plan.count.p, plan.stride, state, slots.p};
         void* args[] = {&a};
         if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(persist), dim3(persistGrid),
                                        dim3(kPersistThreads), args, 0, s) != hipSuccess) {

@@ -60,6 +60,8 @@
 
 #include "cgkernels.hpp"
 
+#include <vector>
+
 namespace fvhip {
 namespace {
 
@@ -417,6 +419,51 @@ __global__ __launch_bounds__(kCgBlock) void k_ghost_plan(int N, int R, int W, in
     if (tid == 0) count[tile] = base;
 }
 
+// The ghosts of a tile, seen by one of its 256 threads: ghost s is thread s % 256's,
+// which holds the places in the vectors of its first K (byte offsets, SIZE bytes a
+// value).
+template <int KG, int SIZE>
+struct GhostWalk {
+    static constexpr int K = KG;
+    const int32_t* list;
+    int n, t;
+    uint32_t place[K];
+    __device__ GhostWalk(const int32_t* ghosts, const int32_t* count, int stride, int tile, int tiles) {
+        t = (int)threadIdx.x & (kCgBlock - 1);
+        n = tile < tiles ? count[tile] : 0;
+        list = ghosts + (int64_t)(tile < tiles ? tile : 0) * stride;
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const int s = t + j * kCgBlock;
+            place[j] = s < n ? (uint32_t)list[s] * (uint32_t)SIZE : 0u;
+        }
+    }
+    // K ghosts at a time: load(j, place) for each, then use(j, s).  The places of the
+    // next K are loaded meanwhile.
+    template <class Load, class Use>
+    __device__ __forceinline__ void each(Load load, Use use) const {
+        uint32_t o[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) o[j] = place[j];
+        for (int s0 = 0; s0 < n; s0 += K * kCgBlock) {
+            uint32_t next[K];
+            if (s0 + K * kCgBlock < n) {
+#pragma unroll
+                for (int j = 0; j < K; ++j)
+                    next[j] = (uint32_t)list[min(s0 + (K + j) * kCgBlock + t, n - 1)] * (uint32_t)SIZE;
+            }
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+                if (s0 + j * kCgBlock + t < n) load(j, o[j]);
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+                if (s0 + j * kCgBlock + t < n) use(j, s0 + j * kCgBlock + t);
+#pragma unroll
+            for (int j = 0; j < K; ++j) o[j] = next[j];
+        }
+    }
+};
+
 // RPT: rows per thread (the rows a tile gives a thread, rounded up to a power
 // of two); W: entries of every slice of the sliced ELL; RES: rows of each thread
 // whose values and columns stay in registers; GL: rows whose g is in LDS too, DLDS: d
@@ -477,42 +524,10 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     };
     auto col = [](const uint32_t (&c)[W / 2], int k) { return k & 1 ? c[k / 2] >> 16 : c[k / 2] & 0xffffu; };
 
-    // Ghost s of the tile is thread s % 256's, which holds the places in the vectors
-    // of its first kGk; its p is kept in LDS and follows p' = r + beta p like its
-    // owner's, so all that a tile reads of another's rows is their r.
-    constexpr int kGk = RPT == 2 || (RPT == 4 && sizeof(S) == 4) ? 6 : 4;
-    const int gt = tid & (kCgBlock - 1), ng = tile < A.tiles ? A.count[tile] : 0;
-    const int32_t* const glist = A.ghosts + (int64_t)(tile < A.tiles ? tile : 0) * A.ghostStride;
-    uint32_t gc[kGk];
-#pragma unroll
-    for (int j = 0; j < kGk; ++j) {
-        const int s = gt + j * kCgBlock;
-        gc[j] = s < ng ? (uint32_t)glist[s] * (uint32_t)sizeof(S) : 0u;
-    }
-    // kGk ghosts at a time: first(j, o) for each, o its byte offset in the vectors,
-    // then then(j, s).  The places of the next kGk are loaded meanwhile.
-    auto each_ghost = [&](auto first, auto then) {
-        uint32_t o[kGk];
-#pragma unroll
-        for (int j = 0; j < kGk; ++j) o[j] = gc[j];
-        for (int s0 = 0; s0 < ng; s0 += kGk * kCgBlock) {
-            uint32_t next[kGk];
-            if (s0 + kGk * kCgBlock < ng) {
-#pragma unroll
-                for (int j = 0; j < kGk; ++j)
-                    next[j] = (uint32_t)glist[min(s0 + (kGk + j) * kCgBlock + gt, ng - 1)] *
-                              (uint32_t)sizeof(S);
-            }
-#pragma unroll
-            for (int j = 0; j < kGk; ++j)
-                if (s0 + j * kCgBlock + gt < ng) first(j, o[j]);
-#pragma unroll
-            for (int j = 0; j < kGk; ++j)
-                if (s0 + j * kCgBlock + gt < ng) then(j, s0 + j * kCgBlock + gt);
-#pragma unroll
-            for (int j = 0; j < kGk; ++j) o[j] = next[j];
-        }
-    };
+    // A ghost's p follows p' = r + beta p like its owner's, so all that a tile reads of
+    // another's rows is their r.
+    const GhostWalk<RPT == 2 || (RPT == 4 && sizeof(S) == 4) ? 6 : 4, sizeof(S)> ghosts(
+        A.ghosts, A.count, A.ghostStride, tile, A.tiles);
 
     // Bit u: row u has a far column.  The pattern is symmetric, so those are the
     // rows that other workgroups read, and only they are published.
@@ -667,9 +682,9 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     rrep = WHOLE ? 0.0 : uniform(st->rrep);
     S beta = S(0);
     {  // the ghosts' p
-        S x[kGk];
-        each_ghost([&](int j, uint32_t o) { x[j] = get_shared(at_byte(A.p, o)); },
-                   [&](int j, int s) { ghost[s] = x[j]; });
+        S x[ghosts.K];
+        ghosts.each([&](int j, uint32_t o) { x[j] = get_shared(at_byte(A.p, o)); },
+                    [&](int j, int s) { ghost[s] = x[j]; });
     }
     // streamed rows: loaded when the row before is done (the first one of an iteration
     // at the end of the one before, across its exchanges); the other waves of the SIMD
@@ -688,9 +703,9 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
         for (int u = 0; u < RES; ++u)
             for (int j = 0; j < W / 2; ++j) opaque(mc[u][j]);
         if (n) {
-            S x[kGk];
-            each_ghost([&](int j, uint32_t o) { x[j] = get_shared(at_byte(A.r, o)); },
-                       [&](int j, int s) { ghost[s] = x[j] + beta * ghost[s]; });
+            S x[ghosts.K];
+            ghosts.each([&](int j, uint32_t o) { x[j] = get_shared(at_byte(A.r, o)); },
+                        [&](int j, int s) { ghost[s] = x[j] + beta * ghost[s]; });
         }
         __syncthreads();
         // q = As p, p.q
@@ -1042,6 +1057,33 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist_far(CgPersist<S> A
         st->pbuf = 0;
     }
 }
+
+// The ghosts of every tile of a system and the columns that refer to them.
+struct GhostPlan {
+    DBuf<uint32_t> words;
+    DBuf<int32_t> ghosts, count;
+    int stride = 0;
+    // False if a tile has more than cap ghosts.  own: rows a tile has places for; size:
+    // bytes a value.
+    bool make(fv_ctx* c, int N, int tiles, int R, int W, int own, int size, int cap,
+              const int32_t* sellCol) {
+        count.alloc(c, tiles);
+        auto plan = [&](uint32_t* w, int32_t* g) {
+            k_ghost_plan<<<tiles, kCgBlock, 0, c->stream>>>(N, R, W, own, size, sellCol, w, g, stride,
+                                                            count.p);
+            FV_LAUNCH_CHECK();
+        };
+        plan(nullptr, nullptr);
+        std::vector<int32_t> n(tiles);
+        count.download(n.data());
+        for (int32_t v : n) stride = v > stride ? v : stride;
+        if (stride > cap) return false;
+        words.alloc(c, ((size_t)N + 63) / 64 * 64 * W / 2);
+        ghosts.alloc(c, (size_t)tiles * (stride > 0 ? stride : 1));
+        plan(words.p, ghosts.p);
+        return true;
+    }
+};
 
 // Workgroups of a persistent launch over `tiles` tiles
 inline int persist_grid(int tiles) {

@@ -52,9 +52,7 @@ struct CgWork : fv_solver_cache {
     int lastLaunches = 0;  // persistent launches of the previous mixed solve
     int lastTotal = 0;     // iterations of the previous solve, in either form
     DBuf<unsigned long long> slots;
-    DBuf<uint32_t> words;  // kc_persist's columns and ghosts
-    DBuf<int32_t> ghosts, ghostCount;
-    int ghostStride = 0;
+    GhostPlan plan;
     uint32_t tag = 1;
 
     CgWork(fv_ctx* c, const fv_linsys* ls) {
@@ -151,7 +149,8 @@ struct CgWork : fv_solver_cache {
     template <int W>
     void choose_kernel(fv_ctx* c, int tiles, int R, int rpt) {
         const int n = rpt <= 1 ? 1 : rpt <= 2 ? 2 : rpt <= 4 ? 4 : 8;
-        if (make_ghosts(c, tiles, R, W, n)) {
+        // (more ghosts than fit: never up to 2 FP64 or 4 FP32 rows per thread)
+        if (plan.make(c, h.N, tiles, R, W, n * kB, (int)sizeof(S), ghost_cap<S>(n, W), h.sellCol)) {
             if constexpr (sizeof(S) == 8)
                 persist = n == 1   ? kc_persist<S, 1, W, 1, 1, true, true>
                           : n == 2 ? kc_persist<S, 2, W, 2, 2, true, true>
@@ -168,26 +167,6 @@ struct CgWork : fv_solver_cache {
             persist = kc_persist_far<S, 8, W, 4, true>;
         }
     }
-    // The ghosts of every tile and the columns that refer to them; false if a tile has
-    // more than fit (never up to 2 FP64 or 4 FP32 rows per thread).
-    bool make_ghosts(fv_ctx* c, int tiles, int R, int W, int rpt) {
-        hipStream_t s = c->stream;
-        ghostCount.alloc(c, tiles);
-        auto plan = [&](uint32_t* w, int32_t* g) {
-            k_ghost_plan<<<tiles, kB, 0, s>>>(h.N, R, W, rpt * kB, (int)sizeof(S), h.sellCol, w, g,
-                                              ghostStride, ghostCount.p);
-            FV_LAUNCH_CHECK();
-        };
-        plan(nullptr, nullptr);
-        std::vector<int32_t> n(tiles);
-        ghostCount.download(n.data());
-        ghostStride = *std::max_element(n.begin(), n.end());
-        if (ghostStride > ghost_cap<S>(rpt, W)) return false;
-        words.alloc(c, ((size_t)h.N + 63) / 64 * 64 * W / 2);
-        ghosts.alloc(c, std::max<size_t>(1, (size_t)tiles * ghostStride));
-        plan(words.p, ghosts.p);
-        return true;
-    }
     // Up to persistIters iterations in one launch; false if the device refuses it.
     // (whole: x, the limits and whether the solve starts.)
     bool run_persist(hipStream_t s, double* x = nullptr, double tol = 0.0, double atol = 0.0,
@@ -195,8 +174,8 @@ struct CgWork : fv_solver_cache {
         const uint32_t uses = 2 * (uint32_t)persistIters + 8;
         if (tag > 0xffffffffu - uses) clear_tags(s);  // sequence numbers start over
         CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persistIters, tag, h.sellCol, h.sval,
-                       h.g, h.d, h.r, h.p, h.p2, words.p, ghosts.p, ghostCount.p, ghostStride,
-                       h.st, slots.p,
+                       h.g, h.d, h.r, h.p, h.p2, plan.words.p, plan.ghosts.p, plan.count.p,
+                       plan.stride, h.st, slots.p,
                        CsrSystem{h.rowOffs, h.diag, h.vals, h.rhs}, x, tol, atol, maxit,
                        fresh ? 1 : 0};
         void* args[] = {&a};

@@ -76,6 +76,7 @@ def test_persistent_is_bitwise_the_kernel_by_kernel_form(ctx, dims, limit, preci
 
 
 GHOST_CASES = [
+    ((64, 64, 63), "random"),     # one row per thread: up to 1536 ghosts for 256 rows
     ((64, 64, 65), "random"),     # 2 rows per thread: a tile of 512 rows has up to 3072 ghosts
     ((101, 100, 61), "random"),   # 3 rows: more ghosts than fit in FP64, not in FP32
     ((128, 128, 70), "block"),    # 5 rows: the same
@@ -83,14 +84,14 @@ GHOST_CASES = [
 ]
 
 
-@pytest.mark.parametrize("precision", ["double", "mixed"])
+@pytest.mark.parametrize("method", ["double", "mixed", "bicgstab"])
 @pytest.mark.parametrize("dims,order", GHOST_CASES, ids=str)
-def test_many_ghosts(ctx, dims, order, precision):
+def test_many_ghosts(ctx, dims, order, method):
     """Tiles whose rows refer to many rows of other tiles: in LDS while they fit, else read
     where the product meets them.  Fewer iterations than one replacement takes."""
     import foamadapter_amd as fa
     from foamadapter_amd import dsl, fvcc, la
-    print(dims, order, precision, flush=True)
+    print(dims, order, method, flush=True)
     m = fa.Mesh.from_poly(ctx, fa.PolyMesh.hex(dims, **({"perm_seed": 3} if order == "random" else {})))
     N, F, B = m.n_cells, m.n_internal_faces, m.n_boundary_faces
     p = fvcc.VolumeField(m, ctx.zeros((N,)), ctx.zeros((B,)),
@@ -101,8 +102,8 @@ def test_many_ghosts(ctx, dims, order, precision):
     got = []
     for graph in (False, True, True):
         x = ctx.uniform(N, -1, 1, 12, 4)
-        st = la.solve_cg(ls, x, {"relTol": 1e-12, "maxIter": 20, "precision": precision, "graph": graph},
-                         raise_on_noconverge=False)
+        opts = {"solver": "PBiCGStab"} if method == "bicgstab" else {"precision": method}
+        st = la.solve_cg(ls, x, dict(opts, relTol=1e-12, maxIter=20, graph=graph), raise_on_noconverge=False)
         got.append((x.numpy(), st.numIter, st.finalResNorm))
     for g in got[1:]:
         assert g[1:] == got[0][1:] and np.array_equal(g[0], got[0][0])

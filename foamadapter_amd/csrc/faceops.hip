@@ -44,6 +44,12 @@ struct ExGeo {
 
 // ---- cell-result operators -------------------------------------------------
 
+// The per-cell stencil walk.  A cell's entries are taken kWalk at a time: their face and
+// cell indices in one round of loads, then everything these lead to in a second, then
+// the arithmetic in the order of the entries; one entry after another, each waited for
+// its own two rounds.
+constexpr int kWalk = 6;
+
 template <typename S>
 __global__ __launch_bounds__(kBlock) void k_grad(int N, int F, const int32_t* __restrict__ off,
                                                  const int32_t* __restrict__ idx,
@@ -52,34 +58,45 @@ __global__ __launch_bounds__(kBlock) void k_grad(int N, int F, const int32_t* __
                                                  S coeff, S* __restrict__ out) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= N) return;
-    const S Tc = T[c];
+    const S Tc = T[c], v = g.V[c];
     S ax = 0, ay = 0, az = 0;
     const int e1 = off[c + 1];
-    for (int k = off[c]; k < e1; ++k) {
-        const int e = idx[k];
-        if (e >= F) {
-            const int b = e - F;
-            const S tb = Tb[b];
-            ax += g.Sfb[3 * b] * tb;
-            ay += g.Sfb[3 * b + 1] * tb;
-            az += g.Sfb[3 * b + 2] * tb;
-        } else {
-            const S To = T[oth[k]];
-            if (e >= 0) {
-                const S tf = g.w[e] * (Tc - To) + To;
-                ax += g.Sf[3 * (int64_t)e] * tf;
-                ay += g.Sf[3 * (int64_t)e + 1] * tf;
-                az += g.Sf[3 * (int64_t)e + 2] * tf;
+    for (int k = off[c]; k < e1; k += kWalk) {
+        int e[kWalk], o[kWalk];
+#pragma unroll
+        for (int j = 0; j < kWalk; ++j) {
+            e[j] = idx[min(k + j, e1 - 1)];
+            o[j] = oth[min(k + j, e1 - 1)];
+        }
+        S t[kWalk], w[kWalk], sx[kWalk], sy[kWalk], sz[kWalk];
+#pragma unroll
+        for (int j = 0; j < kWalk; ++j) {
+            const bool b = e[j] >= F;
+            const int f = b ? e[j] - F : e[j] >= 0 ? e[j] : ~e[j];
+            const S* const s = (b ? g.Sfb : g.Sf) + 3 * (int64_t)f;
+            sx[j] = s[0];
+            sy[j] = s[1];
+            sz[j] = s[2];
+            t[j] = *(b ? Tb + f : T + o[j]);
+            w[j] = b ? S(0) : g.w[f];
+        }
+#pragma unroll
+        for (int j = 0; j < kWalk; ++j) {
+            if (k + j >= e1) break;
+            const S tf = e[j] >= F   ? t[j]
+                         : e[j] >= 0 ? w[j] * (Tc - t[j]) + t[j]
+                                     : w[j] * (t[j] - Tc) + Tc;
+            if (e[j] >= 0) {
+                ax += sx[j] * tf;
+                ay += sy[j] * tf;
+                az += sz[j] * tf;
             } else {
-                const int f = ~e;
-                const S tf = g.w[f] * (To - Tc) + Tc;
-                ax -= g.Sf[3 * (int64_t)f] * tf;
-                ay -= g.Sf[3 * (int64_t)f + 1] * tf;
-                az -= g.Sf[3 * (int64_t)f + 2] * tf;
+                ax -= sx[j] * tf;
+                ay -= sy[j] * tf;
+                az -= sz[j] * tf;
             }
         }
     }
-    const S v = g.V[c];
     out[3 * (int64_t)c] = coeff * (ax / v);
     out[3 * (int64_t)c + 1] = coeff * (ay / v);
     out[3 * (int64_t)c + 2] = coeff * (az / v);
@@ -97,34 +114,42 @@ __global__ __launch_bounds__(kBlock) void k_div(int N, int F, int scheme,
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= N) return;
     S acc = 0;
+    const S vol = g.V[c], Tc = T ? T[c] : S(0);
     const int e1 = off[c + 1];
-    if (T) {
-        const S Tc = T[c];
-        for (int k = off[c]; k < e1; ++k) {
-            const int e = idx[k];
-            if (e >= F) {
-                const int b = e - F;
-                acc += phi[e] * Tb[b];
-            } else {
-                const S To = T[oth[k]];
-                const int f = e >= 0 ? e : ~e;
-                const S ph = phi[f];
-                const S lam = scheme == 0 ? g.w[f] : (ph >= S(0) ? S(1) : S(0));
-                // owner side: P = this cell; neighbour side: P = other cell
-                const S TP = e >= 0 ? Tc : To, TN = e >= 0 ? To : Tc;
-                const S v = ph * (lam * (TP - TN) + TN);
-                if (e >= 0) acc += v; else acc -= v;
+    for (int k = off[c]; k < e1; k += kWalk) {
+        int e[kWalk], o[kWalk];
+#pragma unroll
+        for (int j = 0; j < kWalk; ++j) {
+            e[j] = idx[min(k + j, e1 - 1)];
+            if (T) o[j] = oth[min(k + j, e1 - 1)];
+        }
+        S ph[kWalk], t[kWalk], w[kWalk];
+#pragma unroll
+        for (int j = 0; j < kWalk; ++j) {
+            const bool b = e[j] >= F;
+            const int f = e[j] >= 0 ? e[j] : ~e[j];
+            ph[j] = phi[f];
+            if (T) {
+                t[j] = *(b ? Tb + (f - F) : T + o[j]);
+                w[j] = b || scheme != 0 ? S(0) : g.w[f];
             }
         }
-    } else {
-        for (int k = off[c]; k < e1; ++k) {
-            const int e = idx[k];
-            if (e >= F) acc += phi[e];
-            else if (e >= 0) acc += phi[e];
-            else acc -= phi[~e];
+#pragma unroll
+        for (int j = 0; j < kWalk; ++j) {
+            if (k + j >= e1) break;
+            S v = ph[j];
+            if (T && e[j] >= F) {
+                v = ph[j] * t[j];
+            } else if (T) {
+                const S lam = scheme == 0 ? w[j] : (ph[j] >= S(0) ? S(1) : S(0));
+                // owner side: P = this cell; neighbour side: P = other cell
+                const S TP = e[j] >= 0 ? Tc : t[j], TN = e[j] >= 0 ? t[j] : Tc;
+                v = ph[j] * (lam * (TP - TN) + TN);
+            }
+            if (e[j] >= 0) acc += v; else acc -= v;
         }
     }
-    out[c] = coeff * (acc / g.V[c]);
+    out[c] = coeff * (acc / vol);
 }
 
 template <typename S>
@@ -141,24 +166,43 @@ __global__ __launch_bounds__(kBlock) void k_laplacian(
     const S* __restrict__ Tg, S coeff, S* __restrict__ out) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= N) return;
-    const S Tc = T[c];
+    const S Tc = T[c], vol = g.V[c];
     S acc = 0;
     const int e1 = off[c + 1];
-    for (int k = off[c]; k < e1; ++k) {
-        const int e = idx[k];
-        if (e >= F) {
-            const int b = e - F;
-            const S sn = bnd_sngrad<S>(kind[b], g.dcb[b], Tb[b], Tc, Tg, b);
-            acc += (gamma[e] * g.magSfb[b]) * sn;
-        } else {
-            const S To = T[oth[k]];
-            const int f = e >= 0 ? e : ~e;
-            const S TP = e >= 0 ? Tc : To, TN = e >= 0 ? To : Tc;
-            const S v = (gamma[f] * g.magSf[f]) * (g.nodc[f] * (TN - TP));
-            if (e >= 0) acc += v; else acc -= v;
+    for (int k = off[c]; k < e1; k += kWalk) {
+        int e[kWalk], o[kWalk];
+#pragma unroll
+        for (int j = 0; j < kWalk; ++j) {
+            e[j] = idx[min(k + j, e1 - 1)];
+            o[j] = oth[min(k + j, e1 - 1)];
+        }
+        S ga[kWalk], ms[kWalk], dc[kWalk], t[kWalk], tg[kWalk];
+        int kd[kWalk];
+#pragma unroll
+        for (int j = 0; j < kWalk; ++j) {
+            const bool b = e[j] >= F;
+            const int f = b ? e[j] - F : e[j] >= 0 ? e[j] : ~e[j];
+            ga[j] = gamma[b ? e[j] : f];
+            ms[j] = *(b ? g.magSfb + f : g.magSf + f);
+            dc[j] = *(b ? g.dcb + f : g.nodc + f);
+            t[j] = *(b ? Tb + f : T + o[j]);
+            kd[j] = b ? kind[f] : 0;
+            tg[j] = b && Tg ? Tg[f] : S(0);
+        }
+#pragma unroll
+        for (int j = 0; j < kWalk; ++j) {
+            if (k + j >= e1) break;
+            const S gm = ga[j] * ms[j];
+            if (e[j] >= F) {
+                acc += gm * (kd[j] == FV_BC_FIXED_GRADIENT ? tg[j] : dc[j] * (t[j] - Tc));
+            } else {
+                const S TP = e[j] >= 0 ? Tc : t[j], TN = e[j] >= 0 ? t[j] : Tc;
+                const S v = gm * (dc[j] * (TN - TP));
+                if (e[j] >= 0) acc += v; else acc -= v;
+            }
         }
     }
-    out[c] = coeff * (acc / g.V[c]);
+    out[c] = coeff * (acc / vol);
 }
 
 // ---- LDS-staged cell gathers (meshes in upper-triangular face order) --------
@@ -888,11 +932,27 @@ __global__ __launch_bounds__(kBlock) void k_correct_bc(int B, int nc, const int3
     }
 }
 
-// Operator drivers: the LDS-staged gather on upper-triangular meshes, the
-// stencil walk otherwise (same arithmetic, same order).
+// Operator drivers: the LDS-staged gather on upper-triangular meshes, the stencil walk
+// otherwise and on small meshes (same arithmetic, same order).  The walk has two rounds
+// of loads where the staged gather has four and a barrier, but reads every face from
+// both its cells: with the faces in the L2s its latency counts, beyond them its bytes.
+// FP64 gradient, linear and upwind divergence, laplacian, staged -> walk in us: 16^3
+// in block order 5.3, 5.0, 4.9, 5.4 -> 3.8, 4.1, 4.0, 4.1; 40^3 in Z order 5.6, 5.3,
+// 5.2, 5.4 -> 4.6, 5.1, 5.0, 5.4; 48^3 5.7, 5.2, 5.1, 5.5 -> 6.9, 5.4, 4.6, 6.7.  In
+// the wide form the line lies higher: 64^3 in block order 15.4, 10.0, 8.0, 12.4 ->
+// 12.3, 8.1, 6.4, 11.4; 80^3 24.0, 16.9, 14.8, 20.2 -> 25.6, 17.1, 13.4, 22.5.
+template <typename S>
+bool staged(const fv_mesh* m) {
+    if (!gather_cells(m)) return false;
+    if (m->gatherMode != 0) return true;
+    if (m->nCells <= 1 << 16) return false;
+    return m->nCells > 1 << 18 ||
+           !gather_wide(gather_lists(const_cast<fv_mesh*>(m), 256, sizeof(S) == 4));
+}
+
 template <typename S>
 void run_grad(fv_ctx* ctx, const fv_mesh* m, Geo<S> g, const S* T, const S* Tb, S coeff, S* out) {
-    if (gather_cells(m)) {
+    if (staged<S>(m)) {
         launch_gather<S>(ctx, m, GradOp<S>{{}, T, g.w, g.Sf, g.Sfb, Tb}, g.V, coeff, out);
         return;
     }
@@ -905,7 +965,7 @@ void run_grad(fv_ctx* ctx, const fv_mesh* m, Geo<S> g, const S* T, const S* Tb, 
 template <typename S>
 void run_div(fv_ctx* ctx, const fv_mesh* m, int scheme, Geo<S> g, const S* phi, const S* T,
              const S* Tb, S coeff, S* out) {
-    if (gather_cells(m)) {
+    if (staged<S>(m)) {
         if (!T)
             launch_gather<S>(ctx, m, IntegrateOp<S>{{}, phi, m->nInt}, g.V, coeff, out);
         else if (scheme == FV_LINEAR)
@@ -923,7 +983,7 @@ void run_div(fv_ctx* ctx, const fv_mesh* m, int scheme, Geo<S> g, const S* phi, 
 template <typename S>
 void run_lap(fv_ctx* ctx, const fv_mesh* m, Geo<S> g, const int8_t* kind, const S* gamma,
              const S* T, const S* Tb, const S* Tg, S coeff, S* out) {
-    if (gather_cells(m)) {
+    if (staged<S>(m)) {
         launch_gather<S>(ctx, m,
                          LapOp<S>{{}, T, gamma, g.magSf, g.nodc, g.magSfb, g.dcb, Tb, Tg, kind, m->nInt},
                          g.V, coeff, out);

@@ -55,3 +55,46 @@ def test_block_order_takes_the_staged_path(ctx):
     blocks, over = m.gather_stats(256)
     assert over * 100 <= blocks
     m.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("dims", DIMS + [(1, 1, 1), "refined", (64, 32, 32), (61, 33, 33), (64, 64, 64), (65, 65, 63)], ids=str)
+def test_walk_and_staged_at_the_edges_of_the_rule(ctx, dims, dtype):
+    """Small meshes walk the stencil by themselves (65536 cells, 262144 in a block mesher's
+    order), six entries at a time (the refined mesh has a cell with 400): every mode against the
+    sums over the faces in Python's order (small meshes) and against each other."""
+    import foamadapter_amd as fa
+    from foamadapter_amd import fvcc
+    import oracle_cpu as orc
+    from skewed_meshes import refined_block
+    print(dims, dtype, flush=True)
+    poly = refined_block(20) if dims == "refined" else fa.PolyMesh.hex(dims, jitter=0.0 if dims == (1, 1, 1) else 0.2, jitter_seed=3)
+    poly = poly[0] if isinstance(poly, tuple) else poly
+    m = fa.Mesh.from_poly(ctx, poly)
+    N, F, B = m.n_cells, m.n_internal_faces, m.n_boundary_faces
+    kinds = (["fixedValue", "fixedGradient"] * m.n_patches)[:m.n_patches]
+    T = fvcc.VolumeField(m, ctx.uniform(N, -1, 1, 1, 0, dtype), ctx.uniform(B, -1, 1, 1, 1, dtype),
+                         fa.BoundaryConditions(m, kinds), "T", ctx.uniform(B, -1, 1, 1, 2, dtype))
+    phi = fvcc.SurfaceField(m, ctx.uniform(F + B, -1, 1, 1, 3, dtype))
+    gamma = fvcc.SurfaceField(m, ctx.uniform(F + B, 0.5, 2, 1, 4, dtype))
+
+    def ops():
+        return [fvcc.GaussGreenGrad(ctx, m).grad(T, 1.5).numpy(),
+                fvcc.GaussGreenDiv(ctx, m, ["linear"]).div(None, phi, T, 0.5).numpy(),
+                fvcc.GaussGreenDiv(ctx, m, ["upwind"]).div(None, phi, T).numpy(),
+                fvcc.GaussGreenDiv(ctx, m).div(None, phi).numpy(),
+                fvcc.GaussGreenLaplacian(ctx, m).laplacian(None, gamma, T, 2.0).numpy()]
+
+    got = {}
+    for mode in (1, 0, 2):
+        m.set_gather(mode)
+        got[mode] = ops()
+    for mode in (0, 2):
+        for name, a, b in zip(("grad", "div", "upwind", "integrate", "laplacian"), got[mode], got[1]):
+            assert np.array_equal(a, b), (mode, name)
+    if dtype == np.float64 and N <= 10000:
+        g = orc.geometry(poly)
+        Th, Tb, ph = T.numpy(), T.boundary.numpy(), phi.values.numpy()
+        assert np.array_equal(got[1][0], 1.5 * orc.grad(g, Th, Tb))
+        assert np.array_equal(got[1][1], 0.5 * orc.div(g, ph, Th, Tb))
+    m.close()

@@ -221,5 +221,6 @@ def check(rc: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    fn = getattr(lib, name)
-    check(fn(*args))
+    rc = getattr(lib, name)(*args)
+    if rc:
+        check(rc)

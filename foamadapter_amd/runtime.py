@@ -15,9 +15,14 @@ import numpy as np
 from ._lib import FV_F32, FV_F64, call, lib
 
 _DT = {np.dtype(np.float64): FV_F64, np.dtype(np.float32): FV_F32}
+_F64 = np.dtype(np.float64)
 
 
 def prec_of(dtype) -> int:
+    # numpy's built-in dtypes are single objects; hashing one takes longer than the rest
+    # of an operator's Python
+    if dtype is _F64:
+        return FV_F64
     return _DT[np.dtype(dtype)]
 
 

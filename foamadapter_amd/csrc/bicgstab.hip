@@ -289,14 +289,14 @@ __global__ void kbi_scale(int64_t n, const int32_t* __restrict__ src, const int3
 // no-op iterations behind the stop, which the host reads in doubling steps) and two
 // for the explicit residual; at 64^3 an iteration is 31 us of kernels that move
 // 78 MB, and the launches, reads and no-ops around it take as long again.  Here one
-// cooperative launch scales the matrix, takes the initial residual, iterates and
+// launch (see Meeting) scales the matrix, takes the initial residual, iterates and
 // takes the explicit residual of the result, on the tiles, the exchange and the LDS
 // scheme of cgpersist.hpp: r, rhat, v, t, x and D^-1 of a thread's rows in registers,
 // p and s in LDS, with p, s and v of the tile's ghosts (up to 4 rows per thread).  Each
 // tile publishes v and r of the rows that others refer to, and follows p' = r + beta (p
 // - omega v) and s = r - alpha v for its ghosts, so an iteration has three grid
 // exchanges.  The order of all sums is that of the kernels above (same
-// bits).  Advection step on 110x100x90 cells (about 28 iterations) 2.9 -> 1.18 ms (1.62
+// bits).  Advection step on 110x100x90 cells (about 28 iterations) 2.97 -> 1.13 ms (1.62
 // with the far columns read in the product, as kbi_persist_far does), an icoFoam step
 // at 64^3 (three momentum solves) 5.01 -> 4.25 ms.
 //
@@ -326,6 +326,7 @@ struct BiPersist {
     const uint32_t* words;  // the columns, see k_ghost_plan; ghosts of each tile
     const int32_t *ghosts, *count;
     int32_t ghostStride;
+    unsigned long long meet;  // Meeting::target
     BiState* st;
     unsigned long long* slots;
 };
@@ -352,6 +353,8 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
     const int R = A.rowsPerTile;
     const int tile = gs.place(A.tiles, sub);
     BiState* const st = A.st;
+    const Meeting meeting{A.slots + 2 * kSlotBuffer, A.meet, A.tag0};
+    meeting.arrive();
     if (!A.fresh && st->stop) return;
     if (A.prev && A.prev->stop != 2) {
         if (gs.slot == 0 && tid == 0) st->stop = 0;
@@ -447,6 +450,10 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
                      s2[1] += bi * bi;
                      if (A.fresh) rv[u] = hv[u] = ri;
                  });
+        if (!meeting.met(L)) {
+            if (gs.slot == 0 && tid == 0) st->stop = kStopApart;
+            return;
+        }
         if (A.fresh) {
 #pragma unroll
             for (int u = 0; u < RPT; ++u)
@@ -996,7 +1003,8 @@ struct BiWork : fv_solver_cache {
     // persistent form (null: kernel by kernel)
     void (*persist)(BiPersist) = nullptr;
     int persistGrid = 0, persistIters = 0;
-    DBuf<unsigned long long> slots;
+    PersistSlots slots;
+    bool plain = false;  // kbi_persist, whose workgroups can meet by themselves
     uint32_t tag = 1;
     GhostPlan plan;
     // 1, 2 or 4 rows per thread (2^20 rows); RES, the rows whose matrix stays in
@@ -1004,7 +1012,8 @@ struct BiWork : fv_solver_cache {
     template <int W>
     void choose_kernel(fv_ctx* c, int rpt) {
         const int n = rpt <= 1 ? 1 : rpt <= 2 ? 2 : 4;
-        if (plan.make(c, h.N, h.ntiles, h.rowsPerBlock, W, n * kB, 8, bi_ghost_cap(n), h.sellCol))
+        plain = plan.make(c, h.N, h.ntiles, h.rowsPerBlock, W, n * kB, 8, bi_ghost_cap(n), h.sellCol);
+        if (plain)
             persist = n == 1 ? kbi_persist<1, W, 1> : n == 2 ? kbi_persist<2, W, 2> : kbi_persist<4, W, 0>;
         else
             persist = n == 1   ? kbi_persist_far<1, W, 1>
@@ -1025,8 +1034,8 @@ struct BiWork : fv_solver_cache {
         }
         // about 2 ms a launch, as the CG (an iteration takes 10 to 40 us)
         persistIters = (int)(2000.0 / (10.0 + 30.0 * h.N / (1 << 20)));
-        slots.alloc(c, 2 * (size_t)kSlotBuffer);
-        FV_HIP(hipMemsetAsync(slots.p, 0, slots.n * sizeof(unsigned long long), c->stream));
+        slots.alloc(c);
+        slots.clear(c->stream);
     }
     // One system of a solve: x in place, or component `comp` of `ncomp` interleaved ones
     // (rhs, x), whose x between launches is dinv (the persistent form has no other use
@@ -1040,7 +1049,7 @@ struct BiWork : fv_solver_cache {
     bool run_persist(hipStream_t s, const Target& t, const fv_solve_opts* o, bool fresh, bool chained = false) {
         const uint32_t uses = 3 * (uint32_t)persistIters + 8;
         if (tag > 0xffffffffu - uses) {  // sequence numbers start over
-            FV_HIP(hipMemsetAsync(slots.p, 0, slots.n * sizeof(unsigned long long), s));
+            slots.clear(s);
             tag = 1;
         }
         double* const x = t.x + t.comp;
@@ -1049,11 +1058,8 @@ struct BiWork : fv_solver_cache {
                     o->rel_tol, o->abs_tol, h.sellCol, CsrSystem{h.rowOffs, diag, h.vals, t.rhs + t.comp},
                     t.ncomp, x, t.ncomp > 1 ? x : nullptr, chained ? state - 1 : nullptr, sval.p,
                     t.ncomp > 1 ? dinv.p : x, h.r, h.rhat, h.p, h.v, h.t, h.s, plan.words.p,
-                    plan.ghosts.p, plan.count.p, plan.stride, state, slots.p};
-        void* args[] = {&a};
-        if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(persist), dim3(persistGrid),
-                                       dim3(kPersistThreads), args, 0, s) != hipSuccess) {
-            (void)hipGetLastError();
+                    plan.ghosts.p, plan.count.p, plan.stride, slots.next(persistGrid, plain), state, slots.words.p};
+        if (!PersistSlots::launch(reinterpret_cast<const void*>(persist), persistGrid, &a, a.meet == 0, s)) {
             persist = nullptr;
             return false;
         }
@@ -1109,8 +1115,15 @@ struct BiWork : fv_solver_cache {
     }
     // Goes on until component t.comp, last seen in state h, has stopped.
     BiState finish_persist(fv_ctx* c, const Target& t, const fv_solve_opts* o, BiState h) {
-        while (!h.stop) {
-            FV_REQUIRE(run_persist(c->stream, t, o, false), "a cooperative launch was refused");
+        bool fresh = true;
+        while (!h.stop || h.stop == kStopApart) {
+            if (h.stop == kStopApart) {  // nothing done: the same launch, cooperative
+                slots.apart = true;
+                if (!fresh) FV_HIP(hipMemsetAsync(&st.p[t.comp].stop, 0, sizeof(int32_t), c->stream));
+            } else {
+                fresh = false;
+            }
+            FV_REQUIRE(run_persist(c->stream, t, o, fresh), "a cooperative launch was refused");
             h = states(c, t.comp + 1)[t.comp];
         }
         if (h.stop == kStopSync) {
@@ -1170,7 +1183,7 @@ int fv_solve_bicgstab_vec(fv_linsys* ls, int ncomp, const void* d_rhs, void* d_x
             BiState h[kMaxComp];
             std::copy_n(w.states(ctx, n), n, h);
             for (bool gone_on = false; k < n && !gone_on; ++k) {
-                gone_on = h[k].stop == 0;  // those behind it returned at once
+                gone_on = h[k].stop == 0 || h[k].stop == kStopApart;  // those behind it returned at once
                 h[k] = w.finish_persist(ctx, target(k), o, h[k]);
                 stats[k].true_res = h[k].trueRes;
                 if (h[k].stop != 2) keep_rhs(k);

@@ -46,9 +46,13 @@
 // -> 5.5 us at 32^3 FP64, 9.5 -> 10.7 at 80^3; in FP32 they gained 0.3 us up to 64^3
 // and lost 0.9 at 96^3.)
 //
-// The launch is cooperative, so its workgroups are resident together.  Every
-// wait is bounded by a clock: a workgroup that waits longer than kSyncSeconds
-// sets stop = kStopSync and ends, and so do the others.
+// A cooperative launch keeps its workgroups resident together, but costs about 17 us
+// more than a plain one, as much as a small solve's whole start.  Launches that do a
+// whole solve are therefore plain ones whose workgroups meet first (Meeting): they
+// write nothing before all of them have arrived, and if one has not within
+// kMeetClocks (other work holds its place), all end and the solve is launched again,
+// cooperatively.  Every wait after that is bounded by a clock too: a workgroup that
+// waits longer than kSyncSeconds sets stop = kStopSync and ends, and so do the others.
 //
 // Measured per iteration (pressure equation on jittered cubes in Z order,
 // kernel-by-kernel form -> this one): FP64 32^3 10.8 -> 5.3 us, 64^3 21.6 -> 8.1, 96^3
@@ -71,6 +75,7 @@ constexpr int kPersistGroups = kCgMaxTiles / kPersistSub;  // workgroups at most
 constexpr int kSlotWords = 16;  // up to two doubles as half-payload words; a 128-byte line per slot
 constexpr int kSlotBuffer = (kPersistGroups + 8) * kSlotWords;  // workgroups and groups of them
 constexpr int kStopSync = 4;           // CgState::stop after a timed-out wait
+constexpr int kStopApart = 5;          // after a plain launch whose workgroups did not meet
 constexpr unsigned long long kSyncSeconds = 20;
 constexpr unsigned long long kClockHz = 100000000ull;  // wall_clock64: 100 MHz
 
@@ -104,6 +109,7 @@ struct CgPersist {
     double* x;
     double tol, atol;
     int32_t maxit, fresh;
+    unsigned long long meet;  // Meeting::target
 };
 
 template <typename T>
@@ -179,7 +185,7 @@ __device__ __forceinline__ double from_lane(double x, int lane) {
 struct PersistLds {
     double wave[2][kPersistThreads / 64];  // wave sums of this workgroup's tiles
     double tot[2][2];                      // by parity of the exchange: the grid's sums
-    int bad;
+    int bad, met;
 };
 
 // One workgroup's place in the grid exchange.  sum_slots adds the slots of a
@@ -419,6 +425,49 @@ __global__ __launch_bounds__(kCgBlock) void k_ghost_plan(int N, int R, int W, in
     if (tid == 0) count[tile] = base;
 }
 
+// The meeting of a plain launch's workgroups: words[0] counts arrivals over all
+// launches, `target` is its value after this one's last; words[16] holds the latest
+// decision, 2 * tag + 1 (all have arrived) or 2 * tag (one gave up).  The first to
+// decide wins, so every workgroup sees the same decision, late ones included.
+constexpr int kMeetWords = 32;
+constexpr unsigned long long kMeetClocks = kClockHz / 500;  // 2 ms
+struct Meeting {
+    unsigned long long* words;
+    unsigned long long target;  // 0: a cooperative launch
+    uint32_t tag;
+
+    __device__ unsigned long long decide(bool go) const {
+        const unsigned long long mine = 2ull * tag + (go ? 1 : 0);
+        unsigned long long seen = get_shared(words + 16);
+        while (seen >> 1 != tag && !__hip_atomic_compare_exchange_strong(
+                                       words + 16, &seen, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT)) {
+        }
+        return seen >> 1 != tag ? mine : seen;
+    }
+    __device__ void arrive() const {
+        if (target && threadIdx.x == 0 &&
+            __hip_atomic_fetch_add(words, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == target)
+            decide(true);
+    }
+    // Whether all have arrived, in every thread.
+    __device__ bool met(PersistLds& L) const {
+        if (!target) return true;
+        if (threadIdx.x == 0) {
+            const unsigned long long t0 = wall_clock64();
+            unsigned long long d;
+            while ((d = get_shared(words + 16)) >> 1 != tag)
+                if (wall_clock64() - t0 > kMeetClocks) {
+                    d = decide(false);
+                    break;
+                }
+            L.met = (int)(d & 1);
+        }
+        __syncthreads();
+        return L.met != 0;
+    }
+};
+
 // The ghosts of a tile, seen by one of its 256 threads: ghost s is thread s % 256's,
 // which holds the places in the vectors of its first K (byte offsets, SIZE bytes a
 // value).
@@ -474,8 +523,9 @@ struct GhostWalk {
 // on), takes the initial residual, and after the stop adds the correction to x and
 // takes the explicit residual, which goes to CgState::rrep: on small systems the
 // nine launches around the iterations cost as much as they do (32^3 heat step of 5
-// iterations 144 us with the start and end as kernels in a replayed graph, 103 whole;
-// 16^3 Poisson of 125 iterations 0.82 -> 0.73 ms).
+// iterations 144 us with the start and end as kernels in a replayed graph, 103 whole,
+// 97 with the ghosts in LDS, 78 with a plain launch; 16^3 Poisson of 125 iterations
+// 0.82 -> 0.73 -> 0.56 ms).
 template <typename S, int RPT, int W, int RES, int GL, bool DLDS, bool WHOLE>
 __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     constexpr int kOwn = RPT * kCgBlock, kTile = kOwn + ghost_cap<S>(RPT, W);
@@ -498,6 +548,8 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     const int tile = gs.place(A.tiles, sub);
     CgState* const st = A.st;
     const bool lead = gs.slot == 0 && tid == 0;
+    const Meeting meeting{A.slots + 2 * kSlotBuffer, WHOLE ? A.meet : 0, A.tag0};
+    meeting.arrive();
     if (!WHOLE || !A.fresh) {
         const int entry = st->stop;
         if (entry) {
@@ -629,6 +681,10 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
                      s2[0] += ri * ri;
                      s2[1] += bi * bi;
                  });
+        if (!meeting.met(L)) {
+            if (lead) st->stop = kStopApart;
+            return;
+        }
         if (A.fresh) {
             // ||b||, the relative residual; r = G^-1 r64, p = r, ||G r||^2 and r.r
             if ((ok = gs.sum<2, false>(s2, t2, L))) {
@@ -1082,6 +1138,28 @@ struct GhostPlan {
         ghosts.alloc(c, (size_t)tiles * (stride > 0 ? stride : 1));
         plan(words.p, ghosts.p);
         return true;
+    }
+};
+
+// The exchange buffer of a system and its launches.
+struct PersistSlots {
+    DBuf<unsigned long long> words;
+    unsigned long long meets = 0;  // arrivals of all plain launches
+    bool apart = false;            // a plain launch did not meet: cooperative from then on
+    void alloc(fv_ctx* c) { words.alloc(c, 2 * (size_t)kSlotBuffer + kMeetWords); }
+    void clear(hipStream_t s) {  // no word carries a tag that is still to come
+        FV_HIP(hipMemsetAsync(words.p, 0, words.n * sizeof(unsigned long long), s));
+        meets = 0;
+    }
+    // Meeting::target of the next launch over `grid` workgroups
+    unsigned long long next(int grid, bool plain) { return plain && !apart ? meets += grid : 0; }
+    static bool launch(const void* kernel, int grid, void* args, bool cooperative, hipStream_t s) {
+        void* a[] = {args};
+        const hipError_t e =
+            cooperative ? hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(kPersistThreads), a, 0, s)
+                        : hipLaunchKernel(kernel, dim3(grid), dim3(kPersistThreads), a, 0, s);
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e == hipSuccess;
     }
 };
 

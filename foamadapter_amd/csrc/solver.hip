@@ -51,7 +51,7 @@ struct CgWork : fv_solver_cache {
     int persistGrid = 0, persistIters = 0;
     int lastLaunches = 0;  // persistent launches of the previous mixed solve
     int lastTotal = 0;     // iterations of the previous solve, in either form
-    DBuf<unsigned long long> slots;
+    PersistSlots slots;
     GhostPlan plan;
     uint32_t tag = 1;
 
@@ -127,21 +127,21 @@ struct CgWork : fv_solver_cache {
         // from the smallest to the largest of these systems), so that the work of
         // other streams gets in between
         persistIters = (int)(2000.0 / (6.0 + 32.0 * h.N / (1 << 21)));
-        slots.alloc(c, 2 * (size_t)kSlotBuffer);
+        slots.alloc(c);
         clear_tags(c->stream);
     }
     // A cooperative launch costs about 17 us more than a plain one and is not
-    // replayed as a graph, and an iteration saves 4 us on the smallest systems: unless
+    // replayed as a graph, and an iteration saves 5 us on the smallest systems: unless
     // it is whole, a system whose previous solve took fewer than kPersistMin
     // iterations keeps the kernel-by-kernel form (32^3 heat step of 5 iterations: 157
-    // us, 178 with the iterations alone persistent, 103 whole).
+    // us, 178 with the iterations alone persistent, 78 whole).
     static constexpr int kPersistMin = 12;
     bool use_persist() const {
         return persist && (whole || lastTotal == 0 || lastTotal >= kPersistMin);
     }
     // no word of the exchange carries a tag that is still to come
     void clear_tags(hipStream_t s) {
-        FV_HIP(hipMemsetAsync(slots.p, 0, slots.n * sizeof(unsigned long long), s));
+        slots.clear(s);
         tag = 1;
     }
     // RES, the rows whose matrix stays in registers, and where g and d are, is what
@@ -175,13 +175,10 @@ struct CgWork : fv_solver_cache {
         if (tag > 0xffffffffu - uses) clear_tags(s);  // sequence numbers start over
         CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persistIters, tag, h.sellCol, h.sval,
                        h.g, h.d, h.r, h.p, h.p2, plan.words.p, plan.ghosts.p, plan.count.p,
-                       plan.stride, h.st, slots.p,
+                       plan.stride, h.st, slots.words.p,
                        CsrSystem{h.rowOffs, h.diag, h.vals, h.rhs}, x, tol, atol, maxit,
-                       fresh ? 1 : 0};
-        void* args[] = {&a};
-        if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(persist), dim3(persistGrid),
-                                       dim3(kPersistThreads), args, 0, s) != hipSuccess) {
-            (void)hipGetLastError();
+                       fresh ? 1 : 0, slots.next(persistGrid, whole)};
+        if (!PersistSlots::launch(reinterpret_cast<const void*>(persist), persistGrid, &a, a.meet == 0, s)) {
             persist = nullptr;
             return false;
         }
@@ -462,10 +459,15 @@ bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, doubl
                 FV_REQUIRE(fresh, "a cooperative launch was refused");
                 return false;
             }
-            fresh = false;
             FV_HIP(hipMemcpyAsync(host, w.st.p, sizeof *host, hipMemcpyDeviceToHost, s));
             FV_HIP(hipStreamSynchronize(s));
-        } while (!host->stop);
+            if (host->stop == kStopApart) {  // nothing done: the same launch, cooperative
+                w.slots.apart = true;
+                if (!fresh) FV_HIP(hipMemsetAsync(&w.st.p->stop, 0, sizeof(int32_t), s));
+            } else {
+                fresh = false;
+            }
+        } while (!host->stop || host->stop == kStopApart);
         *out = *host;
         w.check_persist(*out);
         w.lastIters = std::max(out->it, 1);

@@ -216,3 +216,41 @@ def test_vec_boundary_and_mean_magnitude(ctx, dims):
     want = np.sum(V * np.abs(d.numpy())) / np.sum(V)
     assert abs(mean.value - want) <= 4 * N * 2.3e-16 * want  # two pairs of sums of N terms
     m.close()
+
+
+def test_solves_of_several_threads(ctx):
+    """Small solves are plain launches whose workgroups meet; beside the solves of other threads,
+    one of which fills the device, they may not, and are launched again: the same bits."""
+    import threading
+    import foamadapter_amd as fa
+    from foamadapter_amd import la
+    cases = [((128, 128, 70), "PCG", 2, 40), ((41, 40, 40), "PCG", 12, 2000), ((33, 32, 32), "PCG", 12, 2000),
+             ((64, 32, 32), "PBiCGStab", 12, 400)]
+    out, errors = {}, []
+
+    def run(i):
+        try:
+            dims, method, reps, limit = cases[i]
+            with fa.Context(0) as c:
+                m, ls = _system(c, dims)
+                opts = {"solver": method, "relTol": 1e-8, "maxIter": limit}
+                got = []
+                for graph in [False] + [True] * reps:
+                    x = c.zeros((m.n_cells,))
+                    st = la.solve_cg(ls, x, dict(opts, graph=graph), raise_on_noconverge=False)
+                    got.append((x.numpy(), st.numIter, st.finalResNorm))
+                    x.close()
+                out[i] = got
+                m.close()
+        except Exception as e:  # noqa: BLE001
+            errors.append((i, e))
+
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(len(cases))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for i, got in out.items():
+        for g in got[1:]:
+            assert g[1:] == got[0][1:] and np.array_equal(g[0], got[0][0]), cases[i]

@@ -55,9 +55,9 @@
 // waits longer than kSyncSeconds sets stop = kStopSync and ends, and so do the others.
 //
 // Measured per iteration (pressure equation on jittered cubes in Z order,
-// kernel-by-kernel form -> this one): FP64 32^3 10.8 -> 5.3 us, 64^3 21.6 -> 8.1, 96^3
-// 39.6 -> 12.6, 128^3 65.6 -> 28.0; FP32 32^3 10.9 -> 5.8, 64^3 16.4 -> 7.8, 96^3 27.3
-// -> 10.4, 128^3 42.3 -> 15.6.  At 128^3 FP64 12 of the 28 us are the matrix stream
+// kernel-by-kernel form -> this one): FP64 32^3 10.8 -> 5.3 us, 64^3 21.6 -> 7.9, 96^3
+// 39.6 -> 12.0, 128^3 65.6 -> 28.0; FP32 32^3 10.9 -> 5.8, 64^3 16.4 -> 7.3, 96^3 27.3
+// -> 9.9, 128^3 42.3 -> 14.8.  At 128^3 FP64 12 of the 28 us are the matrix stream
 // (126 MB, from the memory-side cache), 16 the rest: two exchanges (2.4 us each on an
 // idle chip) with their waits for the slowest workgroup, the ghosts, the LDS reads.
 #pragma once
@@ -73,7 +73,8 @@ constexpr int kPersistThreads = 1024;  // four tiles of kCgBlock threads
 constexpr int kPersistSub = kPersistThreads / kCgBlock;
 constexpr int kPersistGroups = kCgMaxTiles / kPersistSub;  // workgroups at most
 constexpr int kSlotWords = 16;  // up to two doubles as half-payload words; a 128-byte line per slot
-constexpr int kSlotBuffer = (kPersistGroups + 8) * kSlotWords;  // workgroups and groups of them
+constexpr int kCopies = 8;       // of what many workgroups read
+constexpr int kSlotBuffer = (kPersistGroups + 8 * kCopies) * kSlotWords;  // workgroups; groups of them
 constexpr int kStopSync = 4;           // CgState::stop after a timed-out wait
 constexpr int kStopApart = 5;          // after a plain launch whose workgroups did not meet
 constexpr unsigned long long kSyncSeconds = 20;
@@ -199,7 +200,11 @@ struct PersistLds {
 //    The first of them collects its group's sums and publishes theirs, and every
 //    workgroup reads the eight group sums: the two hops take as long as polling
 //    all 256 slots does on an idle device (2.4 us), with a sixteenth of the
-//    polling, which otherwise slows the stores it waits for;
+//    polling, which otherwise slows the stores it waits for.  The readers of one
+//    line wait for each other, so the group sums are published in kCopies copies
+//    for 32 workgroups each (an iteration at 64^3 FP64: all eight in one line 9.9
+//    us, one copy 8.6, eight 7.9, 16 or 32 8.0; up to 64 workgroups, copies change
+//    nothing).  Polling twice as often costs more than it gains (8.2);
 //  * up to 256 tiles (64 workgroups): a workgroup holds tiles l, l + 16, l + 32,
 //    l + 48 of a wave, the branch of the first two steps, and every workgroup
 //    reads all slots.
@@ -286,12 +291,12 @@ struct GridSum {
                     for (int j = 0; j < NV; ++j) m[j] = 0.0;
                     if (lane < kPersistGroups / 8)
                         ok = collect<NV>(buf + (size_t)(group + 8 * lane) * kSlotWords, tag, m);
-                    for (int j = 0; j < NV; ++j) m[j] = lane_sum<16>(m[j]);
-                    if (lane == 0)
+                    for (int j = 0; j < NV; ++j) m[j] = from_lane(lane_sum<16>(m[j]), 0);
+                    if (lane < kCopies)
                         for (int j = 0; j < NV; ++j)
-                            publish(gbuf + (size_t)group * kSlotWords + 2 * j, m[j], tag);
+                            publish(gbuf + (size_t)(8 * lane + group) * kSlotWords + 2 * j, m[j], tag);
                 }
-                from = gbuf;
+                from = gbuf + (size_t)(8 * (slot & (kCopies - 1))) * kSlotWords;
                 count = 8;
             }
             double g[NV];

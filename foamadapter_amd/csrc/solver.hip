@@ -123,10 +123,10 @@ struct CgWork : fv_solver_cache {
             return;
         }
         whole = sizeof(S) == 8 && rpt <= 2;
-        // a launch holds the device for about 2 ms (an iteration takes 6 to 40 us,
-        // from the smallest to the largest of these systems), so that the work of
-        // other streams gets in between
-        persistIters = (int)(2000.0 / (6.0 + 32.0 * h.N / (1 << 21)));
+        // a launch holds the device for about 2 ms (an iteration takes 5 us on the
+        // smallest of these systems, on the largest 28 in FP64 and 15 in FP32), so that
+        // the work of other streams gets in between
+        persistIters = (int)(2000.0 / (5.0 + (sizeof(S) == 8 ? 23.0 : 10.0) * h.N / (1 << 21)));
         slots.alloc(c);
         clear_tags(c->stream);
     }

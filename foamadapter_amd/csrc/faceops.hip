@@ -939,15 +939,16 @@ __global__ __launch_bounds__(kBlock) void k_correct_bc(int B, int nc, const int3
 // FP64 gradient, linear and upwind divergence, laplacian, staged -> walk in us: 16^3
 // in block order 5.3, 5.0, 4.9, 5.4 -> 3.8, 4.1, 4.0, 4.1; 40^3 in Z order 5.6, 5.3,
 // 5.2, 5.4 -> 4.6, 5.1, 5.0, 5.4; 48^3 5.7, 5.2, 5.1, 5.5 -> 6.9, 5.4, 4.6, 6.7.  In
-// the wide form the line lies higher: 64^3 in block order 15.4, 10.0, 8.0, 12.4 ->
+// block order the line lies higher: 64^3 15.4, 10.0, 8.0, 12.4 ->
 // 12.3, 8.1, 6.4, 11.4; 80^3 24.0, 16.9, 14.8, 20.2 -> 25.6, 17.1, 13.4, 22.5.
 template <typename S>
 bool staged(const fv_mesh* m) {
     if (!gather_cells(m)) return false;
     if (m->gatherMode != 0) return true;
     if (m->nCells <= 1 << 16) return false;
-    return m->nCells > 1 << 18 ||
-           !gather_wide(gather_lists(const_cast<fv_mesh*>(m), 256, sizeof(S) == 4));
+    if (m->nCells > 1 << 18) return true;
+    const GatherLists& L = gather_lists(const_cast<fv_mesh*>(m), 256, sizeof(S) == 4);
+    return 2 * L.nOverflow <= L.nBlocks;  // else lines of cells: nearly all of them wide
 }
 
 template <typename S>

@@ -15,7 +15,7 @@ import numpy as np
 from ._lib import FV_F32, FV_F64, call, lib
 
 _DT = {np.dtype(np.float64): FV_F64, np.dtype(np.float32): FV_F32}
-_F64 = np.dtype(np.float64)
+_F64, _F32 = np.dtype(np.float64), np.dtype(np.float32)
 
 
 def prec_of(dtype) -> int:
@@ -23,6 +23,8 @@ def prec_of(dtype) -> int:
     # of an operator's Python
     if dtype is _F64:
         return FV_F64
+    if dtype is _F32:
+        return FV_F32
     return _DT[np.dtype(dtype)]
 
 

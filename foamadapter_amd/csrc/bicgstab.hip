@@ -328,13 +328,14 @@ struct BiPersist {
     int32_t ghostStride;
     unsigned long long meet;  // Meeting::target
     BiState* st;
+    BiState* host;  // a copy for the host (pinned; not kbi_persist_far)
     unsigned long long* slots;
 };
 
 // Places for ghosts in the LDS of a tile (see cgpersist.hpp): p and s of its rows and
 // ghosts, and the ghosts' v.  Enough for tiles of up to 512 rows in any order a mesher
 // writes (1230 at most), and for 1024 rows in Z order (about 950).
-constexpr int bi_ghost_cap(int rpt) { return rpt == 1 ? 1528 : rpt == 2 ? 1360 : 1016; }
+constexpr int bi_ghost_cap(int rpt) { return rpt == 1 ? 1528 : rpt == 2 ? 1352 : 1016; }
 
 template <int RPT, int W, int RES>
 __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
     meeting.arrive();
     if (!A.fresh && st->stop) return;
     if (A.prev && A.prev->stop != 2) {
-        if (gs.slot == 0 && tid == 0) st->stop = 0;
+        if (gs.slot == 0 && tid == 0) st->stop = A.host->stop = 0;
         return;
     }
     // x at the start of the launch, at stride xs
@@ -451,7 +452,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
                      if (A.fresh) rv[u] = hv[u] = ri;
                  });
         if (!meeting.met(L)) {
-            if (gs.slot == 0 && tid == 0) st->stop = kStopApart;
+            if (gs.slot == 0 && tid == 0) st->stop = A.host->stop = kStopApart;
             return;
         }
         if (A.fresh) {
@@ -637,7 +638,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
         }
     }
     if (!ok) {
-        if (tid == 0) st->stop = kStopSync;
+        if (tid == 0) st->stop = A.host->stop = kStopSync;
         return;
     }
     if (gs.slot == 0 && tid == 0) {
@@ -654,6 +655,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
         o.it = it;
         o.stop = stop;
         *st = o;
+        *A.host = o;
     }
 }
 
@@ -1004,6 +1006,7 @@ struct BiWork : fv_solver_cache {
     void (*persist)(BiPersist) = nullptr;
     int persistGrid = 0, persistIters = 0;
     PersistSlots slots;
+    BiState* host = nullptr;  // the context's pinned poll area
     bool plain = false;  // kbi_persist, whose workgroups can meet by themselves
     uint32_t tag = 1;
     GhostPlan plan;
@@ -1034,6 +1037,8 @@ struct BiWork : fv_solver_cache {
         }
         // about 2 ms a launch, as the CG (an iteration takes 10 to 40 us)
         persistIters = (int)(2000.0 / (10.0 + 30.0 * h.N / (1 << 20)));
+        static_assert(kMaxComp * sizeof(BiState) <= fv_ctx::kPollBytes, "poll area too small");
+        host = static_cast<BiState*>(ctx_poll_host(c));
         slots.alloc(c);
         slots.clear(c->stream);
     }
@@ -1058,7 +1063,9 @@ struct BiWork : fv_solver_cache {
                     o->rel_tol, o->abs_tol, h.sellCol, CsrSystem{h.rowOffs, diag, h.vals, t.rhs + t.comp},
                     t.ncomp, x, t.ncomp > 1 ? x : nullptr, chained ? state - 1 : nullptr, sval.p,
                     t.ncomp > 1 ? dinv.p : x, h.r, h.rhat, h.p, h.v, h.t, h.s, plan.words.p,
-                    plan.ghosts.p, plan.count.p, plan.stride, slots.next(persistGrid, plain), state, slots.words.p};
+                    plan.ghosts.p, plan.count.p, plan.stride, slots.next(persistGrid, plain), state,
+                    host + t.comp, slots.words.p};
+        host[t.comp].stop = -1;
         if (!PersistSlots::launch(reinterpret_cast<const void*>(persist), persistGrid, &a, a.meet == 0, s)) {
             persist = nullptr;
             return false;
@@ -1105,16 +1112,16 @@ struct BiWork : fv_solver_cache {
         diag = sp->diagOffset.p;
         if (!c->shared) choose_persist(c, sp);
     }
-    // The states after the work queued so far (pinned, valid until the next read)
+    // The states after the work queued so far (pinned, valid until the next launch)
     const BiState* states(fv_ctx* c, int n) {
-        static_assert(kMaxComp * sizeof(BiState) <= fv_ctx::kPollBytes, "poll area too small");
-        auto* const host = static_cast<BiState*>(ctx_poll_host(c));
-        FV_HIP(hipMemcpyAsync(host, st.p, n * sizeof(BiState), hipMemcpyDeviceToHost, c->stream));
+        if (!plain)
+            FV_HIP(hipMemcpyAsync(host, st.p, n * sizeof(BiState), hipMemcpyDeviceToHost, c->stream));
         FV_HIP(hipStreamSynchronize(c->stream));
         return host;
     }
     // Goes on until component t.comp, last seen in state h, has stopped.
     BiState finish_persist(fv_ctx* c, const Target& t, const fv_solve_opts* o, BiState h) {
+        FV_REQUIRE(h.stop != -1, "a persistent solve left no state");
         bool fresh = true;
         while (!h.stop || h.stop == kStopApart) {
             if (h.stop == kStopApart) {  // nothing done: the same launch, cooperative

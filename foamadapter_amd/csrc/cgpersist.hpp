@@ -72,7 +72,7 @@ namespace {
 constexpr int kPersistThreads = 1024;  // four tiles of kCgBlock threads
 constexpr int kPersistSub = kPersistThreads / kCgBlock;
 constexpr int kPersistGroups = kCgMaxTiles / kPersistSub;  // workgroups at most
-constexpr int kSlotWords = 16;  // up to two doubles as half-payload words; a 128-byte line per slot
+constexpr int kSlotWords = 16;  // up to four doubles as half-payload words; a 128-byte line per slot
 constexpr int kCopies = 8;       // of what many workgroups read
 constexpr int kSlotBuffer = (kPersistGroups + 8 * kCopies) * kSlotWords;  // workgroups; groups of them
 constexpr int kStopSync = 4;           // CgState::stop after a timed-out wait
@@ -111,6 +111,7 @@ struct CgPersist {
     double tol, atol;
     int32_t maxit, fresh;
     unsigned long long meet;  // Meeting::target
+    CgState* host;            // what the host reads of the state (pinned)
 };
 
 template <typename T>
@@ -184,8 +185,8 @@ __device__ __forceinline__ double from_lane(double x, int lane) {
 }
 
 struct PersistLds {
-    double wave[2][kPersistThreads / 64];  // wave sums of this workgroup's tiles
-    double tot[2][2];                      // by parity of the exchange: the grid's sums
+    double wave[4][kPersistThreads / 64];  // wave sums of this workgroup's tiles
+    double tot[2][4];                      // by parity of the exchange: the grid's sums
     int bad, met;
 };
 
@@ -666,7 +667,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
                 lds(lg, u) = in ? root(A.m.vals[A.m.rowOffs[i] + A.m.diag[i]]) : 0.0;
                 lds(ld, u) = !A.fresh && in ? *mine(A.d, u) : 0.0;
             }
-        double s2[2] = {0.0, 0.0}, t2[2];
+        double s2[2] = {0.0, 0.0};
         residual([&](uint32_t o) { return *at_byte(A.x, o); },
                  [&](int u, bool in, double ri, double bi, const double (&a)[W],
                      const uint32_t (&c)[W]) {
@@ -687,31 +688,30 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
                      s2[1] += bi * bi;
                  });
         if (!meeting.met(L)) {
-            if (lead) st->stop = kStopApart;
+            if (lead) st->stop = A.host->stop = kStopApart;
             return;
         }
         if (A.fresh) {
             // ||b||, the relative residual; r = G^-1 r64, p = r, ||G r||^2 and r.r
-            if ((ok = gs.sum<2, false>(s2, t2, L))) {
-                bnorm = sqrt(t2[1]);
-                if (!(bnorm > 0.0)) bnorm = 1.0;
-                res = res0 = sqrt(t2[0]) / bnorm;
-                double s3[2] = {0.0, 0.0};
+            double s4[4] = {s2[0], s2[1], 0.0, 0.0}, t4[4];
 #pragma unroll
-                for (int u = 0; u < RPT; ++u)
-                    if (live(u)) {
-                        const bool in = iw + u * kCgBlock + lane < A.N;
-                        const double gi = lds(lg, u);
-                        const double ri = in ? rv[u] / gi : 0.0;
-                        rv[u] = ri;
-                        lds(tp, u) = ri;
-                        if (shown >> u & 1) put_shared(mine(A.p, u), ri);
-                        const double ur = ri * gi;
-                        s3[0] += ur * ur;
-                        s3[1] += ri * ri;
-                    }
-                ok = gs.sum<2, true>(s3, t2, L);
-                rho = t2[1];
+            for (int u = 0; u < RPT; ++u)
+                if (live(u)) {
+                    const bool in = iw + u * kCgBlock + lane < A.N;
+                    const double gi = lds(lg, u);
+                    const double ri = in ? rv[u] / gi : 0.0;
+                    rv[u] = ri;
+                    lds(tp, u) = ri;
+                    if (shown >> u & 1) put_shared(mine(A.p, u), ri);
+                    const double ur = ri * gi;
+                    s4[2] += ur * ur;
+                    s4[3] += ri * ri;
+                }
+            if ((ok = gs.sum<4, true>(s4, t4, L))) {
+                bnorm = sqrt(t4[1]);
+                if (!(bnorm > 0.0)) bnorm = 1.0;
+                res = res0 = sqrt(t4[0]) / bnorm;
+                rho = t4[3];
                 rhoPrev = alpha = 0.0;
                 it = 0;
                 // the decision of kc_direction after a start
@@ -851,7 +851,10 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
         }
     }
     if (!ok) {
-        if (tid == 0) st->stop = kStopSync;
+        if (tid == 0) {
+            st->stop = kStopSync;
+            if (WHOLE) A.host->stop = kStopSync;
+        }
         return;
     }
     if (!WHOLE || !stop) {
@@ -876,6 +879,13 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
             st->bnorm = bnorm;
             st->res0 = res0;
             st->rrep = rrep;
+            // straight to the host: a copy behind the launch takes 5 us
+            A.host->res = res;
+            A.host->res0 = res0;
+            A.host->rrep = rrep;
+            A.host->bnorm = bnorm;
+            A.host->it = it;
+            A.host->stop = stop;
         }
     }
 }

@@ -170,14 +170,14 @@ struct CgWork : fv_solver_cache {
     // Up to persistIters iterations in one launch; false if the device refuses it.
     // (whole: x, the limits and whether the solve starts.)
     bool run_persist(hipStream_t s, double* x = nullptr, double tol = 0.0, double atol = 0.0,
-                     int maxit = 0, bool fresh = false) {
+                     int maxit = 0, bool fresh = false, CgState* host = nullptr) {
         const uint32_t uses = 2 * (uint32_t)persistIters + 8;
         if (tag > 0xffffffffu - uses) clear_tags(s);  // sequence numbers start over
         CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persistIters, tag, h.sellCol, h.sval,
                        h.g, h.d, h.r, h.p, h.p2, plan.words.p, plan.ghosts.p, plan.count.p,
                        plan.stride, h.st, slots.words.p,
                        CsrSystem{h.rowOffs, h.diag, h.vals, h.rhs}, x, tol, atol, maxit,
-                       fresh ? 1 : 0, slots.next(persistGrid, whole)};
+                       fresh ? 1 : 0, slots.next(persistGrid, whole), host};
         if (!PersistSlots::launch(reinterpret_cast<const void*>(persist), persistGrid, &a, a.meet == 0, s)) {
             persist = nullptr;
             return false;
@@ -452,15 +452,16 @@ bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, doubl
                     double* x, double* true_res, CgState* out) {
     hipStream_t s = ctx->stream;
     if (w.whole) {
-        CgState* const host = static_cast<CgState*>(ctx_poll_host(ctx));
+        CgState* const host = static_cast<CgState*>(ctx_poll_host(ctx));  // the kernel writes it
         bool fresh = true;
         do {
-            if (!w.run_persist(s, x, tol, atol, maxit, fresh)) {
+            host->stop = -1;
+            if (!w.run_persist(s, x, tol, atol, maxit, fresh, host)) {
                 FV_REQUIRE(fresh, "a cooperative launch was refused");
                 return false;
             }
-            FV_HIP(hipMemcpyAsync(host, w.st.p, sizeof *host, hipMemcpyDeviceToHost, s));
             FV_HIP(hipStreamSynchronize(s));
+            FV_REQUIRE(host->stop != -1, "a persistent solve left no state");
             if (host->stop == kStopApart) {  // nothing done: the same launch, cooperative
                 w.slots.apart = true;
                 if (!fresh) FV_HIP(hipMemsetAsync(&w.st.p->stop, 0, sizeof(int32_t), s));

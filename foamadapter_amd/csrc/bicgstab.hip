@@ -296,7 +296,7 @@ __global__ void kbi_scale(int64_t n, const int32_t* __restrict__ src, const int3
 // tile publishes v and r of the rows that others refer to, and follows p' = r + beta (p
 // - omega v) and s = r - alpha v for its ghosts, so an iteration has three grid
 // exchanges.  The order of all sums is that of the kernels above (same
-// bits).  Advection step on 110x100x90 cells (about 28 iterations) 2.97 -> 1.13 ms (1.62
+// bits).  Advection step on 110x100x90 cells (about 28 iterations) 3.28 -> 1.19 ms (1.77
 // with the far columns read in the product, as kbi_persist_far does), an icoFoam step
 // at 64^3 (three momentum solves) 5.01 -> 4.25 ms.
 //

@@ -530,7 +530,8 @@ struct GhostWalk {
 // takes the explicit residual, which goes to CgState::rrep: on small systems the
 // nine launches around the iterations cost as much as they do (32^3 heat step of 5
 // iterations 144 us with the start and end as kernels in a replayed graph, 103 whole,
-// 97 with the ghosts in LDS, 78 with a plain launch; 16^3 Poisson of 125 iterations
+// 97 with the ghosts in LDS, 78 with a plain launch, 75 with the state written to
+// the host and the start in one exchange; 16^3 Poisson of 125 iterations
 // 0.82 -> 0.73 -> 0.56 ms).
 template <typename S, int RPT, int W, int RES, int GL, bool DLDS, bool WHOLE>
 __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {

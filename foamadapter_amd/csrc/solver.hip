@@ -134,7 +134,7 @@ struct CgWork : fv_solver_cache {
     // replayed as a graph, and an iteration saves 5 us on the smallest systems: unless
     // it is whole, a system whose previous solve took fewer than kPersistMin
     // iterations keeps the kernel-by-kernel form (32^3 heat step of 5 iterations: 157
-    // us, 178 with the iterations alone persistent, 78 whole).
+    // us, 178 with the iterations alone persistent, 75 whole).
     static constexpr int kPersistMin = 12;
     bool use_persist() const {
         return persist && (whole || lastTotal == 0 || lastTotal >= kPersistMin);

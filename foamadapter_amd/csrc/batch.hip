@@ -249,9 +249,11 @@ bool start_members(fv_batch* b) {
     // tile list of the members that (re)start, with their global slots, and
     // their start parameters; one batched start launch covers all of them
     int slot = 0;
+    int rows = 0;  // of the tallest tile: a large member's are taller than b->tileRows
     for (int i = 0; i < (int)b->members.size(); ++i) {
         BMember* m = b->members[i];
         if (m->needStart) {
+            rows = std::max(rows, member_rows(b, m));
             member_tile_list<S>(b, i, slot, st);
             prm[i] = CgStartParam{m->tol > 0.0 ? m->tol : b->tol, b->delta, b->atol,
                                   m->maxit > 0 ? m->maxit : b->maxit, 0};
@@ -277,7 +279,7 @@ bool start_members(fv_batch* b) {
     const int G = cg_grid((int)st.size());
     FV_HIP(hipEventRecord(b->ev[2], s));
     kc_begin<S><<<G, kB, 0, s>>>(g, red, (const CgStartParam*)(dev + oPrm), CgStartParam{});
-    kc_scale<S><<<cg_scale_grid(G, b->tileRows), kB, 0, s>>>(g, red);
+    kc_scale<S><<<cg_scale_grid(G, rows), kB, 0, s>>>(g, red);
     FV_LAUNCH_CHECK();
     FV_HIP(hipEventRecord(b->ev[3], s));
     return true;

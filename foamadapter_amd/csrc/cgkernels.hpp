@@ -657,7 +657,8 @@ __global__ __launch_bounds__(kCgBlock) void kc_begin(const CgGrid<S>* __restrict
 // kc_scale: the scaled sliced-ELL values a_ij / (g_i |g_j|) in S; the first tile
 // sums the partials of kc_begin and decides on the FP64 residual (2 converged, 3
 // non-finite, 1 iteration limit).  No sum runs over a tile's rows here, so long tiles
-// are split over blockIdx.y, kScaleRows each (tiles of 4096 rows unsplit: 118 us).
+// are split over blockIdx.y, kScaleRows each (tiles of 4096 rows unsplit: 118 us); a tile
+// taller than the grid was made for is taken in several rounds.
 constexpr int kScaleRows = 1024;
 inline dim3 cg_scale_grid(int blocks, int tileRows) {
     return dim3(blocks, (tileRows + kScaleRows - 1) / kScaleRows);
@@ -696,9 +697,9 @@ __global__ __launch_bounds__(kCgBlock) void kc_scale(const CgGrid<S>* __restrict
     const int32_t* __restrict__ scol = P.sellCol;
     S* __restrict__ sval = const_cast<S*>(P.sval);
     const int N = P.N;
-    row0 += (int)blockIdx.y * kScaleRows;
-    row1 = min(row1, row0 + kScaleRows);
-    for (int i0 = row0; i0 < row1; i0 += kCgBlock) {
+    static_assert(kScaleRows % kCgBlock == 0, "whole blocks of rows");
+    for (int part = row0 + (int)blockIdx.y * kScaleRows; part < row1; part += (int)gridDim.y * kScaleRows)
+    for (int i0 = part; i0 < min(part + kScaleRows, row1); i0 += kCgBlock) {
         const int i = i0 + (int)threadIdx.x, ic = min(i, N - 1);
         const int base = ro[i0], n = ro[min(min(i0 + kCgBlock, row1), N)] - base;
         const int o = ro[ic] - base, len = i < N ? ro[ic + 1] - base - o : 0, d = dg[ic];

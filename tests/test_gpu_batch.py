@@ -260,3 +260,24 @@ def test_batch_absolute_tolerance(ctx, systems, precision):
         r = np.linalg.norm(ls.rhs() - ls.scipy() @ x.numpy())
         assert st.status == 0 and st.finalResNorm * nb <= atol * 1.0001, (i, st)
         assert r <= atol * 1.01, (i, r, atol)
+
+
+@pytest.mark.parametrize("precision", ["double", "mixed"])
+def test_tiles_taller_than_the_batch_asked_for(ctx, precision):
+    """A system of over 1024 tiles of the batch's height gets taller tiles (102^3 rows in
+    tiles of 1024: 1088).  The same tiles asked for: the same bits, so every row of them is
+    scaled, whatever the memory of the scaled matrix held before."""
+    s = _heat_system(ctx, 102, 3e-2, 7)
+    out = []
+    for tile_rows in (1024, 256, 1088):
+        # a block of the pool, of the size of the scaled matrix (six entries a row), full of NaN
+        rows = (s["mesh"].n_cells + 63) // 64 * 64
+        ctx.upload(np.full(6 * rows, np.nan, np.float64 if precision == "double" else np.float32)).close()
+        (x,), (st,) = _run(ctx, [s], [0], precision, False, tile_rows=tile_rows, chunk=16)
+        out.append((x, st.numIter, st.finalResNorm))
+    assert out[-1][2] <= 1e-8
+    for o in out[:-1]:
+        assert o[1:] == out[-1][1:] and np.array_equal(o[0], out[-1][0])
+    s["ls"].close()
+    s["bc"].close()
+    s["mesh"].close()

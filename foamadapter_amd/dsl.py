@@ -152,7 +152,11 @@ def _assemble_fused(expr: Expression, psi: fvcc.VolumeField, dt: float, ls: Line
             continue
         a, f = tm.args
         if k == 3:
-            t.field = (a.internal if isinstance(a, fvcc.VolumeField) else a).ptr.value
+            arr = a.internal if isinstance(a, fvcc.VolumeField) else a
+            # one value a cell for every component (psi itself: each has its own)
+            if arr.shape != (psi.mesh.n_cells,) or arr.dtype != np.float64:
+                return False
+            t.field = arr.ptr.value
             continue
         t.field = a.values.ptr.value
         if k < 3:

@@ -118,3 +118,25 @@ def test_other_orders_are_assembled_term_by_term(ctx):
         dsl.assemble(eq, psi, 0.0, 0.1, ls)
         assert np.all(np.isfinite(ls.values())) and np.any(ls.values() != 0.0)
     m.close()
+
+
+@pytest.mark.parametrize("coefficient", ["psi", "other"])
+def test_source_with_a_vector_coefficient(ctx, coefficient, monkeypatch):
+    """A Vec3 equation whose source coefficient is the field itself (each component's equation
+    has that component) or an array of another shape than one value a cell: not one for the
+    one-pass kernel, which reads one value a cell for all components."""
+    from foamadapter_amd import dsl, la
+    m = _mesh(ctx, "bricks")
+    psi, phi, gamma, other, sp = _fields(ctx, m, 3, ["fixedValue"] * m.n_patches)
+    wide = ctx.uniform(3 * m.n_cells, 0.0, 1.0, 21, 8)
+    eq = dsl.imp.ddt(psi) - dsl.imp.laplacian(gamma, psi) + dsl.imp.source(psi if coefficient == "psi" else wide, psi)
+    fused = dsl._assemble_fused
+    got = []
+    for one_pass in (True, False):
+        monkeypatch.setattr(dsl, "_assemble_fused", fused if one_pass else (lambda *a: False))
+        ls = la.LinearSystem(la.SparsityPattern.readOrCreate(m))
+        dsl.assemble(eq, psi, 0.0, 0.125, ls)
+        got.append([ls.values(), ls.rhs(), ls.rhs3.numpy()])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    m.close()

@@ -167,6 +167,8 @@ _SIGS = {
     "fv_solve_cg": [_vp, _vp, C.POINTER(FvSolveOpts), C.POINTER(FvSolverStats)],
     "fv_solve_bicgstab_vec": [_vp, C.c_int, _vp, _vp, C.POINTER(FvSolveOpts), C.POINTER(FvSolverStats),
                               C.POINTER(C.c_int)],
+    "fv_linsys_persist_counts": [_vp, C.c_int, _vp],
+    "fv_linsys_persist_fault": [_vp, C.c_int, C.c_int, C.c_int, C.c_int],
     "fv_solve_bicgstab": [_vp, _vp, C.POINTER(FvSolveOpts), C.POINTER(FvSolverStats)],
     "fv_batch_create": [_vp, C.c_int, C.c_int, C.c_int, _pp],
     "fv_batch_destroy": [_vp],

@@ -34,9 +34,25 @@ constexpr int kB = kCgBlock;
 
 struct BiState {
     double rho[2], alpha, omega, bnorm, res, res0, tol, atol;
-    int32_t it, stop, maxit, pad;
+    int32_t it, stop, maxit;
+    int32_t lost;        // as CgState::lost
     double rr, trueRes;  // persistent form: ||r||^2 and the result's explicit residual
 };
+
+// What a persistent launch leaves; `lost` is its lost workgroups'.
+__device__ inline void bi_leave(BiState* st, const BiState& o) {
+    st->rho[0] = o.rho[0];
+    st->rho[1] = o.rho[1];
+    st->alpha = o.alpha;
+    st->omega = o.omega;
+    st->bnorm = o.bnorm;
+    st->res = o.res;
+    st->res0 = o.res0;
+    st->rr = o.rr;
+    st->trueRes = o.trueRes;
+    st->it = o.it;
+    st->stop = o.stop;
+}
 
 struct BiSys {
     int32_t N, ntiles, rowsPerBlock, pad;
@@ -326,10 +342,10 @@ struct BiPersist {
     const uint32_t* words;  // the columns, see k_ghost_plan; ghosts of each tile
     const int32_t *ghosts, *count;
     int32_t ghostStride;
-    unsigned long long meet;  // Meeting::target
     BiState* st;
     BiState* host;  // a copy for the host (pinned; not kbi_persist_far)
     unsigned long long* slots;
+    PersistLaunch launch;
 };
 
 // Places for ghosts in the LDS of a tile (see cgpersist.hpp): p and s of its rows and
@@ -354,17 +370,17 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
     const int R = A.rowsPerTile;
     const int tile = gs.place(A.tiles, sub);
     BiState* const st = A.st;
-    const Meeting meeting{A.slots + 2 * kSlotBuffer, A.meet, A.tag0};
+    const Meeting meeting{A.slots + 2 * kSlotBuffer, A.launch.meet, A.tag0};
     meeting.arrive();
-    if (!A.fresh && st->stop) return;
-    if (A.prev && A.prev->stop != 2) {
+    if (!A.fresh && (st->stop || st->lost)) return;
+    if (A.prev && (A.prev->stop != 2 || A.prev->lost)) {
         if (gs.slot == 0 && tid == 0) st->stop = A.host->stop = 0;
         return;
     }
     // x at the start of the launch, at stride xs
     const double* const xin = A.fresh ? A.x0 : A.x;
     const int xs = A.fresh ? A.stride : 1;
-    if (tid == 0) L.bad = 0;
+    if (tid == 0) L.begin(A.launch);
     const int row0 = tile * R;
     const int row1 = tile < A.tiles ? min(row0 + R, (A.N + 63) & ~63) : row0;
     const int iw = row0 + __builtin_amdgcn_readfirstlane(tid & (kB - 64));
@@ -638,7 +654,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
         }
     }
     if (!ok) {
-        if (tid == 0) st->stop = A.host->stop = kStopSync;
+        if (tid == 0) st->lost = A.host->lost = 1;
         return;
     }
     if (gs.slot == 0 && tid == 0) {
@@ -654,8 +670,8 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
         o.trueRes = trueRes;
         o.it = it;
         o.stop = stop;
-        *st = o;
-        *A.host = o;
+        bi_leave(st, o);
+        bi_leave(A.host, o);
     }
 }
 
@@ -681,15 +697,15 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist_far(BiPersist A) 
     const int tile = gs.place(A.tiles, sub);
     const uint32_t cbase = (uint32_t)tile * R, lofs = (uint32_t)sub * (RPT * kB);
     BiState* const st = A.st;
-    if (!A.fresh && st->stop) return;
-    if (A.prev && A.prev->stop != 2) {
+    if (!A.fresh && (st->stop || st->lost)) return;
+    if (A.prev && (A.prev->stop != 2 || A.prev->lost)) {
         if (gs.slot == 0 && tid == 0) st->stop = 0;
         return;
     }
     // x at the start of the launch, at stride xs
     const double* const xin = A.fresh ? A.x0 : A.x;
     const int xs = A.fresh ? A.stride : 1;
-    if (tid == 0) L.bad = 0;
+    if (tid == 0) L.begin(A.launch);
     const int row0 = tile * R;
     const int row1 = tile < A.tiles ? min(row0 + R, (A.N + 63) & ~63) : row0;
     const int iw = row0 + __builtin_amdgcn_readfirstlane(tid & (kB - 64));
@@ -973,7 +989,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist_far(BiPersist A) 
         }
     }
     if (!ok) {
-        if (tid == 0) st->stop = kStopSync;
+        if (tid == 0) st->lost = 1;
         return;
     }
     if (gs.slot == 0 && tid == 0) {
@@ -989,7 +1005,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist_far(BiPersist A) 
         o.trueRes = trueRes;
         o.it = it;
         o.stop = stop;
-        *st = o;
+        bi_leave(st, o);
     }
 }
 
@@ -1023,13 +1039,22 @@ struct BiWork : fv_solver_cache {
                       : n == 2 ? kbi_persist_far<2, W, 1>
                                : kbi_persist_far<4, W, 0>;
     }
-    void choose_persist(fv_ctx* c, const fv_sparsity* sp) {
+    // Where its buffers find no room, the system runs kernel by kernel.
+    void choose_persist(fv_ctx* c, const fv_sparsity* sp, fv_persist_log* log) {
         const int rpt = (h.rowsPerBlock + kB - 1) / kB;
         if (rpt > 4) return;
-        if (sp->sellWidth == 6)
-            choose_kernel<6>(c, rpt);
-        else if (sp->sellWidth == 4)
-            choose_kernel<4>(c, rpt);
+        const bool room = persist_room([&] {
+            slots.alloc(c, log);
+            if (sp->sellWidth == 6)
+                choose_kernel<6>(c, rpt);
+            else if (sp->sellWidth == 4)
+                choose_kernel<4>(c, rpt);
+        });
+        if (!room) {
+            persist = nullptr;
+            slots.words.release();
+            plan = GhostPlan{};
+        }
         persistGrid = persist_grid(h.ntiles);
         if (!persist || !persist_fits(reinterpret_cast<const void*>(persist), c->device, persistGrid)) {
             persist = nullptr;
@@ -1039,7 +1064,6 @@ struct BiWork : fv_solver_cache {
         persistIters = (int)(2000.0 / (10.0 + 30.0 * h.N / (1 << 20)));
         static_assert(kMaxComp * sizeof(BiState) <= fv_ctx::kPollBytes, "poll area too small");
         host = static_cast<BiState*>(ctx_poll_host(c));
-        slots.alloc(c);
         slots.clear(c->stream);
     }
     // One system of a solve: x in place, or component `comp` of `ncomp` interleaved ones
@@ -1063,10 +1087,10 @@ struct BiWork : fv_solver_cache {
                     o->rel_tol, o->abs_tol, h.sellCol, CsrSystem{h.rowOffs, diag, h.vals, t.rhs + t.comp},
                     t.ncomp, x, t.ncomp > 1 ? x : nullptr, chained ? state - 1 : nullptr, sval.p,
                     t.ncomp > 1 ? dinv.p : x, h.r, h.rhat, h.p, h.v, h.t, h.s, plan.words.p,
-                    plan.ghosts.p, plan.count.p, plan.stride, slots.next(persistGrid, plain), state,
-                    host + t.comp, slots.words.p};
+                    plan.ghosts.p, plan.count.p, plan.stride, state, host + t.comp, slots.words.p, {}};
         host[t.comp].stop = -1;
-        if (!PersistSlots::launch(reinterpret_cast<const void*>(persist), persistGrid, &a, a.meet == 0, s)) {
+        host[t.comp].lost = 0;
+        if (!slots.launch(persist, persistGrid, a, plain, s)) {
             persist = nullptr;
             return false;
         }
@@ -1074,7 +1098,7 @@ struct BiWork : fv_solver_cache {
         return true;
     }
     const int32_t* diag = nullptr;
-    BiWork(fv_ctx* c, const fv_linsys* ls) {
+    BiWork(fv_ctx* c, fv_linsys* ls) {
         const fv_sparsity* sp = ls->sp;
         const int N = sp->nRows;
         const int R = cg_tile_rows(N, kB);
@@ -1110,7 +1134,8 @@ struct BiWork : fv_solver_cache {
         h.pb = parts.p + 5 * (int64_t)tiles;
         h.st = st.p;
         diag = sp->diagOffset.p;
-        if (!c->shared) choose_persist(c, sp);
+        FV_HIP(hipMemsetAsync(st.p, 0, kMaxComp * sizeof(BiState), c->stream));
+        if (!c->shared) choose_persist(c, sp, &ls->persistLog[2]);
     }
     // The states after the work queued so far (pinned, valid until the next launch)
     const BiState* states(fv_ctx* c, int n) {
@@ -1119,26 +1144,33 @@ struct BiWork : fv_solver_cache {
         FV_HIP(hipStreamSynchronize(c->stream));
         return host;
     }
-    // Goes on until component t.comp, last seen in state h, has stopped.
-    BiState finish_persist(fv_ctx* c, const Target& t, const fv_solve_opts* o, BiState h) {
-        FV_REQUIRE(h.stop != -1, "a persistent solve left no state");
+    // Goes on until component t.comp, last seen in state h, has stopped.  False if the
+    // device refuses a launch or one is lost: h.it iterations are in x then (ncomp 1).
+    bool finish_persist(fv_ctx* c, const Target& t, const fv_solve_opts* o, BiState& h) {
         bool fresh = true;
-        while (!h.stop || h.stop == kStopApart) {
+        while (!h.lost && (!h.stop || h.stop == kStopApart)) {
             if (h.stop == kStopApart) {  // nothing done: the same launch, cooperative
-                slots.apart = true;
+                slots.did_not_meet();
                 if (!fresh) FV_HIP(hipMemsetAsync(&st.p[t.comp].stop, 0, sizeof(int32_t), c->stream));
             } else {
                 fresh = false;
             }
-            FV_REQUIRE(run_persist(c->stream, t, o, fresh), "a cooperative launch was refused");
+            if (!run_persist(c->stream, t, o, fresh)) break;
             h = states(c, t.comp + 1)[t.comp];
         }
-        if (h.stop == kStopSync) {
+        if (h.lost) {
+            ++slots.log->lost;
             persist = nullptr;
-            throw Error{FV_EDEVICE, "persistent BiCGStab: the workgroups did not meet in " +
-                                        std::to_string(kSyncSeconds) + " s"};
         }
-        return h;
+        if (!persist) {
+            if (fresh) {  // no launch before this one left anything
+                h.it = 0;
+                h.res0 = -1.0;
+            }
+            return false;
+        }
+        FV_REQUIRE(h.stop != -1, "a persistent solve left no state");
+        return true;
     }
 };
 
@@ -1191,7 +1223,10 @@ int fv_solve_bicgstab_vec(fv_linsys* ls, int ncomp, const void* d_rhs, void* d_x
             std::copy_n(w.states(ctx, n), n, h);
             for (bool gone_on = false; k < n && !gone_on; ++k) {
                 gone_on = h[k].stop == 0 || h[k].stop == kStopApart;  // those behind it returned at once
-                h[k] = w.finish_persist(ctx, target(k), o, h[k]);
+                if (!w.finish_persist(ctx, target(k), o, h[k])) {  // this one kernel by kernel
+                    if (k) keep_rhs(k - 1);
+                    return;
+                }
                 stats[k].true_res = h[k].trueRes;
                 if (h[k].stop != 2) keep_rhs(k);
                 bi_finish(h[k], stats[k]);
@@ -1209,12 +1244,18 @@ int fv_solve_bicgstab(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solve
         fv_sparsity* sp = ls->sp;
         fv_ctx* ctx = sp->mesh->ctx;
         hipStream_t s = ctx->stream;
-        BiState h{};
+        BiState h{}, part{};  // part: of a persistent solve that could not go on
+        part.res0 = -1.0;
         const BiWork::Target t{(double*)d_x, ls->rhs.p, 0, 1};
-        if (!o->eager && w.persist && w.run_persist(s, t, o, true)) {
-            h = w.finish_persist(ctx, t, o, *w.states(ctx, 1));
+        bool through = !o->eager && w.persist && w.run_persist(s, t, o, true);
+        if (through) {
+            h = *w.states(ctx, 1);
+            through = w.finish_persist(ctx, t, o, h);
+            if (!through) part = h;
             local.true_res = h.trueRes;
-        } else {
+        }
+        if (!through) {
+            const int maxIter = part.it ? std::max(o->max_iter - part.it, 1) : o->max_iter;
             w.h.x = (double*)d_x;
             FV_HIP(hipMemcpyAsync(w.sys.p, &w.h, sizeof w.h, hipMemcpyHostToDevice, s));
             kbi_dinv<<<grid_for(sp->nRows, kB), kB, 0, s>>>(sp->nRows, sp->rowOffs.p, sp->diagOffset.p,
@@ -1222,12 +1263,12 @@ int fv_solve_bicgstab(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solve
             kbi_scale<<<grid_for(sp->sellTotal, kB, 8192), kB, 0, s>>>(
                 sp->sellTotal, sp->sellSrc.p, sp->sellCol.p, ls->values.p, w.dinv.p, w.sval.p);
             kbi_start<<<w.G, kB, 0, s>>>(w.sys.p);
-            kbi_start_state<<<1, kB, 0, s>>>(w.sys.p, o->rel_tol, o->abs_tol, o->max_iter);
+            kbi_start_state<<<1, kB, 0, s>>>(w.sys.p, o->rel_tol, o->abs_tol, maxIter);
             FV_LAUNCH_CHECK();
             const int check = o->check_every > 0 ? o->check_every : 8;
             int launched = 0, batch = std::min(2, check);
             while (true) {
-                const int n = std::min(batch, std::max(1, o->max_iter - launched + 1));
+                const int n = std::min(batch, std::max(1, maxIter - launched + 1));
                 batch = std::min(2 * batch, check);
                 for (int i = 0; i < n; ++i) {
                     kbi_dir<<<w.G, kB, 0, s>>>(w.sys.p);
@@ -1241,7 +1282,7 @@ int fv_solve_bicgstab(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solve
                 FV_HIP(hipMemcpyAsync(&h, w.st.p, sizeof h, hipMemcpyDeviceToHost, s));
                 FV_HIP(hipStreamSynchronize(s));
                 if (h.stop) break;
-                FV_REQUIRE(launched <= o->max_iter + 1, "BiCGStab iteration bookkeeping");
+                FV_REQUIRE(launched <= maxIter + 1, "BiCGStab iteration bookkeeping");
             }
             // explicit FP64 residual b - A x of the result
             kbi_start<<<w.G, kB, 0, s>>>(w.sys.p);
@@ -1251,6 +1292,8 @@ int fv_solve_bicgstab(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solve
             FV_HIP(hipMemcpyAsync(&h2, w.st.p, sizeof h2, hipMemcpyDeviceToHost, s));
             FV_HIP(hipStreamSynchronize(s));
             local.true_res = h2.res0;
+            if (part.res0 >= 0.0) h.res0 = part.res0;
+            h.it += part.it;
         }
         bi_finish(h, local);
     });

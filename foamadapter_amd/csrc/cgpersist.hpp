@@ -52,7 +52,9 @@
 // write nothing before all of them have arrived, and if one has not within
 // kMeetClocks (other work holds its place), all end and the solve is launched again,
 // cooperatively.  Every wait after that is bounded by a clock too: a workgroup that
-// waits longer than kSyncSeconds sets stop = kStopSync and ends, and so do the others.
+// waits longer than kSyncSeconds sets `lost` and ends, and so do the others.  A solve
+// whose launch is lost, or refused by the device, goes on kernel by kernel from the x
+// there is.
 //
 // Measured per iteration (pressure equation on jittered cubes in Z order,
 // kernel-by-kernel form -> this one): FP64 32^3 10.8 -> 5.3 us, 64^3 21.6 -> 7.9, 96^3
@@ -75,16 +77,23 @@ constexpr int kPersistGroups = kCgMaxTiles / kPersistSub;  // workgroups at most
 constexpr int kSlotWords = 16;  // up to four doubles as half-payload words; a 128-byte line per slot
 constexpr int kCopies = 8;       // of what many workgroups read
 constexpr int kSlotBuffer = (kPersistGroups + 8 * kCopies) * kSlotWords;  // workgroups; groups of them
-constexpr int kStopSync = 4;           // CgState::stop after a timed-out wait
-constexpr int kStopApart = 5;          // after a plain launch whose workgroups did not meet
-constexpr unsigned long long kSyncSeconds = 20;
-constexpr unsigned long long kClockHz = 100000000ull;  // wall_clock64: 100 MHz
+constexpr int kStopApart = 5;  // CgState::stop after a plain launch whose workgroups did not meet
+constexpr double kSyncSeconds = 20.0, kFailSeconds = 0.005;
+constexpr double kClockHz = 1e8;  // wall_clock64: 100 MHz
 
 // The assembled system, for the persistent forms that scale the matrix and take
 // explicit residuals themselves.
 struct CsrSystem {
     const int32_t *rowOffs, *diag;
     const double *vals, *rhs;
+};
+
+// What PersistSlots::launch says of a launch.
+struct PersistLaunch {
+    unsigned long long meet;  // Meeting::target
+    uint32_t fails;           // exchange workgroups 8 to 15 are missing from (0: none; for
+                              // tests, where a wait ends after kFailSeconds; p.q or the
+                              // result's residual)
 };
 
 // Arguments by value: the kernel reads them from scalar registers instead of
@@ -110,8 +119,8 @@ struct CgPersist {
     double* x;
     double tol, atol;
     int32_t maxit, fresh;
-    unsigned long long meet;  // Meeting::target
     CgState* host;            // what the host reads of the state (pinned)
+    PersistLaunch launch;
 };
 
 template <typename T>
@@ -187,7 +196,15 @@ __device__ __forceinline__ double from_lane(double x, int lane) {
 struct PersistLds {
     double wave[4][kPersistThreads / 64];  // wave sums of this workgroup's tiles
     double tot[2][4];                      // by parity of the exchange: the grid's sums
+    // PersistLaunch's, and how long a wait may last in 65536 clocks: no registers are left
+    // for them in the loop (spills: 128^3 FP32 14.8 -> 15.2 us)
+    uint32_t fails, limit;
     int bad, met;
+    __device__ void begin(const PersistLaunch& a) {  // one thread, before the first barrier
+        fails = a.fails;
+        limit = (uint32_t)((a.fails ? kFailSeconds : kSyncSeconds) * kClockHz / 65536);
+        bad = 0;
+    }
 };
 
 // One workgroup's place in the grid exchange.  sum_slots adds the slots of a
@@ -234,7 +251,7 @@ struct GridSum {
     }
     // The values of slot s once they carry the tag; false after kSyncSeconds.
     template <int NV>
-    __device__ static bool collect(const unsigned long long* s, uint32_t tag, double (&v)[NV]) {
+    __device__ bool collect(const unsigned long long* s, double (&v)[NV], const PersistLds& L) const {
         unsigned long long w[2 * NV], t0 = 0;
         for (int tries = 0;; ++tries) {
             bool ok = true;
@@ -244,7 +261,7 @@ struct GridSum {
             if ((tries & 63) == 63) {
                 const unsigned long long t = wall_clock64();
                 if (!t0) t0 = t;
-                if (t - t0 > kSyncSeconds * kClockHz) return false;
+                if ((uint32_t)((t - t0) >> 16) > L.limit) return false;
             }
         }
         for (int j = 0; j < NV; ++j)
@@ -278,7 +295,9 @@ struct GridSum {
                              p2 = from_lane(part, 2), p3 = from_lane(part, 3);
                 a[j] = large ? ((p0 + p1) + p2) + p3 : (p0 + p2) + (p1 + p3);
             }
-            if (lane == 0)
+            // (only where this is asked, and the BiCGStab's loop has no register for it)
+            const bool there = NV > 1 || PUBLISHED || tag != L.fails || slot >> 3 != 1;
+            if (lane == 0 && there)
                 for (int j = 0; j < NV; ++j)
                     publish(buf + (size_t)slot * kSlotWords + 2 * j, a[j], tag);
             bool ok = true;
@@ -291,7 +310,7 @@ struct GridSum {
                     double m[NV];
                     for (int j = 0; j < NV; ++j) m[j] = 0.0;
                     if (lane < kPersistGroups / 8)
-                        ok = collect<NV>(buf + (size_t)(group + 8 * lane) * kSlotWords, tag, m);
+                        ok = collect<NV>(buf + (size_t)(group + 8 * lane) * kSlotWords, m, L);
                     for (int j = 0; j < NV; ++j) m[j] = from_lane(lane_sum<16>(m[j]), 0);
                     if (lane < kCopies)
                         for (int j = 0; j < NV; ++j)
@@ -302,7 +321,7 @@ struct GridSum {
             }
             double g[NV];
             for (int j = 0; j < NV; ++j) g[j] = 0.0;
-            if (ok && lane < count) ok = collect<NV>(from + (size_t)lane * kSlotWords, tag, g);
+            if (ok && lane < count) ok = collect<NV>(from + (size_t)lane * kSlotWords, g, L);
             for (int j = 0; j < NV; ++j) {
                 double r = 0.0;
                 if (large) {  // lanes 2 w and 2 w + 1: the last step of wave w's tree
@@ -436,7 +455,7 @@ __global__ __launch_bounds__(kCgBlock) void k_ghost_plan(int N, int R, int W, in
 // decision, 2 * tag + 1 (all have arrived) or 2 * tag (one gave up).  The first to
 // decide wins, so every workgroup sees the same decision, late ones included.
 constexpr int kMeetWords = 32;
-constexpr unsigned long long kMeetClocks = kClockHz / 500;  // 2 ms
+constexpr unsigned long long kMeetClocks = (unsigned long long)(kClockHz / 500);  // 2 ms
 struct Meeting {
     unsigned long long* words;
     unsigned long long target;  // 0: a cooperative launch
@@ -555,16 +574,16 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     const int tile = gs.place(A.tiles, sub);
     CgState* const st = A.st;
     const bool lead = gs.slot == 0 && tid == 0;
-    const Meeting meeting{A.slots + 2 * kSlotBuffer, WHOLE ? A.meet : 0, A.tag0};
+    const Meeting meeting{A.slots + 2 * kSlotBuffer, WHOLE ? A.launch.meet : 0, A.tag0};
     meeting.arrive();
     if (!WHOLE || !A.fresh) {
         const int entry = st->stop;
-        if (entry) {
+        if (entry || st->lost) {
             if (lead) st->done = entry;  // as the update kernel of a stopped system
             return;
         }
     }
-    if (tid == 0) L.bad = 0;
+    if (tid == 0) L.begin(A.launch);
     const int row0 = tile * R;
     const int row1 = tile < A.tiles ? min(row0 + R, (A.N + 63) & ~63) : row0;
     // this wave's first row; its row u is iw + 256 u + lane, of slice (iw + 256 u) / 64
@@ -712,6 +731,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
                 bnorm = sqrt(t4[1]);
                 if (!(bnorm > 0.0)) bnorm = 1.0;
                 res = res0 = sqrt(t4[0]) / bnorm;
+                if (lead) A.host->res0 = res0;
                 rho = t4[3];
                 rhoPrev = alpha = 0.0;
                 it = 0;
@@ -853,8 +873,8 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
     }
     if (!ok) {
         if (tid == 0) {
-            st->stop = kStopSync;
-            if (WHOLE) A.host->stop = kStopSync;
+            st->lost = 1;
+            if (WHOLE) A.host->lost = 1;
         }
         return;
     }
@@ -882,7 +902,6 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
             st->rrep = rrep;
             // straight to the host: a copy behind the launch takes 5 us
             A.host->res = res;
-            A.host->res0 = res0;
             A.host->rrep = rrep;
             A.host->bnorm = bnorm;
             A.host->it = it;
@@ -915,11 +934,11 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist_far(CgPersist<S> A
     CgState* const st = A.st;
     const bool lead = gs.slot == 0 && tid == 0;
     const int entry = st->stop;
-    if (entry) {
+    if (entry || st->lost) {
         if (lead) st->done = entry;  // as the update kernel of a stopped system
         return;
     }
-    if (tid == 0) L.bad = 0;
+    if (tid == 0) L.begin(A.launch);
     const int row0 = tile * R;
     const int row1 = tile < A.tiles ? min(row0 + R, (A.N + 63) & ~63) : row0;
     // this wave's first row; its row u is iw + 256 u + lane, of slice (iw + 256 u) / 64
@@ -1108,7 +1127,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist_far(CgPersist<S> A
         __syncthreads();
     }
     if (!ok) {
-        if (tid == 0) st->stop = kStopSync;
+        if (tid == 0) st->lost = 1;
         return;
     }
 #pragma unroll
@@ -1160,24 +1179,59 @@ struct GhostPlan {
 // The exchange buffer of a system and its launches.
 struct PersistSlots {
     DBuf<unsigned long long> words;
+    fv_persist_log* log = nullptr;
     unsigned long long meets = 0;  // arrivals of all plain launches
     bool apart = false;            // a plain launch did not meet: cooperative from then on
-    void alloc(fv_ctx* c) { words.alloc(c, 2 * (size_t)kSlotBuffer + kMeetWords); }
+    void alloc(fv_ctx* c, fv_persist_log* l) {
+        words.alloc(c, 2 * (size_t)kSlotBuffer + kMeetWords);
+        log = l;
+    }
     void clear(hipStream_t s) {  // no word carries a tag that is still to come
         FV_HIP(hipMemsetAsync(words.p, 0, words.n * sizeof(unsigned long long), s));
         meets = 0;
     }
-    // Meeting::target of the next launch over `grid` workgroups
-    unsigned long long next(int grid, bool plain) { return plain && !apart ? meets += grid : 0; }
-    static bool launch(const void* kernel, int grid, void* args, bool cooperative, hipStream_t s) {
-        void* a[] = {args};
-        const hipError_t e =
-            cooperative ? hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(kPersistThreads), a, 0, s)
-                        : hipLaunchKernel(kernel, dim3(grid), dim3(kPersistThreads), a, 0, s);
-        if (e != hipSuccess) (void)hipGetLastError();
-        return e == hipSuccess;
+    // One launch; meeting: as a plain one whose workgroups meet.  False if the device
+    // refuses it.
+    template <typename Args>
+    bool launch(void (*kernel)(Args), int grid, Args& args, bool meeting, hipStream_t s) {
+        const int fault = log->take();
+        const bool plain = meeting && !apart;
+        args.launch = PersistLaunch{plain ? meets + grid : 0, 0};
+        if (fault == FV_PERSIST_APART && plain) ++args.launch.meet;  // never reached
+        if (fault == FV_PERSIST_LOST) args.launch.fails = args.tag0 + (uint32_t)log->exchange;
+        void* a[] = {&args};
+        const void* const k = reinterpret_cast<const void*>(kernel);
+        hipError_t e = hipErrorUnknown;
+        if (fault != FV_PERSIST_REFUSED)
+            e = plain ? hipLaunchKernel(k, dim3(grid), dim3(kPersistThreads), a, 0, s)
+                      : hipLaunchCooperativeKernel(k, dim3(grid), dim3(kPersistThreads), a, 0, s);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            ++log->refused;
+            return false;
+        }
+        ++log->launches;
+        if (plain) meets += grid;
+        return true;
+    }
+    void did_not_meet() {
+        apart = true;
+        ++log->apart;
     }
 };
+
+// Whether alloc() found room for the buffers of a persistent solver.
+template <typename F>
+bool persist_room(F&& alloc) {
+    try {
+        alloc();
+        return true;
+    } catch (const Error&) {
+        (void)hipGetLastError();
+        clear_error();
+        return false;
+    }
+}
 
 // Workgroups of a persistent launch over `tiles` tiles
 inline int persist_grid(int tiles) {

@@ -588,6 +588,27 @@ int fv_linsys_destroy(fv_linsys* ls) {
     return guarded([&] { delete ls; });
 }
 
+int fv_linsys_persist_counts(const fv_linsys* ls, int solver, int64_t* h) {
+    return guarded([&] {
+        FV_REQUIRE(ls && h && solver >= 0 && solver < 3, "bad arguments");
+        const fv_persist_log& l = ls->persistLog[solver];
+        const int64_t c[4] = {l.launches, l.apart, l.refused, l.lost};
+        std::copy_n(c, 4, h);
+    });
+}
+
+int fv_linsys_persist_fault(fv_linsys* ls, int solver, int fault, int after, int exchange) {
+    return guarded([&] {
+        FV_REQUIRE(ls && solver >= 0 && solver < 3 && fault >= 0 && fault <= FV_PERSIST_LOST &&
+                       after >= 0 && exchange >= 0,
+                   "bad arguments");
+        fv_persist_log& l = ls->persistLog[solver];
+        l.fault = fault;
+        l.after = after;
+        l.exchange = exchange;
+    });
+}
+
 void* fv_linsys_values(fv_linsys* ls) { return ls ? (void*)ls->values.p : nullptr; }
 void* fv_linsys_rhs(fv_linsys* ls) { return ls ? (void*)ls->rhs.p : nullptr; }
 

@@ -36,6 +36,20 @@ struct fv_solver_cache {
     virtual ~fv_solver_cache() = default;
 };
 
+// Launches of a system's persistent solver, and the mishap the next ones are to have
+// (fv_linsys_persist_fault).
+struct fv_persist_log {
+    int64_t launches = 0, apart = 0, refused = 0, lost = 0;
+    int fault = 0, after = 0, exchange = 0;
+    // the fault of the launch at hand
+    int take() {
+        if (!fault || after-- > 0) return 0;
+        const int f = fault;
+        fault = 0;
+        return f;
+    }
+};
+
 // la::LinearSystem<scalar, localIdx>: values[nnz], rhs[N] (FP64), with the
 // convention A.x - b = (operator applied to x) * V.
 struct fv_linsys {
@@ -45,6 +59,7 @@ struct fv_linsys {
     // the face flux is bRhs - bMat * x_P (NeoN's la::BoundaryCoefficients,
     // read by updateFaceVelocity, pressureVelocityCoupling.cpp:180-192)
     fvhip::DBuf<double> bMat, bRhs;
+    fv_persist_log persistLog[3];
     std::unique_ptr<fv_solver_cache> cg[3];  // FP64 CG, FP32 CG in FP64 refinement, BiCGStab
 };
 

@@ -55,7 +55,7 @@ struct CgWork : fv_solver_cache {
     GhostPlan plan;
     uint32_t tag = 1;
 
-    CgWork(fv_ctx* c, const fv_linsys* ls) {
+    CgWork(fv_ctx* c, fv_linsys* ls) {
         const fv_sparsity* sp = ls->sp;
         const int N = sp->nRows;
         const int R = cg_tile_rows(N, kB);
@@ -101,21 +101,31 @@ struct CgWork : fv_solver_cache {
         grid.nTiles = tiles;
         grid.rowsPerBlock = R;
         gdev.upload(c, &grid, 1);
+        FV_HIP(hipMemsetAsync(st.p, 0, sizeof(CgState), c->stream));
         FV_HIP(hipStreamSynchronize(c->stream));
         red = CgPartials{pq.p, rz.p, rb.p};
-        if (!c->shared) choose_persist(c, sp, tiles, R);
+        if (!c->shared) choose_persist(c, sp, tiles, R, &ls->persistLog[sizeof(S) == 8 ? 0 : 1]);
     }
 
     // The persistent kernel for this system, when there is one: slices of one
     // width, at most 8 rows per thread (2^21 rows; beyond, the vectors do not fit
     // the registers), and a device that keeps its workgroups resident together.
-    void choose_persist(fv_ctx* c, const fv_sparsity* sp, int tiles, int R) {
+    // Where its buffers find no room, the system runs kernel by kernel.
+    void choose_persist(fv_ctx* c, const fv_sparsity* sp, int tiles, int R, fv_persist_log* log) {
         const int rpt = (R + kB - 1) / kB;
         if (rpt > 8) return;
-        if (sp->sellWidth == 6)
-            choose_kernel<6>(c, tiles, R, rpt);
-        else if (sp->sellWidth == 4)
-            choose_kernel<4>(c, tiles, R, rpt);
+        const bool room = persist_room([&] {
+            slots.alloc(c, log);
+            if (sp->sellWidth == 6)
+                choose_kernel<6>(c, tiles, R, rpt);
+            else if (sp->sellWidth == 4)
+                choose_kernel<4>(c, tiles, R, rpt);
+        });
+        if (!room) {
+            persist = nullptr;
+            slots.words.release();
+            plan = GhostPlan{};
+        }
         if (!persist) return;
         persistGrid = persist_grid(tiles);
         if (!persist_fits(reinterpret_cast<const void*>(persist), c->device, persistGrid)) {
@@ -127,7 +137,6 @@ struct CgWork : fv_solver_cache {
         // smallest of these systems, on the largest 28 in FP64 and 15 in FP32), so that
         // the work of other streams gets in between
         persistIters = (int)(2000.0 / (5.0 + (sizeof(S) == 8 ? 23.0 : 10.0) * h.N / (1 << 21)));
-        slots.alloc(c);
         clear_tags(c->stream);
     }
     // A cooperative launch costs about 17 us more than a plain one and is not
@@ -177,19 +186,20 @@ struct CgWork : fv_solver_cache {
                        h.g, h.d, h.r, h.p, h.p2, plan.words.p, plan.ghosts.p, plan.count.p,
                        plan.stride, h.st, slots.words.p,
                        CsrSystem{h.rowOffs, h.diag, h.vals, h.rhs}, x, tol, atol, maxit,
-                       fresh ? 1 : 0, slots.next(persistGrid, whole), host};
-        if (!PersistSlots::launch(reinterpret_cast<const void*>(persist), persistGrid, &a, a.meet == 0, s)) {
+                       fresh ? 1 : 0, host, {}};
+        if (!slots.launch(persist, persistGrid, a, whole, s)) {
             persist = nullptr;
             return false;
         }
         tag += uses;
         return true;
     }
-    void check_persist(const CgState& h) {
-        if (h.stop != kStopSync) return;
+    // Whether a launch lost its workgroups; this system's solves run kernel by kernel then.
+    bool lost(const CgState& h) {
+        if (!h.lost) return false;
+        ++slots.log->lost;
         persist = nullptr;
-        throw Error{FV_EDEVICE, "persistent CG: the workgroups did not meet in " +
-                                    std::to_string(kSyncSeconds) + " s"};
+        return true;
     }
 
     ~CgWork() override { drop_graph(); }
@@ -446,31 +456,34 @@ CgState run_cg(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, int check,
 // nothing has to be predicted.  A whole solve is one launch and one read (of pinned
 // memory) unless it runs out of a launch's iterations.  Else, a system whose previous solve fitted one launch
 // gets the correction and the explicit residual queued behind it and is read
-// once; otherwise two launches are kept queued until one has stopped.  False
-// (and nothing done) if the device refuses the launch.
+// once; otherwise two launches are kept queued until one has stopped.  False if the
+// device refuses a launch or one is lost: out->it iterations are in x then, and out->res0
+// is the initial residual if it is known (the caller sets -1).
 bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, double atol,
                     double* x, double* true_res, CgState* out) {
     hipStream_t s = ctx->stream;
     if (w.whole) {
         CgState* const host = static_cast<CgState*>(ctx_poll_host(ctx));  // the kernel writes it
         bool fresh = true;
+        host->res0 = -1.0;
         do {
             host->stop = -1;
-            if (!w.run_persist(s, x, tol, atol, maxit, fresh, host)) {
-                FV_REQUIRE(fresh, "a cooperative launch was refused");
+            host->lost = 0;
+            if (!w.run_persist(s, x, tol, atol, maxit, fresh, host)) return false;
+            FV_HIP(hipStreamSynchronize(s));
+            if (w.lost(*host)) {
+                out->res0 = host->res0;
                 return false;
             }
-            FV_HIP(hipStreamSynchronize(s));
             FV_REQUIRE(host->stop != -1, "a persistent solve left no state");
             if (host->stop == kStopApart) {  // nothing done: the same launch, cooperative
-                w.slots.apart = true;
+                w.slots.did_not_meet();
                 if (!fresh) FV_HIP(hipMemsetAsync(&w.st.p->stop, 0, sizeof(int32_t), s));
             } else {
                 fresh = false;
             }
         } while (!host->stop || host->stop == kStopApart);
         *out = *host;
-        w.check_persist(*out);
         w.lastIters = std::max(out->it, 1);
         *true_res = out->rrep;
         return true;
@@ -479,7 +492,7 @@ bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, doubl
     w.start(s, tol, maxit, 0.0, atol);
     if (!w.run_persist(s)) return false;
     CgState h{}, t{};
-    bool haveTrue = false;
+    bool haveTrue = false, refused = false;
     if (w.lastIters > 0 && w.lastIters <= w.persistIters) {
         w.finish(s);
         w.enqueue_true_residual(s);
@@ -487,20 +500,25 @@ bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, doubl
         h = w.state2(s, &t);
         haveTrue = h.stop != 0;
     }
-    if (!h.stop) {
+    if (!h.stop && !h.lost) {
         PollPipe pp{static_cast<CgState*>(ctx_poll_host(ctx)), ctx};
         pp.push(s, w.st.p);
-        while (!h.stop) {
-            while (pp.npend < 2) {
-                FV_REQUIRE(w.run_persist(s), "a cooperative launch was refused");
-                pp.push(s, w.st.p);
+        while (!h.stop && !h.lost) {
+            while (!refused && pp.npend < 2) {
+                refused = !w.run_persist(s);
+                if (!refused) pp.push(s, w.st.p);
             }
+            if (pp.npend == 0) break;
             h = pp.pop();
         }
         while (pp.npend) h = pp.pop();
         w.finish(s);
     }
-    w.check_persist(h);
+    const bool lost = w.lost(h);
+    if (lost || !h.stop) {
+        *out = h;
+        return false;
+    }
     w.lastIters = std::max(h.it, 1);
     *true_res = haveTrue ? t.res : w.true_residual(s);
     *out = h;
@@ -654,24 +672,29 @@ IrOut run_mixed(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, int chunk,
 // run_mixed with the persistent kernel: a round is one launch, which ends at the
 // drop trigger, the tolerance or its iterations, and the replacement kernels,
 // which act only on a stopped CG.  As many rounds as the previous solve took are
-// queued at once, otherwise two at a time.
+// queued at once, otherwise two at a time.  False if the device refuses a launch or one is
+// lost: out->iters iterations, of which x holds those up to the last replacement, and
+// out->init_res as run_cg_persist.
 bool run_mixed_persist(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, double delta,
                        double atol, IrOut* out) {
     hipStream_t s = ctx->stream;
     w.start(s, tol, maxit, delta, atol);
-    if (!w.run_persist(s)) return false;
-    w.replacement(s);
-    int rounds = 1;
+    int rounds = 0;
+    bool refused = false;
     auto round = [&] {
-        FV_REQUIRE(w.run_persist(s), "a cooperative launch was refused");
+        refused = !w.run_persist(s);
+        if (refused) return false;
         w.replacement(s);
         FV_LAUNCH_CHECK();
         ++rounds;
+        return true;
     };
+    if (!round()) return false;
     CgState h{};
-    auto done = [&] { return h.stop >= 2 || h.it >= maxit; };
+    auto done = [&] { return h.stop >= 2 || h.it >= maxit || h.lost; };
     if (w.lastLaunches > 0) {
-        while (rounds < w.lastLaunches) round();
+        while (rounds < w.lastLaunches && round()) {
+        }
         h = w.state(s);
     }
     if (!done()) {
@@ -679,19 +702,18 @@ bool run_mixed_persist(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, dou
         int seen = rounds - 1;
         pp.push(s, w.st.p);
         while (!done()) {
-            while (pp.npend < 2) {
-                round();
-                pp.push(s, w.st.p);
-            }
+            while (!refused && pp.npend < 2)
+                if (round()) pp.push(s, w.st.p);
+            if (pp.npend == 0) break;
             h = pp.pop();
             ++seen;
         }
         while (pp.npend) h = pp.pop();
         rounds = seen;
     }
-    w.check_persist(h);
-    if (h.stop == 2) w.lastLaunches = rounds;
     *out = IrOut{h.res0, h.res, h.bnorm, h.it, h.nrep};
+    if (w.lost(h) || !done()) return false;
+    if (h.stop == 2) w.lastLaunches = rounds;
     return true;
 }
 
@@ -714,10 +736,15 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
             CgWork<double>& w = work_of<double>(ls, false);
             double tr = 0.0;
             CgState h{};
+            h.res0 = -1.0;
             if (o->eager || !w.use_persist() ||
                 !run_cg_persist(ctx, w, o->rel_tol, o->max_iter, o->abs_tol, x, &tr, &h)) {
+                const CgState part = h;  // of a persistent solve that could not go on
                 w.bind(ctx, x);
-                h = run_cg(ctx, w, o->rel_tol, o->max_iter, check, o->abs_tol, o->eager != 0, &tr);
+                h = run_cg(ctx, w, o->rel_tol, part.it ? std::max(o->max_iter - part.it, 1) : o->max_iter,
+                           check, o->abs_tol, o->eager != 0, &tr);
+                if (part.res0 >= 0.0) h.res0 = part.res0;
+                h.it += part.it;
             }
             w.lastTotal = h.it;
             local.init_res = h.res0;
@@ -729,16 +756,21 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
         } else if (o->mode == FV_SOLVE_F32_IR) {
             CgWork<float>& w = work_of<float>(ls, true);
             w.bind(ctx, x);
-            IrOut r{};
+            IrOut r{-1.0, 0.0, 0.0, 0, 0};
             const double delta = o->inner_rel_tol > 0.0 ? o->inner_rel_tol : kIrDelta;
             // max_outer counts rounds of check_every iterations: those solves run
             // kernel by kernel
             if (o->eager || o->max_outer > 0 || !w.use_persist() ||
-                !run_mixed_persist(ctx, w, o->rel_tol, o->max_iter, delta, o->abs_tol, &r))
-                r = run_mixed(ctx, w, o->rel_tol, o->max_iter,
+                !run_mixed_persist(ctx, w, o->rel_tol, o->max_iter, delta, o->abs_tol, &r)) {
+                const IrOut part = r;
+                r = run_mixed(ctx, w, o->rel_tol, part.iters ? std::max(o->max_iter - part.iters, 1) : o->max_iter,
                               o->check_every > 0 ? o->check_every : 64, delta,
                               o->max_outer > 0 ? o->max_outer : (1 << 30), o->abs_tol,
                               o->eager != 0);
+                if (part.init_res >= 0.0) r.init_res = part.init_res;
+                r.iters += part.iters;
+                r.outer += part.outer;
+            }
             w.lastTotal = r.iters;
             local.init_res = r.init_res;
             local.final_res = r.res;

@@ -432,6 +432,17 @@ int fv_solve_bicgstab(fv_linsys* ls, void* d_x, const fv_solve_opts* opts,
  * the component solved last. */
 int fv_solve_bicgstab_vec(fv_linsys* ls, int ncomp, const void* d_rhs, void* d_x,
                           const fv_solve_opts* opts, fv_solver_stats* stats, int* solved);
+/* The persistent solves of a system, by solver: 0 FP64 CG, 1 mixed CG, 2 BiCGStab.
+ * h_counts4: launches; plain launches whose workgroups did not meet (launched again,
+ * cooperatively); launches the device refused, and launches whose workgroups lost each
+ * other (both go on kernel by kernel, from the x there is). */
+int fv_linsys_persist_counts(const fv_linsys* ls, int solver, int64_t* h_counts4);
+/* Makes one of these happen to the launch after the next `after` ones, for tests of what
+ * follows: FV_PERSIST_LOST at the launch's exchange number `exchange` (from 0; one that
+ * sums p.q or the result's residual), to which some workgroups bring nothing; the waits end
+ * after 5 ms and every workgroup by itself. */
+enum { FV_PERSIST_APART = 1, FV_PERSIST_REFUSED = 2, FV_PERSIST_LOST = 3 };
+int fv_linsys_persist_fault(fv_linsys* ls, int solver, int fault, int after, int exchange);
 
 /* ---- pressure-velocity coupling (src/algorithms/pressureVelocityCoupling.cpp) ---
  * FP64.  The momentum matrix is the scalar system ls (the reference reads

@@ -312,7 +312,8 @@ struct GridSum {
                     if (lane < kPersistGroups / 8)
                         ok = collect<NV>(buf + (size_t)(group + 8 * lane) * kSlotWords, m, L);
                     for (int j = 0; j < NV; ++j) m[j] = from_lane(lane_sum<16>(m[j]), 0);
-                    if (lane < kCopies)
+                    ok = __all(ok);  // a sum without one of its members is none
+                    if (ok && lane < kCopies)
                         for (int j = 0; j < NV; ++j)
                             publish(gbuf + (size_t)(8 * lane + group) * kSlotWords + 2 * j, m[j], tag);
                 }

@@ -1025,13 +1025,15 @@ struct BiWork : fv_solver_cache {
     BiState* host = nullptr;  // the context's pinned poll area
     bool plain = false;  // kbi_persist, whose workgroups can meet by themselves
     uint32_t tag = 1;
-    GhostPlan plan;
+    bool chosen = false;  // (or found impossible: at the first solve that may use it)
+    const fv_ghost_plan* plan = nullptr;  // null: kbi_persist_far
     // 1, 2 or 4 rows per thread (2^20 rows); RES, the rows whose matrix stays in
     // registers, as in the CG
     template <int W>
-    void choose_kernel(fv_ctx* c, int rpt) {
+    void choose_kernel(fv_ctx* c, fv_sparsity* sp, int rpt) {
         const int n = rpt <= 1 ? 1 : rpt <= 2 ? 2 : 4;
-        plain = plan.make(c, h.N, h.ntiles, h.rowsPerBlock, W, n * kB, 8, bi_ghost_cap(n), h.sellCol);
+        plan = ghost_plan(c, sp, h.ntiles, h.rowsPerBlock, W, n * kB, 8, bi_ghost_cap(n));
+        plain = plan != nullptr;
         if (plain)
             persist = n == 1 ? kbi_persist<1, W, 1> : n == 2 ? kbi_persist<2, W, 2> : kbi_persist<4, W, 0>;
         else
@@ -1040,20 +1042,22 @@ struct BiWork : fv_solver_cache {
                                : kbi_persist_far<4, W, 0>;
     }
     // Where its buffers find no room, the system runs kernel by kernel.
-    void choose_persist(fv_ctx* c, const fv_sparsity* sp, fv_persist_log* log) {
+    void choose_persist(fv_ctx* c, fv_linsys* ls) {
+        if (chosen || c->shared) return;
+        chosen = true;
+        fv_sparsity* const sp = ls->sp;
         const int rpt = (h.rowsPerBlock + kB - 1) / kB;
         if (rpt > 4) return;
         const bool room = persist_room([&] {
-            slots.alloc(c, log);
+            slots.alloc(c, &ls->persistLog[2]);
             if (sp->sellWidth == 6)
-                choose_kernel<6>(c, rpt);
+                choose_kernel<6>(c, sp, rpt);
             else if (sp->sellWidth == 4)
-                choose_kernel<4>(c, rpt);
+                choose_kernel<4>(c, sp, rpt);
         });
         if (!room) {
             persist = nullptr;
             slots.words.release();
-            plan = GhostPlan{};
         }
         persistGrid = persist_grid(h.ntiles);
         if (!persist || !persist_fits(reinterpret_cast<const void*>(persist), c->device, persistGrid)) {
@@ -1086,8 +1090,9 @@ struct BiWork : fv_solver_cache {
         BiPersist a{h.N, h.ntiles, h.rowsPerBlock, persistIters, fresh ? 1 : 0, o->max_iter, tag,
                     o->rel_tol, o->abs_tol, h.sellCol, CsrSystem{h.rowOffs, diag, h.vals, t.rhs + t.comp},
                     t.ncomp, x, t.ncomp > 1 ? x : nullptr, chained ? state - 1 : nullptr, sval.p,
-                    t.ncomp > 1 ? dinv.p : x, h.r, h.rhat, h.p, h.v, h.t, h.s, plan.words.p,
-                    plan.ghosts.p, plan.count.p, plan.stride, state, host + t.comp, slots.words.p, {}};
+                    t.ncomp > 1 ? dinv.p : x, h.r, h.rhat, h.p, h.v, h.t, h.s, plan ? plan->words.p : nullptr,
+                    plan ? plan->ghosts.p : nullptr, plan ? plan->count.p : nullptr,
+                    plan ? plan->stride : 0, state, host + t.comp, slots.words.p, {}};
         host[t.comp].stop = -1;
         host[t.comp].lost = 0;
         if (!slots.launch(persist, persistGrid, a, plain, s)) {
@@ -1135,7 +1140,6 @@ struct BiWork : fv_solver_cache {
         h.st = st.p;
         diag = sp->diagOffset.p;
         FV_HIP(hipMemsetAsync(st.p, 0, kMaxComp * sizeof(BiState), c->stream));
-        if (!c->shared) choose_persist(c, sp, &ls->persistLog[2]);
     }
     // The states after the work queued so far (pinned, valid until the next launch)
     const BiState* states(fv_ctx* c, int n) {
@@ -1179,7 +1183,9 @@ BiWork& bi_work(fv_linsys* ls, const fv_solve_opts* o) {
     FV_REQUIRE(o->mode == FV_SOLVE_F64, "BiCGStab runs in FP64 only");
     auto& slot = ls->cg[2];
     if (!slot) slot.reset(new BiWork(ls->sp->mesh->ctx, ls));
-    return *static_cast<BiWork*>(slot.get());
+    BiWork& w = *static_cast<BiWork*>(slot.get());
+    if (!o->eager) w.choose_persist(ls->sp->mesh->ctx, ls);
+    return w;
 }
 
 // stats of a stopped solve; throws unless it converged

@@ -66,6 +66,7 @@
 
 #include "cgkernels.hpp"
 
+#include <algorithm>
 #include <vector>
 
 namespace fvhip {
@@ -1150,32 +1151,34 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist_far(CgPersist<S> A
     }
 }
 
-// The ghosts of every tile of a system and the columns that refer to them.
-struct GhostPlan {
-    DBuf<uint32_t> words;
-    DBuf<int32_t> ghosts, count;
-    int stride = 0;
-    // False if a tile has more than cap ghosts.  own: rows a tile has places for; size:
-    // bytes a value.
-    bool make(fv_ctx* c, int N, int tiles, int R, int W, int own, int size, int cap,
-              const int32_t* sellCol) {
-        count.alloc(c, tiles);
-        auto plan = [&](uint32_t* w, int32_t* g) {
-            k_ghost_plan<<<tiles, kCgBlock, 0, c->stream>>>(N, R, W, own, size, sellCol, w, g, stride,
-                                                            count.p);
-            FV_LAUNCH_CHECK();
-        };
+// The ghosts of a pattern's tiles for values of `size` bytes (own: rows a tile has places
+// for); null if a tile has more than cap.  The plan stays with the pattern: its systems and
+// solvers have the same tiles (cg_tile_rows), so one per value size serves them all.
+inline const fv_ghost_plan* ghost_plan(fv_ctx* c, fv_sparsity* sp, int tiles, int R, int W, int own,
+                                       int size, int cap) {
+    fv_ghost_plan& p = sp->ghostPlan[size == 8 ? 0 : 1];
+    auto plan = [&](uint32_t* w, int32_t* g) {
+        k_ghost_plan<<<tiles, kCgBlock, 0, c->stream>>>(sp->nRows, R, W, own, size, sp->sellCol.p, w, g,
+                                                        p.stride, p.count.p);
+        FV_LAUNCH_CHECK();
+    };
+    if (p.stride < 0) {
+        p.count.alloc(c, tiles);
         plan(nullptr, nullptr);
         std::vector<int32_t> n(tiles);
-        count.download(n.data());
-        for (int32_t v : n) stride = v > stride ? v : stride;
-        if (stride > cap) return false;
-        words.alloc(c, ((size_t)N + 63) / 64 * 64 * W / 2);
-        ghosts.alloc(c, (size_t)tiles * (stride > 0 ? stride : 1));
-        plan(words.p, ghosts.p);
-        return true;
+        p.count.download(n.data());
+        p.stride = *std::max_element(n.begin(), n.end());
     }
-};
+    if (p.stride > cap) return nullptr;
+    if (!p.words.p) {
+        p.ghosts.alloc(c, (size_t)tiles * (p.stride > 0 ? p.stride : 1));
+        p.words.alloc(c, ((size_t)sp->nRows + 63) / 64 * 64 * W / 2);
+        plan(p.words.p, p.ghosts.p);
+    }
+    return &p;
+}
+
+constexpr size_t kPersistWords = 2 * (size_t)kSlotBuffer + kMeetWords;
 
 // The exchange buffer of a system and its launches.
 struct PersistSlots {
@@ -1184,7 +1187,7 @@ struct PersistSlots {
     unsigned long long meets = 0;  // arrivals of all plain launches
     bool apart = false;            // a plain launch did not meet: cooperative from then on
     void alloc(fv_ctx* c, fv_persist_log* l) {
-        words.alloc(c, 2 * (size_t)kSlotBuffer + kMeetWords);
+        words.alloc(c, kPersistWords);
         log = l;
     }
     void clear(hipStream_t s) {  // no word carries a tag that is still to come

@@ -5,6 +5,14 @@
 
 #include <memory>
 
+// The rows of other tiles that the persistent solvers' tiles of a pattern refer to, and the
+// columns that refer to them (cgpersist.hpp).
+struct fv_ghost_plan {
+    fvhip::DBuf<uint32_t> words;
+    fvhip::DBuf<int32_t> ghosts, count;
+    int stride = -1;  // ghosts of a tile at most (-1: not counted yet)
+};
+
 // la::SparsityPattern (expression.hpp:35; test_sparsityPattern.cpp:36-62):
 // CSR of the face graph, columns ascending per row; row c is
 // [lower neighbours | c | upper neighbours] in the cell's stencil order.
@@ -29,6 +37,7 @@ struct fv_sparsity {
     int64_t sellTotal = 0;
     fvhip::DBuf<int64_t> sellOff;
     fvhip::DBuf<int32_t> sellCol, sellSrc;
+    fv_ghost_plan ghostPlan[2];  // for FP64, FP32: made by the first solver that uses it
 };
 
 // Solver workspace kept with a linear system between solves (one per precision).
@@ -62,6 +71,14 @@ struct fv_linsys {
     fv_persist_log persistLog[3];
     std::unique_ptr<fv_solver_cache> cg[3];  // FP64 CG, FP32 CG in FP64 refinement, BiCGStab
 };
+
+namespace fvhip {
+// Makes what the systems of a pattern share for fv_solve_cg in a mode (FV_SOLVE_*), for
+// owners that keep patterns and account for their memory; the bytes a system's solver needs
+// beside its vectors and its scaled matrix.
+void cg_prepare(fv_sparsity* sp, int mode);
+size_t cg_extra_bytes();
+}  // namespace fvhip
 
 #ifdef __HIPCC__
 namespace fvhip {

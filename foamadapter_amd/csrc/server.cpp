@@ -171,11 +171,12 @@ void drop_request(fv_server* s, Req* r) {
 size_t estimate_bytes(const fv_server* s, const MeshEntry& me, int kind) {
     const size_t N = me.N, F = me.F, B = me.B, nnz = me.nnz;
     const size_t e = s->opts.mode == FV_SOLVE_F32_IR ? 4 : 8;
-    size_t b = 8 * nnz + 8 * N              // linear system
+    size_t b = 8 * nnz + 8 * N + 16 * B     // linear system, its boundary coefficients
                + 8 * N * 2 + 8 * B           // x, x_old, boundary values
                + 8 * (F + B)                 // face coefficient (kappa or 1)
                + e * (size_t)me.sellTotal    // sliced-ELL matrix copy
-               + 6 * e * N + 8 * N;          // Krylov vectors, correction, FP64 residual
+               + 6 * e * N + 8 * N           // Krylov vectors, correction, FP64 residual
+               + (s->opts.batched ? 0 : cg_extra_bytes());
     if (kind == FV_REQ_POISSON) b += 24 * N + 24 * B + 8 * (F + B) + 8 * N;  // U, phi, div
     return b + (1 << 16);
 }
@@ -420,6 +421,8 @@ void worker_loop(fv_server* s) {
                 std::lock_guard<std::mutex> lk(s->qmu);
                 s->active.erase(std::find(s->active.begin(), s->active.end(), r));
                 s->gpuMs += ms_between(t1, Clock::now());
+                s->laneBytes[0] = s->ctx->in_use;  // with the solver's workspace
+                s->peakBytes = std::max(s->peakBytes, s->laneBytes[0] + s->laneBytes[1]);
             }
             try {
                 finish(s, r, status);
@@ -549,8 +552,10 @@ void solo_loop(fv_server* s) {
 // A resident mesh on context ctx from a (possibly renumbered) description:
 // device mesh, cell map, sparsity, the two boundary-condition sets and the
 // staged-gather lists.  Returns the device bytes it took.
+// solve_mode: the mode of requests solved one by one through fv_solve_cg, whose plan of the
+// pattern is made here (-1: they join the batch).
 size_t make_entry(fv_ctx* ctx, const fv_polymesh_desc* d, const std::vector<int32_t>* cmap,
-                  MeshEntry& me) {
+                  int solve_mode, MeshEntry& me) {
     const size_t used0 = ctx->in_use;
     check(fv_mesh_create_poly(ctx, d, &me.mesh));
     if (cmap) {
@@ -580,6 +585,7 @@ size_t make_entry(fv_ctx* ctx, const fv_polymesh_desc* d, const std::vector<int3
     me.B = me.mesh->nB;
     me.nnz = me.sp->nnz;
     me.sellTotal = me.sp->sellTotal;
+    if (solve_mode >= 0) cg_prepare(me.sp, solve_mode);
     return ctx->in_use - used0;
 }
 
@@ -665,14 +671,15 @@ int fv_server_add_mesh(fv_server* s, const fv_polymesh_desc* d, int renumber, in
         size_t bytes = 0;
         {
             std::lock_guard<std::mutex> g(s->gpumu);
-            bytes += make_entry(s->ctx, &r, renumber ? &cmap : nullptr, *me);
+            bytes += make_entry(s->ctx, &r, renumber ? &cmap : nullptr,
+                                s->opts.batched ? -1 : s->opts.mode, *me);
         }
         if (s->soloCtx && me->N >= s->opts.solo_rows) {
             // the solo lane runs requests on this mesh: resident there too
             auto solo = std::make_unique<MeshEntry>();
             std::lock_guard<std::mutex> g(s->solomu);
             try {
-                bytes += make_entry(s->soloCtx, &r, renumber ? &cmap : nullptr, *solo);
+                bytes += make_entry(s->soloCtx, &r, renumber ? &cmap : nullptr, s->opts.mode, *solo);
             } catch (...) {
                 destroy_entry(*solo);
                 std::lock_guard<std::mutex> g2(s->gpumu);

@@ -52,7 +52,8 @@ struct CgWork : fv_solver_cache {
     int lastLaunches = 0;  // persistent launches of the previous mixed solve
     int lastTotal = 0;     // iterations of the previous solve, in either form
     PersistSlots slots;
-    GhostPlan plan;
+    bool chosen = false;  // (or found impossible: at the first solve that may use it)
+    const fv_ghost_plan* plan = nullptr;  // null: kc_persist_far
     uint32_t tag = 1;
 
     CgWork(fv_ctx* c, fv_linsys* ls) {
@@ -104,27 +105,29 @@ struct CgWork : fv_solver_cache {
         FV_HIP(hipMemsetAsync(st.p, 0, sizeof(CgState), c->stream));
         FV_HIP(hipStreamSynchronize(c->stream));
         red = CgPartials{pq.p, rz.p, rb.p};
-        if (!c->shared) choose_persist(c, sp, tiles, R, &ls->persistLog[sizeof(S) == 8 ? 0 : 1]);
     }
 
     // The persistent kernel for this system, when there is one: slices of one
     // width, at most 8 rows per thread (2^21 rows; beyond, the vectors do not fit
     // the registers), and a device that keeps its workgroups resident together.
     // Where its buffers find no room, the system runs kernel by kernel.
-    void choose_persist(fv_ctx* c, const fv_sparsity* sp, int tiles, int R, fv_persist_log* log) {
+    void choose_persist(fv_ctx* c, fv_linsys* ls) {
+        if (chosen || c->shared) return;
+        chosen = true;
+        fv_sparsity* const sp = ls->sp;
+        const int R = grid.rowsPerBlock, tiles = grid.nTiles;
         const int rpt = (R + kB - 1) / kB;
         if (rpt > 8) return;
         const bool room = persist_room([&] {
-            slots.alloc(c, log);
+            slots.alloc(c, &ls->persistLog[sizeof(S) == 8 ? 0 : 1]);
             if (sp->sellWidth == 6)
-                choose_kernel<6>(c, tiles, R, rpt);
+                choose_kernel<6>(c, sp, rpt);
             else if (sp->sellWidth == 4)
-                choose_kernel<4>(c, tiles, R, rpt);
+                choose_kernel<4>(c, sp, rpt);
         });
         if (!room) {
             persist = nullptr;
             slots.words.release();
-            plan = GhostPlan{};
         }
         if (!persist) return;
         persistGrid = persist_grid(tiles);
@@ -145,7 +148,8 @@ struct CgWork : fv_solver_cache {
     // iterations keeps the kernel-by-kernel form (32^3 heat step of 5 iterations: 157
     // us, 178 with the iterations alone persistent, 75 whole).
     static constexpr int kPersistMin = 12;
-    bool use_persist() const {
+    bool use_persist(fv_ctx* c, fv_linsys* ls) {
+        choose_persist(c, ls);
         return persist && (whole || lastTotal == 0 || lastTotal >= kPersistMin);
     }
     // no word of the exchange carries a tag that is still to come
@@ -155,11 +159,17 @@ struct CgWork : fv_solver_cache {
     }
     // RES, the rows whose matrix stays in registers, and where g and d are, is what
     // fits the 128 registers of a 1024-thread workgroup and its LDS without spills.
+    static const fv_ghost_plan* ghosts(fv_ctx* c, fv_sparsity* sp, int tiles, int R, int W, int n) {
+        return ghost_plan(c, sp, tiles, R, W, n * kB, (int)sizeof(S),
+                          W == 6 ? ghost_cap<S>(n, 6) : ghost_cap<S>(n, 4));
+    }
+    static int kernel_rows(int rpt) { return rpt <= 1 ? 1 : rpt <= 2 ? 2 : rpt <= 4 ? 4 : 8; }
     template <int W>
-    void choose_kernel(fv_ctx* c, int tiles, int R, int rpt) {
-        const int n = rpt <= 1 ? 1 : rpt <= 2 ? 2 : rpt <= 4 ? 4 : 8;
+    void choose_kernel(fv_ctx* c, fv_sparsity* sp, int rpt) {
+        const int n = kernel_rows(rpt);
+        plan = ghosts(c, sp, grid.nTiles, grid.rowsPerBlock, W, n);
         // (more ghosts than fit: never up to 2 FP64 or 4 FP32 rows per thread)
-        if (plan.make(c, h.N, tiles, R, W, n * kB, (int)sizeof(S), ghost_cap<S>(n, W), h.sellCol)) {
+        if (plan) {
             if constexpr (sizeof(S) == 8)
                 persist = n == 1   ? kc_persist<S, 1, W, 1, 1, true, true>
                           : n == 2 ? kc_persist<S, 2, W, 2, 2, true, true>
@@ -183,8 +193,9 @@ struct CgWork : fv_solver_cache {
         const uint32_t uses = 2 * (uint32_t)persistIters + 8;
         if (tag > 0xffffffffu - uses) clear_tags(s);  // sequence numbers start over
         CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persistIters, tag, h.sellCol, h.sval,
-                       h.g, h.d, h.r, h.p, h.p2, plan.words.p, plan.ghosts.p, plan.count.p,
-                       plan.stride, h.st, slots.words.p,
+                       h.g, h.d, h.r, h.p, h.p2, plan ? plan->words.p : nullptr,
+                       plan ? plan->ghosts.p : nullptr, plan ? plan->count.p : nullptr,
+                       plan ? plan->stride : 0, h.st, slots.words.p,
                        CsrSystem{h.rowOffs, h.diag, h.vals, h.rhs}, x, tol, atol, maxit,
                        fresh ? 1 : 0, host, {}};
         if (!slots.launch(persist, persistGrid, a, whole, s)) {
@@ -717,7 +728,27 @@ bool run_mixed_persist(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, dou
     return true;
 }
 
+template <typename S>
+void prepare(fv_sparsity* sp) {
+    const int R = cg_tile_rows(sp->nRows, kB), rpt = (R + kB - 1) / kB;
+    if (rpt > 8 || !sp->sellWidth || sp->mesh->ctx->shared) return;
+    persist_room([&] {
+        CgWork<S>::ghosts(sp->mesh->ctx, sp, (sp->nRows + R - 1) / R, R, sp->sellWidth,
+                          CgWork<S>::kernel_rows(rpt));
+    });
+}
+
 }  // namespace
+
+namespace fvhip {
+void cg_prepare(fv_sparsity* sp, int mode) {
+    if (mode == FV_SOLVE_F64)
+        prepare<double>(sp);
+    else
+        prepare<float>(sp);
+}
+size_t cg_extra_bytes() { return kPersistWords * sizeof(unsigned long long); }
+}  // namespace fvhip
 
 extern "C" {
 
@@ -737,7 +768,7 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
             double tr = 0.0;
             CgState h{};
             h.res0 = -1.0;
-            if (o->eager || !w.use_persist() ||
+            if (o->eager || !w.use_persist(ctx, ls) ||
                 !run_cg_persist(ctx, w, o->rel_tol, o->max_iter, o->abs_tol, x, &tr, &h)) {
                 const CgState part = h;  // of a persistent solve that could not go on
                 w.bind(ctx, x);
@@ -760,7 +791,7 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
             const double delta = o->inner_rel_tol > 0.0 ? o->inner_rel_tol : kIrDelta;
             // max_outer counts rounds of check_every iterations: those solves run
             // kernel by kernel
-            if (o->eager || o->max_outer > 0 || !w.use_persist() ||
+            if (o->eager || o->max_outer > 0 || !w.use_persist(ctx, ls) ||
                 !run_mixed_persist(ctx, w, o->rel_tol, o->max_iter, delta, o->abs_tol, &r)) {
                 const IrOut part = r;
                 r = run_mixed(ctx, w, o->rel_tol, part.iters ? std::max(o->max_iter - part.iters, 1) : o->max_iter,

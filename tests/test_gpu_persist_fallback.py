@@ -174,3 +174,27 @@ def test_no_room_for_the_persistent_buffers(method):
                 rest.close()
             m.close()
     _same(out[1], out[0])
+
+
+def test_systems_of_one_pattern_share_the_plan(ctx):
+    """What depends on the pattern alone is made once: a second system takes less memory than
+    the first, and the BiCGStab of a third uses what the CG made."""
+    from foamadapter_amd import la
+    m, ls = _system(ctx, (64, 64, 40))
+    x = ctx.uniform(m.n_cells, -1, 1, 12, 4)
+    took = []
+    for method in ("double", "double", "bicgstab"):
+        two = la.LinearSystem(ls.sp)
+        from foamadapter_amd._lib import call, lib
+        call("fv_memcpy_d2d", ctx.handle, lib.fv_linsys_values(two.handle), lib.fv_linsys_values(ls.handle), 8 * ls.sp.nnz)
+        call("fv_memcpy_d2d", ctx.handle, lib.fv_linsys_rhs(two.handle), lib.fv_linsys_rhs(ls.handle), 8 * m.n_cells)
+        used = ctx.bytes_in_use
+        opts = {"solver": "PBiCGStab"} if method == "bicgstab" else {}
+        la.solve_cg(two, x, dict(opts, relTol=1e-3, maxIter=2000))
+        assert _counts(two, method)["launches"] >= 1
+        took.append(ctx.bytes_in_use - used)
+        two.close()
+    vectors = 8 * 13 * m.n_cells  # of either solver, with its scaled matrix
+    assert took[0] >= vectors + 12 * m.n_cells
+    assert took[1] <= vectors + (1 << 18) and took[2] <= vectors + (1 << 18)
+    m.close()

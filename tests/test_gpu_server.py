@@ -237,3 +237,21 @@ def test_failures_and_cancellation(polys):
     assert st0.status == 0 and st1.status == 0 and st2.status == 6   # FV_ECANCELLED
     assert srv.stats()["cancelled"] == 1
     srv.close()
+
+
+@pytest.mark.parametrize("precision", ["double", "mixed"])
+def test_plain_requests_stay_within_their_estimate(precision):
+    """Requests solved one by one: what the server counts (resident meshes and the estimate of
+    the request in flight) covers what the device holds, the solver's workspace included."""
+    import foamadapter_amd as fa
+    from foamadapter_amd.serve import HEAT, POISSON
+    print(precision, flush=True)
+    srv, ids = _server([fa.PolyMesh.hex(40, jitter=0.2, jitter_seed=1, perm_seed=2)], batched=False,
+                       precision=precision)
+    for kind, submit in ((HEAT, lambda: srv.submit_heat(ids[0], kappa=1e-2, steps=2, seed=1)),
+                         (POISSON, lambda: srv.submit_poisson(ids[0], seed=1))):
+        assert srv.wait(submit())[1].status == 0
+        s = srv.stats()
+        print(s["peak_bytes"], s["resident_bytes"], srv.request_bytes(ids[0], kind), flush=True)
+        assert s["peak_bytes"] <= s["resident_bytes"] + srv.request_bytes(ids[0], kind)
+    srv.close()

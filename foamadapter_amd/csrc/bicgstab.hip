@@ -648,7 +648,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist(BiPersist A) {
                 residual([&](uint32_t o) { return get_shared(at_byte(A.x, o)); },
                          [&](int, bool, double ri, double, const double (&)[W],
                              const uint32_t (&)[W]) { s1[0] += ri * ri; });
-                ok = gs.sum<1, false>(s1, all, L);
+                ok = gs.sum<1, false, true>(s1, all, L);
                 trueRes = sqrt(all[0]) / bnorm;
             }
         }
@@ -983,7 +983,7 @@ __global__ __launch_bounds__(kPersistThreads) void kbi_persist_far(BiPersist A) 
                 residual([&](uint32_t o) { return get_shared(at_byte(A.x, o)); },
                          [&](int, bool, double ri, double, const double (&)[W],
                              const uint32_t (&)[W]) { s1[0] += ri * ri; });
-                ok = gs.sum<1, false>(s1, all, L);
+                ok = gs.sum<1, false, true>(s1, all, L);
                 trueRes = sqrt(all[0]) / bnorm;
             }
         }
@@ -1152,6 +1152,7 @@ struct BiWork : fv_solver_cache {
     // device refuses a launch or one is lost: h.it iterations are in x then (ncomp 1).
     bool finish_persist(fv_ctx* c, const Target& t, const fv_solve_opts* o, BiState& h) {
         bool fresh = true;
+        h.lost |= slots.doubted;
         while (!h.lost && (!h.stop || h.stop == kStopApart)) {
             if (h.stop == kStopApart) {  // nothing done: the same launch, cooperative
                 slots.did_not_meet();
@@ -1161,6 +1162,7 @@ struct BiWork : fv_solver_cache {
             }
             if (!run_persist(c->stream, t, o, fresh)) break;
             h = states(c, t.comp + 1)[t.comp];
+            h.lost |= slots.doubted;
         }
         if (h.lost) {
             ++slots.log->lost;

@@ -92,9 +92,8 @@ struct CsrSystem {
 // What PersistSlots::launch says of a launch.
 struct PersistLaunch {
     unsigned long long meet;  // Meeting::target
-    uint32_t fails;           // exchange workgroups 8 to 15 are missing from (0: none; for
-                              // tests, where a wait ends after kFailSeconds; p.q or the
-                              // result's residual)
+    uint32_t fails;           // exchange of the result's residual, if workgroups 8 to 15 are
+                              // to miss it and the waits to end after kFailSeconds (tests)
 };
 
 // Arguments by value: the kernel reads them from scalar registers instead of
@@ -197,8 +196,8 @@ __device__ __forceinline__ double from_lane(double x, int lane) {
 struct PersistLds {
     double wave[4][kPersistThreads / 64];  // wave sums of this workgroup's tiles
     double tot[2][4];                      // by parity of the exchange: the grid's sums
-    // PersistLaunch's, and how long a wait may last in 65536 clocks: no registers are left
-    // for them in the loop (spills: 128^3 FP32 14.8 -> 15.2 us)
+    // PersistLaunch's, and how long a wait may last in 65536 clocks (as constants or in
+    // scalar registers they cost the loops registers they do not have)
     uint32_t fails, limit;
     int bad, met;
     __device__ void begin(const PersistLaunch& a) {  // one thread, before the first barrier
@@ -273,8 +272,9 @@ struct GridSum {
 
     // The sum over the grid of every thread's v[], in the order of write_slot
     // and sum_slots.  PUBLISHED: this wave's put_shared stores are complete for
-    // every workgroup once it returns.  False after a timed-out wait.
-    template <int NV, bool PUBLISHED>
+    // every workgroup once it returns.  LAST: the launch's last.  False after a timed-out
+    // wait.
+    template <int NV, bool PUBLISHED, bool LAST = false>
     __device__ bool sum(double (&v)[NV], double (&tot)[NV], PersistLds& L) {
         const int tid = (int)threadIdx.x, lane = tid & 63, wid = tid >> 6;
         for (int j = 0; j < NV; ++j) v[j] = lane_sum<32>(v[j]);
@@ -296,9 +296,7 @@ struct GridSum {
                              p2 = from_lane(part, 2), p3 = from_lane(part, 3);
                 a[j] = large ? ((p0 + p1) + p2) + p3 : (p0 + p2) + (p1 + p3);
             }
-            // (only where this is asked, and the BiCGStab's loop has no register for it)
-            const bool there = NV > 1 || PUBLISHED || tag != L.fails || slot >> 3 != 1;
-            if (lane == 0 && there)
+            if (lane == 0 && (!LAST || tag != L.fails || slot >> 3 != 1))
                 for (int j = 0; j < NV; ++j)
                     publish(buf + (size_t)slot * kSlotWords + 2 * j, a[j], tag);
             bool ok = true;
@@ -868,7 +866,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
                 residual([&](uint32_t o) { return get_shared(at_byte(A.x, o)); },
                          [&](int, bool, double ri, double, const double (&)[W],
                              const uint32_t (&)[W]) { s1[0] += ri * ri; });
-                ok = gs.sum<1, false>(s1, all, L);
+                ok = gs.sum<1, false, true>(s1, all, L);
                 rrep = sqrt(all[0]) / bnorm;
             }
         }
@@ -1186,6 +1184,7 @@ struct PersistSlots {
     fv_persist_log* log = nullptr;
     unsigned long long meets = 0;  // arrivals of all plain launches
     bool apart = false;            // a plain launch did not meet: cooperative from then on
+    bool doubted = false;          // the latest launch's state is to be taken for lost (tests)
     void alloc(fv_ctx* c, fv_persist_log* l) {
         words.alloc(c, kPersistWords);
         log = l;
@@ -1202,7 +1201,8 @@ struct PersistSlots {
         const bool plain = meeting && !apart;
         args.launch = PersistLaunch{plain ? meets + grid : 0, 0};
         if (fault == FV_PERSIST_APART && plain) ++args.launch.meet;  // never reached
-        if (fault == FV_PERSIST_LOST) args.launch.fails = args.tag0 + (uint32_t)log->exchange;
+        doubted = fault == FV_PERSIST_LOST && !log->exchange;
+        if (fault == FV_PERSIST_LOST && log->exchange) args.launch.fails = args.tag0 + (uint32_t)log->exchange;
         void* a[] = {&args};
         const void* const k = reinterpret_cast<const void*>(kernel);
         hipError_t e = hipErrorUnknown;

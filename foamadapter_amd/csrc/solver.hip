@@ -207,7 +207,7 @@ struct CgWork : fv_solver_cache {
     }
     // Whether a launch lost its workgroups; this system's solves run kernel by kernel then.
     bool lost(const CgState& h) {
-        if (!h.lost) return false;
+        if (!h.lost && !slots.doubted) return false;
         ++slots.log->lost;
         persist = nullptr;
         return true;
@@ -511,10 +511,10 @@ bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, doubl
         h = w.state2(s, &t);
         haveTrue = h.stop != 0;
     }
-    if (!h.stop && !h.lost) {
+    if (!h.stop && !h.lost && !w.slots.doubted) {
         PollPipe pp{static_cast<CgState*>(ctx_poll_host(ctx)), ctx};
         pp.push(s, w.st.p);
-        while (!h.stop && !h.lost) {
+        while (!h.stop && !h.lost && !w.slots.doubted) {
             while (!refused && pp.npend < 2) {
                 refused = !w.run_persist(s);
                 if (!refused) pp.push(s, w.st.p);
@@ -702,7 +702,7 @@ bool run_mixed_persist(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, dou
     };
     if (!round()) return false;
     CgState h{};
-    auto done = [&] { return h.stop >= 2 || h.it >= maxit || h.lost; };
+    auto done = [&] { return h.stop >= 2 || h.it >= maxit || h.lost || w.slots.doubted; };
     if (w.lastLaunches > 0) {
         while (rounds < w.lastLaunches && round()) {
         }

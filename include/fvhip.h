@@ -438,9 +438,10 @@ int fv_solve_bicgstab_vec(fv_linsys* ls, int ncomp, const void* d_rhs, void* d_x
  * other (both go on kernel by kernel, from the x there is). */
 int fv_linsys_persist_counts(const fv_linsys* ls, int solver, int64_t* h_counts4);
 /* Makes one of these happen to the launch after the next `after` ones, for tests of what
- * follows: FV_PERSIST_LOST at the launch's exchange number `exchange` (from 0; one that
- * sums p.q or the result's residual), to which some workgroups bring nothing; the waits end
- * after 5 ms and every workgroup by itself. */
+ * follows: FV_PERSIST_LOST with `exchange` the number (from 0) of the launch's last
+ * exchange, the result's residual, to which some workgroups bring nothing then (the waits
+ * end after 5 ms and every workgroup by itself), or 0: the launch runs, and its state is
+ * taken for that of a lost one. */
 enum { FV_PERSIST_APART = 1, FV_PERSIST_REFUSED = 2, FV_PERSIST_LOST = 3 };
 int fv_linsys_persist_fault(fv_linsys* ls, int solver, int fault, int after, int exchange);
 

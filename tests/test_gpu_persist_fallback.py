@@ -99,16 +99,12 @@ CASES = [("double", ONE, 0), ("double", MANY, 0), ("double", MANY, 1), ("double"
 @pytest.mark.parametrize("method,dims,after", CASES, ids=str)
 def test_a_solve_goes_on_kernel_by_kernel(ctx, method, dims, after, fault):
     """After a first launch, x of a system without whole solves holds that launch's
-    iterations, and the solve goes on from there: its own count, the same tolerance.  A
-    BiCGStab launch is lost at its last exchange, when x is written."""
-    if fault == "lost" and method == "bicgstab" and (dims, after) != (ONE, 0):
-        pytest.skip("its launches of several have no exchange to lose")
+    iterations, and the solve goes on from there: its own count, the same tolerance.  (Lost:
+    the host takes a launch's state for that of a lost one.)"""
     print(method, dims, after, fault, flush=True)
     m, ls = _system(ctx, dims)
     ref = _solve(ctx, m, ls, method, graph=False)
-    whole = method == "double" and dims != LARGE
-    exchange = 3 * ref[1].numIter + 2 if method == "bicgstab" else 3 if whole and after == 0 else 2
-    _fault(ls, method, REFUSED if fault == "refused" else LOST, after, exchange)
+    _fault(ls, method, REFUSED if fault == "refused" else LOST, after)
     got = _solve(ctx, m, ls, method)
     c = _counts(ls, method)
     assert c[fault] == 1 and sum(c.values()) == c["launches"] + 1
@@ -116,11 +112,10 @@ def test_a_solve_goes_on_kernel_by_kernel(ctx, method, dims, after, fault):
     res = np.linalg.norm(b - A @ got[0]) / np.linalg.norm(b)
     # the CG recurrence estimates the residual: its bound is that of the reference's
     assert res <= max(1.01e-8, 2 * ref[1].trueResNorm) and abs(got[1].trueResNorm - res) <= 1e-10
-    if method == "bicgstab" and fault == "lost":
-        return
-    assert got[1].initResNorm == ref[1].initResNorm
-    if after == 0 or whole:
-        _same(got, ref)
+    if fault == "refused" or dims == MANY and (after or method == "double"):
+        assert got[1].initResNorm == ref[1].initResNorm
+    if method == "double" and dims == MANY or fault == "refused" and after == 0:
+        _same(got, ref)  # x was not written before
     _, later = _solve(ctx, m, ls, method)  # kernel by kernel
     assert later.finalResNorm <= 1e-8 and _counts(ls, method) == c
     m.close()

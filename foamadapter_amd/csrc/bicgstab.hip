@@ -1054,7 +1054,10 @@ struct BiWork : fv_solver_cache {
                 choose_kernel<6>(c, sp, rpt);
             else if (sp->sellWidth == 4)
                 choose_kernel<4>(c, sp, rpt);
+            if (persist) grow(sval, c, sp->uniTotal());
         });
+        h.sval = sval.p;
+        sellCol = uniform_col(sp);
         if (!room) {
             persist = nullptr;
             slots.words.release();
@@ -1088,7 +1091,7 @@ struct BiWork : fv_solver_cache {
         double* const x = t.x + t.comp;
         BiState* const state = st.p + t.comp;
         BiPersist a{h.N, h.ntiles, h.rowsPerBlock, persistIters, fresh ? 1 : 0, o->max_iter, tag,
-                    o->rel_tol, o->abs_tol, h.sellCol, CsrSystem{h.rowOffs, diag, h.vals, t.rhs + t.comp},
+                    o->rel_tol, o->abs_tol, sellCol, CsrSystem{h.rowOffs, diag, h.vals, t.rhs + t.comp},
                     t.ncomp, x, t.ncomp > 1 ? x : nullptr, chained ? state - 1 : nullptr, sval.p,
                     t.ncomp > 1 ? dinv.p : x, h.r, h.rhat, h.p, h.v, h.t, h.s, plan ? plan->words.p : nullptr,
                     plan ? plan->ghosts.p : nullptr, plan ? plan->count.p : nullptr,
@@ -1103,6 +1106,7 @@ struct BiWork : fv_solver_cache {
         return true;
     }
     const int32_t* diag = nullptr;
+    const int32_t* sellCol = nullptr;  // slices of one width (persistent)
     BiWork(fv_ctx* c, fv_linsys* ls) {
         const fv_sparsity* sp = ls->sp;
         const int N = sp->nRows;

@@ -1149,14 +1149,28 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist_far(CgPersist<S> A
     }
 }
 
+inline const int32_t* uniform_col(const fv_sparsity* sp) {
+    return sp->sellUniform ? sp->sellCol.p : sp->uniCol.p;
+}
+
+// A buffer of at least n elements; the one there is stays if there is no room for another.
+template <typename T>
+inline void grow(DBuf<T>& b, fv_ctx* c, size_t n) {
+    if (b.n >= n) return;
+    DBuf<T> larger;
+    larger.alloc(c, n);
+    b = std::move(larger);
+}
+
 // The ghosts of a pattern's tiles for values of `size` bytes (own: rows a tile has places
 // for); null if a tile has more than cap.  The plan stays with the pattern: its systems and
 // solvers have the same tiles (cg_tile_rows), so one per value size serves them all.
 inline const fv_ghost_plan* ghost_plan(fv_ctx* c, fv_sparsity* sp, int tiles, int R, int W, int own,
                                        int size, int cap) {
     fv_ghost_plan& p = sp->ghostPlan[size == 8 ? 0 : 1];
+    uniform_sell(sp);
     auto plan = [&](uint32_t* w, int32_t* g) {
-        k_ghost_plan<<<tiles, kCgBlock, 0, c->stream>>>(sp->nRows, R, W, own, size, sp->sellCol.p, w, g,
+        k_ghost_plan<<<tiles, kCgBlock, 0, c->stream>>>(sp->nRows, R, W, own, size, uniform_col(sp), w, g,
                                                         p.stride, p.count.p);
         FV_LAUNCH_CHECK();
     };

@@ -400,6 +400,20 @@ __global__ __launch_bounds__(kBlock) void k_residual(int N, const int32_t* __res
     res[r] = s - bi;
 }
 
+// slices of width W from those as wide as their longest row
+__global__ __launch_bounds__(kBlock) void k_uniform_sell(int N, int W, const int64_t* __restrict__ off,
+                                                         const int32_t* __restrict__ col,
+                                                         int64_t* __restrict__ uniOff,
+                                                         int32_t* __restrict__ uniCol) {
+    const int i = blockIdx.x * kBlock + threadIdx.x, l = i & 63, s = i >> 6;
+    if (i == 0) uniOff[0] = 0;
+    if (s >= (N + 63) >> 6) return;
+    const int64_t b = off[s], u = (int64_t)s * 64 * W;
+    const int w = (int)((off[s + 1] - b) >> 6);
+    for (int k = 0; k < W; ++k) uniCol[u + 64 * k + l] = k < w ? col[b + 64 * k + l] : min(i, N - 1);
+    if (l == 0) uniOff[s + 1] = u + 64 * W;
+}
+
 fv_mesh* mesh_of(const fv_linsys* ls) { return ls->sp->mesh; }
 
 void check_ls(const fv_linsys* ls) { FV_REQUIRE(ls && ls->sp && ls->sp->mesh, "NULL linear system"); }
@@ -422,6 +436,19 @@ HeatDesc heat_desc(fv_linsys* ls, const double* Told, double dt, const double* g
 }
 
 }  // namespace
+
+namespace fvhip {
+void uniform_sell(fv_sparsity* sp) {
+    if (sp->sellUniform || sp->uniCol.p) return;
+    fv_ctx* const c = sp->mesh->ctx;
+    const int nS = (sp->nRows + 63) / 64;
+    sp->uniOff.alloc(c, (size_t)nS + 1);
+    sp->uniCol.alloc(c, (size_t)sp->uniTotal());
+    k_uniform_sell<<<grid_for(64 * (int64_t)nS, kBlock), kBlock, 0, c->stream>>>(
+        sp->nRows, sp->sellWidth, sp->sellOff.p, sp->sellCol.p, sp->uniOff.p, sp->uniCol.p);
+    FV_LAUNCH_CHECK();
+}
+}  // namespace fvhip
 
 extern "C" {
 
@@ -492,12 +519,22 @@ int fv_sparsity_create(fv_mesh* m, fv_sparsity** out) {
         const int64_t C = fv_sparsity::kSlice, nS = (N + C - 1) / C;
         int32_t widest = 0;
         for (int64_t r = 0; r < N; ++r) widest = std::max(widest, rowOffs[r + 1] - rowOffs[r] - 1);
-        sp->sellWidth = widest <= 4 ? 4 : widest <= 6 ? 6 : 0;
+        sp->sellWidth = N > fv_sparsity::kUniformRows ? 0 : widest <= 4 ? 4 : widest <= 6 ? 6 : 0;
+        if (sp->sellWidth) {
+            int64_t own = 0;
+            for (int64_t s = 0; s < nS; ++s) {
+                int32_t w = 0;
+                for (int64_t r = s * C; r < std::min<int64_t>(N, (s + 1) * C); ++r)
+                    w = std::max(w, rowOffs[r + 1] - rowOffs[r] - 1);
+                own += C * w;
+            }
+            sp->sellUniform = 20 * sp->uniTotal() <= 21 * own;
+        }
         auto sliced = [&](fvhip::DBuf<int64_t>& offOut, fvhip::DBuf<int32_t>& colOut,
                           fvhip::DBuf<int32_t>& srcOut) -> int64_t {
             std::vector<int64_t> soff(nS + 1, 0);
             for (int64_t s = 0; s < nS; ++s) {
-                int32_t wmax = sp->sellWidth;
+                int32_t wmax = sp->sellUniform ? sp->sellWidth : 0;
                 for (int64_t r = s * C; r < std::min<int64_t>(N, (s + 1) * C); ++r)
                     wmax = std::max(wmax, rowOffs[r + 1] - rowOffs[r] - 1);
                 soff[s + 1] = soff[s] + C * wmax;

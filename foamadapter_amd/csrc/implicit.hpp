@@ -29,14 +29,22 @@ struct fv_sparsity {
     // wavefront each; entry k of row 64s+l at sellOff[s] + 64k + l): column and
     // source CSR index (-1 for padding)
     static constexpr int kSlice = 64;
-    // When no row has more than 6 off-diagonal entries (hexahedra) every slice has
-    // the same width, 4 or 6: entry k of row i is at (i / 64) * 64 w + 64 k + i % 64
-    // and the persistent CG reads it without slice offsets.  0: slices as wide as
-    // their longest row.
-    int32_t sellWidth = 0;
     int64_t sellTotal = 0;
     fvhip::DBuf<int64_t> sellOff;
     fvhip::DBuf<int32_t> sellCol, sellSrc;
+    // The persistent solvers read slices of one width, 4 or 6 (sellWidth; 0: a row has more
+    // off-diagonal entries, or there are more rows than they take), without their offsets:
+    // entry k of row i at (i / 64) * 64 w + 64 k + i % 64.  Where that makes the slices no
+    // more than 5 % larger (hexahedra: those at the mesh's sides), all slices have that
+    // width.  Else (triangles 3 of 4, prisms 5 of 6) they are as wide as their longest row,
+    // for the solvers that stream them, and the first persistent solver makes these
+    // (uniform_sell).
+    static constexpr int64_t kUniformRows = 1 << 21;
+    int32_t sellWidth = 0;
+    bool sellUniform = false;
+    fvhip::DBuf<int64_t> uniOff;
+    fvhip::DBuf<int32_t> uniCol;
+    int64_t uniTotal() const { return ((int64_t)nRows + kSlice - 1) / kSlice * kSlice * sellWidth; }
     fv_ghost_plan ghostPlan[2];  // for FP64, FP32: made by the first solver that uses it
 };
 
@@ -77,6 +85,8 @@ namespace fvhip {
 // owners that keep patterns and account for their memory; the bytes a system's solver needs
 // beside its vectors and its scaled matrix.
 void cg_prepare(fv_sparsity* sp, int mode);
+// The slices of width sellWidth (> 0), made on first use unless the others are such.
+void uniform_sell(fv_sparsity* sp);
 size_t cg_extra_bytes();
 }  // namespace fvhip
 

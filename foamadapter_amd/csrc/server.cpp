@@ -585,7 +585,10 @@ size_t make_entry(fv_ctx* ctx, const fv_polymesh_desc* d, const std::vector<int3
     me.B = me.mesh->nB;
     me.nnz = me.sp->nnz;
     me.sellTotal = me.sp->sellTotal;
-    if (solve_mode >= 0) cg_prepare(me.sp, solve_mode);
+    if (solve_mode >= 0) {
+        cg_prepare(me.sp, solve_mode);
+        me.sellTotal = std::max(me.sellTotal, me.sp->uniTotal());
+    }
     return ctx->in_use - used0;
 }
 

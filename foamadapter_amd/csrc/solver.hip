@@ -33,7 +33,7 @@ struct CgWork : fv_solver_cache {
     DBuf<double> r64, pq, rz, rb;
     DBuf<CgState> st, st2;
     DBuf<CgSys<S>> sys;
-    CgSys<S> h{};
+    CgSys<S> h{}, hu{};  // hu: with the slices of one width (persistent)
     CgGrid<S> grid{};
     DBuf<CgGrid<S>> gdev;  // device copy of grid (the kernels' launch description)
     CgPartials red{};
@@ -124,7 +124,14 @@ struct CgWork : fv_solver_cache {
                 choose_kernel<6>(c, sp, rpt);
             else if (sp->sellWidth == 4)
                 choose_kernel<4>(c, sp, rpt);
+            if (persist && !(sizeof(S) == 8 && rpt <= 2)) grow(sval, c, sp->uniTotal());  // (not whole)
         });
+        h.sval = sval.p;
+        hu = h;
+        if (!sp->sellUniform) {
+            hu.sellOff = sp->uniOff.p;
+            hu.sellCol = sp->uniCol.p;
+        }
         if (!room) {
             persist = nullptr;
             slots.words.release();
@@ -192,7 +199,7 @@ struct CgWork : fv_solver_cache {
                      int maxit = 0, bool fresh = false, CgState* host = nullptr) {
         const uint32_t uses = 2 * (uint32_t)persistIters + 8;
         if (tag > 0xffffffffu - uses) clear_tags(s);  // sequence numbers start over
-        CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persistIters, tag, h.sellCol, h.sval,
+        CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persistIters, tag, hu.sellCol, h.sval,
                        h.g, h.d, h.r, h.p, h.p2, plan ? plan->words.p : nullptr,
                        plan ? plan->ghosts.p : nullptr, plan ? plan->count.p : nullptr,
                        plan ? plan->stride : 0, h.st, slots.words.p,
@@ -223,10 +230,11 @@ struct CgWork : fv_solver_cache {
 
     // Binds the solution vector (the device copy of the system description
     // the kernels read).
-    void bind(fv_ctx* c, double* x) {
-        h.x = x;
-        h.xold = nullptr;
-        FV_HIP(hipMemcpyAsync(sys.p, &h, sizeof h, hipMemcpyHostToDevice, c->stream));
+    void bind(fv_ctx* c, double* x, bool uniform = false) {
+        CgSys<S>& b = uniform ? hu : h;
+        b.x = x;
+        b.xold = nullptr;
+        FV_HIP(hipMemcpyAsync(sys.p, &b, sizeof b, hipMemcpyHostToDevice, c->stream));
     }
     // Runs enqueue() -- kernel launches only, whose by-value arguments `key`
     // determines -- eagerly until the same key has come kCaptureAfter times in
@@ -499,7 +507,7 @@ bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, doubl
         *true_res = out->rrep;
         return true;
     }
-    w.bind(ctx, x);
+    w.bind(ctx, x, true);
     w.start(s, tol, maxit, 0.0, atol);
     if (!w.run_persist(s)) return false;
     CgState h{}, t{};
@@ -687,8 +695,9 @@ IrOut run_mixed(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, int chunk,
 // lost: out->iters iterations, of which x holds those up to the last replacement, and
 // out->init_res as run_cg_persist.
 bool run_mixed_persist(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, double delta,
-                       double atol, IrOut* out) {
+                       double atol, double* x, IrOut* out) {
     hipStream_t s = ctx->stream;
+    w.bind(ctx, x, true);
     w.start(s, tol, maxit, delta, atol);
     int rounds = 0;
     bool refused = false;
@@ -786,14 +795,14 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
             local.true_res = tr;
         } else if (o->mode == FV_SOLVE_F32_IR) {
             CgWork<float>& w = work_of<float>(ls, true);
-            w.bind(ctx, x);
             IrOut r{-1.0, 0.0, 0.0, 0, 0};
             const double delta = o->inner_rel_tol > 0.0 ? o->inner_rel_tol : kIrDelta;
             // max_outer counts rounds of check_every iterations: those solves run
             // kernel by kernel
             if (o->eager || o->max_outer > 0 || !w.use_persist(ctx, ls) ||
-                !run_mixed_persist(ctx, w, o->rel_tol, o->max_iter, delta, o->abs_tol, &r)) {
+                !run_mixed_persist(ctx, w, o->rel_tol, o->max_iter, delta, o->abs_tol, x, &r)) {
                 const IrOut part = r;
+                w.bind(ctx, x);
                 r = run_mixed(ctx, w, o->rel_tol, part.iters ? std::max(o->max_iter - part.iters, 1) : o->max_iter,
                               o->check_every > 0 ? o->check_every : 64, delta,
                               o->max_outer > 0 ? o->max_outer : (1 << 30), o->abs_tol,

@@ -129,3 +129,69 @@ def refined_block(m=3):
                     face_points=np.array([v for r in order for v in r[0]], np.int32),
                     owner=np.array([r[1] for r in order], np.int32),
                     neighbour=np.array([r[2] for r in internal], np.int32), patches=patches)
+
+
+def prism_block(nx, ny, nz):
+    """The unit-spaced nx x ny x nz block, each hexahedron cut into two prisms along the diagonal
+    of its z-faces: cells with 5 neighbours (3 in a plane mesh, nz = 1, whose z-patch is empty).
+    Patches: sides (x and y) and ends (z)."""
+    I, J, K = (a.ravel(order="F") for a in np.meshgrid(*(np.arange(n) for n in (nx, ny, nz)), indexing="ij"))
+
+    def P(i, j, k):
+        return i + (nx + 1) * (j + (ny + 1) * k)
+
+    def cell(i, j, k, t):
+        return 2 * (i + nx * (j + ny * k)) + t
+
+    pts = np.stack([a.ravel(order="F") for a in np.meshgrid(
+        *(np.arange(n + 1.0) for n in (nx, ny, nz)), indexing="ij")], axis=1)
+    recs = []  # vertices [n, 4] (-1: none), owner, neighbour (-1: boundary), patch
+
+    def add(verts, own, nbr, patch):
+        v = np.stack([np.broadcast_to(a, own.shape) for a in verts], axis=1)
+        if v.shape[1] == 3:
+            v = np.concatenate([v, np.full((len(v), 1), -1)], axis=1)
+        recs.append((v, own, np.where(nbr >= 0, nbr, -1), np.where(nbr >= 0, -1, patch)))
+
+    # t = 0 holds the corners (0,0) (1,0) (1,1) of its square, t = 1 (0,0) (1,1) (0,1)
+    def upright(a, b):  # the side over the edge a-b
+        (ai, aj), (bi, bj) = a, b
+        return [P(I + ai, J + aj, K), P(I + bi, J + bj, K), P(I + bi, J + bj, K + 1), P(I + ai, J + aj, K + 1)]
+
+    none = np.full(I.shape, -1)
+    add(upright((0, 0), (1, 1)), cell(I, J, K, 0), cell(I, J, K, 1), 0)
+    add(upright((1, 0), (1, 1)), cell(I, J, K, 0), np.where(I + 1 < nx, cell(I + 1, J, K, 1), -1), 0)
+    add(upright((0, 1), (1, 1)), cell(I, J, K, 1), np.where(J + 1 < ny, cell(I, J + 1, K, 0), -1), 0)
+    for mask, edge, t in ((I == 0, ((0, 0), (0, 1)), 1), (J == 0, ((0, 0), (1, 0)), 0)):
+        v, own = upright(*edge), cell(I, J, K, t)
+        recs.append((np.stack(v, axis=1)[mask], own[mask], none[mask], 0 * none[mask]))
+    for t, tri in ((0, ((0, 0), (1, 0), (1, 1))), (1, ((0, 0), (1, 1), (0, 1)))):
+        top = [P(I + a, J + b, K + 1) for a, b in tri]
+        add(top, cell(I, J, K, t), np.where(K + 1 < nz, cell(I, J, K + 1, t), -1), 1)
+        low = np.stack([P(I + a, J + b, K) for a, b in tri] + [none], axis=1)
+        m = K == 0
+        recs.append((low[m], cell(I, J, K, t)[m], none[m], 0 * none[m] + 1))
+    v, own, nbr, patch = (np.concatenate(c) for c in zip(*recs))
+    swap = (nbr >= 0) & (nbr < own)
+    own, nbr = np.where(swap, nbr, own), np.where(swap, own, nbr)
+    # orient: area vector from owner to neighbour (outward on the boundary)
+    cent = np.zeros((2 * nx * ny * nz, 3))
+    cent[cell(I, J, K, 0)] = np.stack([I + 2 / 3, J + 1 / 3, K + 0.5], axis=1)
+    cent[cell(I, J, K, 1)] = np.stack([I + 1 / 3, J + 2 / 3, K + 0.5], axis=1)
+    tri = v[:, 3] < 0
+    a, b, c = pts[v[:, 0]], pts[v[:, 1]], pts[v[:, 2]]
+    back = np.einsum("ij,ij->i", np.cross(b - a, c - a), a - cent[own]) < 0
+    v[back & ~tri] = v[back & ~tri][:, ::-1]
+    v[back & tri, :3] = v[back & tri, :3][:, ::-1]
+    inner = np.nonzero(nbr >= 0)[0]
+    inner = inner[np.lexsort((nbr[inner], own[inner]))]
+    order, patches = [inner], []
+    for p, name in enumerate(("sides", "ends")):
+        f = np.nonzero(patch == p)[0]
+        patches.append(Patch(name, "empty" if nz == 1 and p == 1 else "wall", sum(map(len, order)), len(f)))
+        order.append(f)
+    order = np.concatenate(order)
+    v = v[order]
+    return PolyMesh(points=pts, face_offsets=np.concatenate([[0], np.cumsum((v >= 0).sum(1))]).astype(np.int32),
+                    face_points=v[v >= 0].astype(np.int32), owner=own[order].astype(np.int32),
+                    neighbour=nbr[inner].astype(np.int32), patches=patches)

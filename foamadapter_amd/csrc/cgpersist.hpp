@@ -455,6 +455,9 @@ __global__ __launch_bounds__(kCgBlock) void k_ghost_plan(int N, int R, int W, in
 // decision, 2 * tag + 1 (all have arrived) or 2 * tag (one gave up).  The first to
 // decide wins, so every workgroup sees the same decision, late ones included.
 constexpr int kMeetWords = 32;
+// Launches after a missed meeting that do not try one: as many as lose together, at 17 us
+// each, what another miss would cost.
+constexpr int kApartLaunches = 128;
 constexpr unsigned long long kMeetClocks = (unsigned long long)(kClockHz / 500);  // 2 ms
 struct Meeting {
     unsigned long long* words;
@@ -1197,7 +1200,7 @@ struct PersistSlots {
     DBuf<unsigned long long> words;
     fv_persist_log* log = nullptr;
     unsigned long long meets = 0;  // arrivals of all plain launches
-    bool apart = false;            // a plain launch did not meet: cooperative from then on
+    int apart = 0;                 // launches that are to be cooperative, after one that did not meet
     bool doubted = false;          // the latest launch's state is to be taken for lost (tests)
     void alloc(fv_ctx* c, fv_persist_log* l) {
         words.alloc(c, kPersistWords);
@@ -1212,7 +1215,8 @@ struct PersistSlots {
     template <typename Args>
     bool launch(void (*kernel)(Args), int grid, Args& args, bool meeting, hipStream_t s) {
         const int fault = log->take();
-        const bool plain = meeting && !apart;
+        const bool plain = meeting && apart == 0;
+        if (meeting && apart > 0) --apart;
         args.launch = PersistLaunch{plain ? meets + grid : 0, 0};
         if (fault == FV_PERSIST_APART && plain) ++args.launch.meet;  // never reached
         doubted = fault == FV_PERSIST_LOST && !log->exchange;
@@ -1233,7 +1237,7 @@ struct PersistSlots {
         return true;
     }
     void did_not_meet() {
-        apart = true;
+        apart = kApartLaunches;
         ++log->apart;
     }
 };

@@ -68,6 +68,22 @@ def test_a_plain_launch_that_does_not_meet(ctx, dims, after, method):
     m.close()
 
 
+def test_plain_launches_are_tried_again(ctx):
+    """After a miss 128 launches are cooperative ones, which cannot miss; the next is plain."""
+    m, ls = _system(ctx, (3, 3, 3))
+    ref = _solve(ctx, m, ls, "double", graph=False)
+    _fault(ls, "double", APART)
+    for i in range(128):
+        if i == 127:
+            _fault(ls, "double", APART)  # of no effect on the last cooperative one
+        _same(_solve(ctx, m, ls, "double"), ref)
+    assert _counts(ls, "double") == {"launches": 129, "apart": 1, "refused": 0, "lost": 0}
+    _fault(ls, "double", APART)
+    _same(_solve(ctx, m, ls, "double"), ref)
+    assert _counts(ls, "double") == {"launches": 131, "apart": 2, "refused": 0, "lost": 0}
+    m.close()
+
+
 @pytest.mark.parametrize("after", [0, 1, 2])
 def test_a_component_whose_launch_does_not_meet(ctx, after):
     import foamadapter_amd as fa

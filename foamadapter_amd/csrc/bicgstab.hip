@@ -1067,8 +1067,8 @@ struct BiWork : fv_solver_cache {
             persist = nullptr;
             return;
         }
-        // about 2 ms a launch, as the CG (an iteration takes 10 to 40 us)
-        persistIters = (int)(2000.0 / (10.0 + 30.0 * h.N / (1 << 20)));
+        // an iteration takes 10 to 40 us
+        persistIters = (int)(1000.0 * kPersistMs / (10.0 + 30.0 * h.N / (1 << 20)));
         static_assert(kMaxComp * sizeof(BiState) <= fv_ctx::kPollBytes, "poll area too small");
         host = static_cast<BiState*>(ctx_poll_host(c));
         slots.clear(c->stream);
@@ -1082,7 +1082,8 @@ struct BiWork : fv_solver_cache {
         int comp, ncomp;
     };
     // Up to persistIters iterations; false if the device refuses the launch.
-    bool run_persist(hipStream_t s, const Target& t, const fv_solve_opts* o, bool fresh, bool chained = false) {
+    bool run_persist(fv_ctx* c, const Target& t, const fv_solve_opts* o, bool fresh, bool chained = false) {
+        hipStream_t s = c->stream;
         const uint32_t uses = 3 * (uint32_t)persistIters + 8;
         if (tag > 0xffffffffu - uses) {  // sequence numbers start over
             slots.clear(s);
@@ -1090,7 +1091,7 @@ struct BiWork : fv_solver_cache {
         }
         double* const x = t.x + t.comp;
         BiState* const state = st.p + t.comp;
-        BiPersist a{h.N, h.ntiles, h.rowsPerBlock, persistIters, fresh ? 1 : 0, o->max_iter, tag,
+        BiPersist a{h.N, h.ntiles, h.rowsPerBlock, persist_iters(c, persistIters), fresh ? 1 : 0, o->max_iter, tag,
                     o->rel_tol, o->abs_tol, sellCol, CsrSystem{h.rowOffs, diag, h.vals, t.rhs + t.comp},
                     t.ncomp, x, t.ncomp > 1 ? x : nullptr, chained ? state - 1 : nullptr, sval.p,
                     t.ncomp > 1 ? dinv.p : x, h.r, h.rhat, h.p, h.v, h.t, h.s, plan ? plan->words.p : nullptr,
@@ -1164,7 +1165,7 @@ struct BiWork : fv_solver_cache {
             } else {
                 fresh = false;
             }
-            if (!run_persist(c->stream, t, o, fresh)) break;
+            if (!run_persist(c, t, o, fresh)) break;
             h = states(c, t.comp + 1)[t.comp];
             h.lost |= slots.doubted;
         }
@@ -1229,7 +1230,7 @@ int fv_solve_bicgstab_vec(fv_linsys* ls, int ncomp, const void* d_rhs, void* d_x
         int& k = *solved;
         while (k < ncomp && w.persist) {
             int n = k;  // components launched
-            while (n < ncomp && w.run_persist(ctx->stream, target(n), o, true, n > k)) ++n;
+            while (n < ncomp && w.run_persist(ctx, target(n), o, true, n > k)) ++n;
             if (n == k) return;
             BiState h[kMaxComp];
             std::copy_n(w.states(ctx, n), n, h);
@@ -1259,7 +1260,7 @@ int fv_solve_bicgstab(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solve
         BiState h{}, part{};  // part: of a persistent solve that could not go on
         part.res0 = -1.0;
         const BiWork::Target t{(double*)d_x, ls->rhs.p, 0, 1};
-        bool through = !o->eager && w.persist && w.run_persist(s, t, o, true);
+        bool through = !o->eager && w.persist && w.run_persist(ctx, t, o, true);
         if (through) {
             h = *w.states(ctx, 1);
             through = w.finish_persist(ctx, t, o, h);

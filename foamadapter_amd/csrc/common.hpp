@@ -104,6 +104,8 @@ void ctx_free(fv_ctx* ctx, void* p);
 // Generation of a live context (0 if it was destroyed); a buffer released after
 // its context is gone was freed with the context and is dropped.
 uint64_t ctx_generation(fv_ctx* ctx);
+// Live contexts on a device.
+int ctx_live_on(int device);
 // The context's pinned poll area (kPollBytes) and its two events, made on first use.
 void* ctx_poll_host(fv_ctx* ctx);
 

@@ -17,6 +17,13 @@ uint64_t ctx_generation(fv_ctx* ctx) {
     return it == g_live.end() ? 0 : it->second;
 }
 
+int ctx_live_on(int device) {
+    std::lock_guard<std::mutex> lk(g_ctx_mu);
+    int n = 0;
+    for (const auto& kv : g_live) n += kv.first->device == device;
+    return n;
+}
+
 void* ctx_poll_host(fv_ctx* ctx) {
     if (!ctx->pollHost) {
         FV_HIP(hipSetDevice(ctx->device));

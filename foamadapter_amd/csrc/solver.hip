@@ -143,10 +143,9 @@ struct CgWork : fv_solver_cache {
             return;
         }
         whole = sizeof(S) == 8 && rpt <= 2;
-        // a launch holds the device for about 2 ms (an iteration takes 5 us on the
-        // smallest of these systems, on the largest 28 in FP64 and 15 in FP32), so that
-        // the work of other streams gets in between
-        persistIters = (int)(2000.0 / (5.0 + (sizeof(S) == 8 ? 23.0 : 10.0) * h.N / (1 << 21)));
+        // an iteration takes 5 us on the smallest of these systems, on the largest 28 in
+        // FP64 and 15 in FP32
+        persistIters = (int)(1000.0 * kPersistMs / (5.0 + (sizeof(S) == 8 ? 23.0 : 10.0) * h.N / (1 << 21)));
         clear_tags(c->stream);
     }
     // A cooperative launch costs about 17 us more than a plain one and is not
@@ -195,11 +194,12 @@ struct CgWork : fv_solver_cache {
     }
     // Up to persistIters iterations in one launch; false if the device refuses it.
     // (whole: x, the limits and whether the solve starts.)
-    bool run_persist(hipStream_t s, double* x = nullptr, double tol = 0.0, double atol = 0.0,
+    bool run_persist(fv_ctx* c, double* x = nullptr, double tol = 0.0, double atol = 0.0,
                      int maxit = 0, bool fresh = false, CgState* host = nullptr) {
+        hipStream_t s = c->stream;
         const uint32_t uses = 2 * (uint32_t)persistIters + 8;
         if (tag > 0xffffffffu - uses) clear_tags(s);  // sequence numbers start over
-        CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persistIters, tag, hu.sellCol, h.sval,
+        CgPersist<S> a{h.N, h.ntiles, grid.rowsPerBlock, persist_iters(c, persistIters), tag, hu.sellCol, h.sval,
                        h.g, h.d, h.r, h.p, h.p2, plan ? plan->words.p : nullptr,
                        plan ? plan->ghosts.p : nullptr, plan ? plan->count.p : nullptr,
                        plan ? plan->stride : 0, h.st, slots.words.p,
@@ -488,7 +488,7 @@ bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, doubl
         do {
             host->stop = -1;
             host->lost = 0;
-            if (!w.run_persist(s, x, tol, atol, maxit, fresh, host)) return false;
+            if (!w.run_persist(ctx, x, tol, atol, maxit, fresh, host)) return false;
             FV_HIP(hipStreamSynchronize(s));
             if (w.lost(*host)) {
                 out->res0 = host->res0;
@@ -509,10 +509,10 @@ bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, doubl
     }
     w.bind(ctx, x, true);
     w.start(s, tol, maxit, 0.0, atol);
-    if (!w.run_persist(s)) return false;
+    if (!w.run_persist(ctx)) return false;
     CgState h{}, t{};
     bool haveTrue = false, refused = false;
-    if (w.lastIters > 0 && w.lastIters <= w.persistIters) {
+    if (w.lastIters > 0 && w.lastIters <= persist_iters(ctx, w.persistIters)) {
         w.finish(s);
         w.enqueue_true_residual(s);
         FV_LAUNCH_CHECK();
@@ -524,7 +524,7 @@ bool run_cg_persist(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, doubl
         pp.push(s, w.st.p);
         while (!h.stop && !h.lost && !w.slots.doubted) {
             while (!refused && pp.npend < 2) {
-                refused = !w.run_persist(s);
+                refused = !w.run_persist(ctx);
                 if (!refused) pp.push(s, w.st.p);
             }
             if (pp.npend == 0) break;
@@ -702,7 +702,7 @@ bool run_mixed_persist(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, dou
     int rounds = 0;
     bool refused = false;
     auto round = [&] {
-        refused = !w.run_persist(s);
+        refused = !w.run_persist(ctx);
         if (refused) return false;
         w.replacement(s);
         FV_LAUNCH_CHECK();

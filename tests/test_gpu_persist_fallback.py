@@ -53,6 +53,19 @@ def _same(got, ref):
     assert np.array_equal(got[0], ref[0])
 
 
+def _short(ctx, dims):
+    """A system solved in a few iterations, in one launch also beside other contexts."""
+    import foamadapter_amd as fa
+    from foamadapter_amd import dsl, fvcc
+    m, ls = _system(ctx, dims)
+    T = fvcc.VolumeField(m, ctx.uniform(m.n_cells, -1, 1, 12, 0), ctx.zeros((m.n_boundary_faces,)),
+                         fa.BoundaryConditions(m, ["fixedValue"] * m.n_patches), "T")
+    gamma = fvcc.SurfaceField(m, ctx.uniform(m.n_internal_faces + m.n_boundary_faces, 0.5, 2.0, 12, 3))
+    dt = 0.05 * float(m.get("V").mean()) ** (2.0 / 3.0)
+    dsl.assemble(dsl.imp.ddt(T) - dsl.imp.laplacian(gamma, T), T, 0.0, dt, ls)
+    return m, ls
+
+
 @pytest.mark.parametrize("method", ["double", "bicgstab"])
 @pytest.mark.parametrize("dims,after", [(ONE, 0), (MANY, 0), (MANY, 1)], ids=str)
 def test_a_plain_launch_that_does_not_meet(ctx, dims, after, method):
@@ -89,7 +102,7 @@ def test_a_component_whose_launch_does_not_meet(ctx, after):
     import foamadapter_amd as fa
     from foamadapter_amd import dsl, fvcc
     print(after, flush=True)
-    m, ls = _system(ctx, ONE)
+    m, ls = _short(ctx, ONE)
     N = m.n_cells
     got = []
     for graph in (False, True):
@@ -142,15 +155,8 @@ def test_a_group_without_one_of_its_workgroups(ctx, method):
     """More than 256 tiles: the sums of 32 workgroups each are collected and published by one of
     them.  One of each group is missing from the last exchange, the result's residual: the
     launch is lost, and the residual reported is the result's, not one of the others' rows."""
-    import foamadapter_amd as fa
-    from foamadapter_amd import dsl, fvcc
     print(method, flush=True)
-    m, ls = _system(ctx, (64, 64, 17))
-    T = fvcc.VolumeField(m, ctx.uniform(m.n_cells, -1, 1, 12, 0), ctx.zeros((m.n_boundary_faces,)),
-                         fa.BoundaryConditions(m, ["fixedValue"] * m.n_patches), "T")
-    gamma = fvcc.SurfaceField(m, ctx.uniform(m.n_internal_faces + m.n_boundary_faces, 0.5, 2.0, 12, 3))
-    dt = float(m.get("V").mean()) ** (2.0 / 3.0)  # a few iterations, in one launch
-    dsl.assemble(dsl.imp.ddt(T) - dsl.imp.laplacian(gamma, T), T, 0.0, dt, ls)
+    m, ls = _short(ctx, (64, 64, 17))
     ref = _solve(ctx, m, ls, method, graph=False)
     n = ref[1].numIter
     _same(_solve(ctx, m, ls, method), ref)
@@ -208,4 +214,19 @@ def test_systems_of_one_pattern_share_the_plan(ctx):
     vectors = 8 * 13 * m.n_cells  # of either solver, with its scaled matrix
     assert took[0] >= vectors + 12 * m.n_cells
     assert took[1] <= vectors + (1 << 18) and took[2] <= vectors + (1 << 18)
+    m.close()
+
+
+@pytest.mark.parametrize("method", ["double", "mixed", "bicgstab"])
+def test_launches_are_short_beside_another_context(ctx, method):
+    """Where another context lives on the device a launch holds it for a quarter of a
+    millisecond (an iteration takes 5 us and more): the same bits."""
+    import foamadapter_amd as fa
+    print(method, flush=True)
+    m, ls = _system(ctx, MANY)
+    ref = _solve(ctx, m, ls, method, graph=False)
+    with fa.Context(0):
+        got = _solve(ctx, m, ls, method)
+    _same(got, ref)
+    assert _counts(ls, method)["launches"] >= got[1].numIter / 50
     m.close()

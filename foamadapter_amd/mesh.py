@@ -299,8 +299,8 @@ class Mesh:
         return dst
 
     def set_gather(self, mode: int):
-        """0: LDS-staged face blocks when possible, each operator's default workgroup
-        size (default); 1: per-cell stencil walk; 2/3/4: staged with 256/512/1024
+        """0 (default): each operator's choice, the per-cell stencil walk on small meshes,
+        LDS-staged face blocks on others; 1: the walk; 2/3/4: staged with 256/512/1024
         cells per workgroup."""
         call("fv_mesh_set_gather", self.handle, int(mode))
 
@@ -311,6 +311,7 @@ class Mesh:
 
     @property
     def gather_kernel(self) -> str:
+        """What the mode stands for ("staged" for 0, which walks small meshes)."""
         m = C.c_int()
         call("fv_mesh_get_gather", self.handle, C.byref(m))
         return {1: "stencil-walk", 2: "staged-256", 3: "staged", 4: "staged-1024"}[m.value]

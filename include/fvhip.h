@@ -221,13 +221,15 @@ typedef enum {
 } fv_geom;
 int fv_mesh_get(const fv_mesh* mesh, fv_geom which, void* h_out);
 
-/* Kernel choice for the cell-result operators (grad, div, laplacian): mode 0
- * picks the LDS-staged face-block gather (default workgroup size) when the
- * faces are in upper-triangular order, mode 1 forces the per-cell stencil walk,
- * modes 2/3/4 the staged gather with 256/512/1024 cells per workgroup (same
- * arithmetic and order: bit-identical results).  fv_mesh_get_gather reports the
- * kernel in use: 1 stencil walk, 2/3/4 staged with 256/512/1024 cells.  No
- * counterpart in the reference: a tuning knob. */
+/* Kernel choice for the cell-result operators (grad, div, laplacian): mode 1
+ * forces the per-cell stencil walk, modes 2/3/4 the LDS-staged face-block gather with
+ * 256/512/1024 cells per workgroup, mode 0 leaves it to each operator: on meshes of up
+ * to 65536 cells (262144 in a block mesher's order) the walk, on larger ones the staged
+ * gather with the workgroup size that suits the operator and the mesh.  Meshes whose faces
+ * are not in upper-triangular order take the walk in every mode.  Same arithmetic and
+ * order: bit-identical results.  fv_mesh_get_gather reports what the mode stands for: 1
+ * walk, 2/3/4 staged with 256/512/1024 cells; 3 for mode 0, whose choice on a mesh it does
+ * not make.  No counterpart in the reference: a tuning knob. */
 int fv_mesh_set_gather(fv_mesh* mesh, int mode);
 int fv_mesh_get_gather(const fv_mesh* mesh, int* mode);
 /* Order in which the staged gather's workgroups take the mesh's bricks: each

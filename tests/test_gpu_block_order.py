@@ -98,3 +98,54 @@ def test_walk_and_staged_at_the_edges_of_the_rule(ctx, dims, dtype):
         assert np.array_equal(got[1][0], 1.5 * orc.grad(g, Th, Tb))
         assert np.array_equal(got[1][1], 0.5 * orc.div(g, ph, Th, Tb))
     m.close()
+
+
+def _crowded(poly, cells=256):
+    """The workgroups of `cells` cells that the default lists do not hold: more than 256 lower
+    faces from outside, 128 boundary faces or 8 lower faces of a cell from inside."""
+    F = len(poly.neighbour)
+    ow, nb = poly.owner[:F] // cells, poly.neighbour // cells
+    n = -(-poly.n_cells // cells)
+    live = np.concatenate([np.zeros(0, np.int64)] + [np.arange(p.start, p.start + p.size) for p in poly.patches if not p.empty])
+    outside = np.bincount(nb[ow != nb], minlength=n)
+    boundary = np.bincount(poly.owner[live] // cells, minlength=n)
+    inside = np.zeros(n, np.int64)
+    np.maximum.at(inside, np.arange(poly.n_cells) // cells, np.bincount(poly.neighbour[ow == nb], minlength=poly.n_cells))
+    owned = np.bincount(ow, minlength=n)
+    return int(np.sum((outside > 256) | (boundary > 128) | (inside > 8) | (owned > 832))), n
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("dims,order", [(d, "block") for d in DIMS] + [((97, 83, 61), "block"), ((33, 20, 27), "zorder"),
+                                                                      ((65, 65, 63), "zorder")], ids=str)
+def test_every_form_gives_the_bits_of_the_walk(ctx, dims, order, dtype):
+    """Each workgroup size asked for (small meshes walk the stencil unless it is), the wide form
+    of the 256-cell workgroup where a mesh in lines takes it, and mode 0's own choice, on the two
+    large meshes a staged one."""
+    import foamadapter_amd as fa
+    from foamadapter_amd import fvcc
+    print(dims, order, dtype, flush=True)
+    poly = fa.PolyMesh.hex(dims, jitter=0.2, jitter_seed=3, **({"perm_seed": 2} if order == "zorder" else {}))
+    m = fa.Mesh.from_poly(ctx, poly, renumber=order == "zorder")
+    if order == "block":
+        crowded, n = _crowded(poly)
+        _, over = m.gather_stats(256)
+        assert crowded * 100 > n and over < crowded  # the rule of the wide form
+    N, F, B = m.n_cells, m.n_internal_faces, m.n_boundary_faces
+    T = fvcc.VolumeField(m, ctx.uniform(N, -1, 1, 1, 0, dtype), ctx.uniform(B, -1, 1, 1, 1, dtype),
+                         fa.BoundaryConditions(m, ["fixedValue", "fixedGradient"] * 3), "T",
+                         ctx.uniform(B, -1, 1, 1, 2, dtype))
+    phi = fvcc.SurfaceField(m, ctx.uniform(F + B, -1, 1, 1, 3, dtype))
+    gamma = fvcc.SurfaceField(m, ctx.uniform(F + B, 0.5, 2, 1, 4, dtype))
+    got = {}
+    for mode in (1, 0, 2, 3, 4):
+        m.set_gather(mode)
+        got[mode] = [fvcc.GaussGreenGrad(ctx, m).grad(T, 1.5).numpy(),
+                     fvcc.GaussGreenDiv(ctx, m, ["linear"]).div(None, phi, T, 0.5).numpy(),
+                     fvcc.GaussGreenDiv(ctx, m, ["upwind"]).div(None, phi, T).numpy(),
+                     fvcc.GaussGreenDiv(ctx, m).div(None, phi).numpy(),
+                     fvcc.GaussGreenLaplacian(ctx, m).laplacian(None, gamma, T, 2.0).numpy()]
+    for mode in (0, 2, 3, 4):
+        for name, a, b in zip(("grad", "div", "upwind", "integrate", "laplacian"), got[mode], got[1]):
+            assert np.array_equal(a, b), (mode, name)
+    m.close()

@@ -202,8 +202,9 @@ def solver_opts(solver: dict | None) -> _lib.FvSolveOpts:
     relTol -> relative_residual_norm, maxIter -> iteration, default 1000, tolerance ->
     absolute_residual_norm), or its mapped Ginkgo form, to solver options.
     'precision': 'mixed' selects FP32 CG inside FP64 iterative refinement;
-    'graph': False launches a CG solve kernel by kernel instead of as a persistent
-    kernel or a captured hipGraph (the same bits)."""
+    'graph': False launches a solve kernel by kernel instead of as a persistent kernel or
+    a captured hipGraph (the same bits; a mixed solve cut by maxIter after a residual
+    replacement runs fewer iterations so, see fv_solve_opts)."""
     d = dict(solver or {})
     crit = d.get("criteria", {})
     o = _lib.FvSolveOpts()

@@ -400,7 +400,15 @@ typedef struct {
     int32_t eager;        /* 1 launches the kernels of every phase one by one; 0 (default)
                              runs many iterations in one persistent kernel where the
                              system fits the chip, and else (CG) replays a repeated solve
-                             as a hipGraph once the same schedule repeats (same bits) */
+                             as a hipGraph once the same schedule repeats.  Same bits, but
+                             for two things: a mixed solve cut by max_iter after a residual
+                             replacement has run as many iterations as it was given in the
+                             persistent form, up to max_iter in the others, which count what
+                             was queued behind the replacement's stop towards it (if they
+                             end before a replacement then, x holds what the last one left
+                             and final_res estimates the iterations since); and a repeated FP64 CG solve that takes more iterations than the
+                             one before adds its correction to x in two parts unless it
+                             is persistent */
 } fv_solve_opts;
 typedef struct {
     double init_res;      /* SolverStats::initResNorm, relative */

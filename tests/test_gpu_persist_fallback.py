@@ -230,3 +230,23 @@ def test_launches_are_short_beside_another_context(ctx, method):
     _same(got, ref)
     assert _counts(ls, method)["launches"] >= got[1].numIter / 50
     m.close()
+
+
+@pytest.mark.parametrize("dims,limit", [((256, 16, 16), 700), ((257, 16, 16), 700), ((64, 32, 32), 150),
+                                        ((41, 40, 40), 130)], ids=str)
+def test_a_mixed_solve_cut_by_its_limit_reports_its_residual(ctx, dims, limit):
+    """The persistent form runs the iterations it was given, whatever replacements came before
+    them, and reports the FP64 residual of the x it leaves.  The rows are summed in the host's
+    order: the norms differ by a sum of N terms."""
+    from foamadapter_amd import la
+    print(dims, limit, flush=True)
+    m, ls = _system(ctx, dims)
+    A, b = ls.scipy(), ls.rhs()
+    for _ in range(2):
+        x = ctx.uniform(m.n_cells, -1, 1, 12, 4)
+        st = la.solve_cg(ls, x, {"relTol": 1e-12, "maxIter": limit, "precision": "mixed"},
+                         raise_on_noconverge=False)
+        res = np.linalg.norm(b - A @ x.numpy()) / np.linalg.norm(b)
+        assert st.status != 0 and st.numIter == limit and _counts(ls, "mixed")["launches"] > 0
+        assert abs(st.finalResNorm - res) <= m.n_cells * 2.3e-16 * res
+    m.close()

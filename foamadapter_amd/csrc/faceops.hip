@@ -940,7 +940,11 @@ __global__ __launch_bounds__(kBlock) void k_correct_bc(int B, int nc, const int3
 // in block order 5.3, 5.0, 4.9, 5.4 -> 3.8, 4.1, 4.0, 4.1; 40^3 in Z order 5.6, 5.3,
 // 5.2, 5.4 -> 4.6, 5.1, 5.0, 5.4; 48^3 5.7, 5.2, 5.1, 5.5 -> 6.9, 5.4, 4.6, 6.7.  In
 // block order the line lies higher: 64^3 15.4, 10.0, 8.0, 12.4 ->
-// 12.3, 8.1, 6.4, 11.4; 80^3 24.0, 16.9, 14.8, 20.2 -> 25.6, 17.1, 13.4, 22.5.
+// 12.3, 8.1, 6.4, 11.4; 80^3 24.0, 16.9, 14.8, 20.2 -> 25.6, 17.1, 13.4, 22.5.  FP32, the
+// divergences and the laplacian (256-cell workgroups): 16^3 in block order 4.8, 4.7, 5.1 ->
+// 3.8, 3.8, 4.0; 40^3 in Z order 4.8, 4.7, 5.0 -> 3.9, 3.9, 4.0; 64^3 6.0, 5.8, 6.5 -> 7.3,
+// 6.2, 9.3; in block order 64^3 6.9, 6.4, 8.1 -> 6.5, 5.7, 7.5, 80^3 12.9, 11.9, 15.2 -> 12.1,
+// 9.9, 14.5, so its lines lie a little higher still.
 template <typename S>
 bool staged(const fv_mesh* m) {
     if (!gather_cells(m)) return false;

@@ -151,8 +151,12 @@ struct CgWork : fv_solver_cache {
     // A cooperative launch costs about 17 us more than a plain one and is not
     // replayed as a graph, and an iteration saves 5 us on the smallest systems: unless
     // it is whole, a system whose previous solve took fewer than kPersistMin
-    // iterations keeps the kernel-by-kernel form (32^3 heat step of 5 iterations: 157
-    // us, 178 with the iterations alone persistent, 75 whole).
+    // iterations keeps the kernel-by-kernel form.  Solves of 4, 8 and 11 iterations,
+    // kernel by kernel -> persistent, in us: FP32 32^3 99, 143, 185 -> 143, 165, 179; 64^3
+    // 141, 206, 266 -> 177, 206, 226; 128^3 405, 574, 713 -> 433, 489, 532; FP64 96^3
+    // 296, 452, 571 -> 229, 273, 308.  So the line is that of the small FP32 systems; it
+    // lies too high for FP32 above 64^3 and for all FP64 systems that are not whole,
+    // which lose by it after a first solve of that few iterations.
     static constexpr int kPersistMin = 12;
     bool use_persist(fv_ctx* c, fv_linsys* ls) {
         choose_persist(c, ls);
@@ -473,8 +477,8 @@ CgState run_cg(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, int check,
 
 // run_cg with the persistent kernel: a launch ends at the stop by itself, so
 // nothing has to be predicted.  A whole solve is one launch and one read (of pinned
-// memory) unless it runs out of a launch's iterations.  Else, a system whose previous solve fitted one launch
-// gets the correction and the explicit residual queued behind it and is read
+// memory) unless it runs out of a launch's iterations.  Else, a system whose previous solve
+// fitted one launch gets the correction and the explicit residual queued behind it and is read
 // once; otherwise two launches are kept queued until one has stopped.  False if the
 // device refuses a launch or one is lost: out->it iterations are in x then, and out->res0
 // is the initial residual if it is known (the caller sets -1).

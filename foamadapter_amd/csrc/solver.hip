@@ -774,6 +774,8 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
         fv_sparsity* sp = ls->sp;
         fv_ctx* ctx = sp->mesh->ctx;
         const int check = o->check_every > 0 ? o->check_every : 8;
+        // nothing to iterate: the state is that of the kernel-by-kernel start
+        const bool byKernel = o->eager || o->max_iter == 0;
         double* x = (double*)d_x;
         double bnorm = 0.0;
         if (o->mode == FV_SOLVE_F64) {
@@ -781,7 +783,7 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
             double tr = 0.0;
             CgState h{};
             h.res0 = -1.0;
-            if (o->eager || !w.use_persist(ctx, ls) ||
+            if (byKernel || !w.use_persist(ctx, ls) ||
                 !run_cg_persist(ctx, w, o->rel_tol, o->max_iter, o->abs_tol, x, &tr, &h)) {
                 const CgState part = h;  // of a persistent solve that could not go on
                 w.bind(ctx, x);
@@ -803,7 +805,7 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
             const double delta = o->inner_rel_tol > 0.0 ? o->inner_rel_tol : kIrDelta;
             // max_outer counts rounds of check_every iterations: those solves run
             // kernel by kernel
-            if (o->eager || o->max_outer > 0 || !w.use_persist(ctx, ls) ||
+            if (byKernel || o->max_outer > 0 || !w.use_persist(ctx, ls) ||
                 !run_mixed_persist(ctx, w, o->rel_tol, o->max_iter, delta, o->abs_tol, x, &r)) {
                 const IrOut part = r;
                 w.bind(ctx, x);

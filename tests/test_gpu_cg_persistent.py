@@ -254,3 +254,34 @@ def test_solves_of_several_threads(ctx):
     for i, got in out.items():
         for g in got[1:]:
             assert g[1:] == got[0][1:] and np.array_equal(g[0], got[0][0]), cases[i]
+
+
+@pytest.mark.parametrize("method", ["double", "mixed", "bicgstab"])
+def test_a_solve_without_iterations(ctx, method):
+    """maxIter 0, first and repeated, before and after a solve: the forms agree, x stays, and a
+    residual above the tolerance is not reported as convergence (FP64 CG, which reads no state
+    when it runs nothing, reports the residual of x as its explicit one)."""
+    from foamadapter_amd import la
+    print(method, flush=True)
+    opts = {"solver": "PBiCGStab"} if method == "bicgstab" else {"precision": method}
+    got = []
+    for graph in (False, True):
+        m, ls = _system(ctx, (17, 16, 16))
+        A, b = ls.scipy(), ls.rhs()
+        x = ctx.uniform(m.n_cells, -1, 1, 12, 4)
+        x0 = x.numpy()
+        res = np.linalg.norm(b - A @ x0) / np.linalg.norm(b)
+        out = []
+        for limit in (0, 0, 30, 0):
+            if limit:
+                la.solve_cg(ls, ctx.uniform(m.n_cells, -1, 1, 12, 5), dict(opts, relTol=1e-12, maxIter=limit, graph=graph),
+                            raise_on_noconverge=False)
+                continue
+            st = la.solve_cg(ls, x, dict(opts, relTol=1e-8, maxIter=0, graph=graph), raise_on_noconverge=False)
+            assert np.array_equal(x.numpy(), x0) and abs(st.trueResNorm - res) <= m.n_cells * 2.3e-16 * res
+            if method != "double":
+                assert st.status != 0 and st.finalResNorm == st.trueResNorm
+            out.append((st.numIter, st.initResNorm, st.finalResNorm, st.trueResNorm, st.status))
+        got.append(out)
+        m.close()
+    assert got[0] == got[1]

@@ -470,7 +470,7 @@ CgState run_cg(fv_ctx* ctx, CgWork<double>& w, double tol, int maxit, int check,
     while (pp.npend) h = pp.pop();  // chunks queued behind the stop ran as no-ops
     // a system that needed no iteration polls (blocking) after the first
     w.lastIters = h.stop ? std::max(h.it, 1) : h.it;
-    if (!haveTrue) w.finish(s);
+    if (!haveTrue && launched > 0) w.finish(s);  // (else d is zero, and g may be NaN)
     *true_res = haveTrue ? t.res : w.true_residual(s);
     return h;
 }

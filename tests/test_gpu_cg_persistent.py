@@ -285,3 +285,25 @@ def test_a_solve_without_iterations(ctx, method):
         got.append(out)
         m.close()
     assert got[0] == got[1]
+
+
+def test_a_solve_without_iterations_leaves_x(ctx):
+    """A diagonal of both signs, which the scaling cannot take: x is not touched and its residual
+    reported all the same."""
+    import foamadapter_amd as fa
+    from foamadapter_amd import dsl, fvcc, la
+    m = fa.Mesh.from_poly(ctx, fa.PolyMesh.hex((11, 9, 8)))
+    N, F, B = m.n_cells, m.n_internal_faces, m.n_boundary_faces
+    T = fvcc.VolumeField(m, ctx.uniform(N, -1, 1, 3, 0), ctx.uniform(B, -1, 1, 3, 1),
+                         fa.BoundaryConditions(m, ["fixedValue"] * m.n_patches), "T")
+    phi = fvcc.SurfaceField(m, ctx.uniform(F + B, -1, 1, 3, 2))
+    ls = dsl.assemble(dsl.imp.ddt(T) + dsl.imp.div(phi, T), T, 0.0, 1.0)
+    A, b = ls.scipy(), ls.rhs()
+    assert A.diagonal().min() < 0 < A.diagonal().max()
+    for graph in (False, True):
+        x = ctx.uniform(N, -1, 1, 12, 4)
+        x0 = x.numpy()
+        st = la.solve_cg(ls, x, {"relTol": 1e-8, "maxIter": 0, "graph": graph}, raise_on_noconverge=False)
+        res = np.linalg.norm(b - A @ x0) / np.linalg.norm(b)
+        assert np.array_equal(x.numpy(), x0) and abs(st.trueResNorm - res) <= N * 2.3e-16 * res
+    m.close()

@@ -899,6 +899,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist(CgPersist<S> A) {
         st->stop = stop;
         st->done = 0;
         st->pbuf = 0;
+        if (!WHOLE) st->runs += 1;
         if (WHOLE) {
             st->bnorm = bnorm;
             st->res0 = res0;
@@ -1149,6 +1150,7 @@ __global__ __launch_bounds__(kPersistThreads) void kc_persist_far(CgPersist<S> A
         st->stop = stop;
         st->done = 0;
         st->pbuf = 0;
+        st->runs += 1;
     }
 }
 

@@ -37,6 +37,7 @@ constexpr double kIrDelta = 1e-5;
 //            latest update (written by the update kernel)
 //   nrep     FP64 residual replacements so far (advanced by the replacement
 //            kernel; read by the host)
+//   runs     persistent launches that found the system running
 //   lost     set by a workgroup of a persistent launch whose wait for the others
 //            ended by its clock, and by nothing else: the launch's results are void
 struct CgState {
@@ -44,7 +45,7 @@ struct CgState {
     int32_t it, done, maxit, stop;
     double tol, atol;  // relative and absolute (0: off) residual targets
     int32_t pbuf, nrep;
-    int32_t lost, pad;
+    int32_t lost, runs;
 };
 
 // Fixed-shape block reduction of NV values at once: wavefront shuffles, then

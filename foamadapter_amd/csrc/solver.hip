@@ -723,21 +723,18 @@ bool run_mixed_persist(fv_ctx* ctx, CgWork<float>& w, double tol, int maxit, dou
     }
     if (!done()) {
         PollPipe pp{static_cast<CgState*>(ctx_poll_host(ctx)), ctx};
-        int seen = rounds - 1;
         pp.push(s, w.st.p);
         while (!done()) {
             while (!refused && pp.npend < 2)
                 if (round()) pp.push(s, w.st.p);
             if (pp.npend == 0) break;
             h = pp.pop();
-            ++seen;
         }
         while (pp.npend) h = pp.pop();
-        rounds = seen;
     }
     *out = IrOut{h.res0, h.res, h.bnorm, h.it, h.nrep};
     if (w.lost(h) || !done()) return false;
-    if (h.stop == 2) w.lastLaunches = rounds;
+    if (h.stop == 2) w.lastLaunches = h.runs;  // (not those queued behind the stop)
     return true;
 }
 

@@ -232,6 +232,24 @@ def test_launches_are_short_beside_another_context(ctx, method):
     m.close()
 
 
+def test_a_mixed_solve_queues_the_launches_it_needs(ctx):
+    """A solve queues as many launches as the one before took, at once: after one of many, a
+    short one queues as many once, and the next as many as that took."""
+    from foamadapter_amd import la
+    m, ls = _system(ctx, MANY)
+    took = []
+    for tol in (1e-8, 1e-8, 1e-1, 1e-1, 1e-1):
+        before = _counts(ls, "mixed")["launches"]
+        x = ctx.uniform(m.n_cells, -1, 1, 12, 4)
+        st = la.solve_cg(ls, x, {"relTol": tol, "maxIter": 4000, "precision": "mixed"})
+        assert st.finalResNorm <= tol and st.numIter >= 12
+        took.append(_counts(ls, "mixed")["launches"] - before)
+    print(took, flush=True)
+    assert took[0] > 3 and took[1] <= took[0] and took[2] == took[1]
+    assert took[3] < took[2] and took[4] == took[3]
+    m.close()
+
+
 @pytest.mark.parametrize("dims,limit", [((256, 16, 16), 700), ((257, 16, 16), 700), ((64, 32, 32), 150),
                                         ((41, 40, 40), 130)], ids=str)
 def test_a_mixed_solve_cut_by_its_limit_reports_its_residual(ctx, dims, limit):

@@ -379,6 +379,7 @@ void batch_remove(fv_batch* b, BMember* m) {
 void batch_restart(fv_batch*, BMember* m) { m->needStart = true; }
 
 void batch_step(fv_batch* b, std::vector<CgState>& states) {
+    ctx_touch(b->ctx);
     if (b->prec == FV_SOLVE_F32_IR)
         step_t<float>(b, states);
     else

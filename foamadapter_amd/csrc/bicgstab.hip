@@ -1291,6 +1291,7 @@ int fv_solve_bicgstab(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solve
                     kbi_update<<<w.G, kB, 0, s>>>(w.sys.p);
                 }
                 FV_LAUNCH_CHECK();
+                ctx_touch(ctx);
                 launched += n;
                 FV_HIP(hipMemcpyAsync(&h, w.st.p, sizeof h, hipMemcpyDeviceToHost, s));
                 FV_HIP(hipStreamSynchronize(s));

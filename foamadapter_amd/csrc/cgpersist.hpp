@@ -1258,15 +1258,16 @@ bool persist_room(F&& alloc) {
 }
 
 // Iterations a launch may run, of those that take kPersistMs.  A launch holds up to every CU
-// until it ends, and the work of other streams waits; where other contexts live on the
-// device it is an eighth as long.  Two threads, a Poisson solve at 128^3 beside heat steps at
-// 32^3, a second of each: kernel by kernel 35 and 3600, launches of 2 ms 89 and 870, of 0.25
-// ms 72 and 3870, of 0.1 ms 53 and 7210; gradients at 64^3 beside it 24000, 1390, 4560, 8430.
-// Solves beside solves lose by short launches (two at 128^3 45 a second each, 38; kernel by
-// kernel 19).
+// until it ends, and the work of other streams waits; while another thread uses another
+// context of the device it is an eighth as long.  Two threads, a Poisson solve at 128^3 beside
+// heat steps at 32^3, a second of each: kernel by kernel 35 and 3600, launches of 2 ms 89 and
+// 870, of 0.25 ms 72 and 3870, of 0.1 ms 53 and 7210; gradients at 64^3 beside it 24000,
+// 1390, 4560, 8430.  Solves beside solves lose by short launches (two at 128^3 45 a second
+// each, 38; kernel by kernel 19).
 constexpr double kPersistMs = 2.0;
-inline int persist_iters(const fv_ctx* c, int whole) {
-    return ctx_live_on(c->device) > 1 ? std::max(whole / 8, 1) : whole;
+inline int persist_iters(fv_ctx* c, int whole) {
+    ctx_touch(c);
+    return ctx_beside(c) ? std::max(whole / 8, 1) : whole;
 }
 
 // Workgroups of a persistent launch over `tiles` tiles

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <string>
@@ -94,6 +95,9 @@ struct fv_ctx {
     // another context of the same owner works on the device at the same time (the
     // server's two lanes): no kernel of this one may hold every CU for long
     bool shared = false;
+    // when (CLOCK_MONOTONIC_COARSE, ns) and by which thread it was last used (ctx_touch)
+    std::atomic<int64_t> usedAt{0};
+    std::atomic<const void*> usedBy{nullptr};
 };
 
 namespace fvhip {
@@ -104,8 +108,10 @@ void ctx_free(fv_ctx* ctx, void* p);
 // Generation of a live context (0 if it was destroyed); a buffer released after
 // its context is gone was freed with the context and is dropped.
 uint64_t ctx_generation(fv_ctx* ctx);
-// Live contexts on a device.
-int ctx_live_on(int device);
+// Notes that this thread uses the context now: called by what enqueues work or waits.
+void ctx_touch(fv_ctx* ctx);
+// Whether another thread has used another context of the device in the last 20 ms.
+bool ctx_beside(const fv_ctx* ctx);
 // The context's pinned poll area (kPollBytes) and its two events, made on first use.
 void* ctx_poll_host(fv_ctx* ctx);
 

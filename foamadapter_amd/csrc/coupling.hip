@@ -289,7 +289,10 @@ double* scratch_on(int device) {
     return g_scratch_ptr[device];
 }
 
-void check_ls(const fv_linsys* ls) { FV_REQUIRE(ls && ls->sp && ls->sp->mesh, "NULL linear system"); }
+void check_ls(const fv_linsys* ls) {
+    FV_REQUIRE(ls && ls->sp && ls->sp->mesh, "NULL linear system");
+    ctx_touch(ls->sp->mesh->ctx);
+}
 
 // one value through the context's pinned area: a copy into pageable memory is staged
 double read_double(fv_ctx* ctx, const double* d) {

@@ -1004,6 +1004,7 @@ void check_common(fv_ctx* ctx, const fv_mesh* m, fv_prec prec) {
     FV_REQUIRE(ctx && m, "NULL ctx/mesh");
     FV_REQUIRE(m->ctx == ctx, "mesh belongs to another context");
     FV_REQUIRE(prec == FV_F64 || prec == FV_F32, "unknown precision");
+    ctx_touch(ctx);
 }
 
 void check_bc(const fv_mesh* m, const fv_bc* bc) {

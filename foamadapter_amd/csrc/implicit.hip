@@ -416,7 +416,10 @@ __global__ __launch_bounds__(kBlock) void k_uniform_sell(int N, int W, const int
 
 fv_mesh* mesh_of(const fv_linsys* ls) { return ls->sp->mesh; }
 
-void check_ls(const fv_linsys* ls) { FV_REQUIRE(ls && ls->sp && ls->sp->mesh, "NULL linear system"); }
+void check_ls(const fv_linsys* ls) {
+    FV_REQUIRE(ls && ls->sp && ls->sp->mesh, "NULL linear system");
+    ctx_touch(ls->sp->mesh->ctx);
+}
 
 void check_bc(const fv_linsys* ls, const fv_bc* bc) {
     FV_REQUIRE(bc && bc->mesh == mesh_of(ls), "boundary conditions belong to another mesh");

@@ -17,11 +17,35 @@ uint64_t ctx_generation(fv_ctx* ctx) {
     return it == g_live.end() ? 0 : it->second;
 }
 
-int ctx_live_on(int device) {
+// (a coarse clock: 5 ns, steps of a few ms)
+static int64_t coarse_now() {
+    timespec t{};
+    (void)clock_gettime(CLOCK_MONOTONIC_COARSE, &t);
+    return (int64_t)t.tv_sec * 1000000000 + t.tv_nsec;
+}
+
+static const void* this_thread() {
+    static thread_local char here;
+    return &here;
+}
+
+void ctx_touch(fv_ctx* ctx) {
+    ctx->usedAt.store(coarse_now(), std::memory_order_relaxed);
+    ctx->usedBy.store(this_thread(), std::memory_order_relaxed);
+}
+
+bool ctx_beside(const fv_ctx* ctx) {
+    constexpr int64_t kRecent = 20000000;
+    const int64_t now = coarse_now();
     std::lock_guard<std::mutex> lk(g_ctx_mu);
-    int n = 0;
-    for (const auto& kv : g_live) n += kv.first->device == device;
-    return n;
+    for (const auto& kv : g_live) {
+        const fv_ctx* const c = kv.first;
+        if (c != ctx && c->device == ctx->device &&
+            c->usedBy.load(std::memory_order_relaxed) != this_thread() &&
+            now - c->usedAt.load(std::memory_order_relaxed) < kRecent)
+            return true;
+    }
+    return false;
 }
 
 void* ctx_poll_host(fv_ctx* ctx) {
@@ -327,6 +351,7 @@ int fv_ctx_destroy(fv_ctx* ctx) {
 int fv_sync(fv_ctx* ctx) {
     return guarded([&] {
         FV_REQUIRE(ctx, "ctx is NULL");
+        ctx_touch(ctx);
         FV_HIP(hipStreamSynchronize(ctx->stream));
     });
 }
@@ -374,6 +399,7 @@ int fv_memcpy_h2d(fv_ctx* ctx, void* d_dst, const void* h_src, size_t bytes) {
         FV_REQUIRE(ctx, "ctx is NULL");
         if (!bytes) return;
         FV_REQUIRE(d_dst && h_src, "NULL pointer");
+        ctx_touch(ctx);
         FV_HIP(hipMemcpyAsync(d_dst, h_src, bytes, hipMemcpyHostToDevice, ctx->stream));
         FV_HIP(hipStreamSynchronize(ctx->stream));
     });
@@ -384,6 +410,7 @@ int fv_memcpy_d2h(fv_ctx* ctx, void* h_dst, const void* d_src, size_t bytes) {
         FV_REQUIRE(ctx, "ctx is NULL");
         if (!bytes) return;
         FV_REQUIRE(h_dst && d_src, "NULL pointer");
+        ctx_touch(ctx);
         FV_HIP(hipMemcpyAsync(h_dst, d_src, bytes, hipMemcpyDeviceToHost, ctx->stream));
         FV_HIP(hipStreamSynchronize(ctx->stream));
     });
@@ -436,6 +463,7 @@ int fv_permute(fv_ctx* ctx, fv_prec prec, int64_t n, int ncomp, int mode, int or
         FV_REQUIRE(ctx && n >= 0 && ncomp >= 1 && (mode == 0 || mode == 1), "bad argument");
         if (!n) return;
         FV_REQUIRE(map && src && dst && src != dst, "NULL or aliased pointer");
+        ctx_touch(ctx);
         FV_REQUIRE(n <= (int64_t)0xFFFFFFFF * 256 * kPermU, "too many elements");
         if (prec == FV_F64)
             launch_permute<double>(ctx->stream, n, ncomp, mode, oriented, map,

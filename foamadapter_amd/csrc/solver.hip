@@ -384,6 +384,7 @@ struct PollPipe {
     fv_ctx* ctx;
     int pend[2] = {-1, -1}, npend = 0, slot = 0;
     void push(hipStream_t s, const CgState* dev) {
+        ctx_touch(ctx);
         FV_HIP(hipMemcpyAsync(&mirror[slot], dev, sizeof(CgState), hipMemcpyDeviceToHost, s));
         FV_HIP(hipEventRecord(ctx->pollEv[slot], s));
         pend[npend++] = slot;
@@ -774,6 +775,7 @@ int fv_solve_cg(fv_linsys* ls, void* d_x, const fv_solve_opts* o, fv_solver_stat
         // nothing to iterate: the state is that of the kernel-by-kernel start
         const bool byKernel = o->eager || o->max_iter == 0;
         double* x = (double*)d_x;
+        ctx_touch(ctx);
         double bnorm = 0.0;
         if (o->mode == FV_SOLVE_F64) {
             CgWork<double>& w = work_of<double>(ls, false);

@@ -218,17 +218,44 @@ def test_systems_of_one_pattern_share_the_plan(ctx):
 
 
 @pytest.mark.parametrize("method", ["double", "mixed", "bicgstab"])
-def test_launches_are_short_beside_another_context(ctx, method):
-    """Where another context lives on the device a launch holds it for a quarter of a
-    millisecond (an iteration takes 5 us and more): the same bits."""
+def test_launches_are_short_beside_another_thread(ctx, method):
+    """While another thread uses a context of its own a launch holds the device for a quarter of
+    a millisecond (an iteration takes 5 us and more): the same bits.  A context that is idle, or
+    used by this thread, changes nothing."""
+    import threading
+    import time
     import foamadapter_amd as fa
     print(method, flush=True)
     m, ls = _system(ctx, MANY)
     ref = _solve(ctx, m, ls, method, graph=False)
-    with fa.Context(0):
+
+    def launches():
+        before = _counts(ls, method)["launches"]
         got = _solve(ctx, m, ls, method)
-    _same(got, ref)
-    assert _counts(ls, method)["launches"] >= got[1].numIter / 50
+        _same(got, ref)
+        return _counts(ls, method)["launches"] - before
+
+    with fa.Context(0) as other:
+        other.sync()
+        time.sleep(0.1)  # other tests' threads are long gone
+        idle = launches()
+        stop = threading.Event()
+
+        def use():
+            while not stop.is_set():
+                other.sync()
+                time.sleep(0.001)
+        t = threading.Thread(target=use)
+        t.start()
+        time.sleep(0.05)
+        busy = launches()
+        stop.set()
+        t.join()
+        time.sleep(0.1)
+        launches()  # (a mixed solve queues as many as the one before)
+        again = launches()
+    assert busy >= ref[1].numIter / 50 and idle <= ref[1].numIter / 100 + 8
+    assert again <= idle + 2
     m.close()
 
 

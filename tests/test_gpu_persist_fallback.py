@@ -120,6 +120,30 @@ def test_a_component_whose_launch_does_not_meet(ctx, after):
     m.close()
 
 
+@pytest.mark.parametrize("after,fault", [(0, REFUSED), (1, REFUSED), (2, REFUSED), (2, LOST)])
+def test_a_component_goes_on_kernel_by_kernel(ctx, after, fault):
+    """The components behind a refused or lost launch are solved one by one: each to its
+    tolerance, the system's right-hand side that of the last."""
+    from foamadapter_amd import dsl, fvcc
+    print(after, fault, flush=True)
+    m, ls = _short(ctx, ONE)
+    N = m.n_cells
+    A = ls.scipy()
+    x3, b3 = ctx.uniform(3 * N, -1, 1, 13, 2), ctx.uniform(3 * N, -1, 1, 13, 1)
+    x3.shape = b3.shape = (N, 3)
+    ls.rhs3 = b3
+    _fault(ls, "bicgstab", fault, after)
+    st = dsl._solve_vec(ls, fvcc.VolumeField(m, x3, None), {"solver": "PBiCGStab", "relTol": 1e-9, "maxIter": 400})
+    c = _counts(ls, "bicgstab")
+    assert c["refused" if fault == REFUSED else "lost"] == 1 and len(st) == 3
+    x, b = x3.numpy(), b3.numpy()
+    for k in range(3):
+        res = np.linalg.norm(b[:, k] - A @ x[:, k]) / np.linalg.norm(b[:, k])
+        assert st[k].status == 0 and res <= 1.01e-9 and abs(st[k].trueResNorm - res) <= 1e-12
+    assert np.array_equal(ls.rhs(), b[:, 2])
+    m.close()
+
+
 CASES = [("double", ONE, 0), ("double", MANY, 0), ("double", MANY, 1), ("double", LARGE, 0), ("double", LARGE, 1),
          ("mixed", ONE, 0), ("mixed", ONE, 1), ("bicgstab", ONE, 0), ("bicgstab", MANY, 0), ("bicgstab", MANY, 1)]
 
